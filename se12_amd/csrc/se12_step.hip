@@ -33,6 +33,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "se12_step.h"
 #include "se12_step_math.hpp"
 
@@ -201,6 +203,9 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t v) {
     return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
+// A block barrier for LDS data that leaves global loads in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // Makes the wave wait for a loaded value here: issued before a branch on the
 // position, loads would otherwise be sunk past it and wait for it.
 __device__ __forceinline__ void pin(float v) { asm volatile("" ::"v"(v)); }
@@ -290,15 +295,15 @@ __device__ __forceinline__ void chunk_key_dots(const uint4 (&raw)[kMaxHeadDim / 
 // For thread t < 64 (one wave): the score of position j0 + t for each head
 // (the 4 waves' dots in order, scaling, soft-capping, -inf outside
 // [lo, p]) and the chunk's max m and sum l of exp(score - m).
-template <int G>
+template <int G, int STRIDE = kChunk>
 __device__ __forceinline__ void chunk_scores(const float* red, const AttnArgs& a, int t, int j0, int p, int lo,
                                              float (&sc)[G], float (&m)[G], float (&l)[G]) {
     const int jq = j0 + t;
     const bool valid = jq <= p && jq >= lo;
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-        const float dot = red[(0 * G + h) * kChunk + t] + red[(1 * G + h) * kChunk + t] +
-                          red[(2 * G + h) * kChunk + t] + red[(3 * G + h) * kChunk + t];
+        const float dot = red[(0 * G + h) * STRIDE + t] + red[(1 * G + h) * STRIDE + t] +
+                          red[(2 * G + h) * STRIDE + t] + red[(3 * G + h) * STRIDE + t];
         float v = round_bf16(round_bf16(dot) * a.scaling);
         if (a.softcap > 0.0f) v = round_bf16(round_bf16(tanhf(round_bf16(v / a.softcap))) * a.softcap);
         if (!valid) v = -INFINITY;
@@ -581,6 +586,316 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(const int64_t* po
 }
 
 // ---------------------------------------------------------------------------
+// attention over many positions: launches of more score blocks than
+// kLongBlocks (sequences x KV heads x chunks), e.g. a batch over a long
+// cache. The blocks of the kernels above load their share of the cache before
+// they know the position, one round trip less on a cache nearly all in use,
+// but a launch of many blocks then reads the whole cache whatever part is in
+// use, rotates q once per 64 positions, and computes each probability once
+// per 8 columns. Here a block reads the position first (other blocks of the
+// CU hide that), and the positions in use, not the cache's length, are cut
+// among the grid's blocks:
+//   scores  a run of units of 64 to 256 positions per block (by head_dim,
+//           so that a unit is a few KB of keys per wave): q rotated once, the
+//           next batch of keys in flight while one is used, a wave for each
+//           of the unit's chunks at its end.
+//   pv      a run of positions per block over all head-dim columns: whole
+//           V rows per load, each probability computed once and shared
+//           through LDS; the runs' FP32 sums meet as the spans above do.
+// Bound by the cache's bytes in use. Two launches in a graph, cold cache, the
+// short kernels above against these: 8 sequences x 8 KV heads of 256 x 2
+// queries, cache of 8,192: position 8,190 145.6 -> 136 us (3.9 TB/s; the key
+// rows are 16 KB apart, and a cache of 8,064 takes 17 us less), 3,000 121 ->
+// 56 us, 300 114 -> 18.6, a window of 1,024 at 8,000 128 -> 32; 32 x 8 x 128,
+// 2,048 long at 700 68 -> 31; 32 x 8 x 64, 4,096 long at 4,000 80 -> 66. Units
+// of 128 / 256 at head_dim 256 took 60 / 62 us at position 3,000, 64 / 128 at
+// head_dim 64 79 / 69; 2,048 blocks instead of 1,024 3-7% more, nontemporal
+// loads 126 at 8,190 but 40 and 97 on the smaller caches. Below kLongBlocks the
+// short kernels stay: at 512-1,024 blocks these took 29 / 34 / 41 us against
+// 19 / 25 / 24 (4 x 4 x 2,048, 8 x 8 x 1,024, 1 x 4 x 8,192).
+// ---------------------------------------------------------------------------
+
+constexpr int kLongBlocks = 1024;
+constexpr int kLongGrid = 1024;    // blocks aimed at, over all (sequence, KV head) pairs
+constexpr int kUnitLoads = 8;      // 16-byte loads of one batch per thread, two batches in flight
+constexpr int kPvStep = 64;        // positions of one step of a pv block: 8 V rows per thread, two steps in flight
+
+template <int G, int DT, int UNIT>
+__global__ __launch_bounds__(kAttnThreads) void attn_scores_long_kernel(AttnArgs a) {
+    __shared__ float qk[(G + 1) * kMaxHeadDim];
+    __shared__ float red[4 * G * UNIT];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int kvb = blockIdx.x, b = kvb / a.kvh, kh = kvb % a.kvh;
+    const int d = a.d, half = d / 2, L = a.max_len;
+    const int64_t p64 = uniform_i64(__hip_atomic_load(a.pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (p64 < 0 || p64 >= L) return;
+    const int p = (int)p64, lo = window_lo(p, a.window);
+    // units u0 .. u1 - 1 of the nu in use
+    const int u_lo = lo / UNIT, nu = p / UNIT - u_lo + 1;
+    const int Y = (int)gridDim.y, y = (int)blockIdx.y;
+    const int u0 = u_lo + (int)((int64_t)y * nu / Y), u1 = u_lo + (int)((int64_t)(y + 1) * nu / Y);
+    if (u0 >= u1) return;
+
+    // lane group pg: 8 consecutive positions (UNIT contiguous positions of
+    // one head-dim element's row per kLanes lanes); slice es: every
+    // kSlices-th element, kUnitLoads of them in flight twice over
+    constexpr int kLanes = UNIT / 8, kSlices = kAttnThreads / kLanes;
+    const int pg = t % kLanes, es = t / kLanes;
+    const int nb = (d + kSlices * kUnitLoads - 1) / (kSlices * kUnitLoads);   // load batches per unit
+    auto load = [&](uint4 (&raw)[kUnitLoads], int u, int k) {
+        const int jg = u * UNIT + 8 * pg;
+        const uint16_t* kb = a.kt + (int64_t)kvb * d * L + (jg + 8 <= L ? jg : L - 8);
+#pragma unroll
+        for (int i = 0; i < kUnitLoads; ++i) {
+            const int e = es + kSlices * (kUnitLoads * k + i);
+            raw[i] = *reinterpret_cast<const uint4*>(kb + (int64_t)(e < d ? e : d - 1) * L);
+        }
+    };
+    uint4 r0[kUnitLoads], r1[kUnitLoads];
+    float x[G + 1], y0[G + 1];
+    const int tc = t < d ? t : d - 1;
+#pragma unroll
+    for (int h = 0; h < G; ++h)
+        x[h] = load_as_bf16<DT>(a.q, (int64_t)b * a.q_stride + (int64_t)(kh * G + h) * d + tc);
+    x[G] = load_as_bf16<DT>(a.k, (int64_t)b * a.kv_stride + (int64_t)kh * d + tc);
+    const float vv = load_as_bf16<DT>(a.v, (int64_t)b * a.kv_stride + (int64_t)kh * d + tc);
+    const float fr = a.inv_freq[tc % half];
+    load(r0, u0, 0);
+    rotate_qk<G>(qk, x, fr, p, d, t, y0);
+    if (t < d && u1 == u_lo + nu) {
+        a.kt[((int64_t)kvb * d + t) * L + p] = f_to_bf16(y0[G]);
+        a.vc[((int64_t)kvb * L + p) * d + t] = f_to_bf16(vv);
+    }
+    __syncthreads();
+    float acc[8][G];
+    auto clear = [&]() {
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+#pragma unroll
+            for (int h = 0; h < G; ++h) acc[m][h] = 0.0f;
+    };
+    auto dots = [&](const uint4 (&raw)[kUnitLoads], int u, int k) {
+        const int jg = u * UNIT + 8 * pg, jgl = jg + 8 <= L ? jg : L - 8;
+        const bool holds = p < (u + 1) * UNIT;   // block-uniform: the unit of the new token
+#pragma unroll
+        for (int i = 0; i < kUnitLoads; ++i) {
+            const int e = es + kSlices * (kUnitLoads * k + i);
+            if (e < d) {
+                float kv[8];
+                unpack8(raw[i], kv);
+                if (holds) {
+#pragma unroll
+                    for (int m = 0; m < 8; ++m)
+                        if (jgl + m == p) kv[m] = qk[G * d + e];
+                }
+#pragma unroll
+                for (int h = 0; h < G; ++h) {
+                    const float qv = qk[h * d + e];
+#pragma unroll
+                    for (int m = 0; m < 8; ++m) acc[m][h] += qv * kv[m];
+                }
+            }
+        }
+    };
+    const int64_t lp = (int64_t)a.chunks * kChunk;
+    const int64_t row0 = (int64_t)b * a.kvh * G + kh * G;
+    // the unit's scores: the wave's two slices, then the four waves in order,
+    // each wave taking one of the unit's chunks
+    auto finish = [&](int u) {
+#pragma unroll
+        for (int h = 0; h < G; ++h)
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+                float v = acc[m][h];
+#pragma unroll
+                for (int o = kLanes; o < 64; o *= 2) v += __shfl_xor(v, o, 64);
+                if (lane < kLanes) red[(w * G + h) * UNIT + 8 * pg + m] = v;
+            }
+        lds_barrier();
+        const int c = u * (UNIT / kChunk) + w;
+        if (w < UNIT / kChunk && c >= lo / kChunk && c <= p / kChunk) {
+            float sc[G], m[G], l[G];
+            chunk_scores<G, UNIT>(red + w * kChunk, a, lane, c * kChunk, p, lo, sc, m, l);
+#pragma unroll
+            for (int h = 0; h < G; ++h) {
+                a.scores[(row0 + h) * lp + c * kChunk + lane] = sc[h];
+                if (lane == 0) {
+                    a.stats[((row0 + h) * a.chunks + c) * 2 + 0] = m[h];
+                    a.stats[((row0 + h) * a.chunks + c) * 2 + 1] = l[h];
+                }
+            }
+        }
+        lds_barrier();
+    };
+    int u = u0, k = 0;
+    auto step = [&](const uint4 (&cur)[kUnitLoads], uint4 (&next)[kUnitLoads]) {
+        const bool last = k + 1 == nb;
+        const int un = last ? u + 1 : u, kn = last ? 0 : k + 1;
+        if (un < u1) load(next, un, kn);
+        __builtin_amdgcn_sched_barrier(0);   // in flight while this batch is used
+        if (k == 0) clear();
+        dots(cur, u, k);
+        if (last) finish(u);
+        u = un;
+        k = kn;
+        return u < u1;
+    };
+    while (step(r0, r1) && step(r1, r0)) {
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(kAttnThreads) void attn_pv_long_kernel(AttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [position slices][G][d] sums
+    __shared__ float ms[2 * G];
+    __shared__ float pr[2][G * kPvStep];
+    __shared__ int flag;
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int kvb = blockIdx.x, b = kvb / a.kvh, kh = kvb % a.kvh;
+    const int d = a.d, L = a.max_len;
+    const int Y = (int)gridDim.y, sp = (int)blockIdx.y;
+    const int64_t obase = (int64_t)b * a.kvh * G * d + (int64_t)kh * G * d;
+    const int64_t row0 = (int64_t)b * a.kvh * G + kh * G;
+    const int64_t lp = (int64_t)a.chunks * kChunk;
+    const int64_t p64 = uniform_i64(__hip_atomic_load(a.pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (p64 < 0 || p64 >= L) {  // no cache slot: zeros, no cache or counter touched
+        if (sp == 0)
+            for (int i = t; i < G * d; i += kAttnThreads) a.out[obase + i] = 0;
+        return;
+    }
+    const int p = (int)p64, lo = window_lo(p, a.window);
+    // span sp of the positions in use: whole steps, the same for every block
+    const int len = p - lo + 1;
+    const int span = ((len + Y - 1) / Y + kPvStep - 1) / kPvStep * kPvStep;
+    const int nspans = (len + span - 1) / span;
+    if (sp >= nspans) return;
+    const int j0 = lo + sp * span, j1 = j0 + span < p + 1 ? j0 + span : p + 1;
+
+    // thread: columns 8 cq .. + 7 of position slice ps of rpp
+    const int tpr = d / 8, rpp = kAttnThreads / tpr;
+    const int cq = t % tpr, ps = t / tpr;
+    const bool mine = ps < rpp;
+    const uint16_t* vb = a.vc + (int64_t)kvb * L * d + 8 * cq;
+    constexpr int kRows = kPvStep / 8;   // V rows per thread and step at head_dim 256 (fewer below)
+    constexpr int kProbs = (G * kPvStep + kAttnThreads - 1) / kAttnThreads;
+    const int rows = (kPvStep + rpp - 1) / rpp;
+    auto load = [&](uint4 (&vr)[kRows], float (&sc)[kProbs], int j) {
+#pragma unroll
+        for (int i = 0; i < kProbs; ++i) {
+            const int o = t + i * kAttnThreads, jj = j + o % kPvStep, h = o / kPvStep;
+            sc[i] = a.scores[(row0 + (h < G ? h : G - 1)) * lp + (jj < j1 ? jj : j1 - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < kRows; ++i)
+            if (i < rows) {
+                const int jj = j + ps + rpp * i;
+                vr[i] = *reinterpret_cast<const uint4*>(vb + (int64_t)(jj < j1 ? jj : j1 - 1) * d);
+            }
+    };
+    uint4 v0[kRows], v1[kRows];
+    float s0[kProbs], s1[kProbs];
+    load(v0, s0, j0);
+    // global max and sum of each head over its chunks (one wave per head)
+    const int c_lo = lo / kChunk, c_hi = p / kChunk;
+    for (int h = w; h < G; h += 4) {
+        const float* st = a.stats + (row0 + h) * a.chunks * 2;
+        float m = -INFINITY;
+        for (int cc = c_lo + lane; cc <= c_hi; cc += 64) m = fmaxf(m, st[cc * 2]);
+        m = wave_max(m);
+        float s = 0.0f;
+        for (int cc = c_lo + lane; cc <= c_hi; cc += 64) s += st[cc * 2 + 1] * expf(st[cc * 2] - m);
+        s = wave_sum(s);
+        if (lane == 0) {
+            ms[2 * h] = m;
+            ms[2 * h + 1] = s;
+        }
+    }
+    float acc[8][G];
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+        for (int h = 0; h < G; ++h) acc[m][h] = 0.0f;
+    lds_barrier();
+    int j = j0, buf = 0;
+    auto step = [&](const uint4 (&vr)[kRows], const float (&sc)[kProbs], uint4 (&vn)[kRows], float (&sn)[kProbs]) {
+        // the step's probabilities, once each
+#pragma unroll
+        for (int i = 0; i < kProbs; ++i) {
+            const int o = t + i * kAttnThreads, h = o / kPvStep;
+            if (h < G)
+                pr[buf][o] = j + o % kPvStep < j1 ? round_bf16(expf(sc[i] - ms[2 * h]) / ms[2 * h + 1]) : 0.0f;
+        }
+        if (j + kPvStep < j1) load(vn, sn, j + kPvStep);
+        // (one barrier per step: a buffer is written again two steps later)
+        lds_barrier();
+        if (mine) {
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) {
+                const int o = ps + rpp * i;
+                if (o < kPvStep && j + o < j1) {
+                    float v[8];
+                    unpack8(vr[i], v);
+#pragma unroll
+                    for (int h = 0; h < G; ++h) {
+                        const float q = pr[buf][h * kPvStep + o];
+#pragma unroll
+                        for (int m = 0; m < 8; ++m) acc[m][h] += q * v[m];
+                    }
+                }
+            }
+        }
+        buf ^= 1;
+        j += kPvStep;
+        return j < j1;
+    };
+    while (step(v0, s0, v1, s1) && step(v1, s1, v0, s0)) {
+    }
+    // the position slices in ascending order
+    if (mine) {
+#pragma unroll
+        for (int h = 0; h < G; ++h)
+#pragma unroll
+            for (int m = 0; m < 8; ++m) lds[(ps * G + h) * d + 8 * cq + m] = acc[m][h];
+    }
+    __syncthreads();
+    float* part = a.partial + row0 * (int64_t)a.chunks * d;   // [G][chunks][d]
+    for (int i = t; i < G * d; i += kAttnThreads) {
+        float o = 0.0f;
+        for (int r = 0; r < rpp; ++r) o += lds[r * G * d + i];
+        if (nspans == 1)
+            a.out[obase + i] = f_to_bf16(o);
+        else
+            __hip_atomic_store(&part[((int64_t)(i / d) * a.chunks + sp) * d + i % d], o, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (nspans == 1) return;
+    // several spans: the last block of the (sequence, KV head) adds them in order
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* counter = &a.counters[kvb];
+    if (t == 0) flag = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nspans - 1;
+    __syncthreads();
+    if (!flag) return;
+    for (int i = t; i < G * d; i += kAttnThreads) {
+        const float* q = part + (int64_t)(i / d) * a.chunks * d + i % d;
+        float sum = 0.0f;
+        for (int s0 = 0; s0 < nspans; s0 += 8) {   // 8 loads in flight, added in span order
+            float v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int s = s0 + k < nspans ? s0 + k : nspans - 1;
+                v[k] = __hip_atomic_load(&q[(int64_t)s * d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (s0 + k < nspans) sum += v[k];
+        }
+        a.out[obase + i] = f_to_bf16(sum);
+    }
+    if (t == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---------------------------------------------------------------------------
 // gelu(tanh) x up
 // ---------------------------------------------------------------------------
 
@@ -766,8 +1081,31 @@ bool attn_shape_ok(int32_t batch, int32_t heads, int32_t kv_heads, int32_t head_
     return g == 1 || g == 2 || g == 4 || g == 8;
 }
 
+template <int G, int UNIT>
+void launch_scores_long(const AttnArgs& a, dim3 grid, hipStream_t stream) {
+    if (a.dtype == SE12_STEP_F32)
+        hipLaunchKernelGGL((attn_scores_long_kernel<G, SE12_STEP_F32, UNIT>), grid, dim3(kAttnThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL((attn_scores_long_kernel<G, SE12_STEP_BF16, UNIT>), grid, dim3(kAttnThreads), 0, stream, a);
+}
+
 template <int G>
 void launch_attention(const AttnArgs& a, int blocks_x, hipStream_t stream) {
+    if ((int64_t)blocks_x * a.chunks > kLongBlocks) {
+        // a chunk, and a step of the pv kernel, is the least a block takes
+        const int y = std::max(1, std::min(a.chunks, kLongGrid / blocks_x));
+        const dim3 grid(blocks_x, y);
+        // about 16 K key elements per unit
+        if (a.d > 128)
+            launch_scores_long<G, 64>(a, grid, stream);
+        else if (a.d > 64)
+            launch_scores_long<G, 128>(a, grid, stream);
+        else
+            launch_scores_long<G, 256>(a, grid, stream);
+        const size_t sums = (size_t)(kAttnThreads / (a.d / 8)) * G * a.d * sizeof(float);
+        hipLaunchKernelGGL(attn_pv_long_kernel<G>, grid, dim3(kAttnThreads), sums, stream, a);
+        return;
+    }
     const dim3 grid(blocks_x, a.chunks);
     const int32_t qs = (int32_t)a.q_stride, kvs = (int32_t)a.kv_stride;
     if (a.dtype == SE12_STEP_F32)

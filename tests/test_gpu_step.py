@@ -192,6 +192,48 @@ def test_attention_step(gpu, batch, heads, kvh, d, L, pos, window, dtype):
     assert torch.equal(out, out2)
 
 
+# more than 1,024 (sequence, KV head, 64-position chunk) blocks, the kernels for long caches: positions at the edges of
+# units (64 / 128 / 256 at head_dim 256 / 128 / up to 64), of pv steps and spans, windows across them, head dims whose
+# value rows leave threads idle, every query-group size, a cache length off the unit
+ATTN_LONG_CASES = [
+    (32, 16, 8, 256, 320, 0, 0, torch.float32),
+    (32, 16, 8, 256, 320, 63, 0, torch.bfloat16),
+    (32, 16, 8, 256, 320, 64, 0, torch.float32),
+    (32, 16, 8, 256, 328, 327, 100, torch.float32),
+    (16, 8, 8, 128, 600, 599, 0, torch.float32),
+    (16, 8, 8, 128, 600, 128, 65, torch.bfloat16),
+    (32, 32, 8, 64, 520, 511, 0, torch.float32),
+    (32, 32, 8, 64, 520, 512, 300, torch.float32),
+    (4, 8, 4, 256, 8192, 8191, 0, torch.float32),
+    (4, 8, 4, 256, 8192, 5000, 4096, torch.bfloat16),
+    (3, 8, 1, 128, 32768, 20000, 0, torch.float32),      # 8 query heads per KV head
+    (32, 8, 4, 40, 1000, 777, 0, torch.float32),
+    (64, 4, 4, 8, 400, 390, 30, torch.float32),
+]
+
+
+@pytest.mark.parametrize("batch,heads,kvh,d,L,pos,window,dtype", ATTN_LONG_CASES)
+def test_attention_step_over_many_blocks(gpu, batch, heads, kvh, d, L, pos, window, dtype):
+    assert batch * kvh * -(-L // 64) > 1024
+    test_attention_step(gpu, batch, heads, kvh, d, L, pos, window, dtype)
+
+
+def test_attention_over_many_blocks_position_outside_the_cache_touches_nothing(gpu):
+    batch, heads, kvh, d, L = 64, 8, 4, 64, 384
+    q = torch.ones((batch, heads * d), device=gpu)
+    k = torch.ones((batch, kvh * d), device=gpu)
+    kt = torch.full((batch, kvh, d, L), 3.0, device=gpu).to(torch.bfloat16)
+    vc = torch.full((batch, kvh, L, d), 5.0, device=gpu).to(torch.bfloat16)
+    out = torch.full((batch, heads * d), 7.0, device=gpu).to(torch.bfloat16)
+    ws = _workspace(gpu, batch, heads, kvh, d, L)
+    for p in (L, -1):
+        _attention(q, k, k, torch.float32, heads * d, kvh * d, kt, vc, torch.ones(d // 2, device=gpu),
+                   torch.tensor(p, dtype=torch.int64, device=gpu), out, batch, heads, kvh, d, L, 1.0, 0.0, 0, ws)
+        torch.cuda.synchronize()
+        assert bool((out == 0).all()) and bool((kt == 3).all()) and bool((vc == 5).all())
+    assert bool((ws == 0).all())
+
+
 @pytest.mark.parametrize("L", [80, 1096])
 def test_attention_position_outside_the_cache_touches_nothing(gpu, L):
     batch, heads, kvh, d = 1, 4, 2, 64
