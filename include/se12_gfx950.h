@@ -71,7 +71,10 @@ typedef struct se12_streams_out {
 } se12_streams_out;
 
 /* Launch shape of the GEMV: `threads_per_block` = 64 * waves per workgroup.
- * Its `blocks` depend on the kernel the batch runs:
+ * Its `blocks` depend on the kernel the batch runs (FP32 x: a configuration
+ * names the dot2 kernel's shape at any batch; without one, 5 rows and more
+ * run the x-slab MFMA kernel on three BF16 planes of x, which together hold
+ * every bit of it):
  *  - dot2 kernel (batch 1..4 per launch, FP32 x): 1..16 waves, `blocks` =
  *    tile_rows * k_splits, k_splits cutting the K tiles into contiguous
  *    ranges;
@@ -237,11 +240,11 @@ int se12_gemv_grouped(se12_handle* const* handles, int32_t count, const void* x_
  * rows <= 8192.
  *
  * Where the product runs the dot2 kernel (batch rows per launch <= 4, or FP32
- * x) and, for the norm, rows % 4 == 0, y, w1, w2, residual and out are
+ * x under a given launch configuration) and, for the norm, rows % 4 == 0, y, w1, w2, residual and out are
  * 8-byte aligned and the row fits a block's LDS (10 bytes per row of W;
  * gfx950 blocks take up to 160 KiB), the block completing the inputs of the
  * step runs it;
- * otherwise (MFMA launches for BF16 x with batch >= 5, longer rows) the
+ * otherwise (MFMA launches, batch >= 5, longer rows) the
  * separate step kernel follows the product. Same stream, allocation and
  * ordering rules as se12_gemv. */
 int se12_gemv_gelu_mul(se12_handle* const* gate_up, const void* x_dev, int32_t x_dtype, int32_t batch,

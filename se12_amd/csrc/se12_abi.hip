@@ -320,9 +320,13 @@ int se12_handle_shape(const se12_handle* h, int64_t* rows, int64_t* cols, int64_
 // kernel variant (one tile per round, no prefetch) of the fused kernel and of
 // its raw twin must fit its VGPR budget.
 // BF16 activations with kGemmMinBatch or more rows take the MFMA kernel (one
-// launch, one pass over the weights); FP32 activations and smaller batches
-// the dot2 kernel, 4 rows per launch.
-static bool uses_mfma(int32_t batch, bool xf32) { return !xf32 && batch >= kGemmMinBatch; }
+// launch, one pass over the weights); smaller batches the dot2 kernel, 4 rows
+// per launch. FP32 activations: the x-slab MFMA kernel (three BF16 planes of
+// x) from kGemmMinBatch rows under the default launch; a launch
+// configuration given for them names the dot2 kernel's shape.
+static bool uses_mfma(int32_t batch, bool xf32, bool default_launch = true) {
+    return batch >= kGemmMinBatch && (!xf32 || default_launch);
+}
 static bool rx_fits(se12_handle* const* hs, int32_t count, int32_t batch);
 static void rx_default_launch(se12_handle* const* hs, int32_t count, int32_t batch, int32_t* waves_out,
                               int32_t* blocks_out);
@@ -520,6 +524,29 @@ static void gemm_default_launch(se12_handle* const* hs, int32_t count, int32_t b
     *splits_out = (int32_t)best_s;
 }
 
+// Default launch of the x-slab MFMA kernel for FP32 x: one K group, and K
+// splits for about kF32WavesPerCu waves per CU, which is what its registers
+// let a CU hold (2 waves per SIMD): 3584x14336 B = 8 / 32 28.4 / 53 us with
+// 8, 29.6 / 54 with 6, 34.5 / 66.5 with 12; 14336x3584 27.7 / 45 with 8, 31.5
+// / 60 with 12.
+constexpr int64_t kF32WavesPerCu = 8;
+static void gemm_f32_default_launch(se12_handle* const* hs, int32_t count, int32_t batch, int64_t max_partials,
+                                    int32_t* waves_out, int32_t* splits_out) {
+    const se12_handle* h0 = hs[0];
+    const int64_t cus = std::max<int32_t>(1, h0->cu_count);
+    const int32_t rows = gemm_min_waves(batch, true);
+    const int64_t row_waves = gemm_row_blocks(hs, count, rows) * rows;
+    int64_t splits = (kF32WavesPerCu * cus + row_waves / 2) / row_waves;
+    // 3+ K tiles each, fewer only to give every CU a block (1024x2304 B = 8 /
+    // 32 11.2 / 22.3 us against 12.2 / 24.8 with 3 splits)
+    const int64_t cap = std::max<int64_t>(h0->TC / 3, std::min<int64_t>(h0->TC, cus * rows / row_waves));
+    splits = std::min<int64_t>({splits, cap, (int64_t)kGemmMaxSplits, (int64_t)h0->s_cap});
+    // what the caller's scratch holds
+    if (max_partials > 0) splits = std::min<int64_t>(splits, max_partials / (batch * h0->Np));
+    *waves_out = rows;
+    *splits_out = (int32_t)std::max<int64_t>(1, splits);
+}
+
 int se12_read_probe(const void* buf_dev, int64_t bytes, uint32_t* out_dev, int64_t out_elems, void* stream) {
     if (!buf_dev || !out_dev) return fail(SE12_E_INVALID, "se12_read_probe: NULL argument");
     if (bytes < 16 || !aligned16(buf_dev))
@@ -588,22 +615,23 @@ static GemvPlan plan_gemv(int64_t tr, int64_t tc, bool raw, int32_t bl, bool xf3
     return p;
 }
 
-static GemvPlan plan_gemm(int64_t row_blocks, bool raw, int32_t batch, bool generic, int32_t waves, int32_t splits,
-                          int32_t tile_cols, int64_t lds_per_block) {
+static GemvPlan plan_gemm(int64_t row_blocks, bool raw, int32_t batch, bool xf32, bool generic, int32_t waves,
+                          int32_t splits, int32_t tile_cols, int64_t lds_per_block) {
     GemvPlan p{};
     p.batch = batch;
+    p.xf32 = xf32;
     p.raw = raw;
     p.generic = generic;
     p.waves = waves;
     p.blocks = (int32_t)(row_blocks * splits);
     // steps of a wave: its K group's share of the split's K tiles
-    const int32_t kgroups = std::max(1, waves / gemm_min_waves(batch));
+    const int32_t kgroups = std::max(1, waves / gemm_min_waves(batch, xf32));
     const int64_t steps = ceil_div(ceil_div(tile_cols, splits), kgroups);
     p.slab_ring = !generic && steps >= kGemmSlabRingMinSteps &&
-                          (int64_t)(gemm_lds_bytes(waves, batch, kGemmSlabRing) + kLutBytes) <= lds_per_block
+                          (int64_t)(gemm_lds_bytes(waves, batch, kGemmSlabRing, xf32) + kLutBytes) <= lds_per_block
                       ? kGemmSlabRing
                       : 0;
-    p.lds = gemm_lds_bytes(waves, batch, p.slab_ring);
+    p.lds = gemm_lds_bytes(waves, batch, p.slab_ring, xf32);
     p.g = 1;
     p.pf = 1;
     return p;
@@ -809,15 +837,19 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
     bool generic = xf32 || h0->K % SE12_TILE_COLS != 0 || !aligned16(x);
     for (int32_t i = 0; i < count; ++i)
         generic = generic || (raw && (hs[i]->N % SE12_TILE_ROWS != 0 || !aligned16(hs[i]->wraw)));
-    const bool mfma = uses_mfma(batch, xf32);
+    bool mfma = uses_mfma(batch, xf32, launch == nullptr);
+    // the edge-handling MFMA variants read x 16 bytes at a time: an x of
+    // fewer (one column, a few rows) goes to the dot2 kernel
+    const bool tiny = mfma && generic && (int64_t)batch * h0->K * (int64_t)esize < 16;
     const RxLayout rx_lay = mfma && !generic ? rx_layout(hs, count, batch) : RxLayout{0, 0};
     const int32_t rx_rows = rx_lay.staged;  // x rows in LDS
     const int32_t rx_splits = std::max<int32_t>(1, rx_lay.splits);
     const int64_t rx_k = ceil_div(h0->TC, rx_splits) * SE12_TILE_COLS;  // x columns a block holds
     const bool rx = rx_rows > 0;
     const int rx_max_threads = rx_rows < batch ? kRxMaxThreadsXG : kRxMaxThreads;
-    const int32_t step = mfma ? batch : kGemvMaxBatchPerLaunch;
-    const int32_t b_first = std::min<int32_t>(batch, step);
+    const int32_t mfma_rows = gemm_min_waves(batch, xf32);  // x-slab kernel: tile rows per block
+    int32_t step = mfma ? batch : kGemvMaxBatchPerLaunch;
+    int32_t b_first = std::min<int32_t>(batch, step);
     int32_t waves, splits;
     int32_t rx_blocks = 0;
     int64_t grid_rows = tr_total;  // grid rows per split: tile rows, or row blocks (MFMA)
@@ -842,16 +874,16 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
     } else if (launch) {
         const int max_threads = mfma ? (generic ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
                                      : max_threads_for(b_first, xf32, generic);
-        const int min_threads = mfma ? 64 * gemm_min_waves(batch) : 64;
+        const int min_threads = mfma ? 64 * mfma_rows : 64;
         if (launch->threads_per_block < min_threads || launch->threads_per_block > max_threads ||
             launch->threads_per_block % 64 != 0)
             return fail(SE12_E_INVALID, "%s: threads_per_block %d must be a multiple of 64 in [%d, %d] at batch %d", fn,
                         launch->threads_per_block, min_threads, max_threads, batch);
         waves = launch->threads_per_block / 64;
-        if (mfma && waves % gemm_min_waves(batch) != 0)
+        if (mfma && waves % mfma_rows != 0)
             return fail(SE12_E_INVALID, "%s: %d waves per block at batch %d: the MFMA kernel takes %d tile rows per block "
-                        "times K groups", fn, waves, batch, gemm_min_waves(batch));
-        if (mfma) grid_rows = gemm_row_blocks(hs, count, gemm_min_waves(batch));
+                        "times K groups", fn, waves, batch, mfma_rows);
+        if (mfma) grid_rows = gemm_row_blocks(hs, count, mfma_rows);
         if (launch->blocks <= 0 || launch->blocks % grid_rows != 0)
             return fail(SE12_E_INVALID, "%s: blocks %d must be a positive multiple of the %lld %s", fn, launch->blocks,
                         (long long)grid_rows, mfma ? "row blocks (tile rows / waves, rounded up, per matrix)" : "tile rows");
@@ -861,8 +893,11 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
             return fail(SE12_E_CAPACITY, "%s: %d K splits exceed the limit %d at batch %d", fn, splits, cap, batch);
     } else {
         if (mfma) {
-            gemm_default_launch(hs, count, batch, generic, &waves, &splits);
-            grid_rows = gemm_row_blocks(hs, count, gemm_min_waves(batch));
+            if (xf32)
+                gemm_f32_default_launch(hs, count, batch, ws ? ws->partial_elems : 0, &waves, &splits);
+            else
+                gemm_default_launch(hs, count, batch, generic, &waves, &splits);
+            grid_rows = gemm_row_blocks(hs, count, mfma_rows);
         } else {
             default_launch(tr_total, h0->TC, h0->cu_count, h0->s_cap, batch, xf32, generic, pro != nullptr, &waves,
                            &splits);
@@ -875,6 +910,13 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
                 if (h0->TC % even == 0 && even >= waves - 2) waves = even;
             }
         }
+    }
+    if (tiny) {
+        mfma = false;
+        step = kGemvMaxBatchPerLaunch;
+        b_first = std::min<int32_t>(batch, step);
+        waves = splits = 1;
+        grid_rows = tr_total;
     }
     if (grid_rows * splits > INT32_MAX) return fail(SE12_E_INVALID, "%s: grid too large", fn);
     DeviceScope ds;
@@ -924,7 +966,7 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
         const int32_t bl = std::min<int32_t>(step, batch - b0);
         GemvGroupArgs g{};
         g.count = count;
-        g.rows_per_block = mfma ? gemm_min_waves(bl) : 1;
+        g.rows_per_block = mfma ? mfma_rows : 1;
         int32_t start = 0;
         size_t rx_lds = 0;
         for (int32_t i = 0; i < count; ++i) {
@@ -950,12 +992,12 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
             a.S = rx ? rx_kgroups(h->TR, h->TC / rx_splits, waves, rx_blocks / (count * rx_splits)) : splits;
             rx_lds = std::max(rx_lds, rx ? rx_lds_total(rx_k, rx_rows, bl, waves, a.S) : 0);
             g.tr_start[i] = start;
-            start += mfma ? (int32_t)ceil_div(h->TR, gemm_min_waves(bl)) : h->TR;
+            start += mfma ? (int32_t)ceil_div(h->TR, mfma_rows) : h->TR;
         }
         for (int32_t i = count; i <= kMaxGroup; ++i) g.tr_start[i] = start;
         const bool gen = generic || !aligned16(g.m[0].x);
         GemvPlan p = rx     ? plan_rx(raw, bl, rx_rows, rx_splits, waves, rx_blocks, rx_k, rx_lds)
-                     : mfma ? plan_gemm(grid_rows, raw, bl, gen, waves, splits, h0->TC, h0->lds_per_block)
+                     : mfma ? plan_gemm(grid_rows, raw, bl, xf32, gen, waves, splits, h0->TC, h0->lds_per_block)
                             : plan_gemv(tr_total, h0->TC, raw, bl, xf32, gen, waves, splits);
         if (fuse_pro) {
             g.pro = *pro;

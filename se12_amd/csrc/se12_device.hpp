@@ -73,7 +73,7 @@ __device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballo
 // launches measured, against plain loads (same box, interleaved): 2304x9216
 // 8.49 -> 8.28 us, 2 x 9216x2304 grouped 14.13 -> 13.41, 14336x3584 16.69
 // -> 15.56, 4608x36864 50.5 -> 45.2 us. Where an instruction reads half of
-// each line and the next one the other half (the x-slab kernel's row layout,
+// each line and the next one the other half (a layout of one tile row per lane,
 // the raw twin's 32 bytes per lane as two loads, side records of 64 bytes)
 // the hint makes the second read fetch the line again: the x-slab kernel at
 // 14336x3584, batch 32, took 31.3 us with it against 26.5 without, the raw
@@ -92,6 +92,13 @@ __device__ __forceinline__ T stream_load(const T* p) {
         static_assert(sizeof(T) == 4, "stream_load: 4, 8 or 16 bytes");
         return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p)));
     }
+}
+
+// 16 bytes at any address (gfx950 global loads take unaligned addresses)
+__device__ __forceinline__ uint4 load16_unaligned(const void* p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, sizeof v);
+    return v;
 }
 
 // inclusive prefix sum over the 64 lanes with DPP: shifts of 1, 2, 4, 8
@@ -318,20 +325,18 @@ __device__ __forceinline__ void or_pattern_word(uint32_t pat[4][8], uint32_t wor
 // Patches the n (1..kListedEscapes) listed escapes of a tile: escape k sits
 // at pos_k = row * 256 + col and takes esc slot k. Everything but the final
 // OR is wave-uniform (scalar), so an escape costs a few instructions.
-// Three lane layouts of a tile's 16 x 256 weights, 16 consecutive columns
+// Two lane layouts of a tile's 16 x 256 weights, 16 consecutive columns
 // of one row (a column block, col / 16) per lane in each of 4 parts
 // (pat[part][word], word = pair of columns):
 //   chunk layout (dot2, decode): part j = rows 4j..4j+3, lane 16 (row % 4) +
 //     block;
-//   row layout (se12_gemm.hip): part p = columns 64p..64p+63, lane row + 16
-//     (block % 4);
-//   block layout (se12_gemm_rx.hip): part = block % 4, lane row + 16 (block
+//   block layout (the MFMA kernels): part = block % 4, lane row + 16 (block
 //     / 4).
 // and one of 8 columns per lane in each of 8 parts:
 //   half layout (the decode-only kernel): part p = rows 2p, 2p+1, lane 32
 //     (row % 2) + col / 8, word (col % 8) / 2 of the part's 4, stored as
 //     pattern word 4p + word (pat[p / 2][4 (p % 2) + word]).
-enum TileLayout { kChunkLayout, kRowLayout, kBlockLayout, kHalfLayout };
+enum TileLayout { kChunkLayout, kBlockLayout, kHalfLayout };
 
 template <int LAYOUT>
 __device__ __forceinline__ void patch_listed_escapes(uint32_t pat[4][8], uint4 pos, uint4 esc, uint32_t n,
@@ -341,10 +346,9 @@ __device__ __forceinline__ void patch_listed_escapes(uint32_t pat[4][8], uint4 p
         const uint32_t p = (k & 1u) ? (w >> 16) : (w & 0xFFFFu);
         const uint32_t row = (p >> 8) & 15u, col = p & 255u, block = col >> 4;
         const uint32_t owner = LAYOUT == kChunkLayout ? (((row & 3u) << 4) | block)
-                               : LAYOUT == kRowLayout ? (row | ((block & 3u) << 4))
                                : LAYOUT == kHalfLayout ? (((row & 1u) << 5) | (col >> 3))
                                                        : (row | ((block >> 2) << 4));
-        const uint32_t part = LAYOUT == kChunkLayout ? (row >> 2) : LAYOUT == kRowLayout ? (block >> 2) : (block & 3u);
+        const uint32_t part = LAYOUT == kChunkLayout ? (row >> 2) : (block & 3u);
         const uint32_t word = LAYOUT == kHalfLayout ? (((row >> 1) << 2) | ((col & 7u) >> 1))
                                                     : ((part << 3) | ((col & 15u) >> 1));
         const uint32_t v = esc_byte(esc, k) << ((col & 1u) ? 23u : 7u);

@@ -20,21 +20,17 @@
 // (slabs of step i + 1 written during step i), or, on launches of 12 or more
 // steps where LDS holds it, a ring of 8 slabs written 4 steps ahead with a
 // barrier every 4 steps. Each wave requests its tile streams two tiles ahead
-// of the decode (the edge-handling variants load and use in turn).
+// of the decode (the edge-handling and FP32 variants one).
 //
-// FAST variants load each tile whole-line (a kilobyte of sm holding 4 tile
-// rows per load instruction, as the resident-x kernel does) and move it into
+// Each tile is loaded whole-line (a kilobyte of sm holding 4 tile
+// rows per load instruction, as the resident-x kernel does) and moved into
 // the block layout with DPP exchanges: lane l holds, in part p, the 16
 // columns 16 (4 (l / 16) + p) .. + 15 of row l % 16, decoded through the
 // pair table with listed escapes and raw tiles. Each part's first and second
 // 8 columns are the A operands of two v_mfma_f32_16x16x32_bf16 (MFMA row =
 // tile row); their K positions differ between lane groups, and the B
 // operands (lane l: batch row 16 g + l % 16) read the same 8 columns of the
-// x slab. GENERIC variants load row-wise: lane l takes row l % 16 and the 16
-// columns 64 p + 16 (l / 16) .. + 15 of part p, and two lane-row swaps
-// (v_permlane16_swap, v_permlane32_swap) leave each lane holding its A
-// operands for the part's two 32-column slices s (lane l: columns 32 s + 8
-// (l / 16) .. + 7). Either way the decoded tile never goes through memory;
+// x slab. The decoded tile never goes through memory;
 // 8 MFMAs per tile and group of 16 batch rows, FP32 accumulate, in a fixed
 // order. Rows of the LDS x slabs are padded to 528 bytes so that the 16-byte
 // reads of 8 lanes per cycle hit distinct banks. Batch rows past the batch
@@ -48,10 +44,14 @@
 // shape (W, S) fixes every sum: the raw-BF16 twin (same kernel, RAW) is
 // bit-identical under one shape.
 //
-// FAST variants need K % 256 == 0 and 16-byte aligned x rows (and, for the
-// raw twin, N % 16 == 0 and an aligned W); GENERIC variants guard loads by
-// the matrix edges and zero weights and x past K (padding can decode to
-// +inf when codebook[0] = 255).
+// How x is read (XMode): whole K tiles of 16-byte aligned BF16 rows; BF16 of
+// any K and alignment (16-byte loads at any address, the columns past K cut
+// where they are stored to LDS, weights past K zeroed: the SE12 streams
+// themselves are whole, aligned tiles; loading the tiles whole-line and one
+// ahead instead of element-wise x with each tile loaded and used in turn:
+// 5003x2887 at 6 / 16 / 32 rows 21.5 / 25.0 / 28.2 -> 13.9 / 15.1 / 16.4 us,
+// 14337x3585 at 8 / 24 56.6 / 72.1 -> 27.9 / 31.2); FP32 of any K (three BF16
+// planes, below). The raw twin's W is guarded by its edges in the last two.
 #include <algorithm>
 
 #include "se12_device.hpp"
@@ -69,10 +69,30 @@ constexpr int x_slab_bytes() {
     return 16 * BG * kRowBytes;
 }
 
-// the 16-byte pieces p = tid + k * threads (k < kGemmXPieces) of an x slab:
-// batch row p / 32, columns 8 (p % 32) .. + 7
+// How a launch reads x: kXFast, BF16 in whole K tiles and 16-byte aligned rows;
+// kXEdge, BF16 of any K and alignment; kXF32, FP32 of any K.
+enum XMode { kXFast, kXEdge, kXF32 };
+
+// FP32 x goes to LDS as three BF16 planes, x = h + m + l exactly: each plane
+// is the top 16 bits of what the ones before it leave (8 of the 24
+// significand bits). The product is then three MFMAs per part whose BF16
+// products are exact, summed in FP32: h in one accumulator that is emptied
+// into the row's sum after each K tile, m and l (2^-8 and 2^-16 of it) in
+// another. The edge-handling dot2 kernel it replaces at 5 and more rows reads
+// the weights once per 4 rows. Bound by the conversion and LDS traffic of the
+// planes beside the weights' stream. Cold weights, before and after: 3584x14336
+// at 8 / 16 / 32 rows 214 / 427 / 855 -> 28.4 / 34 / 53 us, 2304x9216 100 / 200 /
+// 400 -> 18.4 / 22 / 37, 14336x3584 210 / 420 / 840 -> 27.7 / 32 / 45; error
+// against 64 bits 1.0e-7 to 1.2e-7 (1.0e-7 to 2.8e-7 before).
+constexpr int x_planes(XMode xm) { return xm == kXF32 ? 3 : 1; }
+// a piece is 16 bytes of x: 8 BF16 or 4 FP32 columns of one batch row
+constexpr int x_piece_cols(XMode xm) { return xm == kXF32 ? 4 : 8; }
+constexpr int x_row_pieces(XMode xm) { return kTileCols / x_piece_cols(xm); }
+
+// the pieces p = tid + k * threads (k < PC) of a step's slabs
+template <int PC>
 struct XPieces {
-    uint4 v[kGemmXPieces];
+    uint4 v[PC];
 };
 
 // Every load here and below is issued unconditionally (indexes clamped into
@@ -81,107 +101,142 @@ struct XPieces {
 // prefetched tiles included - before the next decode.
 // The slabs of one step: K group g's slab is x at K tile kb + g + KG i
 // (clamped into the split; a clamped slab is loaded but not used). Piece p
-// of the step: group p / (batch * 32), batch row (p % (batch * 32)) / 32,
-// columns 8 (p % 32) .. + 7.
-template <bool GENERIC>
-__device__ __forceinline__ XPieces load_x_slab(const GemvArgs& a, int batch, int kb, int n, int KG, int i, int tid,
-                                               int threads) {
-    XPieces xr;
-    const int per = batch * 32;
+// of the step: group g = p / (batch * pieces per row), batch row and piece of
+// the row from the remainder. Where a piece runs past the end of x (kXEdge and
+// kXF32, the last row's end) the 16 bytes that end there are read instead;
+// store_x_slab moves them down. The host sends x of fewer than one piece
+// elsewhere.
+struct XPiece {
+    int g, row, c;  // K group, batch row, piece of the tile's 256 columns
+    int kt;
+};
+template <XMode XM>
+__device__ __forceinline__ XPiece x_piece(int batch, int kb, int n, int KG, int i, int p) {
+    constexpr int kPer = x_row_pieces(XM);
+    p = min(p, KG * batch * kPer - 1);
+    XPiece r;
+    r.g = p / (batch * kPer);
+    const int q = p - r.g * (batch * kPer);
+    r.row = q / kPer;
+    r.c = q % kPer;
+    const int t = r.g + KG * i;
+    r.kt = kb + (t < n ? t : n - 1);
+    return r;
+}
+
+template <XMode XM, int PC>
+__device__ __forceinline__ XPieces<PC> load_x_slab(const GemvArgs& a, int batch, int kb, int n, int KG, int i, int tid,
+                                                   int threads) {
+    XPieces<PC> xr;
+    constexpr int kCols = x_piece_cols(XM), kBytes = 16 / kCols;
 #pragma unroll
-    for (int k = 0; k < kGemmXPieces; ++k) {
-        const int p = min(tid + k * threads, KG * per - 1);
-        const int g = p / per, q = p - g * per;
-        const int t = g + KG * i;
-        const int kt = kb + (t < n ? t : n - 1);
-        const uint16_t* row = static_cast<const uint16_t*>(a.x) + (int64_t)(q >> 5) * a.K;
-        const int64_t col = (int64_t)kt * kTileCols + 8 * (q & 31);
-        if constexpr (!GENERIC) {
-            xr.v[k] = *reinterpret_cast<const uint4*>(row + col);
-        } else {
-            uint32_t e[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const uint32_t lo = row[min(col + 2 * t, a.K - 1)];
-                const uint32_t hi = row[min(col + 2 * t + 1, a.K - 1)];
-                e[t] = (col + 2 * t < a.K ? lo : 0u) | (col + 2 * t + 1 < a.K ? hi << 16 : 0u);
-            }
-            xr.v[k] = make_uint4(e[0], e[1], e[2], e[3]);
-        }
+    for (int k = 0; k < PC; ++k) {
+        const XPiece r = x_piece<XM>(batch, kb, n, KG, i, tid + k * threads);
+        int64_t at = (int64_t)r.row * a.K + (int64_t)r.kt * kTileCols + kCols * r.c;
+        if constexpr (XM != kXFast) at = min(at, (int64_t)batch * a.K - kCols);
+        const char* src = static_cast<const char*>(a.x) + at * kBytes;
+        if constexpr (XM == kXFast)
+            xr.v[k] = *reinterpret_cast<const uint4*>(src);
+        else
+            xr.v[k] = load16_unaligned(src);
     }
     return xr;
 }
 
-// pieces past the step's slabs repeat the last piece: the same bytes to the
-// same address as the thread that owns it. Group g's slab sits at xb + g *
-// slab_bytes.
-__device__ __forceinline__ void store_x_slab(char* xb, int slab_bytes, const XPieces& xr, int batch, int KG, int tid,
-                                             int threads) {
-    const int per = batch * 32;
+// v's elements from `shift` on, moved down to 0, those at or past `valid`
+// zero: the columns past K of a piece at a row's end (16-bit elements, or
+// 32-bit ones with WORDS)
+template <bool WORDS>
+__device__ __forceinline__ uint4 cut_piece(uint4 v, int shift, int valid) {
+    uint32_t e[5] = {v.x, v.y, v.z, v.w, 0u};
+    const int dw = WORDS ? shift : shift >> 1;
+    uint32_t o[5];
 #pragma unroll
-    for (int k = 0; k < kGemmXPieces; ++k) {
-        const int p = min(tid + k * threads, KG * per - 1);
-        const int g = p / per, q = p - g * per;
-        *reinterpret_cast<uint4*>(xb + g * slab_bytes + (q >> 5) * kRowBytes + 16 * (q & 31)) = xr.v[k];
-    }
-}
-
-// The row layout: lane l holds row l % 16 and, in part p, the 16 columns
-// 64 p + 16 (l / 16) .. + 15 of the tile.
-__device__ __forceinline__ int row_layout_col(int p, uint32_t lane) { return 64 * p + 16 * (int)(lane >> 4); }
-
-// One tile's sm and ec bytes in the row layout (per part: 16 sm bytes, 8 ec
-// bytes of the lane's row).
-__device__ __forceinline__ void load_tile_rows(TileLoads& t, const uint8_t* sm, const uint8_t* ec, int64_t tile,
-                                               uint32_t lane) {
-    const uint8_t* smt = sm + tile * kTile + (lane & 15u) * kTileCols + 16u * (lane >> 4);
-    const uint8_t* ect = ec + tile * (kTile / 2) + (lane & 15u) * (kTileCols / 2) + 8u * (lane >> 4);
+    for (int i = 0; i < 5; ++i) {
+        o[i] = 0u;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        t.sm[p] = *reinterpret_cast<const uint4*>(smt + 64 * p);
-        t.ec[p] = *reinterpret_cast<const uint2*>(ect + 32 * p);
+        for (int j = i; j < 4; ++j)
+            if (j - i == dw) o[i] = e[j];
     }
-}
-
-// Raw BF16 of part p of a raw tile (tile-local row-major) in the row layout.
-__device__ __forceinline__ void load_raw_part(const int16_t* tile_raw, int p, uint32_t lane, uint32_t w[8]) {
-    const uint4* q = reinterpret_cast<const uint4*>(tile_raw + (lane & 15u) * kTileCols + row_layout_col(p, lane));
-    const uint4 a = q[0], b = q[1];
-    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w;
-    w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
-}
-
-// The lane's 16 decoded weights of a part (8 BF16 pairs: w[0..3] columns
-// c..c+7, w[4..7] columns c+8..c+15) become the A operands of the part's two
-// slices: a v_permlane16_swap (odd rows of the first register with even rows
-// of the second) and a v_permlane32_swap (upper half of the first with lower
-// half of the second) per register pair.
-__device__ __forceinline__ void rows_to_operands(const uint32_t w[8], bf16x8_t& a0, bf16x8_t& a1) {
-    uint32_t u[4], v[4];
+    if constexpr (!WORDS) {
+        if (shift & 1) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = (o[i] >> 16) | (o[i + 1] << 16);
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const auto s16 = __builtin_amdgcn_permlane16_swap(w[i], w[4 + i], false, false);
-        const auto s32 = __builtin_amdgcn_permlane32_swap(s16[0], s16[1], false, false);
-        u[i] = s32[0];
-        v[i] = s32[1];
+        if constexpr (WORDS)
+            o[i] = i < valid ? o[i] : 0u;
+        else
+            o[i] = 2 * i + 1 < valid ? o[i] : 2 * i < valid ? (o[i] & 0xFFFFu) : 0u;
     }
-    a0 = __builtin_bit_cast(bf16x8_t, make_uint4(u[0], u[1], u[2], u[3]));
-    a1 = __builtin_bit_cast(bf16x8_t, make_uint4(v[0], v[1], v[2], v[3]));
+    return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// Raw-twin rows in the row layout (per part: the lane's 16 columns).
-template <bool GENERIC>
-__device__ __forceinline__ void load_raw_rows(uint4 r[4][2], const GemvArgs& a, int tr, int kt, uint32_t lane) {
+// One FP32 value as three BF16 planes (bits in the high half): h + m + l == x
+// for every finite x whose l is not below BF16's range; an infinity or a NaN
+// goes to h alone (a NaN quiet, so that it stays one in 16 bits).
+__device__ __forceinline__ void split3(uint32_t u, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const float x = __uint_as_float(u);
+    const bool finite = (u & 0x7F800000u) != 0x7F800000u;
+    h = x != x ? 0x7FC00000u : (u & 0xFFFF0000u);
+    const float r = finite ? x - __uint_as_float(u & 0xFFFF0000u) : 0.0f;
+    m = __float_as_uint(r) & 0xFFFF0000u;
+    l = __float_as_uint(r - __uint_as_float(m));
+}
+
+// pieces past the step's slabs repeat the last piece: the same bytes to the
+// same address as the thread that owns it. Group g's slab sits at xb + g *
+// slab_bytes, its planes plane_bytes apart.
+template <XMode XM, int PC>
+__device__ __forceinline__ void store_x_slab(const GemvArgs& a, char* xb, int slab_bytes, int plane_bytes,
+                                             const XPieces<PC>& xr, int batch, int kb, int n, int KG, int i, int tid,
+                                             int threads) {
+    constexpr int kCols = x_piece_cols(XM);
+#pragma unroll
+    for (int k = 0; k < PC; ++k) {
+        const XPiece r = x_piece<XM>(batch, kb, n, KG, i, tid + k * threads);
+        char* dst = xb + r.g * slab_bytes + r.row * kRowBytes + 2 * kCols * r.c;
+        uint4 v = xr.v[k];
+        if constexpr (XM != kXFast) {
+            const int64_t col = (int64_t)r.kt * kTileCols + kCols * r.c;
+            if (col + kCols > a.K) {
+                const int64_t past = (int64_t)r.row * a.K + col + kCols - (int64_t)batch * a.K;
+                const int64_t valid = a.K - col;
+                v = cut_piece<XM == kXF32>(v, (int)min(max(past, (int64_t)0), (int64_t)kCols),
+                                           (int)max(valid, (int64_t)0));
+            }
+        }
+        if constexpr (XM == kXF32) {
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+            uint32_t h[4], m[4], l[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) split3(u[e], h[e], m[e], l[e]);
+            // the high halves of two values side by side
+            *reinterpret_cast<uint2*>(dst) = make_uint2(perm(h[1], h[0], 0x07060302u), perm(h[3], h[2], 0x07060302u));
+            *reinterpret_cast<uint2*>(dst + plane_bytes) =
+                make_uint2(perm(m[1], m[0], 0x07060302u), perm(m[3], m[2], 0x07060302u));
+            *reinterpret_cast<uint2*>(dst + 2 * plane_bytes) =
+                make_uint2(perm(l[1], l[0], 0x07060302u), perm(l[3], l[2], 0x07060302u));
+        } else {
+            *reinterpret_cast<uint4*>(dst) = v;
+        }
+    }
+}
+
+// Raw-twin rows in the block layout, guarded by the matrix edges and of any
+// alignment: the edge-handling form of load_raw_blocks.
+__device__ __forceinline__ void load_raw_blocks_edge(uint4 r[4][2], const GemvArgs& a, int tr, int kt, uint32_t lane) {
     const int64_t row = (int64_t)tr * kTileRows + (lane & 15u);
+    const uint16_t* p = a.wraw + min(row, a.N - 1) * a.K;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int64_t col = (int64_t)kt * kTileCols + row_layout_col(j, lane);
-        if constexpr (!GENERIC) {
-            const uint16_t* p = a.wraw + row * a.K + col;
-            r[j][0] = reinterpret_cast<const uint4*>(p)[0];
-            r[j][1] = reinterpret_cast<const uint4*>(p)[1];
+        const int64_t col = (int64_t)kt * kTileCols + block_layout_col(j, lane);
+        if (row < a.N && col + 16 <= a.K) {
+            r[j][0] = load16_unaligned(p + col);
+            r[j][1] = load16_unaligned(p + col + 8);
         } else {
-            const uint16_t* p = a.wraw + min(row, a.N - 1) * a.K;
             uint32_t h[8];
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
@@ -196,7 +251,8 @@ __device__ __forceinline__ void load_raw_rows(uint4 r[4][2], const GemvArgs& a, 
     }
 }
 
-// weights at columns >= lim of the tile are zeroed
+// weights at columns >= lim of the tile are zeroed (padding can decode to
+// +inf when codebook[0] = 255)
 __device__ __forceinline__ void zero_past_k(uint32_t w[8], int c0, int lim) {
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -205,26 +261,20 @@ __device__ __forceinline__ void zero_past_k(uint32_t w[8], int c0, int lim) {
     }
 }
 
-// The MFMAs of part p (slices 2p and 2p + 1) for every batch group, the x
-// slab (B operands) read from LDS.
-template <int BG>
-__device__ __forceinline__ void mfma_part(const bf16x8_t& a0, const bf16x8_t& a1, const char* xb, int p, uint32_t lane,
-                                          floatx4_t acc[BG]) {
-    const int off = (int)(lane & 15u) * kRowBytes + 16 * (int)(lane >> 4);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int s = 2 * p + h;
-#pragma unroll
-        for (int g = 0; g < BG; ++g) {
-            const uint4 bv = *reinterpret_cast<const uint4*>(xb + g * 16 * kRowBytes + off + 64 * s);
-            acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h ? a1 : a0, __builtin_bit_cast(bf16x8_t, bv), acc[g], 0, 0,
-                                                              0);
-        }
-    }
+// infinities and NaNs of a BF16 pair zeroed: the m and l planes of a finite x
+// may be zero, and must add nothing to what the h plane gives
+__device__ __forceinline__ uint32_t finite_pair(uint32_t w) {
+    const uint32_t lo = (w & 0x7F80u) == 0x7F80u ? 0u : (w & 0xFFFFu);
+    const uint32_t hi = (w & 0x7F800000u) == 0x7F800000u ? 0u : (w & 0xFFFF0000u);
+    return lo | hi;
 }
+__device__ __forceinline__ bool pair_not_finite(uint32_t w) {
+    return (w & 0x7F80u) == 0x7F80u || (w & 0x7F800000u) == 0x7F800000u;
+}
+__device__ __forceinline__ bool has_byte_ff(uint32_t w) { return ((~w - 0x01010101u) & w & 0x80808080u) != 0u; }
 
-// The MFMAs of part p of a tile in the block layout (FAST variants; lane l
-// holds row l % 16, columns 16 (4 (l / 16) + p) .. + 15 as 8 BF16 pairs):
+// The MFMAs of part p of a tile in the block layout (lane l holds row l % 16,
+// columns 16 (4 (l / 16) + p) .. + 15 as 8 BF16 pairs):
 // its first and second 8 columns are the A operands of two MFMAs whose B
 // operands are the same 8 columns of the x slab (batch row 16 g + l % 16).
 // The MFMA's K positions differ between lane groups; A and B agree on them.
@@ -250,10 +300,9 @@ struct GemmTile {
     uint4 r[RAW ? 4 : 1][2];
 };
 
-template <int BG, bool RAW, bool GENERIC, int M>
-__global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
-                                                                                                  int batch) {
-    static_assert(M == 0 || (!GENERIC && M >= 1), "the slab ring serves the FAST variants");
+template <int BG, bool RAW, XMode XM, int M, int PC = kGemmXPieces>
+__global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga, int batch) {
+    static_assert(M == 0 || (XM == kXFast && M >= 1), "the slab ring serves the FAST variants");
     SE12_DECLARE_LUT(lut);
     extern __shared__ __attribute__((aligned(16))) char gsm[];
     // the matrix comes from the grid; every argument the block needs goes out
@@ -281,7 +330,8 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
     const int n = ke - kb;
     const int steps = (n + KG - 1) / KG;  // K group kg takes the split's tiles kg, kg + KG, ...
     const int64_t row_tiles = (int64_t)trl * a.TC;
-    const int slab_bytes = x_slab_bytes<BG>();
+    constexpr int plane_bytes = x_slab_bytes<BG>();
+    constexpr int slab_bytes = x_planes(XM) * plane_bytes;
     // [NB buffers][KG slabs] of x: two with a block barrier per step, or a
     // ring of 2 M with a barrier every M steps
     constexpr int NB = M > 0 ? 2 * M : 2;
@@ -290,17 +340,20 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
     floatx4_t acc[BG];
 #pragma unroll
     for (int g = 0; g < BG; ++g) acc[g] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    floatx4_t low[XM == kXF32 ? BG : 1];  // the m and l planes' sums
+    if constexpr (XM == kXF32) {
+#pragma unroll
+        for (int g = 0; g < BG; ++g) low[g] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    bool lut_special = false;  // the codebook holds exponent 255
 
     auto load_tile_i = [&](GemmTile<RAW>& t, int i) {
         const int j = kg + KG * i;
         const int kt = kb + (j < n ? j : n - 1);
-        if constexpr (RAW && GENERIC) {
-            load_raw_rows<true>(t.r, a, trl, kt, lane);
+        if constexpr (RAW && XM != kXFast) {
+            load_raw_blocks_edge(t.r, a, trl, kt, lane);
         } else if constexpr (RAW) {
             load_raw_blocks(t.r, a.wraw, a.K, trl, kt, lane);
-        } else if constexpr (GENERIC) {
-            load_side(t.side, a.side, row_tiles + kt, lane);
-            load_tile_rows(t.t, a.sm, a.ec, row_tiles + kt, lane);
         } else {
             load_tile_block_order(t.t, t.side, a.sm, a.ec, a.side, row_tiles + kt, lane);
         }
@@ -308,52 +361,60 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
     auto use_tile = [&](GemmTile<RAW>& t, int i) {
         const int kt = kb + kg + KG * i;
         const char* xb = xbuf + ((i % NB) * KG + kg) * slab_bytes;
-        if constexpr (GENERIC) {
-            const int lim = (int)(a.K - (int64_t)kt * kTileCols);
-            // one part: weights (row layout) -> A operands -> the part's MFMAs
-            auto part = [&](int p, uint32_t wv[8]) {
-                zero_past_k(wv, row_layout_col(p, lane), lim);
-                bf16x8_t a0, a1;
-                rows_to_operands(wv, a0, a1);
-                mfma_part<BG>(a0, a1, xb, p, lane, acc);
-            };
-            if constexpr (RAW) {
+        // a decoded tile's (or raw tile's) 4 parts: edge columns zeroed, then
+        // the MFMAs; `special` (wave-uniform): it may hold an infinity or NaN
+        auto mfma_tile = [&](uint32_t (&wv)[4][8], bool special) {
+            if constexpr (XM != kXFast) {
+                const int64_t lim = a.K - (int64_t)kt * kTileCols;
+                if (lim < kTileCols) {
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) zero_past_k(wv[p], block_layout_col(p, lane), (int)lim);
+                }
+            }
+            if constexpr (XM != kXF32) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) mfma_block_part<BG>(wv[p], xb, p, lane, acc);
+            } else {
+                floatx4_t tile[BG];
+#pragma unroll
+                for (int g = 0; g < BG; ++g) tile[g] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int p = 0; p < 4; ++p) mfma_block_part<BG>(wv[p], xb, p, lane, tile);
+                if (special) {
+#pragma unroll
+                    for (int p = 0; p < 4; ++p)
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) wv[p][q] = finite_pair(wv[p][q]);
+                }
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
-                    uint32_t wv[8] = {t.r[p][0].x, t.r[p][0].y, t.r[p][0].z, t.r[p][0].w,
-                                      t.r[p][1].x, t.r[p][1].y, t.r[p][1].z, t.r[p][1].w};
-                    part(p, wv);
+                    mfma_block_part<BG>(wv[p], xb + plane_bytes, p, lane, low);
+                    mfma_block_part<BG>(wv[p], xb + 2 * plane_bytes, p, lane, low);
                 }
-            } else {
-                const uint32_t info = side_info(t.side, 0);
-                if (info_is_fallback(info)) {
-                    const int16_t* raw = raw_tile_ptr(info, a.fb_raw, a.ovf_raw);
-                    uint32_t wv[4][8];
 #pragma unroll
-                    for (int p = 0; p < 4; ++p) load_raw_part(raw, p, lane, wv[p]);
-                    wait_vector_loads();  // rare path: keeps the common path's waits exact
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) part(p, wv[p]);
-                } else {
-                    uint32_t pat[4][8];
-                    lookup_tile(lut, t.t, pat);
-                    patch_tile_escapes<kRowLayout>(pat, info, t.side, 0, lane);
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) {
-                        uint32_t wv[8];
-                        merge_chunk(pat[p], t.t.sm[p], wv);
-                        part(p, wv);
-                    }
-                }
+                for (int g = 0; g < BG; ++g) acc[g] += tile[g];
             }
-        } else if constexpr (RAW) {
+        };
+        // raw words: looked at one by one (FP32 x only)
+        auto raw_special = [&](const uint32_t (&wv)[4][8]) {
+            bool any = false;
+            if constexpr (XM == kXF32) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) any = any || pair_not_finite(wv[p][q]);
+            }
+            return wave_any(any);
+        };
+        if constexpr (RAW) {
             // block layout: each part's 16 columns are the A operands as loaded
+            uint32_t wv[4][8];
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
-                const uint32_t wv[8] = {t.r[p][0].x, t.r[p][0].y, t.r[p][0].z, t.r[p][0].w,
-                                        t.r[p][1].x, t.r[p][1].y, t.r[p][1].z, t.r[p][1].w};
-                mfma_block_part<BG>(wv, xb, p, lane, acc);
+                wv[p][0] = t.r[p][0].x; wv[p][1] = t.r[p][0].y; wv[p][2] = t.r[p][0].z; wv[p][3] = t.r[p][0].w;
+                wv[p][4] = t.r[p][1].x; wv[p][5] = t.r[p][1].y; wv[p][6] = t.r[p][1].z; wv[p][7] = t.r[p][1].w;
             }
+            mfma_tile(wv, raw_special(wv));
         } else {
             const uint32_t info = side_info(t.side, 0);
             if (info_is_fallback(info)) {
@@ -362,8 +423,7 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
 #pragma unroll
                 for (int p = 0; p < 4; ++p) raw_block_part(raw, p, lane, wv[p]);
                 wait_vector_loads();  // rare path: keeps the common path's waits exact
-#pragma unroll
-                for (int p = 0; p < 4; ++p) mfma_block_part<BG>(wv[p], xb, p, lane, acc);
+                mfma_tile(wv, raw_special(wv));
             } else {
                 // whole-line loads (4 tile rows per instruction) into the block
                 // layout, in place (the slot is reloaded next); each part's
@@ -379,8 +439,15 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
                     merge_chunk(pat, t.t.sm[p], wv[p]);
                 }
                 patch_tile_escapes<kBlockLayout>(wv, info, t.side, 0, lane);
-#pragma unroll
-                for (int p = 0; p < 4; ++p) mfma_block_part<BG>(wv[p], xb, p, lane, acc);
+                bool special = false;
+                if constexpr (XM == kXF32) {
+                    special = lut_special;
+                    if (info_escapes(info) != 0u) {
+                        const uint4 e = side_esc(t.side, 0);
+                        special = special || has_byte_ff(e.x) || has_byte_ff(e.y) || has_byte_ff(e.z) || has_byte_ff(e.w);
+                    }
+                }
+                mfma_tile(wv, special);
             }
         }
     };
@@ -391,15 +458,22 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
     // rings of three: tile i's streams are requested two steps before its
     // decode, x slab i's pieces two steps before they are stored to LDS
     // Tile streams and x pieces are requested D - 1 steps ahead of their
-    // use (D = 3; the GENERIC variants, whose element-wise loads are packed
-    // as they arrive, load and use in turn): under a full-bandwidth stream
+    // use (D = 3): under a full-bandwidth stream
     // even the L2 hits of x take about a step to return. The loop body holds
     // D steps so that every step's loads are issued on every path that goes
     // on (loads past the last tile reload it): a load skipped on some path
     // would make the compiler wait for all loads in flight. Slab i + 1 is
     // stored to LDS at the end of step i.
-    constexpr int D = GENERIC ? 1 : 3;
-    auto x_step = [&](int i) { return load_x_slab<GENERIC>(a, batch, kb, n, KG, i, tid, threads); };
+    auto x_step = [&](int i) { return load_x_slab<XM, PC>(a, batch, kb, n, KG, i, tid, threads); };
+    auto x_store = [&](char* to, const XPieces<PC>& xr, int i) {
+        store_x_slab<XM, PC>(a, to, slab_bytes, plane_bytes, xr, batch, kb, n, KG, i, tid, threads);
+    };
+    // FP32 x: exponent 255 in the pair table (each lane's 4 entries)
+    auto note_lut = [&]() {
+        if constexpr (XM == kXF32 && !RAW)
+            lut_special = wave_any(pair_not_finite(lutv.x) || pair_not_finite(lutv.y) || pair_not_finite(lutv.z) ||
+                                   pair_not_finite(lutv.w));
+    };
     auto has_tile = [&](int i) { return kg + KG * i < n; };
     if constexpr (M > 0) {
         // Slab ring: the slabs of step j sit in buffer j % NB (NB = 2 M);
@@ -418,20 +492,20 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
         GemmTile<RAW> t0, t1, t2;
         load_tile_i(t0, 0);
         load_tile_i(t1, 1);
-        XPieces xp[L];
+        XPieces<PC> xp[L];
 #pragma unroll
         for (int j = 0; j < L; ++j) xp[j] = x_step(j);
-        XPieces x0 = x_step(L), x1, x2;
+        XPieces<PC> x0 = x_step(L), x1, x2;
         if constexpr (!RAW) store_block_lut(lut, lutv, lane);
 #pragma unroll
-        for (int j = 0; j < L; ++j) store_x_slab(buf(j), slab_bytes, xp[j], batch, KG, tid, threads);
+        for (int j = 0; j < L; ++j) x_store(buf(j), xp[j], j);
         lds_barrier();  // the pair table and the slabs of steps 0 .. L - 1 are in LDS
-        auto step = [&](GemmTile<RAW>& cur, GemmTile<RAW>& ahead, const XPieces& x_next, XPieces& x_ahead, int i) {
+        auto step = [&](GemmTile<RAW>& cur, GemmTile<RAW>& ahead, const XPieces<PC>& x_next, XPieces<PC>& x_ahead, int i) {
             x_ahead = x_step(i + L + 1);
             load_tile_i(ahead, i + 2);
             if (i > 0 && i % M == 0) lds_barrier();
             if (has_tile(i)) use_tile(cur, i);  // an idle wave decodes row trl; its sums are dropped
-            store_x_slab(buf(i + L), slab_bytes, x_next, batch, KG, tid, threads);
+            x_store(buf(i + L), x_next, i + L);
         };
         int i = 0;
         while (true) {
@@ -442,22 +516,48 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
             step(t2, t1, x2, x0, i);
             if (++i >= steps) break;
         }
-    } else if constexpr (D == 3) {
+    } else if constexpr (XM != kXFast) {
+        // the edge-handling variants: tiles one step ahead (their x address
+        // and cut arithmetic leaves no registers for a third tile)
+        GemmTile<RAW> t0, t1;
+        load_tile_i(t0, 0);
+        XPieces<PC> x0 = x_step(0), x1 = x_step(1);
+        if constexpr (!RAW) store_block_lut(lut, lutv, lane);
+        note_lut();
+        x_store(xbuf, x0, 0);
+        lds_barrier();
+        auto step = [&](GemmTile<RAW>& cur, GemmTile<RAW>& ahead, const XPieces<PC>& x_next, XPieces<PC>& x_ahead, int i) {
+            load_tile_i(ahead, i + 1);
+            x_ahead = x_step(i + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            if (has_tile(i)) use_tile(cur, i);
+            __builtin_amdgcn_sched_barrier(0);
+            x_store(xbuf + ((i + 1) & 1) * KG * slab_bytes, x_next, i + 1);
+            lds_barrier();
+        };
+        int i = 0;
+        while (true) {
+            step(t0, t1, x1, x0, i);
+            if (++i >= steps) break;
+            step(t1, t0, x0, x1, i);
+            if (++i >= steps) break;
+        }
+    } else {
         GemmTile<RAW> t0, t1, t2;
         load_tile_i(t0, 0);
-        XPieces x0 = x_step(0);
+        XPieces<PC> x0 = x_step(0);
         load_tile_i(t1, 1);
-        XPieces x1 = x_step(1);
-        XPieces x2;
+        XPieces<PC> x1 = x_step(1);
+        XPieces<PC> x2;
         if constexpr (!RAW) store_block_lut(lut, lutv, lane);
-        store_x_slab(xbuf, slab_bytes, x0, batch, KG, tid, threads);
+        x_store(xbuf, x0, 0);
         lds_barrier();
-        auto step = [&](GemmTile<RAW>& cur, GemmTile<RAW>& ahead, const XPieces& x_next, XPieces& x_ahead,
+        auto step = [&](GemmTile<RAW>& cur, GemmTile<RAW>& ahead, const XPieces<PC>& x_next, XPieces<PC>& x_ahead,
                         int i) {
             x_ahead = x_step(i + 2);
             load_tile_i(ahead, i + 2);
             if (has_tile(i)) use_tile(cur, i);  // an idle wave decodes row trl; its sums are dropped
-            store_x_slab(xbuf + ((i + 1) & 1) * KG * slab_bytes, slab_bytes, x_next, batch, KG, tid, threads);
+            x_store(xbuf + ((i + 1) & 1) * KG * slab_bytes, x_next, i + 1);
             lds_barrier();
         };
         // the loop leaves after the last step (not after a group of three):
@@ -471,19 +571,10 @@ __global__ __launch_bounds__(GENERIC ? kGemmMaxThreadsGeneric : kGemmMaxThreads)
             step(t2, t1, x0, x1, i);
             if (++i >= steps) break;
         }
-    } else {
-        GemmTile<RAW> t0;
-        XPieces xr = x_step(0);
-        if constexpr (!RAW) store_block_lut(lut, lutv, lane);
-        store_x_slab(xbuf, slab_bytes, xr, batch, KG, tid, threads);
-        lds_barrier();
-        for (int i = 0; i < steps; ++i) {
-            xr = x_step(i + 1);
-            load_tile_i(t0, i);
-            if (has_tile(i)) use_tile(t0, i);
-            store_x_slab(xbuf + ((i + 1) & 1) * KG * slab_bytes, slab_bytes, xr, batch, KG, tid, threads);
-            lds_barrier();
-        }
+    }
+    if constexpr (XM == kXF32) {
+#pragma unroll
+        for (int g = 0; g < BG; ++g) acc[g] += low[g];
     }
     // the K groups of a tile row: groups 1..KG-1 hand their sums to group 0
     // through LDS (the x slabs are no longer read: every wave passed the
@@ -577,28 +668,35 @@ namespace {
 template <int BG, bool RAW>
 hipError_t gemm_b(const GemvGroupArgs& a, int batch, const GemvPlan& p, hipStream_t stream) {
     const dim3 grid(group_grid_x(a), a.m[0].S, a.count), block(p.waves * 64);
-    if (p.generic)
-        hipLaunchKernelGGL((gemm_kernel<BG, RAW, true, 0>), grid, block, p.lds, stream, a, batch);
+    const int pieces = (batch * x_row_pieces(kXF32) + p.waves * 64 - 1) / (p.waves * 64);   // FP32 x: per thread and step
+    if (p.xf32 && BG == 1 && pieces <= 1)
+        hipLaunchKernelGGL((gemm_kernel<1, RAW, kXF32, 0, 1>), grid, block, p.lds, stream, a, batch);
+    else if (p.xf32 && BG == 1 && pieces <= 2)
+        hipLaunchKernelGGL((gemm_kernel<1, RAW, kXF32, 0, 2>), grid, block, p.lds, stream, a, batch);
+    else if (p.xf32)
+        hipLaunchKernelGGL((gemm_kernel<BG, RAW, kXF32, 0>), grid, block, p.lds, stream, a, batch);
+    else if (p.generic)
+        hipLaunchKernelGGL((gemm_kernel<BG, RAW, kXEdge, 0>), grid, block, p.lds, stream, a, batch);
     else if (p.slab_ring == kGemmSlabRing)
-        hipLaunchKernelGGL((gemm_kernel<BG, RAW, false, kGemmSlabRing>), grid, block, p.lds, stream, a, batch);
+        hipLaunchKernelGGL((gemm_kernel<BG, RAW, kXFast, kGemmSlabRing>), grid, block, p.lds, stream, a, batch);
     else
-        hipLaunchKernelGGL((gemm_kernel<BG, RAW, false, 0>), grid, block, p.lds, stream, a, batch);
+        hipLaunchKernelGGL((gemm_kernel<BG, RAW, kXFast, 0>), grid, block, p.lds, stream, a, batch);
     return hipGetLastError();
 }
 
 }  // namespace
 
-size_t gemm_lds_bytes(int waves, int batch, int slab_ring) {
-    const int bg = batch > 16 ? 2 : 1;
-    const int rows = gemm_min_waves(batch), kgroups = std::max(1, waves / rows);
+size_t gemm_lds_bytes(int waves, int batch, int slab_ring, bool xf32) {
+    const int bg = batch > 16 ? 2 : 1, planes = x_planes(xf32 ? kXF32 : kXFast);
+    const int rows = gemm_min_waves(batch, xf32), kgroups = std::max(1, waves / rows);
     const size_t sums = (size_t)(kgroups - 1) * rows * 64 * bg * 4 * sizeof(float);
     if (slab_ring > 0) return (size_t)2 * slab_ring * kgroups * 16 * bg * kRowBytes + sums;
-    const size_t slabs = (size_t)2 * kgroups * 16 * bg * kRowBytes;
+    const size_t slabs = (size_t)2 * kgroups * planes * 16 * bg * kRowBytes;
     return std::max(slabs, sums);
 }
 
 hipError_t launch_gemm(const GemvGroupArgs& a, int batch, const GemvPlan& p, hipStream_t stream) {
-    const int rows = gemm_min_waves(batch);
+    const int rows = gemm_min_waves(batch, p.xf32);
     if (batch < 1 || batch > 32 || p.waves % rows != 0 || a.rows_per_block != rows) return hipErrorInvalidValue;
     if (batch > 16) return p.raw ? gemm_b<2, true>(a, batch, p, stream) : gemm_b<2, false>(a, batch, p, stream);
     return p.raw ? gemm_b<1, true>(a, batch, p, stream) : gemm_b<1, false>(a, batch, p, stream);

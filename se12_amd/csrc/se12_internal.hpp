@@ -220,8 +220,8 @@ hipError_t launch_row_sumsq(const float* y, int64_t N, int32_t TR, int32_t batch
 // units.
 constexpr int kGemmMinBatch = 5;
 constexpr int kGemmMaxThreads = 512;
-// the edge-handling (GENERIC) MFMA variants, whose element-wise loads need
-// more registers, take at most 4 waves per block (enough for 32 batch rows)
+// launches of BF16 x in part K tiles or of any alignment take at most 4 waves
+// per block (enough for 32 batch rows)
 constexpr int kGemmMaxThreadsGeneric = 256;
 
 constexpr int kGemmMaxSplits = 16;
@@ -230,10 +230,15 @@ constexpr int kGemmXPieces = 4;
 // slab (batch / 8, rounded up), rounded up to a power of two (3 waves leave a
 // SIMD of the CU without a row: 14336x3584 at B = 24 took 32.4 us with 3,
 // B = 32 26.2 with 4)
-constexpr int gemm_min_waves(int batch) {
-    return (batch * 32 + 64 * kGemmXPieces - 1) / (64 * kGemmXPieces) == 3 ? 4
-                                                                            : (batch * 32 + 64 * kGemmXPieces - 1) /
-                                                                                  (64 * kGemmXPieces);
+// FP32 x: 4 rows share each conversion to planes (8 rows where 32 batch rows
+// need their threads): 3584x14336, 8 batch rows, 28.3 us with 4, 30.9 with 8,
+// 43 with 2; 2304x9216 18.4 / 21.8 / 25.0
+constexpr int gemm_min_waves(int batch, bool xf32 = false) {
+    if (xf32) return batch > 16 ? 8 : 4;
+    const int fewest = (batch * 32 + 64 * kGemmXPieces - 1) / (64 * kGemmXPieces);
+    int waves = 1;
+    while (waves < fewest) waves *= 2;
+    return waves;
 }
 // The FAST variants' x slabs on launches of kGemmSlabRingMinSteps or more
 // steps, where LDS allows: a ring of 2 M buffers per K group (M =
@@ -246,7 +251,7 @@ constexpr int gemm_min_waves(int batch) {
 // / 32 78.4 / 81.5 us against 76.3 / 79.8).
 constexpr int kGemmSlabRing = 4;
 constexpr int kGemmSlabRingMinSteps = 12;
-size_t gemm_lds_bytes(int waves, int batch, int slab_ring);
+size_t gemm_lds_bytes(int waves, int batch, int slab_ring, bool xf32);
 hipError_t launch_gemm(const GemvGroupArgs& a, int batch, const GemvPlan& p, hipStream_t stream);
 
 // Resident-x batched path (se12_gemm_rx.hip): BF16 x with up to 32 rows on

@@ -117,6 +117,100 @@ def test_float32_activations_through_the_pair_tree(gpu, batch):
     assert max_rel_error(y1, o.gemv_reference(enc, xf)) <= REL_TOL
 
 
+# The MFMA variants that read x 16 bytes at a time at any address: K below, at and above a piece (8 BF16 or 4 FP32
+# columns), a tile and a tile's part, batches at the edges of the 16-row groups and of the rows per block; x so small
+# that it holds no piece (the dot2 kernel takes it)
+EDGE_SHAPES = [(1, 1), (5, 2), (16, 3), (33, 7), (33, 8), (17, 9), (48, 255), (40, 256), (70, 257), (100, 300), (129, 511),
+               (300, 2887), (64, 4099)]
+
+
+def _edge_check(y, w, x):
+    """|y - y64| against FP32 sums of K products: (K + 16) 2^-23 sum |w x| (products exact or one rounding each, K
+    additions in any order)."""
+    w64, x64 = w.double(), x.double()
+    ref = x64 @ w64.t().contiguous()
+    bound = (w.shape[1] + 16) * 2.0 ** -23 * (x64.abs() @ w64.abs().t().contiguous())
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", EDGE_SHAPES)
+def test_edge_handling_mfma_products(gpu, rows, cols, dtype):
+    """Batches 5..32 over part tiles, x at an odd offset of its buffer (BF16: 2-byte aligned; FP32: 4-byte) with huge
+    values around it (nothing of them may reach a result), the raw twin bit-identical."""
+    from se12_amd.hip import RawBf16MatVecKernel, Se12MatVecKernel, encode_on_device
+
+    g = torch.Generator(device=gpu)
+    g.manual_seed(rows * 31 + cols)
+    w = (torch.randn((rows, cols), generator=g, device=gpu) * 0.02).to(torch.bfloat16)
+    k, r = Se12MatVecKernel(encode_on_device(w)), RawBf16MatVecKernel(w)
+    for batch in (5, 6, 8, 9, 16, 17, 24, 32):
+        buf = torch.full((batch * cols + 40,), float("inf"), device=gpu, dtype=dtype)
+        x = buf[17:17 + batch * cols].view(batch, cols)
+        x.copy_(torch.randn((batch, cols), generator=g, device=gpu))
+        y = k.multiply(x)
+        _edge_check(y, w, x)
+        assert torch.equal(y, r.multiply(x)), batch
+        assert torch.equal(y, k.multiply(x)), batch
+
+
+@pytest.mark.parametrize("batch", [5, 16, 32])
+def test_float32_activations_keep_infinities_and_nans(gpu, batch):
+    """FP32 x through the three BF16 planes: infinities and NaNs of W and x give what FP32 products give (an infinite
+    weight times a value whose lower planes are zero stays infinite), values near FP32's largest do not overflow, and
+    neither format of W differs."""
+    from se12_amd.hip import RawBf16MatVecKernel, Se12MatVecKernel, encode_on_device
+
+    rows, cols = 96, 700
+    g = torch.Generator(device=gpu)
+    g.manual_seed(batch)
+    w = (torch.randn((rows, cols), generator=g, device=gpu) * 0.02).to(torch.bfloat16)
+    w[3, 5], w[20, 699], w[37, 256], w[50, 80] = float("inf"), float("-inf"), float("nan"), float("inf")
+    w[50, 81] = float("-inf")
+    w[64:80, :256] = float("inf")                        # more escapes than slots: a raw tile
+    w[80:96] = w[80:96].abs() * 2.0 ** -20
+    x = torch.randn((batch, cols), generator=g, device=gpu)
+    x[:, 5] = 1.0                                        # lower planes zero
+    x[0, 699] = 2.0 ** -3
+    x[1, 10], x[2, 11] = float("inf"), float("nan")
+    x[3] = 3.0e38                                        # rounds up to infinity in BF16
+    k, r = Se12MatVecKernel(encode_on_device(w)), RawBf16MatVecKernel(w)
+    y = k.multiply(x)
+    assert torch.equal(y.isnan(), r.multiply(x).isnan()) and torch.equal(y.nan_to_num(), r.multiply(x).nan_to_num())
+    terms = x.double().cpu()[:, None, :] * w.double().cpu()[None, :, :]
+    pos, neg, nan = (terms == float("inf")).any(-1), (terms == float("-inf")).any(-1), terms.isnan().any(-1)
+    want_nan = nan | (pos & neg)
+    y = y.cpu()
+    assert torch.equal(y.isnan(), want_nan)
+    assert bool((y[pos & ~want_nan] == float("inf")).all()) and bool((y[neg & ~want_nan] == float("-inf")).all())
+    fine = ~(pos | neg | nan)
+    ref, bound = terms.nan_to_num().sum(-1), (cols + 16) * 2.0 ** -23 * terms.nan_to_num().abs().sum(-1)
+    small = fine & (bound < 1e30) | fine & (torch.arange(rows) >= 80)[None, :]
+    assert bool(((y.double() - ref).abs()[small] <= bound[small]).all()) and int(small.sum()) > 60 * (batch - 3)
+
+
+def test_float32_activations_grouped_and_without_allocation(gpu):
+    """The FP32 MFMA path under a grouped launch and in the static scratch: the results of single calls."""
+    from se12_amd.hip import Se12MatVecKernel, encode_on_device, multiply_grouped
+
+    g = torch.Generator(device=gpu)
+    g.manual_seed(3)
+    ws = [(torch.randn((n, 2304), generator=g, device=gpu) * 0.02).to(torch.bfloat16) for n in (2048, 1024, 1000)]
+    ks = [Se12MatVecKernel(encode_on_device(w)) for w in ws]
+    x = torch.randn((9, 2304), generator=g, device=gpu)
+    for w, k, y in zip(ws, ks, multiply_grouped(ks, x)):
+        _edge_check(y, w, x)
+        out = torch.empty((9, k.rows), device=gpu)
+        assert torch.equal(k.multiply_noalloc(x, out), k.multiply(x))
+    # splits x 32 rows x 40,960 rows of partial sums are cut to what the scratch holds
+    w = (torch.randn((40960, 1024), generator=g, device=gpu) * 0.02).to(torch.bfloat16)
+    k = Se12MatVecKernel(encode_on_device(w))
+    x = torch.randn((32, 1024), generator=g, device=gpu)
+    out = torch.empty((32, 40960), device=gpu)
+    k.multiply_noalloc(x, out)
+    _edge_check(out, w, x)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (17, 257), (33, 300), (100, 2304), (2048, 2304), (64, 9216)])
 def test_gemv_ragged_and_escape_heavy(gpu, rows, cols):
     from se12_amd.hip import Se12MatVecKernel
