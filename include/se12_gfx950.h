@@ -324,6 +324,27 @@ int se12_encode(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld,
                 const uint8_t codebook[15], const se12_streams_out* out, int64_t* fallback_tiles_out,
                 void* stream);
 
+/* The whole encoder in one call: histogram, codebook, sm / ec / esc and the
+ * fallback bitmap of w, without a round trip to the host in between. Writes the
+ * streams of `out` except fallback_raw (out->fallback_raw_* may be NULL / 0),
+ * the codebook to codebook_dev[15] (device) and codebook_out (host) and the
+ * number of fallback tiles; the caller then gives se12_encode_fallback a buffer
+ * of that many tiles. `workspace`: device memory of se12_encode_workspace()
+ * bytes, 16-byte aligned, contents indifferent. Synchronizes `stream` (the count
+ * and the codebook are results). Same bytes as se12_encode_prepare +
+ * se12_encode, which allocate their own scratch and read w twice more. */
+int64_t se12_encode_workspace(void);
+int se12_encode_streams(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld, const se12_streams_out* out,
+                        uint8_t* codebook_dev, uint8_t codebook_out[15], int64_t* fallback_tiles_out, void* workspace,
+                        int64_t workspace_bytes, void* stream);
+
+/* The raw bits of the tiles that fallback_bitmap_dev marks, in tile order, to
+ * fallback_raw_dev [fallback_raw_tiles * 4096] (tiles past its capacity are
+ * left out). Asynchronous on `stream`. */
+int se12_encode_fallback(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld,
+                         const uint8_t* fallback_bitmap_dev, int16_t* fallback_raw_dev, int64_t fallback_raw_tiles,
+                         void* stream);
+
 #ifdef __cplusplus
 }
 #endif

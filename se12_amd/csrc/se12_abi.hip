@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -1302,55 +1303,10 @@ static int encode_args(EncodeArgs& a, const uint16_t* w, int64_t rows, int64_t c
     a.TR = (int32_t)ceil_div(rows, SE12_TILE_ROWS);
     a.TC = (int32_t)ceil_div(cols, SE12_TILE_COLS);
     a.T = (int64_t)a.TR * a.TC;
-    a.w_vec_ok = (aligned16(w) && ld % 8 == 0) ? 1 : 0;
     return SE12_OK;
 }
 
-static void pack_codebook(EncodeArgs& a, const uint8_t cb[15]) {
-    uint8_t b[16] = {0};
-    std::memcpy(b, cb, 15);
-    std::memcpy(a.codebook, b, 16);
-}
-
-int se12_encode_prepare(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, uint8_t codebook_out[15],
-                        int64_t* fallback_tiles_out, void* stream) {
-    if (!codebook_out || !fallback_tiles_out) return fail(SE12_E_INVALID, "se12_encode_prepare: NULL output");
-    EncodeArgs a;
-    if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    uint64_t* hist = nullptr;
-    int32_t* counts = nullptr;
-    SE12_HIP(hipMalloc(&hist, 256 * sizeof(uint64_t)));
-    hipError_t e = hipMalloc(&counts, (size_t)a.T * sizeof(int32_t));
-    uint64_t hh[256];
-    std::vector<int32_t> ch((size_t)a.T);
-    if (e == hipSuccess) e = hipMemsetAsync(hist, 0, 256 * sizeof(uint64_t), st);
-    a.histogram = hist;
-    a.tile_escapes = counts;
-    if (e == hipSuccess) e = launch_encode_histogram(a, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(hh, hist, sizeof hh, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess) {
-        se12_codebook_from_histogram(hh, codebook_out);
-        pack_codebook(a, codebook_out);
-        e = launch_encode_count(a, st);
-    }
-    if (e == hipSuccess) e = hipMemcpyAsync(ch.data(), counts, (size_t)a.T * sizeof(int32_t), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    (void)hipFree(hist);
-    if (counts) (void)hipFree(counts);
-    if (e != hipSuccess) return fail(SE12_E_HIP, "se12_encode_prepare: %s", hipGetErrorString(e));
-    int64_t nfb = 0;
-    for (int32_t c : ch) nfb += c > SE12_ESCAPE_BUDGET ? 1 : 0;
-    *fallback_tiles_out = nfb;
-    return SE12_OK;
-}
-
-int se12_encode(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, const uint8_t codebook[15],
-                const se12_streams_out* out, int64_t* fallback_tiles_out, void* stream) {
-    if (!codebook || !out) return fail(SE12_E_INVALID, "se12_encode: NULL argument");
-    EncodeArgs a;
-    if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
+static int encode_streams_args(EncodeArgs& a, const se12_streams_out* out) {
     if (!out->sm_dev || !out->ec_dev || !out->esc_dev || !out->fallback_bitmap_dev)
         return fail(SE12_E_INVALID, "se12_encode: a required output stream is NULL");
     if (!aligned16(out->sm_dev) || !aligned16(out->ec_dev) ||
@@ -1359,27 +1315,111 @@ int se12_encode(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, const
     if (out->fallback_raw_tiles < 0) return fail(SE12_E_INVALID, "se12_encode: negative fallback capacity");
     if (out->fallback_raw_tiles > 0 && !out->fallback_raw_dev)
         return fail(SE12_E_INVALID, "se12_encode: fallback_raw is NULL but has capacity");
-    pack_codebook(a, codebook);
     a.sm = out->sm_dev;
     a.ec = out->ec_dev;
     a.esc = out->esc_dev;
     a.bitmap = out->fallback_bitmap_dev;
     a.raw = out->fallback_raw_dev;
+    a.raw_tiles = out->fallback_raw_tiles;
+    return SE12_OK;
+}
+
+static int compute_units(int* cus) {
+    int dev = 0;
+    SE12_HIP(hipGetDevice(&dev));
+    SE12_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return SE12_OK;
+}
+
+namespace {
+// what the host reads of an EncodeWork, in one copy
+struct EncodeResult {
+    uint8_t codebook[16];
+    unsigned long long fallback_tiles;
+};
+static_assert(offsetof(EncodeWork, fallback_tiles) == offsetof(EncodeWork, codebook) + offsetof(EncodeResult, fallback_tiles),
+              "EncodeResult mirrors EncodeWork");
+hipError_t read_result(EncodeResult* r, const EncodeWork* ws, hipStream_t st) {
+    hipError_t e = hipMemcpyAsync(r, ws->codebook, sizeof *r, hipMemcpyDeviceToHost, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+}
+}  // namespace
+
+int64_t se12_encode_workspace(void) { return (int64_t)sizeof(EncodeWork); }
+
+int se12_encode_streams(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, const se12_streams_out* out,
+                        uint8_t* codebook_dev, uint8_t codebook_out[15], int64_t* fallback_tiles_out, void* workspace,
+                        int64_t workspace_bytes, void* stream) {
+    if (!out || !codebook_dev || !codebook_out || !fallback_tiles_out || !workspace)
+        return fail(SE12_E_INVALID, "se12_encode_streams: NULL argument");
+    if (workspace_bytes < (int64_t)sizeof(EncodeWork) || !aligned16(workspace))
+        return fail(SE12_E_CAPACITY, "se12_encode_streams: needs a 16-byte aligned workspace of %zu bytes", sizeof(EncodeWork));
+    EncodeArgs a;
+    if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
+    if (int rc = encode_streams_args(a, out)) return rc;
+    int cus = 0;
+    if (int rc = compute_units(&cus)) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    int32_t* counts = nullptr;
-    int32_t* rank = nullptr;
-    int64_t* totals = nullptr;
-    int64_t total = 0;
-    hipError_t e = hipMalloc(&counts, (size_t)a.T * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&rank, (size_t)a.T * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&totals, sizeof(int64_t));
-    a.tile_escapes = counts;
-    a.fb_rank = rank;
-    a.totals = totals;
-    if (e == hipSuccess) e = launch_encode_count(a, st);
-    if (e == hipSuccess) e = launch_encode_scan(a, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(&total, totals, sizeof total, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    a.ws = static_cast<EncodeWork*>(workspace);
+    EncodeResult r;
+    SE12_HIP(launch_encode_histogram(a, cus, codebook_dev, st));
+    SE12_HIP(launch_encode_tiles(a, true, st));
+    SE12_HIP(read_result(&r, a.ws, st));
+    std::memcpy(codebook_out, r.codebook, SE12_CODEBOOK_SIZE);
+    *fallback_tiles_out = (int64_t)r.fallback_tiles;
+    return SE12_OK;
+}
+
+int se12_encode_fallback(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, const uint8_t* fallback_bitmap_dev,
+                         int16_t* fallback_raw_dev, int64_t fallback_raw_tiles, void* stream) {
+    EncodeArgs a;
+    if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
+    if (fallback_raw_tiles == 0) return SE12_OK;
+    if (!fallback_bitmap_dev || !fallback_raw_dev || fallback_raw_tiles < 0 || !aligned16(fallback_raw_dev))
+        return fail(SE12_E_INVALID, "se12_encode_fallback: needs the bitmap and a 16-byte aligned output");
+    a.bitmap = const_cast<uint8_t*>(fallback_bitmap_dev);
+    a.raw = fallback_raw_dev;
+    a.raw_tiles = fallback_raw_tiles;
+    SE12_HIP(launch_encode_raw(a, static_cast<hipStream_t>(stream)));
+    return SE12_OK;
+}
+
+int se12_encode_prepare(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, uint8_t codebook_out[15],
+                        int64_t* fallback_tiles_out, void* stream) {
+    if (!codebook_out || !fallback_tiles_out) return fail(SE12_E_INVALID, "se12_encode_prepare: NULL output");
+    EncodeArgs a;
+    if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
+    int cus = 0;
+    if (int rc = compute_units(&cus)) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    SE12_HIP(hipMalloc(&a.ws, sizeof(EncodeWork)));
+    EncodeResult r;
+    hipError_t e = launch_encode_histogram(a, cus, nullptr, st);
+    if (e == hipSuccess) e = launch_encode_tiles(a, false, st);
+    if (e == hipSuccess) e = read_result(&r, a.ws, st);
+    (void)hipFree(a.ws);
+    if (e != hipSuccess) return fail(SE12_E_HIP, "se12_encode_prepare: %s", hipGetErrorString(e));
+    std::memcpy(codebook_out, r.codebook, SE12_CODEBOOK_SIZE);
+    *fallback_tiles_out = (int64_t)r.fallback_tiles;
+    return SE12_OK;
+}
+
+int se12_encode(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, const uint8_t codebook[15],
+                const se12_streams_out* out, int64_t* fallback_tiles_out, void* stream) {
+    if (!codebook || !out) return fail(SE12_E_INVALID, "se12_encode: NULL argument");
+    EncodeArgs a;
+    if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
+    if (int rc = encode_streams_args(a, out)) return rc;
+    uint8_t cb[16] = {0};
+    std::memcpy(cb, codebook, SE12_CODEBOOK_SIZE);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    SE12_HIP(hipMalloc(&a.ws, sizeof(EncodeWork)));
+    EncodeResult r{};
+    // counted before anything is written
+    hipError_t e = launch_encode_codes(a, cb, st);
+    if (e == hipSuccess) e = launch_encode_tiles(a, false, st);
+    if (e == hipSuccess) e = read_result(&r, a.ws, st);
+    const int64_t total = (int64_t)r.fallback_tiles;
     int rc = SE12_OK;
     if (e != hipSuccess) {
         rc = fail(SE12_E_HIP, "se12_encode: %s", hipGetErrorString(e));
@@ -1387,14 +1427,13 @@ int se12_encode(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, const
         rc = fail(SE12_E_CAPACITY, "se12_encode: %lld fallback tiles, fallback_raw holds %lld", (long long)total,
                   (long long)out->fallback_raw_tiles);
     } else {
-        e = launch_encode_write(a, st);
+        e = launch_encode_tiles(a, true, st);
+        if (e == hipSuccess && total > 0) e = launch_encode_raw(a, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) rc = fail(SE12_E_HIP, "se12_encode write: %s", hipGetErrorString(e));
     }
     if (fallback_tiles_out) *fallback_tiles_out = total;
-    if (counts) (void)hipFree(counts);
-    if (rank) (void)hipFree(rank);
-    if (totals) (void)hipFree(totals);
+    (void)hipFree(a.ws);
     return rc;
 }
 

@@ -114,6 +114,24 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
     return v;
 }
 
+// The rank of fallback tile `tile` (the set bits before it in the MSB-first
+// bitmap), counted by a whole wave: 8 bytes per lane and step.
+__device__ __forceinline__ int64_t fallback_rank(const uint8_t* bitmap, int64_t tile, uint32_t lane) {
+    const int64_t bytes = tile >> 3;
+    uint32_t n = 0;
+    for (int64_t b = 8 * (int64_t)lane; b < bytes; b += 8 * kWave) {
+        if (b + 8 <= bytes) {
+            uint64_t v;
+            __builtin_memcpy(&v, bitmap + b, sizeof v);
+            n += __popcll(v);
+        } else {
+            for (int64_t i = b; i < bytes; ++i) n += __popc((uint32_t)bitmap[i]);
+        }
+    }
+    const uint32_t total = __builtin_amdgcn_readlane(wave_incl_scan(n), kWave - 1);
+    return (int64_t)total + __popc((uint32_t)bitmap[bytes] >> (8 - (tile & 7)));
+}
+
 // LDS barrier that does not wait for outstanding global loads (a plain
 // __syncthreads would also drain vmcnt and kill the prefetch).
 __device__ __forceinline__ void lds_barrier() {

@@ -1,61 +1,177 @@
 // SE12 encoder on the GPU, byte-identical to the reference encoder
 // lws/domain/se12/codec.py:111-141 (which runs numpy on the host at pack time,
-// lws/application/codec/pack_model.py:113-120). Four kernels:
-//   histogram  - 256-bin exponent histogram over the real weights
-//                (the host then picks the codebook, codebook.py:41-59)
-//   count      - escapes per tile (weights whose exponent is not in the
-//                codebook; padding never escapes, codec.py:119-125)
-//   scan       - fallback flag (count > 16, codec.py:132-133), rank among
-//                fallback tiles, MSB-first bitmap (codec.py:351-353)
-//   write      - sm / ec / esc / fallback_raw, one wave per tile with the same
-//                lane mapping as the decoder: escapes take slots in tile-local
-//                row-major order (codec.py:131,332-343); fallback tiles keep
-//                their padded bits raw (codec.py:363-365) and zero esc slots.
+// lws/application/codec/pack_model.py:113-120). Kernels:
+//   histogram  - 256-bin exponent histogram over the real weights, one partial
+//                histogram per block
+//   select     - the histogram, and from it the codebook (codebook.py:41-59)
+//                and the code of every exponent value, on the device, so that
+//                the next kernel follows without a round trip to the host
+//   tiles      - sm / ec / esc of every tile, one wave per tile with the same
+//                lane mapping as the decoder: escapes (weights whose exponent
+//                is not in the codebook; padding never escapes, codec.py:
+//                119-125) take slots in tile-local row-major order (codec.py:
+//                131,332-343); the fallback bitmap (more than 16 escapes,
+//                MSB first, codec.py:132-133,351-353) and its count. Fallback
+//                tiles have zero esc slots.
+//   raw        - the fallback tiles' padded bits (codec.py:363-365), ranked by
+//                the bitmap: launched only where there are any.
+//
+// Bound by the weights' bytes: read once for the histogram, once (from the
+// last-level cache where they fit) for the streams.
+// 9216x2304 as the packer's call issues it 253 -> 73 us (histogram 78 -> 10.2:
+// it read 2 bytes per load, divided 64-bit indexes and queued on shared LDS
+// counters; select 7.2; tiles 17.2 + 2 x 11 of counting + 9.4 of scanning ->
+// 19; the rest is the call's one synchronisation, was 4, and its allocations);
+// 256000x2304 2,024 -> 626 us, 5.2 TB/s of weights read twice and streams.
+#include <algorithm>
+
 #include "se12_device.hpp"
 #include "se12_internal.hpp"
 
 namespace se12 {
 
-constexpr int kEncWaves = 4;
-constexpr int kHistThreads = 256;
+constexpr int kTilesThreads = 512;                     // 8 waves: one bitmap byte per block
+constexpr int kHistThreads = 1024;
+constexpr int kHistCopies = 32;                        // per bin, by lane: no LDS bank conflicts
+constexpr int kBins = 256;
 
-__device__ __forceinline__ uint32_t cb_byte(const EncodeArgs& a, int i) {
-    return (a.codebook[i >> 2] >> (8 * (i & 3))) & 0xFFu;
+// Adds the exponents of two BF16 weights: the bin's row of copies is at byte
+// (exponent << 7), which is where the exponent sits in the low half.
+__device__ __forceinline__ void count_pair(uint32_t v, char* mine) {
+    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(mine + (v & 0x7F80u)), 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(mine + ((v >> 16) & 0x7F80u)), 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// code of each exponent value (15 = escape)
-__device__ __forceinline__ void build_code_lut(uint8_t* code_of, const EncodeArgs& a, int tid, int nthreads) {
-    for (int e = tid; e < 256; e += nthreads) {
-        uint32_t c = 15;
-        for (int i = kCodebook - 1; i >= 0; --i)
-            if (cb_byte(a, i) == (uint32_t)e) c = i;
-        code_of[e] = (uint8_t)c;
-    }
-}
-
+// Each lane counts in its own copy of the bins (lane % 32, the copies of a bin
+// side by side): weights share a handful of exponents, so lanes adding to one
+// counter would queue. 16 bytes per load; a matrix whose rows follow each
+// other without gaps is read as one row.
 __global__ __launch_bounds__(kHistThreads) void encode_histogram_kernel(EncodeArgs a) {
-    __shared__ uint32_t hist[256];
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) hist[i] = 0;
+    static_assert(kHistCopies * sizeof(uint32_t) == 128, "a bin's copies span 1 << 7 bytes");
+    __shared__ __attribute__((aligned(16))) uint32_t hist[kBins * kHistCopies];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < kBins * kHistCopies / 4; i += kHistThreads)
+        reinterpret_cast<uint4*>(hist)[i] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
-    const int64_t total = a.N * a.K;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-         idx += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t row = idx / a.K;
-        const int64_t col = idx - row * a.K;
-        const uint32_t v = a.w[row * a.ld + col];
-        atomicAdd(&hist[(v >> 7) & 0xFFu], 1u);
+    char* mine = reinterpret_cast<char*>(hist) + 4 * (tid & (kHistCopies - 1));
+    const bool flat = a.ld == a.K;
+    const int64_t rows = flat ? 1 : a.N, cols = flat ? a.N * a.K : a.K;
+    // blocks along a row, then over the rows
+    const int64_t row_blocks = std::min<int64_t>((cols + 8 * kHistThreads - 1) / (8 * kHistThreads), gridDim.x);
+    const int64_t lanes = row_blocks * kHistThreads, block = blockIdx.x % row_blocks;
+    const int64_t row_step = gridDim.x / row_blocks;
+    for (int64_t r = blockIdx.x / row_blocks; r < rows && blockIdx.x < row_step * row_blocks; r += row_step) {
+        const uint16_t* p = a.w + r * a.ld;
+        const int64_t whole = cols / 8;
+        int64_t c = block * kHistThreads + tid;
+        // four loads in flight
+        for (; c + 3 * lanes < whole; c += 4 * lanes) {
+            uint4 v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = load16_unaligned(p + 8 * (c + k * lanes));
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                count_pair(v[k].x, mine);
+                count_pair(v[k].y, mine);
+                count_pair(v[k].z, mine);
+                count_pair(v[k].w, mine);
+            }
+        }
+        for (; c < whole; c += lanes) {
+            const uint4 v = load16_unaligned(p + 8 * c);
+            count_pair(v.x, mine);
+            count_pair(v.y, mine);
+            count_pair(v.z, mine);
+            count_pair(v.w, mine);
+        }
+        if (block == 0 && tid < cols - 8 * whole)
+            __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(mine + (p[8 * whole + tid] & 0x7F80u)), 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 256; i += blockDim.x)
-        if (hist[i]) atomicAdd(reinterpret_cast<unsigned long long*>(&a.histogram[i]), (unsigned long long)hist[i]);
+    if (tid < kBins) {
+        uint32_t n = 0;
+#pragma unroll
+        for (int k = 0; k < kHistCopies; ++k) n += hist[tid * kHistCopies + ((tid + k) & (kHistCopies - 1))];
+        a.ws->partial[(int64_t)blockIdx.x * kBins + tid] = n;
+    }
+}
+
+// One block: the partial histograms' sum, each exponent's rank (more weights
+// first, the larger exponent on a tie: the order of se12_codebook_from_
+// histogram), and from it the codebook and the codes (15 = escape).
+__global__ __launch_bounds__(kHistThreads) void encode_select_kernel(EncodeWork* ws, int blocks, uint8_t* codebook_out) {
+    __shared__ uint64_t part[kHistThreads];
+    __shared__ __attribute__((aligned(16))) uint64_t key[kBins];   // count << 8 | exponent
+    const int tid = threadIdx.x, e = tid & (kBins - 1), s = tid / kBins;
+    constexpr int kSlices = kHistThreads / kBins, kFlight = 32;
+    uint64_t n = 0;
+    // one block waits for its loads alone: many in flight (7.2 us with 32 and
+    // the one-key ranks below, 20.6 with 16 and two-field ranks)
+    for (int b0 = s; b0 < blocks; b0 += kSlices * kFlight) {
+        uint32_t v[kFlight];
+#pragma unroll
+        for (int k = 0; k < kFlight; ++k) {
+            const int b = b0 + k * kSlices;
+            v[k] = ws->partial[(int64_t)(b < blocks ? b : s) * kBins + e];
+        }
+#pragma unroll
+        for (int k = 0; k < kFlight; ++k) n += b0 + k * kSlices < blocks ? v[k] : 0u;
+    }
+    part[tid] = n;
+    __syncthreads();
+    if (tid < kBins) {
+#pragma unroll
+        for (int k = 1; k < kSlices; ++k) n += part[tid + k * kBins];
+        key[tid] = (n << 8) | (uint64_t)tid;
+        ws->histogram[tid] = n;
+    }
+    __syncthreads();
+    // four threads per exponent, each against a quarter of the others
+    int before = 0;
+    const uint64_t mine = key[e];
+    const ulonglong2* quarter = reinterpret_cast<const ulonglong2*>(key + s * (kBins / kSlices));
+#pragma unroll
+    for (int k = 0; k < kBins / kSlices / 2; ++k) {
+        const ulonglong2 u = quarter[k];
+        before += (u.x > mine ? 1 : 0) + (u.y > mine ? 1 : 0);
+    }
+    part[tid] = (uint64_t)before;
+    __syncthreads();
+    if (tid < kBins) {
+        int rank = 0;
+#pragma unroll
+        for (int k = 0; k < kSlices; ++k) rank += (int)part[tid + k * kBins];
+        ws->code_of[tid] = (uint8_t)(rank < kCodebook ? rank : 15);
+        if (rank < kCodebook) {
+            ws->codebook[rank] = (uint8_t)tid;
+            if (codebook_out) codebook_out[rank] = (uint8_t)tid;
+        }
+    }
+    if (tid == 0) {
+        ws->codebook[kCodebook] = 0;
+        ws->fallback_tiles = 0;
+    }
+}
+
+// the codes of a codebook given by the caller
+__global__ __launch_bounds__(kBins) void encode_codes_kernel(EncodeWork* ws, uint4 codebook) {
+    const uint32_t cb[4] = {codebook.x, codebook.y, codebook.z, codebook.w};
+    const int e = threadIdx.x;
+    uint32_t c = 15;
+    for (int i = kCodebook - 1; i >= 0; --i)
+        if (((cb[i >> 2] >> (8 * (i & 3))) & 0xFFu) == (uint32_t)e) c = i;
+    ws->code_of[e] = (uint8_t)c;
+    if (e == 0) ws->fallback_tiles = 0;
 }
 
 // the lane's 16 weights of chunk j (zero outside the matrix = padding)
 __device__ __forceinline__ void load_weights16(const EncodeArgs& a, int64_t row, int64_t col, uint32_t v[8]) {
     const uint16_t* p = a.w + row * a.ld + col;
-    if (a.w_vec_ok && row < a.N && col + 16 <= a.K) {
-        uint4 u0 = reinterpret_cast<const uint4*>(p)[0];
-        uint4 u1 = reinterpret_cast<const uint4*>(p)[1];
+    if (row < a.N && col + 16 <= a.K) {
+        const uint4 u0 = load16_unaligned(p), u1 = load16_unaligned(p + 8);
         v[0] = u0.x; v[1] = u0.y; v[2] = u0.z; v[3] = u0.w;
         v[4] = u1.x; v[5] = u1.y; v[6] = u1.z; v[7] = u1.w;
     } else {
@@ -72,116 +188,75 @@ __device__ __forceinline__ void load_weights16(const EncodeArgs& a, int64_t row,
 __device__ __forceinline__ void chunk_codes(const EncodeArgs& a, const uint8_t* code_of, int64_t row, int64_t col,
                                             const uint32_t v[8], uint32_t codes[16], uint32_t& escmask) {
     escmask = 0;
+    if (row < a.N && col + 16 <= a.K) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const uint32_t bits = (v[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-        const bool valid = row < a.N && col + i < a.K;
-        const uint32_t c = valid ? (uint32_t)code_of[(bits >> 7) & 0xFFu] : 0u;
-        codes[i] = c;
-        if (c == 15u) escmask |= 1u << i;
-    }
-}
-
-__global__ __launch_bounds__(kEncWaves * kWave) void encode_count_kernel(EncodeArgs a) {
-    __shared__ uint8_t code_of[256];
-    const int tid = threadIdx.x;
-    const uint32_t lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    build_code_lut(code_of, a, tid, blockDim.x);
-    __syncthreads();
-    const int64_t tile = (int64_t)blockIdx.x * kEncWaves + w;
-    if (tile >= a.T) return;
-    const int tr = (int)(tile / a.TC);
-    const int kt = (int)(tile - (int64_t)tr * a.TC);
-    const int64_t col = (int64_t)kt * kTileCols + 16 * (lane & 15u);
-    uint32_t count = 0;
+        for (int i = 0; i < 16; ++i) codes[i] = (uint32_t)code_of[((v[i >> 1] >> (16 * (i & 1))) >> 7) & 0xFFu];
+    } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int64_t row = (int64_t)tr * kTileRows + 4 * j + (lane >> 4);
-        uint32_t v[8], codes[16], m;
-        load_weights16(a, row, col, v);
-        chunk_codes(a, code_of, row, col, v, codes, m);
-        count += __popc(m);
-    }
-    const uint32_t total = __builtin_amdgcn_readlane(wave_incl_scan(count), kWave - 1);
-    if (lane == 0) a.tile_escapes[tile] = (int32_t)total;
-}
-
-constexpr int kScanThreads = 1024;
-
-__global__ __launch_bounds__(kScanThreads) void encode_scan_kernel(EncodeArgs a) {
-    __shared__ int64_t tmp[kScanThreads];
-    const int tid = threadIdx.x;
-    int64_t chunk = (a.T + kScanThreads - 1) / kScanThreads;
-    chunk = (chunk + 7) & ~int64_t(7);
-    const int64_t t0 = (int64_t)tid * chunk;
-    const int64_t t1 = t0 + chunk < a.T ? t0 + chunk : a.T;
-    int64_t count = 0;
-    for (int64_t t = t0; t < t1; ++t) count += a.tile_escapes[t] > kEscBudget ? 1 : 0;
-    tmp[tid] = count;
-    __syncthreads();
-    for (int d = 1; d < kScanThreads; d <<= 1) {
-        int64_t u = tid >= d ? tmp[tid - d] : 0;
-        __syncthreads();
-        tmp[tid] += u;
-        __syncthreads();
-    }
-    int64_t base = tmp[tid] - count;
-    for (int64_t t = t0; t < t1; t += 8) {
-        uint32_t byte = 0;
-        for (int i = 0; i < 8 && t + i < t1; ++i) {
-            const bool fb = a.tile_escapes[t + i] > kEscBudget;
-            a.fb_rank[t + i] = (int32_t)base;
-            base += fb ? 1 : 0;
-            byte |= (fb ? 1u : 0u) << (7 - i);
+        for (int i = 0; i < 16; ++i) {
+            const bool valid = row < a.N && col + i < a.K;
+            codes[i] = valid ? (uint32_t)code_of[((v[i >> 1] >> (16 * (i & 1))) >> 7) & 0xFFu] : 0u;
         }
-        a.bitmap[t >> 3] = (uint8_t)byte;
     }
-    if (tid == kScanThreads - 1) a.totals[0] = tmp[kScanThreads - 1];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        if (codes[i] == 15u) escmask |= 1u << i;
 }
 
-__global__ __launch_bounds__(kEncWaves * kWave) void encode_write_kernel(EncodeArgs a) {
-    __shared__ uint8_t code_of[256];
-    __shared__ uint8_t esc_buf[kEncWaves][kEscBudget];
+// WRITE = false: the count of fallback tiles only
+template <bool WRITE>
+__global__ __launch_bounds__(kTilesThreads) __attribute__((amdgpu_waves_per_eu(4))) void encode_tiles_kernel(EncodeArgs a) {
+    constexpr int kWaves = kTilesThreads / kWave;
+    __shared__ __attribute__((aligned(4))) uint8_t code_of[kBins];
+    __shared__ uint8_t esc_buf[kWaves][kEscBudget];
+    __shared__ uint32_t fallback[kWaves];
     const int tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    build_code_lut(code_of, a, tid, blockDim.x);
-    __syncthreads();
-    const int64_t tile = (int64_t)blockIdx.x * kEncWaves + w;
-    if (tile >= a.T) return;
-    const int tr = (int)(tile / a.TC);
-    const int kt = (int)(tile - (int64_t)tr * a.TC);
+    const int64_t tile = (int64_t)blockIdx.x * kWaves + w;
+    const bool here = tile < a.T;
+    const int64_t t = here ? tile : a.T - 1;   // a wave past the last tile works on it, and stores nothing
+    const int tr = (int)(t / a.TC);
+    const int kt = (int)(t - (int64_t)tr * a.TC);
     const int64_t col = (int64_t)kt * kTileCols + 16 * (lane & 15u);
-
     uint32_t v[4][8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) load_weights16(a, (int64_t)tr * kTileRows + 4 * j + (lane >> 4), col, v[j]);
+    if (tid < kBins / 4)
+        reinterpret_cast<uint32_t*>(code_of)[tid] = reinterpret_cast<const uint32_t*>(a.ws->code_of)[tid];
+    lds_barrier();
+
     uint32_t escm[4];
     uint32_t cnt[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int64_t row = (int64_t)tr * kTileRows + 4 * j + (lane >> 4);
         uint32_t codes[16];
-        load_weights16(a, row, col, v[j]);
         chunk_codes(a, code_of, row, col, v[j], codes, escm[j]);
         cnt[j] = __popc(escm[j]);
-        // sm bytes: ((b >> 8) & 0x80) | (b & 0x7F) for each weight
-        uint32_t smw[4];
+        if constexpr (WRITE) {
+            // sm bytes: ((b >> 8) & 0x80) | (b & 0x7F) for each weight
+            uint32_t smw[4];
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            uint32_t word = 0;
+            for (int d = 0; d < 4; ++d) {
+                uint32_t word = 0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int i = 4 * d + k;
-                const uint32_t bits = (v[j][i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-                word |= (((bits >> 8) & 0x80u) | (bits & 0x7Fu)) << (8 * k);
+                for (int k = 0; k < 2; ++k) {
+                    const uint32_t u = v[j][2 * d + k];
+                    const uint32_t both = ((u >> 8) & 0x00800080u) | (u & 0x007F007Fu);
+                    word |= ((both & 0xFFu) | (both >> 8)) << (16 * k);
+                }
+                smw[d] = word;
             }
-            smw[d] = word;
-        }
-        uint32_t ecw[2] = {0u, 0u};
+            uint32_t ecw[2] = {0u, 0u};
 #pragma unroll
-        for (int q = 0; q < 8; ++q) ecw[q >> 2] |= (codes[2 * q] | (codes[2 * q + 1] << 4)) << (8 * (q & 3));
-        *reinterpret_cast<uint4*>(a.sm + tile * kTile + 1024 * j + 16 * lane) = make_uint4(smw[0], smw[1], smw[2], smw[3]);
-        *reinterpret_cast<uint2*>(a.ec + tile * (kTile / 2) + 512 * j + 8 * lane) = make_uint2(ecw[0], ecw[1]);
+            for (int q = 0; q < 8; ++q) ecw[q >> 2] |= (codes[2 * q] | (codes[2 * q + 1] << 4)) << (8 * (q & 3));
+            if (here) {
+                *reinterpret_cast<uint4*>(a.sm + tile * kTile + 1024 * j + 16 * lane) =
+                    make_uint4(smw[0], smw[1], smw[2], smw[3]);
+                *reinterpret_cast<uint2*>(a.ec + tile * (kTile / 2) + 512 * j + 8 * lane) = make_uint2(ecw[0], ecw[1]);
+            }
+        }
     }
 
     // escape ranks: chunk j, then lane, then position (tile-local row-major)
@@ -192,62 +267,97 @@ __global__ __launch_bounds__(kEncWaves * kWave) void encode_write_kernel(EncodeA
     const uint32_t tot[4] = {t01 & 0xFFFFu, t01 >> 16, t23 & 0xFFFFu, t23 >> 16};
     const uint32_t incl[4] = {s01 & 0xFFFFu, s01 >> 16, s23 & 0xFFFFu, s23 >> 16};
     const uint32_t total = tot[0] + tot[1] + tot[2] + tot[3];
-    uint8_t* esc_out = a.esc + tile * kEscBudget;
-
-    if (total <= (uint32_t)kEscBudget) {
-        uint32_t run = 0;
+    const bool over = here && total > (uint32_t)kEscBudget;
+    if constexpr (WRITE) {
+        if (total <= (uint32_t)kEscBudget) {
+            uint32_t run = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t r = run + incl[j] - cnt[j];
-            uint32_t m = escm[j];
-            while (m) {
-                const int i = __builtin_ctz(m);
-                m &= m - 1u;
-                const uint32_t bits = (v[j][i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-                esc_buf[w][r] = (uint8_t)((bits >> 7) & 0xFFu);
-                ++r;
+            for (int j = 0; j < 4; ++j) {
+                uint32_t r = run + incl[j] - cnt[j];
+                uint32_t m = escm[j];
+                while (m) {
+                    const int i = __builtin_ctz(m);
+                    m &= m - 1u;
+                    const uint32_t bits = (v[j][i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
+                    esc_buf[w][r] = (uint8_t)((bits >> 7) & 0xFFu);
+                    ++r;
+                }
+                run += tot[j];
             }
-            run += tot[j];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (lane < (uint32_t)kEscBudget) esc_out[lane] = lane < total ? esc_buf[w][lane] : (uint8_t)0;
-    } else {
-        if (lane < (uint32_t)kEscBudget) esc_out[lane] = 0;
-        int16_t* raw = a.raw + (int64_t)a.fb_rank[tile] * kTile;
+        if (here && lane < (uint32_t)kEscBudget)
+            a.esc[tile * kEscBudget + lane] = lane < total && !over ? esc_buf[w][lane] : (uint8_t)0;
+    }
+    if (lane == 0) fallback[w] = over ? 1u : 0u;
+    lds_barrier();
+    if (tid == 0) {
+        uint32_t byte = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint4* p = reinterpret_cast<uint4*>(raw + 1024 * j + 16 * lane);
-            p[0] = make_uint4(v[j][0], v[j][1], v[j][2], v[j][3]);
-            p[1] = make_uint4(v[j][4], v[j][5], v[j][6], v[j][7]);
-        }
+        for (int k = 0; k < kWaves; ++k) byte |= fallback[k] << (7 - k);
+        if constexpr (WRITE) a.bitmap[blockIdx.x] = (uint8_t)byte;
+        if (byte)
+            __hip_atomic_fetch_add(&a.ws->fallback_tiles, (unsigned long long)__popc(byte), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
-hipError_t launch_encode_histogram(const EncodeArgs& a, hipStream_t stream) {
-    int64_t total = a.N * a.K;
-    int64_t blocks = (total + kHistThreads * 16 - 1) / (kHistThreads * 16);
-    if (blocks < 1) blocks = 1;
-    if (blocks > 4096) blocks = 4096;
+// One wave per tile: a fallback tile's rank is the number of set bitmap bits
+// before it, counted by the wave.
+__global__ __launch_bounds__(kTilesThreads) void encode_raw_kernel(EncodeArgs a) {
+    const uint32_t lane = threadIdx.x & 63;
+    const int64_t tile = (int64_t)blockIdx.x * (kTilesThreads / kWave) + (threadIdx.x >> 6);
+    if (tile >= a.T || !((a.bitmap[tile >> 3] >> (7 - (tile & 7))) & 1u)) return;
+    const int64_t rank = fallback_rank(a.bitmap, tile, lane);
+    if (rank >= a.raw_tiles) return;
+    const int tr = (int)(tile / a.TC);
+    const int kt = (int)(tile - (int64_t)tr * a.TC);
+    const int64_t col = (int64_t)kt * kTileCols + 16 * (lane & 15u);
+    int16_t* raw = a.raw + rank * kTile;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        uint32_t v[8];
+        load_weights16(a, (int64_t)tr * kTileRows + 4 * j + (lane >> 4), col, v);
+        uint4* p = reinterpret_cast<uint4*>(raw + 1024 * j + 16 * lane);
+        p[0] = make_uint4(v[0], v[1], v[2], v[3]);
+        p[1] = make_uint4(v[4], v[5], v[6], v[7]);
+    }
+}
+
+int encode_histogram_blocks(const EncodeArgs& a, int cu_count) {
+    // one block per CU (its waves fill it), fewer where the weights are few
+    const int64_t blocks = (a.N * a.K + 8 * kHistThreads - 1) / (8 * kHistThreads);
+    return (int)std::max<int64_t>(1, std::min<int64_t>({blocks, (int64_t)cu_count, (int64_t)kEncodeHistBlocks}));
+}
+
+hipError_t launch_encode_histogram(const EncodeArgs& a, int cu_count, uint8_t* codebook_out, hipStream_t stream) {
+    const int blocks = encode_histogram_blocks(a, cu_count);
     hipLaunchKernelGGL(encode_histogram_kernel, dim3((uint32_t)blocks), dim3(kHistThreads), 0, stream, a);
+    hipLaunchKernelGGL(encode_select_kernel, dim3(1), dim3(kHistThreads), 0, stream, a.ws, blocks, codebook_out);
     return hipGetLastError();
 }
 
-hipError_t launch_encode_count(const EncodeArgs& a, hipStream_t stream) {
-    const int64_t blocks = (a.T + kEncWaves - 1) / kEncWaves;
-    hipLaunchKernelGGL(encode_count_kernel, dim3((uint32_t)blocks), dim3(kEncWaves * kWave), 0, stream, a);
+hipError_t launch_encode_codes(const EncodeArgs& a, const uint8_t codebook[16], hipStream_t stream) {
+    uint4 cb;
+    __builtin_memcpy(&cb, codebook, sizeof cb);
+    hipLaunchKernelGGL(encode_codes_kernel, dim3(1), dim3(kBins), 0, stream, a.ws, cb);
     return hipGetLastError();
 }
 
-hipError_t launch_encode_scan(const EncodeArgs& a, hipStream_t stream) {
-    hipLaunchKernelGGL(encode_scan_kernel, dim3(1), dim3(kScanThreads), 0, stream, a);
+hipError_t launch_encode_tiles(const EncodeArgs& a, bool write, hipStream_t stream) {
+    const dim3 grid((uint32_t)((a.T + kTilesThreads / kWave - 1) / (kTilesThreads / kWave))), block(kTilesThreads);
+    if (write)
+        hipLaunchKernelGGL(encode_tiles_kernel<true>, grid, block, 0, stream, a);
+    else
+        hipLaunchKernelGGL(encode_tiles_kernel<false>, grid, block, 0, stream, a);
     return hipGetLastError();
 }
 
-hipError_t launch_encode_write(const EncodeArgs& a, hipStream_t stream) {
-    const int64_t blocks = (a.T + kEncWaves - 1) / kEncWaves;
-    hipLaunchKernelGGL(encode_write_kernel, dim3((uint32_t)blocks), dim3(kEncWaves * kWave), 0, stream, a);
+hipError_t launch_encode_raw(const EncodeArgs& a, hipStream_t stream) {
+    const dim3 grid((uint32_t)((a.T + kTilesThreads / kWave - 1) / (kTilesThreads / kWave)));
+    hipLaunchKernelGGL(encode_raw_kernel, grid, dim3(kTilesThreads), 0, stream, a);
     return hipGetLastError();
 }
 

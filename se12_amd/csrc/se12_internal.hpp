@@ -154,22 +154,28 @@ struct DecodeArgs {
     int32_t out_vec_ok;
 };
 
+// Device scratch of the encoder (se12_encode_workspace bytes).
+constexpr int kEncodeHistBlocks = 512;
+struct EncodeWork {
+    uint64_t histogram[256];
+    uint8_t code_of[256];
+    uint8_t codebook[16];                 // read back by the host with fallback_tiles
+    unsigned long long fallback_tiles;
+    uint32_t partial[kEncodeHistBlocks * 256];
+};
+
 struct EncodeArgs {
     const uint16_t* w;
     int64_t N, K, ld;
     int32_t TR, TC;
     int64_t T;
-    uint32_t codebook[4];     // 15 bytes, little-endian packed
-    uint64_t* histogram;      // [256]
-    int32_t* tile_escapes;    // [T]
-    int32_t* fb_rank;         // [T]
-    int64_t* totals;          // [1] fallback tile count
+    EncodeWork* ws;
     uint8_t* sm;
     uint8_t* ec;
     uint8_t* esc;
     uint8_t* bitmap;
     int16_t* raw;
-    int32_t w_vec_ok;
+    int64_t raw_tiles;                    // tiles `raw` holds
 };
 
 constexpr int kGemvMaxBatchPerLaunch = 4;
@@ -301,10 +307,11 @@ hipError_t launch_tile_info(const uint8_t* bitmap, const uint8_t* ec, int64_t T,
 hipError_t launch_overflow_decode(const DecodeArgs& a, int16_t* raw, hipStream_t stream);
 hipError_t launch_side_records(const uint32_t* info, const uint8_t* esc, const uint4* escpos, int64_t T, uint32_t* side,
                                hipStream_t stream);
-hipError_t launch_encode_histogram(const EncodeArgs& a, hipStream_t stream);
-hipError_t launch_encode_count(const EncodeArgs& a, hipStream_t stream);
-hipError_t launch_encode_scan(const EncodeArgs& a, hipStream_t stream);
-hipError_t launch_encode_write(const EncodeArgs& a, hipStream_t stream);
+// histogram and codebook (also to codebook_out on the device unless NULL)
+hipError_t launch_encode_histogram(const EncodeArgs& a, int cu_count, uint8_t* codebook_out, hipStream_t stream);
+hipError_t launch_encode_codes(const EncodeArgs& a, const uint8_t codebook[16], hipStream_t stream);
+hipError_t launch_encode_tiles(const EncodeArgs& a, bool write, hipStream_t stream);
+hipError_t launch_encode_raw(const EncodeArgs& a, hipStream_t stream);
 // Streaming-read probe (se12_probe.hip): its grid for a device and the launch.
 int64_t read_probe_blocks(int32_t compute_units);
 hipError_t launch_read_probe(const void* buf, int64_t n16, uint32_t* out, int64_t blocks, hipStream_t stream);

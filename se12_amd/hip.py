@@ -460,22 +460,24 @@ def encode_on_device(weights: torch.Tensor) -> Se12DeviceTensor:
     lib = nat.lib()
     with torch.cuda.device(dev):
         st = nat.stream_ptr()
-        nat.check(lib.se12_encode_prepare(nat.ptr(w), rows, cols, cols, cb, ctypes.byref(nfb), st))
         sm = torch.empty(t * TILE_SIZE, dtype=torch.uint8, device=dev)
         ec = torch.empty(t * TILE_SIZE // 2, dtype=torch.uint8, device=dev)
         esc = torch.empty(t * ESCAPE_BUDGET, dtype=torch.uint8, device=dev)
         bitmap = torch.empty(bitmap_bytes(t), dtype=torch.uint8, device=dev)
-        raw = torch.empty(nfb.value * TILE_SIZE, dtype=torch.int16, device=dev)
+        codebook_dev = torch.empty(CODEBOOK_SIZE, dtype=torch.uint8, device=dev)
+        ws = torch.empty(lib.se12_encode_workspace(), dtype=torch.uint8, device=dev)
         out = nat.StreamsOut(
             sm_dev=sm.data_ptr(), ec_dev=ec.data_ptr(), esc_dev=esc.data_ptr(), fallback_bitmap_dev=bitmap.data_ptr(),
-            fallback_raw_dev=raw.data_ptr() if raw.numel() else None, fallback_raw_tiles=nfb.value,
+            fallback_raw_dev=None, fallback_raw_tiles=0,
         )
-        got = ctypes.c_int64()
-        nat.check(lib.se12_encode(nat.ptr(w), rows, cols, cols, cb, ctypes.byref(out), ctypes.byref(got), st))
-    codebook = tuple(int(c) for c in cb)
+        nat.check(lib.se12_encode_streams(nat.ptr(w), rows, cols, cols, ctypes.byref(out), nat.ptr(codebook_dev), cb,
+                                          ctypes.byref(nfb), nat.ptr(ws), ws.numel(), st))
+        raw = torch.empty(nfb.value * TILE_SIZE, dtype=torch.int16, device=dev)
+        if nfb.value:
+            nat.check(lib.se12_encode_fallback(nat.ptr(w), rows, cols, cols, nat.ptr(bitmap), nat.ptr(raw), nfb.value, st))
     return Se12DeviceTensor(
-        sm=sm, ec=ec, esc=esc, codebook=torch.tensor(codebook, dtype=torch.uint8, device=dev),
-        fallback_bitmap=bitmap, fallback_raw=raw, rows=int(rows), cols=int(cols), codebook_host=codebook,
+        sm=sm, ec=ec, esc=esc, codebook=codebook_dev, fallback_bitmap=bitmap, fallback_raw=raw, rows=int(rows),
+        cols=int(cols), codebook_host=tuple(cb),
     )
 
 

@@ -47,3 +47,61 @@ def test_encoder_matches_oracle(gpu, rows, cols, kind):
     else:
         bits = heavy_tailed_bf16(rows, cols, seed=2)
     _assert_same(_encode(bits, gpu), o.encode(bits.reshape(-1), rows, cols))
+
+
+def _streams(dt):
+    return {"sm": dt.sm, "ec": dt.ec, "esc": dt.esc, "fallback_bitmap": dt.fallback_bitmap,
+            "fallback_raw": dt.fallback_raw, "codebook": dt.codebook}
+
+
+@pytest.mark.parametrize("rows,cols,kind", [
+    (1, 1, "normal"), (1, 7, "uniform"), (16, 256, "heavy"), (15, 255, "uniform"), (17, 257, "heavy"),
+    (1000, 8, "normal"), (1000, 9, "heavy"), (128, 256, "uniform"), (129, 256, "uniform"),     # 8 and 9 tiles: bitmap bytes
+    (9000, 700, "mixed"),       # 1,689 tiles, more bitmap bytes than one step of a wave's rank count
+])
+def test_encoder_at_tile_and_bitmap_edges(gpu, rows, cols, kind):
+    """Byte equality with the oracle for an aligned tensor and for one at an odd offset of its buffer, and of the two-call
+    C interface on rows further apart than their length."""
+    import ctypes
+
+    import torch
+
+    from se12_amd import _native as nat
+    from se12_amd.hip import encode_on_device
+
+    if kind == "normal":
+        bits = o.normal_bf16(rows, cols, seed=rows, std=0.02)
+    elif kind == "uniform":
+        bits = uniform_bits(rows, cols, seed=rows)
+    else:
+        bits = heavy_tailed_bf16(rows, cols, seed=rows)
+    if kind == "mixed":          # every third tile row full of escapes
+        u = uniform_bits(rows, cols, seed=1)
+        pick = (np.arange(rows) // 16) % 3 == 1
+        bits = np.where(pick[:, None], u, bits)
+    want = o.encode(bits.reshape(-1), rows, cols)
+    _assert_same(_encode(bits, gpu), want)
+    buf = torch.full((rows * cols + 9,), float("inf"), dtype=torch.bfloat16, device=gpu)
+    w = buf[3:3 + rows * cols].view(rows, cols)
+    w.copy_(bf16_tensor(bits, gpu))
+    odd = _streams(encode_on_device(w))
+    aligned = _streams(encode_on_device(bf16_tensor(bits, gpu)))
+    for k, v in aligned.items():
+        assert torch.equal(odd[k], v), k
+    ld = cols + 5
+    wide = torch.full((rows, ld), float("nan"), dtype=torch.bfloat16, device=gpu)
+    wide[:, :cols] = w
+    cb, n = (ctypes.c_uint8 * 15)(), ctypes.c_int64()
+    nat.check(nat.lib().se12_encode_prepare(nat.ptr(wide), rows, cols, ld, cb, ctypes.byref(n), nat.stream_ptr()))
+    assert tuple(cb) == tuple(aligned["codebook"].tolist()) and n.value * 4096 == aligned["fallback_raw"].numel()
+    got = {k: torch.empty_like(v) for k, v in aligned.items()}
+    out = nat.StreamsOut(sm_dev=got["sm"].data_ptr(), ec_dev=got["ec"].data_ptr(), esc_dev=got["esc"].data_ptr(),
+                         fallback_bitmap_dev=got["fallback_bitmap"].data_ptr(),
+                         fallback_raw_dev=got["fallback_raw"].data_ptr() if n.value else None, fallback_raw_tiles=n.value)
+    total = ctypes.c_int64()
+    nat.check(nat.lib().se12_encode(nat.ptr(wide), rows, cols, ld, cb, ctypes.byref(out), ctypes.byref(total),
+                                    nat.stream_ptr()))
+    assert total.value == n.value
+    for k in got:
+        if k != "codebook":
+            assert torch.equal(got[k], aligned[k]), k
