@@ -304,6 +304,12 @@ int se12_decode(se12_handle* h, uint16_t* out_dev, void* stream);
 int se12_decode_rows(se12_handle* h, const int64_t* rows_dev, int64_t nrows, uint16_t* out_dev,
                      void* stream);
 
+/* se12_decode_rows with each weight times `scale` (rounded to BF16 first; finite
+ * and not zero in BF16), the product rounded to BF16: a scaled embedding lookup
+ * (Gemma multiplies its rows by sqrt(hidden)) in one launch. */
+int se12_decode_rows_scaled(se12_handle* h, const int64_t* rows_dev, int64_t nrows, float scale, uint16_t* out_dev,
+                            void* stream);
+
 /* Host-only: the 15-entry codebook from a 256-bin exponent histogram of the
  * real weights: descending count, equal counts to the larger exponent value,
  * zero-count values last (lws/domain/se12/codebook.py:41-59). */

@@ -1257,26 +1257,43 @@ int se12_decode(se12_handle* h, uint16_t* out, void* stream) {
     SE12_HIP(ds.enter(h->device));
     DecodeArgs a = decode_args(h, out);
     a.items = h->T;
-    hipError_t e = launch_decode(a, false, static_cast<hipStream_t>(stream), h->cu_count);
+    hipError_t e = launch_decode(a, static_cast<hipStream_t>(stream), h->cu_count);
     if (e != hipSuccess) return fail(SE12_E_HIP, "se12_decode launch: %s", hipGetErrorString(e));
     return SE12_OK;
 }
 
-int se12_decode_rows(se12_handle* h, const int64_t* rows, int64_t nrows, uint16_t* out, void* stream) {
-    if (!h) return fail(SE12_E_INVALID, "se12_decode_rows: NULL handle");
-    if (h->format != SE12_FORMAT_SE12) return fail(SE12_E_INVALID, "se12_decode_rows: handle is not SE12");
-    if (nrows < 0) return fail(SE12_E_INVALID, "se12_decode_rows: negative row count");
+static int decode_rows(const char* fn, se12_handle* h, const int64_t* rows, int64_t nrows, float scale, uint16_t* out,
+                       void* stream) {
+    if (!h) return fail(SE12_E_INVALID, "%s: NULL handle", fn);
+    if (h->format != SE12_FORMAT_SE12) return fail(SE12_E_INVALID, "%s: handle is not SE12", fn);
+    if (nrows < 0) return fail(SE12_E_INVALID, "%s: negative row count", fn);
     if (nrows == 0) return SE12_OK;
-    if (!rows || !out) return fail(SE12_E_INVALID, "se12_decode_rows: NULL rows or out");
+    if (!rows || !out) return fail(SE12_E_INVALID, "%s: NULL rows or out", fn);
     DeviceScope ds;
     SE12_HIP(ds.enter(h->device));
     DecodeArgs a = decode_args(h, out);
     a.rows = rows;
     a.nrows = nrows;
-    a.items = nrows * h->TC;
-    hipError_t e = launch_decode(a, true, static_cast<hipStream_t>(stream), h->cu_count);
-    if (e != hipSuccess) return fail(SE12_E_HIP, "se12_decode_rows launch: %s", hipGetErrorString(e));
+    hipError_t e = launch_decode_rows(a, scale, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(SE12_E_HIP, "%s launch: %s", fn, hipGetErrorString(e));
     return SE12_OK;
+}
+
+int se12_decode_rows(se12_handle* h, const int64_t* rows, int64_t nrows, uint16_t* out, void* stream) {
+    return decode_rows("se12_decode_rows", h, rows, nrows, 0.0f, out, stream);
+}
+
+int se12_decode_rows_scaled(se12_handle* h, const int64_t* rows, int64_t nrows, float scale, uint16_t* out, void* stream) {
+    // the BF16 value nearest to scale (ties to even)
+    uint32_t u;
+    std::memcpy(&u, &scale, sizeof u);
+    if (!(scale - scale == 0.0f)) return fail(SE12_E_INVALID, "se12_decode_rows_scaled: scale is not finite");
+    u = (u + 0x7FFFu + ((u >> 16) & 1u)) & 0xFFFF0000u;
+    float s;
+    std::memcpy(&s, &u, sizeof s);
+    if (s == 0.0f || !(s - s == 0.0f))
+        return fail(SE12_E_INVALID, "se12_decode_rows_scaled: scale %g is zero or infinite in BF16", (double)scale);
+    return decode_rows("se12_decode_rows_scaled", h, rows, nrows, s, out, stream);
 }
 
 int se12_codebook_from_histogram(const uint64_t counts[256], uint8_t codebook_out[15]) {

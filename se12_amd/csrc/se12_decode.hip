@@ -2,8 +2,8 @@
 // reference decoder (lws/domain/se12/codec.py:144-186). A wave decodes a
 // 16x256 tile with the same per-lane routine as the fused GEMV and writes its
 // rows straight to the cropped [rows, cols] output (the whole-matrix decode
-// streams several tiles per wave; the row decode takes one (row, K tile) per
-// wave), replacing the reference's
+// streams several tiles per wave; the row decode takes one row of four K
+// tiles per wave), replacing the reference's
 // one-thread-per-tile kernel plus device untile/crop
 // (lws/adapters/cuda/kernels/se12_decode.cu:12-43,
 // lws/adapters/cuda/se12_decoder.py:147-185).
@@ -15,6 +15,7 @@
 // tile reads the tile's `ec` bytes). The kernels read it instead of the bitmap.
 #include "se12_device.hpp"
 #include "se12_internal.hpp"
+#include "se12_step_math.hpp"
 
 namespace se12 {
 
@@ -29,43 +30,6 @@ __device__ __forceinline__ void store16(uint16_t* out_row, int64_t col, int64_t 
         for (int i = 0; i < 16; ++i)
             if (col + i < K) out_row[col + i] = (uint16_t)(w[i >> 1] >> (16 * (i & 1)));
     }
-}
-
-// Decodes a loaded tile for this lane; calls sink(j, w) for each chunk j.
-template <typename Sink>
-__device__ __forceinline__ void decode_loaded(const DecodeArgs& a, const uint32_t* lut, const TileSide& side,
-                                              const TileLoads& t, uint32_t lane, Sink&& sink) {
-    const uint32_t info = side_info(side, 0);
-    if (info_is_fallback(info)) {
-        const int16_t* raw = raw_tile_ptr(info, a.fb_raw, a.ovf_raw);
-        uint32_t w[4][8];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) load_raw_chunk(raw, j, lane, w[j]);
-        wait_vector_loads();  // rare path: keeps the common path's waits exact
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sink(j, w[j]);
-    } else {
-        uint32_t pat[4][8];
-        lookup_tile(lut, t, pat);
-        patch_tile_escapes(pat, info, side, 0, lane);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t w[8];
-            merge_chunk(pat[j], t.sm[j], w);
-            sink(j, w);
-        }
-    }
-}
-
-// Loads and decodes tile `tile` for this lane; calls sink(j, w) for each chunk j.
-template <typename Sink>
-__device__ __forceinline__ void decode_tile(const DecodeArgs& a, const uint32_t* lut, int64_t tile, uint32_t lane,
-                                            Sink&& sink) {
-    TileSide side;
-    TileLoads t;
-    load_side(side, a.side, tile, lane);
-    load_tile(t, a.sm, a.ec, tile, lane);
-    decode_loaded(a, lut, side, t, lane, sink);
 }
 
 // 8 decoded weights (4 BF16 pairs) to out_row[col .. col + 8) clipped at K:
@@ -188,44 +152,66 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Dec
     }
 }
 
-template <bool ROWS>
-__global__ __launch_bounds__(kDecodeWaves * kWave) void decode_kernel(DecodeArgs a) {
+// Decodes single rows, in request order: one wave per (row, 4 K tiles). Lane
+// 16 s + c takes 16 columns of the row in the wave's s-th tile, so the wave
+// reads the row's own 256 bytes of sm and 128 of ec per tile (not the tile's
+// 6 KB) and the four tiles' side records in one 256-byte load; the record's
+// fields reach the 16 lanes of its tile by lane shuffles. Rows outside the
+// matrix give zeros. SCALED: each weight times `scale` (a BF16 value), rounded
+// to BF16. Bound by latency and the scattered 128..256-byte reads: 2,048 rows of
+// 256000x2304 25.9 -> 6.3 us against a wave decoding the whole tile for one of
+// its rows (and no separate multiply, 6.8 us, with a factor copied from the host).
+constexpr int kRowTiles = 4;
+
+template <bool SCALED>
+__global__ __launch_bounds__(kDecodeWaves * kWave) void decode_rows_kernel(DecodeArgs a, float scale) {
     SE12_DECLARE_LUT(lut);
     const int tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    store_block_lut(lut, reinterpret_cast<const uint4*>(a.lut)[lane], lane);
+    const uint4 lutv = reinterpret_cast<const uint4*>(a.lut)[lane];
+    const int64_t groups = (a.TC + kRowTiles - 1) / kRowTiles;
+    const int64_t item = (int64_t)blockIdx.x * kDecodeWaves + w;
+    const bool here = item < a.items;
+    const int64_t ri = (here ? item : a.items - 1) / groups;
+    const int64_t row = a.rows[ri];
+    const int kt = (int)((here ? item : a.items - 1) - ri * groups) * kRowTiles + (int)(lane >> 4);
+    const bool inside = row >= 0 && row < a.N;
+    const int64_t tile = (inside ? row / kTileRows : 0) * a.TC + (kt < a.TC ? kt : a.TC - 1);
+    const uint32_t lr = (uint32_t)row & (kTileRows - 1), c = lane & 15u;
+    const uint32_t rec = a.side[tile * kSideWords + c];
+    const uint4 sm = *reinterpret_cast<const uint4*>(a.sm + tile * kTile + lr * kTileCols + 16 * c);
+    const uint2 ec = *reinterpret_cast<const uint2*>(a.ec + tile * (kTile / 2) + lr * (kTileCols / 2) + 8 * c);
+    store_block_lut(lut, lutv, lane);
     lds_barrier();
 
-    const int64_t item = (int64_t)blockIdx.x * kDecodeWaves + w;
-    if (item >= a.items) return;
-    const bool vec_ok = a.out_vec_ok != 0;
-    if constexpr (!ROWS) {
-        const int64_t tile = item;
-        const int tr = (int)(tile / a.TC);
-        const int kt = (int)(tile - (int64_t)tr * a.TC);
-        const int64_t col = (int64_t)kt * kTileCols + 16 * (lane & 15u);
-        decode_tile(a, lut, tile, lane, [&](int j, const uint32_t* wv) {
-            const int64_t row = (int64_t)tr * kTileRows + 4 * j + (lane >> 4);
-            if (row < a.N) store16(a.out + row * a.K, col, a.K, vec_ok, wv);
-        });
-    } else {
-        const int64_t ri = item / a.TC;
-        const int kt = (int)(item - ri * a.TC);
-        const int64_t row = a.rows[ri];
-        const int64_t col = (int64_t)kt * kTileCols + 16 * (lane & 15u);
-        uint16_t* out_row = a.out + ri * a.K;
-        if (row < 0 || row >= a.N) {
-            const uint32_t zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            if ((lane >> 4) == 0) store16(out_row, col, a.K, vec_ok, zero);
-            return;
-        }
-        const int lr = (int)(row & (kTileRows - 1));
-        const int64_t tile = (row / kTileRows) * a.TC + kt;
-        decode_tile(a, lut, tile, lane, [&](int j, const uint32_t* wv) {
-            if (4 * j + (int)(lane >> 4) == lr) store16(out_row, col, a.K, vec_ok, wv);
-        });
+    // word k of this lane's record, from the lane of its 16 that loaded it
+    auto word = [&](int k) { return (uint32_t)__shfl((int)rec, (int)(lane & 48u) + k, 64); };
+    const uint32_t info = word(0);
+    uint32_t pat[8], v[8];
+    lookup_chunk(lut, ec, pat);
+    const uint32_t n = info_is_fallback(info) ? 0u : info_escapes(info);
+    // the tile's listed escapes that fall on this lane's columns of this row
+    for (uint32_t k = 0; wave_any(k < n); ++k) {
+        const uint32_t p = (word(5 + (int)(k >> 1)) >> (16 * (k & 1u))) & 0xFFFFu;
+        const uint32_t e = (word(1 + (int)(k >> 2)) >> (8 * (k & 3u))) & 0xFFu;
+        if (k < n && (p >> 4) == ((lr << 4) | c)) patch_exponent(pat, p & 15u, e);
     }
+    merge_chunk(pat, sm, v);
+    if (info_is_fallback(info)) {
+        const uint4* raw = reinterpret_cast<const uint4*>(raw_tile_ptr(info, a.fb_raw, a.ovf_raw) + lr * kTileCols + 16 * c);
+        const uint4 r0 = raw[0], r1 = raw[1];
+        v[0] = r0.x; v[1] = r0.y; v[2] = r0.z; v[3] = r0.w;
+        v[4] = r1.x; v[5] = r1.y; v[6] = r1.z; v[7] = r1.w;
+    }
+    if (!here || kt >= a.TC) return;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if constexpr (SCALED)
+            v[i] = se12step::f_to_bf16x2(__uint_as_float(v[i] << 16) * scale, __uint_as_float(v[i] & 0xFFFF0000u) * scale);
+        if (!inside) v[i] = 0u;
+    }
+    store16(a.out + ri * a.K, (int64_t)kt * kTileCols + 16 * c, a.K, a.out_vec_ok != 0, v);
 }
 
 // waves of the whole-matrix decode per CU (MI355X, cold HBM, half layout:
@@ -233,16 +219,22 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_kernel(DecodeArgs
 // 14336x3584 33.5 / 36.5 / 33.6 / 33.9)
 constexpr int kDecodeStreamWavesPerCu = 4;
 
-hipError_t launch_decode(const DecodeArgs& a, bool rows, hipStream_t stream, int cu_count) {
+hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream, int cu_count) {
+    const int64_t nw = std::min<int64_t>(a.T, (int64_t)std::max(1, cu_count) * kDecodeStreamWavesPerCu);
+    const int64_t blocks = (nw + kDecodeWaves - 1) / kDecodeWaves;
+    hipLaunchKernelGGL(decode_stream_kernel, dim3((uint32_t)blocks), dim3(kDecodeWaves * kWave), 0, stream, a, nw);
+    return hipGetLastError();
+}
+
+hipError_t launch_decode_rows(const DecodeArgs& args, float scale, hipStream_t stream) {
+    DecodeArgs a = args;
+    a.items = a.nrows * ((a.TC + kRowTiles - 1) / kRowTiles);
     if (a.items <= 0) return hipSuccess;
-    if (rows) {
-        const int64_t blocks = (a.items + kDecodeWaves - 1) / kDecodeWaves;
-        hipLaunchKernelGGL(decode_kernel<true>, dim3((uint32_t)blocks), dim3(kDecodeWaves * kWave), 0, stream, a);
-    } else {
-        const int64_t nw = std::min<int64_t>(a.T, (int64_t)std::max(1, cu_count) * kDecodeStreamWavesPerCu);
-        const int64_t blocks = (nw + kDecodeWaves - 1) / kDecodeWaves;
-        hipLaunchKernelGGL(decode_stream_kernel, dim3((uint32_t)blocks), dim3(kDecodeWaves * kWave), 0, stream, a, nw);
-    }
+    const dim3 grid((uint32_t)((a.items + kDecodeWaves - 1) / kDecodeWaves)), block(kDecodeWaves * kWave);
+    if (scale != 0.0f)
+        hipLaunchKernelGGL(decode_rows_kernel<true>, grid, block, 0, stream, a, scale);
+    else
+        hipLaunchKernelGGL(decode_rows_kernel<false>, grid, block, 0, stream, a, scale);
     return hipGetLastError();
 }
 

@@ -298,7 +298,9 @@ constexpr size_t rx_lds_total(int64_t k, int staged, int batch, int waves, int k
     return rx_lds_bytes(k, staged) > sums ? rx_lds_bytes(k, staged) : sums;
 }
 hipError_t launch_gemm_rx(const GemvGroupArgs& a, int batch, const GemvPlan& p, hipStream_t stream);
-hipError_t launch_decode(const DecodeArgs& a, bool rows, hipStream_t stream, int cu_count);
+hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream, int cu_count);
+// scale 0: the weights as they are
+hipError_t launch_decode_rows(const DecodeArgs& a, float scale, hipStream_t stream);
 // Bind-time sidecar: one word per tile (fallback rank, or the chunks holding
 // escape codes) and the fallback tile count.
 // total[0] = fallback tiles, total[1] = tiles with more than the listed escapes

@@ -246,6 +246,16 @@ class Se12MatVecKernel(_GemvBase):
         nat.check(nat.lib().se12_decode_rows(self.handle.raw, nat.ptr(idx), idx.numel(), nat.ptr(out), nat.stream_ptr()))
         return out
 
+    def decode_rows_scaled_into(self, rows: torch.Tensor, out: torch.Tensor, scale: float) -> torch.Tensor:
+        """`decode_rows_into` with each row times `scale` (as a BF16 value),
+        rounded to BF16: out * torch.tensor(scale, dtype=torch.bfloat16)."""
+        idx = rows.reshape(-1)
+        _require(idx, "rows", torch.int64, (idx.numel(),), self.device)
+        _require(out, "out", torch.bfloat16, (idx.numel(), self.cols), self.device)
+        nat.check(nat.lib().se12_decode_rows_scaled(self.handle.raw, nat.ptr(idx), idx.numel(), float(scale), nat.ptr(out),
+                                                    nat.stream_ptr()))
+        return out
+
 
 class RawBf16MatVecKernel(_GemvBase):
     """The same-skeleton raw-BF16 twin bound to a [N, K] BF16 matrix (gemv.py:143-172)."""

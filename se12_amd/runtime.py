@@ -246,6 +246,13 @@ class CompressedLinear(nn.Module):
         return f"in_features={self.in_features}, out_features={self.out_features}, mode={self.mode}, se12"
 
 
+def _scales_in_bf16(scale: float) -> bool:
+    """Whether `scale` is a finite BF16 value other than zero once rounded
+    (2^-133 is half the smallest such value's spacing from zero, 3.38e38 below
+    the values that round to infinity): what the library's scaled lookup takes."""
+    return 2.0 ** -133 <= abs(scale) <= 3.38e38
+
+
 class CompressedEmbedding(nn.Module):
     """nn.Embedding replacement: looks rows up by decoding only their tiles.
     `scale` reproduces scaled embeddings (Gemma's: rows x sqrt(hidden), the
@@ -265,9 +272,13 @@ class CompressedEmbedding(nn.Module):
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
         idx = ids.reshape(-1).to(device=self.kernel.device, dtype=torch.int64).contiguous()
         out = torch.empty((idx.numel(), self.embedding_dim), dtype=torch.bfloat16, device=self.kernel.device)
-        self.kernel.decode_rows_into(idx, out)
-        if self.scale is not None:
-            out = out * torch.tensor(self.scale, dtype=torch.bfloat16, device=out.device)
+        scaled = getattr(self.kernel, "decode_rows_scaled_into", None)
+        if self.scale is not None and scaled is not None and _scales_in_bf16(self.scale):
+            scaled(idx, out, self.scale)
+        else:
+            self.kernel.decode_rows_into(idx, out)
+            if self.scale is not None:
+                out = out * torch.tensor(self.scale, dtype=torch.bfloat16, device=out.device)
         return out.view(*ids.shape, self.embedding_dim)
 
     def stream_bytes(self) -> int:

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from conftest import GOLDEN_NAMES, golden_as_encoding, load_golden
-from gpu_helpers import escape_count_bf16, heavy_tailed_bf16, normal_case, to_device, uniform_bits
+from gpu_helpers import bf16_tensor, escape_count_bf16, heavy_tailed_bf16, normal_case, to_device, uniform_bits
 from oracle import se12_codec as o
 
 pytestmark = pytest.mark.gpu
@@ -132,3 +132,30 @@ def test_bind_stats_count_the_raw_decoded_tiles(gpu):
     a, b = ctypes.c_int64(-1), ctypes.c_int64(-1)
     nat.check(nat.lib().se12_handle_bind_stats(rk.handle.raw, ctypes.byref(a), ctypes.byref(b)))
     assert (a.value, b.value) == (0, 0)
+
+
+@pytest.mark.parametrize("rows,cols,kind", [
+    (1, 1, "normal"), (16, 15, "uniform"), (17, 256, "heavy"), (33, 257, "heavy"), (48, 1024, "heavy"),     # 1, 1, 1, 2, 4 K tiles
+    (40, 1025, "uniform"), (64, 2304, "normal"), (64, 2304, "heavy"), (32, 1288, "uniform"),                # 5, 9, 9, 6
+])
+def test_decode_rows_equals_the_oracle_at_tile_edges(gpu, rows, cols, kind):
+    """Every row (each position of a tile, escapes, tiles kept raw), repeated and out-of-range ones, plain and scaled."""
+    from se12_amd.hip import Se12MatVecKernel
+
+    bits = {"normal": lambda: o.normal_bf16(rows, cols, seed=3, std=0.02), "uniform": lambda: uniform_bits(rows, cols, seed=3),
+            "heavy": lambda: heavy_tailed_bf16(rows, cols, seed=3)}[kind]()
+    enc = o.encode(bits.reshape(-1), rows, cols)
+    k = Se12MatVecKernel(to_device(enc, gpu))
+    idx = torch.cat([torch.arange(rows), torch.tensor([rows - 1, 0, -1, rows, 2 ** 40])]).to(gpu)
+    out = torch.empty((idx.numel(), cols), dtype=torch.bfloat16, device=gpu)
+    got = k.decode_rows_into(idx, out).view(torch.int16).cpu().numpy()
+    want = np.concatenate([bits, bits[[rows - 1, 0]], np.zeros((3, cols), dtype=bits.dtype)])
+    assert np.array_equal(got, want.astype(np.int16))
+    w = bf16_tensor(want, gpu)
+    for scale in (48.0, 70.7107, -0.3):
+        scaled = k.decode_rows_scaled_into(idx, torch.empty_like(out), scale)
+        ref = w * torch.tensor(scale, dtype=torch.bfloat16, device=gpu)
+        assert torch.equal(scaled.isnan(), ref.isnan())
+        assert torch.equal(scaled.nan_to_num(), ref.nan_to_num())      # (0 == -0 in a row outside the matrix)
+    with pytest.raises(Exception):
+        k.decode_rows_scaled_into(idx, out, float("inf"))
