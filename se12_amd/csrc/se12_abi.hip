@@ -77,8 +77,9 @@ struct se12_handle {
     int32_t TR, TC;
     se12_streams s;
     const uint16_t* wraw;
-    uint32_t* info;      // [T] per-tile sidecar word (bind time only)
-    uint4* escpos;       // [T] listed escape positions (bind time only)
+    void* arena;         // the device memory the pointers below but ovf_raw lie in
+    bool owns_arena;     // allocated here, not the caller's
+    uint8_t codebook[SE12_CODEBOOK_SIZE];  // as bind read it
     uint32_t* side;      // [T, 16] per-tile side records read by the kernels
     int16_t* ovf_raw;    // tiles with more than the listed escapes, decoded at bind
     int64_t n_overflow;
@@ -134,7 +135,46 @@ int se12_device_info_get(int32_t device, se12_device_info* out) {
     return SE12_OK;
 }
 
-static int bind_common(se12_handle* h, int64_t rows, int64_t cols, int32_t max_batch) {
+// The device memory of a handle, in one allocation: first what must be zero
+// before use (bind's result, arrival counters, dot2 pair slots), then the side
+// records and pair table (SE12 only) and the split-K partial sums.
+namespace {
+struct ArenaLayout {
+    int64_t counters, pairs, zeroed, side, lut, partial, total;  // byte offsets
+    int64_t partial_elems, pair_elems;
+    int32_t s_cap;
+};
+}  // namespace
+
+static ArenaLayout arena_layout(int64_t rows, int64_t cols, int32_t max_batch, bool se12) {
+    const int64_t tr = ceil_div(rows, SE12_TILE_ROWS), tc = ceil_div(cols, SE12_TILE_COLS), np = tr * SE12_TILE_ROWS;
+    auto up = [](int64_t n) { return (n + 255) & ~(int64_t)255; };
+    ArenaLayout l{};
+    l.s_cap = (int32_t)std::min<int64_t>(tc, kMaxSplits);
+    // split-K workspace: S x (rows per launch) x Np floats, for the dot2
+    // path (up to 4 rows per launch, any split count) and the MFMA path (all
+    // rows in one launch, at most kGemmMaxSplits splits); the dot2 kernel's
+    // pair slots: S - 1 per output, zero between launches
+    if (l.s_cap > 1) {
+        int64_t pe = (int64_t)l.s_cap * std::min<int32_t>(max_batch, kGemvMaxBatchPerLaunch);
+        if (max_batch >= kGemmMinBatch) pe = std::max<int64_t>(pe, (int64_t)std::min(l.s_cap, kGemmMaxSplits) * max_batch);
+        l.partial_elems = pe * np;
+        l.pair_elems = (int64_t)(l.s_cap - 1) * std::min<int32_t>(max_batch, kGemvMaxBatchPerLaunch) * np;
+    }
+    l.counters = up((int64_t)sizeof(BindResult));
+    // arrival counters: split-K per tile row and the fused step tails'
+    l.pairs = l.counters + up(gemv_counter_count(tr) * (int64_t)sizeof(int32_t));
+    l.zeroed = l.side = l.pairs + up(l.pair_elems * (int64_t)sizeof(uint64_t));
+    l.lut = l.side + (se12 ? up(tr * tc * (int64_t)kSideBytes) : 0);
+    l.partial = l.lut + (se12 ? (int64_t)kLutBytes : 0);
+    l.total = l.partial + up(l.partial_elems * (int64_t)sizeof(float));
+    return l;
+}
+
+// Fills in the handle's shape and its device memory (`arena`, or an allocation
+// of its own), the zeroed part cleared on `stream`.
+static int bind_common(se12_handle* h, int64_t rows, int64_t cols, int32_t max_batch, void* arena, int64_t arena_bytes,
+                       hipStream_t stream) {
     h->N = rows;
     h->K = cols;
     h->TR = (int32_t)ceil_div(rows, SE12_TILE_ROWS);
@@ -142,42 +182,42 @@ static int bind_common(se12_handle* h, int64_t rows, int64_t cols, int32_t max_b
     h->Np = (int64_t)h->TR * SE12_TILE_ROWS;
     h->T = (int64_t)h->TR * h->TC;
     h->max_batch = max_batch;
-    h->s_cap = std::min<int32_t>(h->TC, kMaxSplits);
     SE12_HIP(hipGetDevice(&h->device));
-    hipDeviceProp_t p;
-    SE12_HIP(hipGetDeviceProperties(&p, h->device));
-    h->cu_count = p.multiProcessorCount;
-    h->lds_per_block = (int64_t)p.sharedMemPerBlock;
-    // split-K workspace: S x (rows per launch) x Np floats, for the dot2
-    // path (up to 4 rows per launch, any split count) and the MFMA path (all
-    // rows in one launch, at most kGemmMaxSplits splits)
-    if (h->s_cap > 1) {
-        int64_t pe = (int64_t)h->s_cap * std::min<int32_t>(max_batch, kGemvMaxBatchPerLaunch);
-        if (max_batch >= kGemmMinBatch) pe = std::max<int64_t>(pe, (int64_t)std::min(h->s_cap, kGemmMaxSplits) * max_batch);
-        h->partial_elems = pe * h->Np;
-        SE12_HIP(hipMalloc(&h->partial, (size_t)h->partial_elems * sizeof(float)));
-        // the dot2 kernel's pair slots: S - 1 per output, zero between launches
-        h->pair_elems = (int64_t)(h->s_cap - 1) * std::min<int32_t>(max_batch, kGemvMaxBatchPerLaunch) * h->Np;
-        SE12_HIP(hipMalloc(&h->pairs, (size_t)h->pair_elems * sizeof(uint64_t)));
-        SE12_HIP(hipMemset(h->pairs, 0, (size_t)h->pair_elems * sizeof(uint64_t)));
+    int cus = 0, lds = 0;
+    SE12_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
+    SE12_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, h->device));
+    h->cu_count = cus;
+    h->lds_per_block = lds;
+    const bool se12 = h->format == SE12_FORMAT_SE12;
+    const ArenaLayout l = arena_layout(rows, cols, max_batch, se12);
+    h->s_cap = l.s_cap;
+    h->partial_elems = l.partial_elems;
+    h->pair_elems = l.pair_elems;
+    if (arena) {
+        if (arena_bytes < l.total || reinterpret_cast<uintptr_t>(arena) % 256 != 0)
+            return fail(SE12_E_CAPACITY, "bind: needs 256-byte aligned memory of %lld bytes, got %lld", (long long)l.total,
+                        (long long)arena_bytes);
+        h->arena = arena;
+    } else {
+        SE12_HIP(hipMalloc(&h->arena, (size_t)l.total));
+        h->owns_arena = true;
     }
-    // arrival counters: split-K per tile row and the fused step tails'
-    const size_t counter_bytes = (size_t)gemv_counter_count(h->TR) * sizeof(int32_t);
-    SE12_HIP(hipMalloc(&h->counters, counter_bytes));
-    SE12_HIP(hipMemset(h->counters, 0, counter_bytes));
+    char* base = static_cast<char*>(h->arena);
+    SE12_HIP(hipMemsetAsync(base, 0, (size_t)l.zeroed, stream));
+    h->counters = reinterpret_cast<int32_t*>(base + l.counters);
+    h->pairs = l.pair_elems ? reinterpret_cast<uint64_t*>(base + l.pairs) : nullptr;
+    h->partial = l.partial_elems ? reinterpret_cast<float*>(base + l.partial) : nullptr;
+    if (se12) {
+        h->side = reinterpret_cast<uint32_t*>(base + l.side);
+        h->lut = reinterpret_cast<uint32_t*>(base + l.lut);
+    }
     return SE12_OK;
 }
 
 static void free_handle(se12_handle* h) {
     if (!h) return;
-    if (h->info) (void)hipFree(h->info);
-    if (h->escpos) (void)hipFree(h->escpos);
-    if (h->side) (void)hipFree(h->side);
+    if (h->owns_arena) (void)hipFree(h->arena);
     if (h->ovf_raw) (void)hipFree(h->ovf_raw);
-    if (h->lut) (void)hipFree(h->lut);
-    if (h->partial) (void)hipFree(h->partial);
-    if (h->counters) (void)hipFree(h->counters);
-    if (h->pairs) (void)hipFree(h->pairs);
     delete h;
 }
 
@@ -195,8 +235,15 @@ static int check_shape(int64_t rows, int64_t cols, int32_t max_batch) {
 
 static DecodeArgs decode_args(const se12_handle* h, uint16_t* out);
 
-int se12_bind(const se12_streams* s, int64_t rows, int64_t cols, int32_t max_batch, void* stream,
-              se12_handle** out) {
+int64_t se12_bind_workspace(int64_t rows, int64_t cols, int32_t max_batch, int32_t format) {
+    if (int rc = check_shape(rows, cols, max_batch)) return rc;
+    if (format != SE12_FORMAT_SE12 && format != SE12_FORMAT_RAW_BF16)
+        return fail(SE12_E_INVALID, "se12_bind_workspace: unknown format %d", format);
+    return arena_layout(rows, cols, max_batch, format == SE12_FORMAT_SE12).total;
+}
+
+static int bind_se12(const se12_streams* s, int64_t rows, int64_t cols, int32_t max_batch, void* arena, int64_t arena_bytes,
+                     void* stream, se12_handle** out) {
     if (!s || !out) return fail(SE12_E_INVALID, "se12_bind: NULL argument");
     *out = nullptr;
     if (int rc = check_shape(rows, cols, max_batch)) return rc;
@@ -214,64 +261,59 @@ int se12_bind(const se12_streams* s, int64_t rows, int64_t cols, int32_t max_bat
     std::memset(h, 0, sizeof *h);
     h->format = SE12_FORMAT_SE12;
     h->s = *s;
-    if (int rc = bind_common(h, rows, cols, max_batch)) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (int rc = bind_common(h, rows, cols, max_batch, arena, arena_bytes, st)) {
         free_handle(h);
         return rc;
     }
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    int64_t* total_dev = nullptr;
-    int64_t totals[2] = {0, 0};  // fallback tiles, tiles with more than the listed escapes
-    uint8_t cb[SE12_CODEBOOK_SIZE] = {0};
-    uint32_t lut[256];
-    hipError_t e = hipMalloc(&h->info, (size_t)h->T * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&h->escpos, (size_t)h->T * sizeof(uint4));
-    if (e == hipSuccess) e = hipMemsetAsync(h->escpos, 0, (size_t)h->T * sizeof(uint4), st);
-    if (e == hipSuccess) e = hipMalloc(&h->side, (size_t)h->T * kSideBytes);
-    if (e == hipSuccess) e = hipMalloc(&h->lut, sizeof lut);
-    if (e == hipSuccess) e = hipMalloc(&total_dev, sizeof totals);
-    if (e == hipSuccess) e = hipMemsetAsync(total_dev, 0, sizeof totals, st);
-    if (e == hipSuccess) e = launch_tile_info(s->fallback_bitmap_dev, s->ec_dev, h->T, h->info, h->escpos, total_dev, st);
-    if (e == hipSuccess) e = launch_side_records(h->info, s->esc_dev, h->escpos, h->T, h->side, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(totals, total_dev, sizeof totals, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(cb, s->codebook_dev, sizeof cb, hipMemcpyDeviceToHost, st);
+    BindResult* result = static_cast<BindResult*>(h->arena);
+    BindResult r{};
+    hipError_t e = launch_bind_tiles(s->fallback_bitmap_dev, s->ec_dev, s->esc_dev, s->codebook_dev, h->T, h->side, h->lut,
+                                     result, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(&r, result, sizeof r, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess) {
-        for (uint32_t b = 0; b < 256; ++b) lut[b] = pair_lut_entry(cb, b);
-        e = hipMemcpyAsync(h->lut, lut, sizeof lut, hipMemcpyHostToDevice, st);
-    }
     // tiles with more escapes than the sidecar lists are decoded once here and
     // read as raw tiles by every kernel
-    if (e == hipSuccess && totals[1] > 0) {
-        e = hipMalloc(&h->ovf_raw, (size_t)totals[1] * SE12_TILE_SIZE * sizeof(int16_t));
+    if (e == hipSuccess && r.overflow_tiles > 0) {
+        e = hipMalloc(&h->ovf_raw, (size_t)r.overflow_tiles * SE12_TILE_SIZE * sizeof(int16_t));
         if (e == hipSuccess) e = launch_overflow_decode(decode_args(h, nullptr), h->ovf_raw, st);
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (total_dev) (void)hipFree(total_dev);
-    // the side records hold everything the kernels read
-    if (e == hipSuccess) {
-        (void)hipFree(h->info);
-        (void)hipFree(h->escpos);
-        h->info = nullptr;
-        h->escpos = nullptr;
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
     }
     if (e != hipSuccess) {
         free_handle(h);
         return fail(SE12_E_HIP, "se12_bind: %s", hipGetErrorString(e));
     }
-    if (totals[0] * SE12_TILE_SIZE != s->fallback_raw_elems) {
+    if ((int64_t)r.fallback_tiles * SE12_TILE_SIZE != s->fallback_raw_elems) {
         free_handle(h);
         return fail(SE12_E_INVALID, "se12_bind: bitmap marks %lld fallback tiles but fallback_raw holds %lld elements",
-                    (long long)totals[0], (long long)s->fallback_raw_elems);
+                    (long long)r.fallback_tiles, (long long)s->fallback_raw_elems);
     }
-    h->n_fallback = totals[0];
-    h->n_overflow = totals[1];
+    h->n_fallback = (int64_t)r.fallback_tiles;
+    h->n_overflow = (int64_t)r.overflow_tiles;
+    std::memcpy(h->codebook, r.codebook, sizeof h->codebook);
     *out = h;
     return SE12_OK;
 }
 
-int se12_bind_raw_bf16(const uint16_t* w, int64_t rows, int64_t cols, int32_t max_batch, void* stream,
-                       se12_handle** out) {
-    (void)stream;
+int se12_bind(const se12_streams* s, int64_t rows, int64_t cols, int32_t max_batch, void* stream, se12_handle** out) {
+    return bind_se12(s, rows, cols, max_batch, nullptr, 0, stream, out);
+}
+
+int se12_bind_in(const se12_streams* s, int64_t rows, int64_t cols, int32_t max_batch, void* workspace,
+                 int64_t workspace_bytes, void* stream, se12_handle** out) {
+    if (!workspace) return fail(SE12_E_INVALID, "se12_bind_in: NULL workspace");
+    return bind_se12(s, rows, cols, max_batch, workspace, workspace_bytes, stream, out);
+}
+
+int se12_handle_codebook(const se12_handle* h, uint8_t codebook_out[15]) {
+    if (!h || !codebook_out) return fail(SE12_E_INVALID, "se12_handle_codebook: NULL argument");
+    if (h->format != SE12_FORMAT_SE12) return fail(SE12_E_INVALID, "se12_handle_codebook: handle is not SE12");
+    std::memcpy(codebook_out, h->codebook, SE12_CODEBOOK_SIZE);
+    return SE12_OK;
+}
+
+static int bind_raw(const uint16_t* w, int64_t rows, int64_t cols, int32_t max_batch, void* arena, int64_t arena_bytes,
+                    void* stream, se12_handle** out) {
     if (!w || !out) return fail(SE12_E_INVALID, "se12_bind_raw_bf16: NULL argument");
     *out = nullptr;
     if (int rc = check_shape(rows, cols, max_batch)) return rc;
@@ -279,12 +321,30 @@ int se12_bind_raw_bf16(const uint16_t* w, int64_t rows, int64_t cols, int32_t ma
     std::memset(h, 0, sizeof *h);
     h->format = SE12_FORMAT_RAW_BF16;
     h->wraw = w;
-    if (int rc = bind_common(h, rows, cols, max_batch)) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    int rc = bind_common(h, rows, cols, max_batch, arena, arena_bytes, st);
+    // the counters are clear before any stream's first product
+    if (rc == SE12_OK) {
+        const hipError_t e = hipStreamSynchronize(st);
+        if (e != hipSuccess) rc = fail(SE12_E_HIP, "se12_bind_raw_bf16: %s", hipGetErrorString(e));
+    }
+    if (rc != SE12_OK) {
         free_handle(h);
         return rc;
     }
     *out = h;
     return SE12_OK;
+}
+
+int se12_bind_raw_bf16(const uint16_t* w, int64_t rows, int64_t cols, int32_t max_batch, void* stream,
+                       se12_handle** out) {
+    return bind_raw(w, rows, cols, max_batch, nullptr, 0, stream, out);
+}
+
+int se12_bind_raw_bf16_in(const uint16_t* w, int64_t rows, int64_t cols, int32_t max_batch, void* workspace,
+                          int64_t workspace_bytes, void* stream, se12_handle** out) {
+    if (!workspace) return fail(SE12_E_INVALID, "se12_bind_raw_bf16_in: NULL workspace");
+    return bind_raw(w, rows, cols, max_batch, workspace, workspace_bytes, stream, out);
 }
 
 int se12_release(se12_handle* h) {
@@ -1235,8 +1295,6 @@ static DecodeArgs decode_args(const se12_handle* h, uint16_t* out) {
     a.codebook = h->s.codebook_dev;
     a.bitmap = h->s.fallback_bitmap_dev;
     a.lut = h->lut;
-    a.info = h->info;
-    a.escpos = h->escpos;
     a.side = h->side;
     a.fb_raw = h->s.fallback_raw_dev;
     a.ovf_raw = h->ovf_raw;

@@ -8,11 +8,11 @@
 // (lws/adapters/cuda/kernels/se12_decode.cu:12-43,
 // lws/adapters/cuda/se12_decoder.py:147-185).
 //
-// Also here: the bind-time per-tile sidecar word. For a fallback tile it holds
-// the tile's rank among all fallback tiles (cumsum(bitmap bits) - 1, as in
-// lws/adapters/cuda/gemv.py:47-53, computed by a single-block scan); for any
-// other tile, which of its four 4-row chunks hold escape codes (one wave per
-// tile reads the tile's `ec` bytes). The kernels read it instead of the bitmap.
+// Also here: bind's per-tile side records. A fallback tile's word holds the
+// tile's rank among all fallback tiles (cumsum(bitmap bits) - 1, as in
+// lws/adapters/cuda/gemv.py:47-53); any other tile's which of its four 4-row
+// chunks hold escape codes, their count and positions (one wave per tile reads
+// the tile's `ec` bytes). The kernels read the records instead of the bitmap.
 #include "se12_device.hpp"
 #include "se12_internal.hpp"
 #include "se12_step_math.hpp"
@@ -239,73 +239,55 @@ hipError_t launch_decode_rows(const DecodeArgs& args, float scale, hipStream_t s
 }
 
 // ---------------------------------------------------------------------------
-// bind-time sidecar words
+// bind: the per-tile side records, the pair table and the tile counts
 // ---------------------------------------------------------------------------
 
-constexpr int kScanThreads = 1024;
+// One wave per tile. Escapes are ranked in row-major order (chunk, then lane,
+// then weight within the lane), the order in which they take the tile's esc
+// slots; the first kListedEscapes positions go into the tile's record. A
+// fallback tile's word holds its rank in the bitmap (counted by its wave:
+// there are few), a tile with more escapes than listed the next free place
+// of the raw buffer bind decodes those into (in no fixed order: the place is
+// only looked up). One kernel for what were a one-block scan of the bitmap, the
+// escape positions, a one-block scan of the counts and the record writes:
+// 9216x2304 __BIND_FIGURES__
+constexpr int kBindThreads = 512;
 
-// exclusive scan of one value per thread over the block (1024 threads)
-__device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* tmp, int64_t* total) {
+__global__ __launch_bounds__(kBindThreads) void bind_tiles_kernel(const uint8_t* bitmap, const uint8_t* ec,
+                                                                   const uint8_t* esc, const uint8_t* codebook, int64_t T,
+                                                                   uint32_t* side, uint32_t* lut, BindResult* result) {
+    constexpr int kWaves = kBindThreads / kWave;
+    __shared__ uint32_t pos[kWaves][kListedEscapes / 2];
+    __shared__ uint32_t over[kWaves], fall[kWaves], base;
     const int tid = threadIdx.x;
-    tmp[tid] = v;
-    __syncthreads();
-    for (int d = 1; d < kScanThreads; d <<= 1) {
-        int64_t u = tid >= d ? tmp[tid - d] : 0;
-        __syncthreads();
-        tmp[tid] += u;
-        __syncthreads();
+    const uint32_t lane = tid & 63u;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (blockIdx.x == 0) {
+        if (tid < 256) lut[tid] = pair_lut_entry(codebook, (uint32_t)tid);
+        if (tid < kCodebook) result->codebook[tid] = codebook[tid];
     }
-    const int64_t incl = tmp[tid];
-    *total = tmp[kScanThreads - 1];
-    __syncthreads();
-    return incl - v;
-}
-
-// fallback tiles: kInfoFallback | rank; other tiles: 0 (escape bits come next)
-__global__ __launch_bounds__(kScanThreads) void fallback_info_kernel(const uint8_t* bitmap, int64_t T, uint32_t* info,
-                                                                     int64_t* total_out) {
-    __shared__ int64_t tmp[kScanThreads];
-    const int tid = threadIdx.x;
-    int64_t chunk = (T + kScanThreads - 1) / kScanThreads;
-    chunk = (chunk + 7) & ~int64_t(7);
-    const int64_t t0 = (int64_t)tid * chunk;
-    const int64_t t1 = t0 + chunk < T ? t0 + chunk : T;
-    int64_t count = 0;
-    for (int64_t t = t0; t < t1; ++t) count += (bitmap[t >> 3] >> (7 - (t & 7))) & 1;
-    int64_t total;
-    int64_t base = block_exclusive_scan(count, tmp, &total);
-    for (int64_t t = t0; t < t1; ++t) {
-        const int bit = (bitmap[t >> 3] >> (7 - (t & 7))) & 1;
-        info[t] = bit ? (kInfoFallback | (uint32_t)base) : 0u;
-        base += bit;
-    }
-    if (tid == 0) *total_out = total;
-}
-
-// escape chunk bits, escape count and listed escape positions of every
-// non-fallback tile: one wave per tile. Escapes are ranked in row-major
-// order (chunk, then lane, then weight within the lane), the order in which
-// they take the tile's esc slots.
-constexpr int kInfoWaves = 4;
-
-__global__ __launch_bounds__(kInfoWaves * kWave) void escape_info_kernel(const uint8_t* ec, int64_t T, uint32_t* info,
-                                                                          uint4* escpos) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const int64_t tile = (int64_t)blockIdx.x * kInfoWaves + (threadIdx.x >> 6);
-    if (tile >= T) return;
-    const uint8_t* ect = ec + tile * (kTile / 2) + 8u * lane;
-    uint16_t* pos = reinterpret_cast<uint16_t*>(escpos + tile);
+    const int64_t tile = (int64_t)blockIdx.x * kWaves + w;
+    const bool here = tile < T;
+    const int64_t t = here ? tile : T - 1;   // a wave past the last tile works on it, and stores nothing
+    const uint8_t* ect = ec + t * (kTile / 2) + 8u * lane;
+    uint2 e[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) e[j] = *reinterpret_cast<const uint2*>(ect + 512 * j);
+    const uint32_t slots = reinterpret_cast<const uint32_t*>(esc + t * kEscBudget)[(lane - 1u) & 3u];
+    const bool fallback = here && ((bitmap[t >> 3] >> (7 - (t & 7))) & 1u) != 0u;
+    if (lane < kListedEscapes / 2) pos[w][lane] = 0u;
+    __builtin_amdgcn_wave_barrier();
+    uint16_t* listed = reinterpret_cast<uint16_t*>(pos[w]);
     uint32_t mask = 0, run = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const uint2 e = *reinterpret_cast<const uint2*>(ect + 512 * j);
-        uint32_t t0 = escape_nibbles(e.x), t1 = escape_nibbles(e.y);
+        uint32_t t0 = escape_nibbles(e[j].x), t1 = escape_nibbles(e[j].y);
         const uint32_t cnt = __popc(t0) + __popc(t1);
         const uint32_t incl = wave_incl_scan(cnt);
         const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
         if (total) mask |= 1u << j;
         uint32_t r = run + incl - cnt;
-        const uint32_t base = (4u * j + (lane >> 4)) * kTileCols + 16u * (lane & 15u);
+        const uint32_t first = (4u * j + (lane >> 4)) * kTileCols + 16u * (lane & 15u);
         while (t0 | t1) {
             uint32_t p;
             if (t0) {
@@ -315,39 +297,52 @@ __global__ __launch_bounds__(kInfoWaves * kWave) void escape_info_kernel(const u
                 p = 8u + ((uint32_t)__builtin_ctz(t1) >> 2);
                 t1 &= t1 - 1u;
             }
-            if (r < kListedEscapes) pos[r] = (uint16_t)(base + p);
+            if (r < kListedEscapes) listed[r] = (uint16_t)(first + p);
             ++r;
         }
         run += total;
     }
-    if (lane == 0 && !info_is_fallback(info[tile]))
-        info[tile] = mask | ((run < kInfoCountMax ? run : kInfoCountMax) << kInfoCountShift);
+    const bool too_many = here && !fallback && run > kListedEscapes;
+    if (lane == 0) {
+        over[w] = too_many ? 1u : 0u;
+        fall[w] = fallback ? 1u : 0u;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t n_over = 0, n_fall = 0;
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) {
+            n_over += over[k];
+            n_fall += fall[k];
+        }
+        base = n_over ? (uint32_t)__hip_atomic_fetch_add(&result->overflow_tiles, (unsigned long long)n_over,
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                      : 0u;
+        if (n_fall)
+            __hip_atomic_fetch_add(&result->fallback_tiles, (unsigned long long)n_fall, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    uint32_t info = mask | ((run < kInfoCountMax ? run : kInfoCountMax) << kInfoCountShift);
+    if (fallback) {
+        info = kInfoFallback | (uint32_t)fallback_rank(bitmap, t, lane);
+    } else if (too_many) {
+        uint32_t rank = base;
+        for (int k = 0; k < w; ++k) rank += over[k];
+        info = kInfoFallback | kInfoOverflow | rank;
+    }
+    if (here && lane < kSideWords)
+        side[tile * kSideWords + lane] = lane == 0   ? info
+                                         : lane <= 4 ? slots
+                                         : lane <= 8 ? pos[w][lane - 5]
+                                                     : 0u;
 }
 
-// Tiles with more than kListedEscapes escapes become raw tiles: rank them
-// (kInfoFallback | kInfoOverflow | rank) and count them.
-__global__ __launch_bounds__(kScanThreads) void overflow_info_kernel(int64_t T, uint32_t* info, int64_t* total_out) {
-    __shared__ int64_t tmp[kScanThreads];
-    const int tid = threadIdx.x;
-    const int64_t chunk = (T + kScanThreads - 1) / kScanThreads;
-    const int64_t t0 = (int64_t)tid * chunk;
-    const int64_t t1 = t0 + chunk < T ? t0 + chunk : T;
-    auto over = [&](int64_t t) {
-        const uint32_t v = info[t];
-        return !info_is_fallback(v) && info_escapes(v) > kListedEscapes;
-    };
-    int64_t count = 0;
-    for (int64_t t = t0; t < t1; ++t) count += over(t) ? 1 : 0;
-    int64_t total;
-    int64_t base = block_exclusive_scan(count, tmp, &total);
-    for (int64_t t = t0; t < t1; ++t)
-        if (over(t)) info[t] = kInfoFallback | kInfoOverflow | (uint32_t)base++;
-    if (tid == 0) *total_out = total;
-}
+// Decodes every tile with more than the listed escapes into raw[rank]
+// (tile-local order, the layout of the format's fallback tiles), ranking its
+// escapes per chunk (lanes, then weights within a lane): one wave per tile.
+constexpr int kInfoWaves = 4;
 
-// Decodes every overflow tile into raw[rank] (tile-local order, the layout of
-// the format's fallback tiles), ranking its escapes per chunk (lanes, then
-// weights within a lane): one wave per tile.
 __global__ __launch_bounds__(kInfoWaves * kWave) void overflow_decode_kernel(DecodeArgs a, int16_t* raw) {
     SE12_DECLARE_LUT(lut);
     const uint32_t lane = threadIdx.x & 63u;
@@ -355,7 +350,7 @@ __global__ __launch_bounds__(kInfoWaves * kWave) void overflow_decode_kernel(Dec
     lds_barrier();
     const int64_t tile = (int64_t)blockIdx.x * kInfoWaves + (threadIdx.x >> 6);
     if (tile >= a.T) return;
-    const uint32_t info = a.info[tile];
+    const uint32_t info = a.side[tile * kSideWords];
     if (!info_is_overflow(info)) return;
     TileLoads t;
     load_tile(t, a.sm, a.ec, tile, lane);
@@ -374,49 +369,17 @@ __global__ __launch_bounds__(kInfoWaves * kWave) void overflow_decode_kernel(Dec
     }
 }
 
-// The side record of every tile (one thread per record word).
-__global__ void side_record_kernel(const uint32_t* info, const uint8_t* esc, const uint4* escpos, int64_t T,
-                                   uint32_t* side) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= T * kSideWords) return;
-    const int64_t t = i / kSideWords;
-    const int k = (int)(i % kSideWords);
-    uint32_t v = 0;
-    if (k == 0)
-        v = info[t];
-    else if (k <= 4)
-        v = reinterpret_cast<const uint32_t*>(esc + t * kEscBudget)[k - 1];
-    else if (k <= 8)
-        v = reinterpret_cast<const uint32_t*>(escpos + t)[k - 5];
-    side[i] = v;
-}
-
-hipError_t launch_side_records(const uint32_t* info, const uint8_t* esc, const uint4* escpos, int64_t T, uint32_t* side,
-                               hipStream_t stream) {
-    if (T == 0) return hipSuccess;
-    const int64_t n = T * kSideWords;
-    hipLaunchKernelGGL(side_record_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, stream, info, esc, escpos, T,
-                       side);
-    return hipGetLastError();
-}
-
 hipError_t launch_overflow_decode(const DecodeArgs& a, int16_t* raw, hipStream_t stream) {
     const int64_t blocks = (a.T + kInfoWaves - 1) / kInfoWaves;
     hipLaunchKernelGGL(overflow_decode_kernel, dim3((uint32_t)blocks), dim3(kInfoWaves * kWave), 0, stream, a, raw);
     return hipGetLastError();
 }
 
-hipError_t launch_tile_info(const uint8_t* bitmap, const uint8_t* ec, int64_t T, uint32_t* info, uint4* escpos,
-                            int64_t* total, hipStream_t stream) {
-    hipLaunchKernelGGL(fallback_info_kernel, dim3(1), dim3(kScanThreads), 0, stream, bitmap, T, info, total);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || T == 0) return e;
-    const int64_t blocks = (T + kInfoWaves - 1) / kInfoWaves;
-    hipLaunchKernelGGL(escape_info_kernel, dim3((uint32_t)blocks), dim3(kInfoWaves * kWave), 0, stream, ec, T, info,
-                       escpos);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(overflow_info_kernel, dim3(1), dim3(kScanThreads), 0, stream, T, info, total + 1);
+hipError_t launch_bind_tiles(const uint8_t* bitmap, const uint8_t* ec, const uint8_t* esc, const uint8_t* codebook, int64_t T,
+                             uint32_t* side, uint32_t* lut, BindResult* result, hipStream_t stream) {
+    const int64_t blocks = (T + kBindThreads / kWave - 1) / (kBindThreads / kWave);
+    hipLaunchKernelGGL(bind_tiles_kernel, dim3((uint32_t)blocks), dim3(kBindThreads), 0, stream, bitmap, ec, esc, codebook, T,
+                       side, lut, result);
     return hipGetLastError();
 }
 

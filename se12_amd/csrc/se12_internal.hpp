@@ -142,8 +142,6 @@ struct DecodeArgs {
     const uint8_t* codebook;
     const uint8_t* bitmap;
     const uint32_t* lut;      // [256] pair table built at bind time
-    const uint32_t* info;     // [T] per-tile sidecar word
-    const uint4* escpos;      // [T] listed escape positions
     const uint32_t* side;     // [T, 16] per-tile side records
     const int16_t* fb_raw;
     const int16_t* ovf_raw;
@@ -301,14 +299,15 @@ hipError_t launch_gemm_rx(const GemvGroupArgs& a, int batch, const GemvPlan& p, 
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream, int cu_count);
 // scale 0: the weights as they are
 hipError_t launch_decode_rows(const DecodeArgs& a, float scale, hipStream_t stream);
-// Bind-time sidecar: one word per tile (fallback rank, or the chunks holding
-// escape codes) and the fallback tile count.
-// total[0] = fallback tiles, total[1] = tiles with more than the listed escapes
-hipError_t launch_tile_info(const uint8_t* bitmap, const uint8_t* ec, int64_t T, uint32_t* info, uint4* escpos, int64_t* total,
-                            hipStream_t stream);
+// What bind reads back: zero before launch_bind_tiles (but the codebook).
+struct BindResult {
+    unsigned long long fallback_tiles;
+    unsigned long long overflow_tiles;    // tiles with more than the listed escapes
+    uint8_t codebook[16];
+};
+hipError_t launch_bind_tiles(const uint8_t* bitmap, const uint8_t* ec, const uint8_t* esc, const uint8_t* codebook, int64_t T,
+                             uint32_t* side, uint32_t* lut, BindResult* result, hipStream_t stream);
 hipError_t launch_overflow_decode(const DecodeArgs& a, int16_t* raw, hipStream_t stream);
-hipError_t launch_side_records(const uint32_t* info, const uint8_t* esc, const uint4* escpos, int64_t T, uint32_t* side,
-                               hipStream_t stream);
 // histogram and codebook (also to codebook_out on the device unless NULL)
 hipError_t launch_encode_histogram(const EncodeArgs& a, int cu_count, uint8_t* codebook_out, hipStream_t stream);
 hipError_t launch_encode_codes(const EncodeArgs& a, const uint8_t codebook[16], hipStream_t stream);

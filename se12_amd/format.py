@@ -248,12 +248,14 @@ def validate_streams(tensor: Any) -> None:
         raise ValueError(f"bitmap marks {nfb} fallback tiles but fallback_raw holds {raw.size // TILE_SIZE}")
 
 
-def validate_device_streams(dt: "Se12DeviceTensor") -> None:
+def validate_device_streams(dt: "Se12DeviceTensor", codebook: bool = True) -> None:
     """The device-side counterpart of `validate_streams`: every stream a torch
     tensor on one GPU, contiguous, of the right dtype and size for the shape
     (the library binds to these pointers and its kernels read every byte the
     shape implies). The fallback count against the bitmap is checked by the
-    library at bind."""
+    library at bind. codebook=False leaves out the comparison of the host
+    codebook with the device's, which copies the device's to the host
+    (`check_codebook`: bind compares what the library read)."""
     import torch
 
     if dt.rows <= 0 or dt.cols <= 0:
@@ -279,7 +281,12 @@ def validate_device_streams(dt: "Se12DeviceTensor") -> None:
     if not isinstance(raw, torch.Tensor) or raw.device != device or raw.dtype != torch.int16 \
             or raw.numel() % TILE_SIZE != 0 or not raw.is_contiguous():
         raise ValueError(f"stream fallback_raw must be whole contiguous int16 tiles on {device}")
-    if tuple(int(c) for c in dt.codebook_host) != tuple(int(c) for c in dt.codebook.cpu().tolist()):
+    if codebook:
+        check_codebook(dt, dt.codebook.cpu().tolist())
+
+
+def check_codebook(dt: "Se12DeviceTensor", device_codebook) -> None:
+    if tuple(int(c) for c in dt.codebook_host) != tuple(int(c) for c in device_codebook):
         raise ValueError("codebook_host differs from the device codebook")
 
 

@@ -36,6 +36,7 @@ from .format import (
     Bf16Weights,
     Se12DeviceTensor,
     bitmap_bytes,
+    check_codebook,
     tile_grid,
     validate_device_streams,
 )
@@ -51,7 +52,7 @@ def _device_of(t: torch.Tensor) -> torch.device:
 
 def _as_device_tensor(tensor: Any, device=None) -> Se12DeviceTensor:
     if isinstance(tensor, Se12DeviceTensor):
-        validate_device_streams(tensor)
+        validate_device_streams(tensor, codebook=False)   # bind_se12 compares the codebook bind reads
         if device is not None and tensor.sm.device != torch.device(device):
             raise ValueError(f"SE12 streams on {tensor.sm.device}, requested {device}")
         return tensor
@@ -73,16 +74,21 @@ def _require(t: Any, name: str, dtype: torch.dtype, shape: tuple, device: torch.
 
 
 class _Handle:
-    """Owns one se12_handle*; released when garbage-collected."""
+    """Owns one se12_handle*; released when garbage-collected. `workspace` is
+    the tensor the library keeps the handle's device data in: it goes back to
+    torch's allocator once the release has waited for the device, so no stream
+    the handle was used on can still read it."""
 
-    def __init__(self, raw: ctypes.c_void_p, keepalive: tuple) -> None:
+    def __init__(self, raw: ctypes.c_void_p, keepalive: tuple, workspace: torch.Tensor | None = None) -> None:
         self.raw = raw
         self._keepalive = keepalive  # the tensors the handle points into
+        self._workspace = workspace
 
     def release(self) -> None:
         if self.raw:
             nat.lib().se12_release(self.raw)
             self.raw = ctypes.c_void_p(None)
+            self._workspace = None
 
     def __del__(self) -> None:
         try:
@@ -107,9 +113,23 @@ def bind_se12(dt: Se12DeviceTensor, max_batch: int = nat.MAX_BATCH) -> _Handle:
         fallback_raw_elems=int(dt.fallback_raw.numel()),
     )
     h = ctypes.c_void_p()
+    lib = nat.lib()
     with torch.cuda.device(dt.sm.device):
-        nat.check(nat.lib().se12_bind(ctypes.byref(s), dt.rows, dt.cols, max_batch, nat.stream_ptr(), ctypes.byref(h)))
-    return _Handle(h, (dt,))
+        ws = _bind_workspace(dt.rows, dt.cols, max_batch, nat.FORMAT_SE12, dt.sm.device)
+        nat.check(lib.se12_bind_in(ctypes.byref(s), dt.rows, dt.cols, max_batch, nat.ptr(ws), ws.numel(), nat.stream_ptr(),
+                                   ctypes.byref(h)))
+    handle = _Handle(h, (dt,), ws)
+    cb = (ctypes.c_uint8 * CODEBOOK_SIZE)()
+    nat.check(lib.se12_handle_codebook(h, cb))
+    check_codebook(dt, cb)
+    return handle
+
+
+def _bind_workspace(rows: int, cols: int, max_batch: int, fmt: int, device) -> torch.Tensor:
+    n = nat.lib().se12_bind_workspace(rows, cols, max_batch, fmt)
+    if n < 0:
+        nat.check(n)
+    return torch.empty(n, dtype=torch.uint8, device=device)
 
 
 def bind_raw_bf16(w: torch.Tensor, max_batch: int = nat.MAX_BATCH) -> _Handle:
@@ -118,8 +138,10 @@ def bind_raw_bf16(w: torch.Tensor, max_batch: int = nat.MAX_BATCH) -> _Handle:
     w = w.contiguous()
     h = ctypes.c_void_p()
     with torch.cuda.device(w.device):
-        nat.check(nat.lib().se12_bind_raw_bf16(nat.ptr(w), w.shape[0], w.shape[1], max_batch, nat.stream_ptr(), ctypes.byref(h)))
-    return _Handle(h, (w,))
+        ws = _bind_workspace(w.shape[0], w.shape[1], max_batch, nat.FORMAT_RAW_BF16, w.device)
+        nat.check(nat.lib().se12_bind_raw_bf16_in(nat.ptr(w), w.shape[0], w.shape[1], max_batch, nat.ptr(ws), ws.numel(),
+                                                  nat.stream_ptr(), ctypes.byref(h)))
+    return _Handle(h, (w,), ws)
 
 
 def _launch_struct(launch: LaunchConfiguration | None):
