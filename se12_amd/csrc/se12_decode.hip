@@ -250,7 +250,7 @@ hipError_t launch_decode_rows(const DecodeArgs& args, float scale, hipStream_t s
 // of the raw buffer bind decodes those into (in no fixed order: the place is
 // only looked up). One kernel for what were a one-block scan of the bitmap, the
 // escape positions, a one-block scan of the counts and the record writes:
-// 9216x2304 __BIND_FIGURES__
+// 9216x2304 18 us in four launches -> 5.5.
 constexpr int kBindThreads = 512;
 
 __global__ __launch_bounds__(kBindThreads) void bind_tiles_kernel(const uint8_t* bitmap, const uint8_t* ec,
