@@ -100,6 +100,26 @@ int se12_step_logits_argmax_advance(const void* logits, int32_t dtype, int64_t s
                                     int64_t token_stride, int64_t* step, int64_t* pos, void* workspace,
                                     int64_t workspace_bytes, void* stream);
 
+/* Attention of a whole prompt: qkv [batch, tokens, stride] BF16 holds each
+ * token's heads query heads, then kv_heads key and kv_heads value heads of
+ * head_dim (64, 128 or 256). q (in place) and k are rotated (x cos +
+ * rotate_half(x) sin, each product and the sum rounded to BF16; cos, sin
+ * [tokens, head_dim] BF16), the keys and values written to the caches of
+ * se12_step_attention at positions 0 .. tokens - 1, and out [batch, tokens,
+ * heads * head_dim] BF16 = softmax(softcap tanh(q . k scaling / softcap)) v over
+ * positions max(0, t - window + 1) .. t (window 0 = all), scores and sums in
+ * FP32, probabilities rounded to BF16. 0 < softcap <= 64; max_len >= tokens and
+ * a multiple of 8; stride a multiple of 8; tensors 16-byte aligned (out 8).
+ * `workspace`: se12_step_prefill_workspace() bytes, contents indifferent; calls
+ * sharing it must not run concurrently. Two launches; not for use under
+ * concurrent writes to the caches. */
+int64_t se12_step_prefill_workspace(int32_t batch, int32_t tokens, int32_t heads, int32_t kv_heads, int32_t head_dim);
+
+int se12_step_prefill_attention(uint16_t* qkv, int64_t stride, const uint16_t* cos, const uint16_t* sin,
+                                uint16_t* k_cache_t, uint16_t* v_cache, uint16_t* out, int32_t batch, int32_t tokens,
+                                int32_t heads, int32_t kv_heads, int32_t head_dim, int32_t max_len, float scaling,
+                                float softcap, int32_t window, void* workspace, int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

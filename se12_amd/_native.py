@@ -174,6 +174,11 @@ SIGNATURES = {
         [c_void_p, c_void_p, c_void_p, c_i32, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i32, c_i32,
          c_i32, c_i32, c_i32, ctypes.c_float, ctypes.c_float, c_i32, c_void_p, c_i64, c_void_p],
     ),
+    "se12_step_prefill_workspace": (c_i64, [c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "se12_step_prefill_attention": (
+        c_i32, [c_void_p, c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
+                ctypes.c_float, ctypes.c_float, c_i32, c_void_p, c_i64, c_void_p],
+    ),
     "se12_step_gelu_mul": (c_i32, [c_void_p, c_void_p, c_i32, c_i64, c_void_p, c_i32, c_i32, c_void_p]),
     "se12_step_logits_workspace": (c_i64, [c_i32, c_i32]),
     "se12_step_logits_argmax": (

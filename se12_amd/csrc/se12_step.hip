@@ -907,6 +907,40 @@ __global__ void gelu_mul_kernel(const void* gate, const void* up, int64_t stride
     out[i] = gelu_mul_bf16(load_as_bf16<DT>(gate, r * stride + c), load_as_bf16<DT>(up, r * stride + c));
 }
 
+// 8 consecutive values of an FP32 or BF16 tensor, rounded to BF16 (16-byte
+// aligned)
+template <int DT>
+__device__ __forceinline__ void load8_as_bf16(const void* p, int64_t i, float* v) {
+    if constexpr (DT == SE12_STEP_F32) {
+        const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i);
+        const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i + 4);
+        v[0] = round_bf16(a.x); v[1] = round_bf16(a.y); v[2] = round_bf16(a.z); v[3] = round_bf16(a.w);
+        v[4] = round_bf16(b.x); v[5] = round_bf16(b.y); v[6] = round_bf16(b.z); v[7] = round_bf16(b.w);
+    } else {
+        unpack8(*reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + i), v);
+    }
+}
+
+// Rows of whole 8-column pieces (cols and stride multiples of 8, 16-byte
+// aligned tensors) on more values than a wave per CU holds: a piece per
+// thread, the row from the grid. Bound by the bytes and the tanh: 1,024 x 9,216
+// BF16 18.7 -> 11.4 us (5 TB/s) against an element per thread.
+template <int DT>
+__global__ __launch_bounds__(256) void gelu_mul8_kernel(const void* gate, const void* up, int64_t stride, uint16_t* out,
+                                                        int cols) {
+    const int64_t r = blockIdx.y;
+    const int c = 8 * (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (c >= cols) return;
+    float g[8], u[8];
+    load8_as_bf16<DT>(gate, r * stride + c, g);
+    load8_as_bf16<DT>(up, r * stride + c, u);
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        o[k] = f_to_bf16x2(gelu_tanh_bf16(g[2 * k]) * u[2 * k], gelu_tanh_bf16(g[2 * k + 1]) * u[2 * k + 1]);
+    *reinterpret_cast<uint4*>(out + r * cols + c) = make_uint4(o[0], o[1], o[2], o[3]);
+}
+
 // ---------------------------------------------------------------------------
 // logits: blocks over vocabulary slices of kArgmaxPer x 256 logits per row
 // ---------------------------------------------------------------------------
@@ -1027,11 +1061,9 @@ __global__ void advance_kernel(int64_t* pos, int64_t* step) {
 
 }  // namespace se12step
 
-using namespace se12step;
+namespace se12step {
 
-namespace {
-
-thread_local char g_step_err[256] = "";
+static thread_local char g_step_err[256] = "";
 
 int step_fail(const char* msg) {
     snprintf(g_step_err, sizeof g_step_err, "%s", msg);
@@ -1052,9 +1084,20 @@ int step_launched() {
     return SE12_STEP_OK;
 }
 
+const char* step_error() { return g_step_err; }
+
+}  // namespace se12step
+
+using namespace se12step;
+
+namespace {
+
 bool dtype_ok(int32_t d) { return d == SE12_STEP_F32 || d == SE12_STEP_BF16; }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// values from which gelu_mul8_kernel fills the CUs (256 x 4 waves x 64 lanes x 8)
+constexpr int64_t kGelu8Min = 524288;
 
 int64_t up256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
@@ -1137,7 +1180,7 @@ ArgmaxLayout argmax_layout(int32_t rows, int32_t vocab) {
 
 extern "C" {
 
-const char* se12_step_last_error(void) { return g_step_err; }
+const char* se12_step_last_error(void) { return step_error(); }
 
 int se12_step_rmsnorm(const void* in, int32_t in_dtype, int64_t in_stride, const uint16_t* w1, uint16_t* residual,
                       const uint16_t* w2, uint16_t* out, int32_t rows, int32_t hidden, float eps, float in_scale,
@@ -1229,6 +1272,15 @@ int se12_step_gelu_mul(const void* gate, const void* up, int32_t dtype, int64_t 
     const int64_t n = (int64_t)rows * cols;
     const dim3 grid((unsigned)((n + 255) / 256));
     const hipStream_t st = static_cast<hipStream_t>(stream);
+    if (n >= kGelu8Min && rows <= 65535 && cols % 8 == 0 && stride % 8 == 0 && aligned16(gate) && aligned16(up) &&
+        aligned16(out)) {
+        const dim3 grid8((unsigned)((cols / 8 + 255) / 256), rows);
+        if (dtype == SE12_STEP_F32)
+            hipLaunchKernelGGL(gelu_mul8_kernel<SE12_STEP_F32>, grid8, dim3(256), 0, st, gate, up, stride, out, cols);
+        else
+            hipLaunchKernelGGL(gelu_mul8_kernel<SE12_STEP_BF16>, grid8, dim3(256), 0, st, gate, up, stride, out, cols);
+        return step_launched();
+    }
     if (dtype == SE12_STEP_F32)
         hipLaunchKernelGGL(gelu_mul_kernel<SE12_STEP_F32>, grid, dim3(256), 0, st, gate, up, stride, out, rows, cols);
     else

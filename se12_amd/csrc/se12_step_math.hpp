@@ -89,4 +89,10 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
     return r;
 }
 
+// host: the calling thread's error message (se12_step.hip) and the status of
+// a launch
+int step_fail(const char* msg);
+int step_fail(const char* who, const char* msg);
+int step_launched();
+
 }  // namespace se12step

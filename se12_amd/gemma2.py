@@ -58,6 +58,8 @@ class Gemma2Shape:
 
 GEMMA2_2B = Gemma2Shape()
 PROJECTIONS = ("q", "k", "v", "o", "gate", "up", "down")
+# projections of one input, multiplied as one matrix in the prompt pass
+PREFILL_GROUPS = (("q", "k", "v"), ("o",), ("gate", "up"), ("down",))
 
 
 def projection_shapes(s: Gemma2Shape) -> dict[str, tuple[int, int]]:
@@ -138,8 +140,8 @@ class _Backend:
         self.w = w
         self.layers = []
         if kind == "se12":
-            biggest = max(max(t.numel() for n, t in lw.items() if n in PROJECTIONS) for lw in w.layers)
-            self.scratch = scratch if scratch is not None else torch.empty(
+            biggest = max(sum(lw[n].numel() for n in group) for lw in w.layers for group in PREFILL_GROUPS)
+            self.scratch = scratch if scratch is not None and scratch.numel() >= biggest else torch.empty(
                 biggest, dtype=torch.bfloat16, device=w.embed.device)
         for li, lw in enumerate(w.layers):
             if kind == "se12":
@@ -157,11 +159,20 @@ class _Backend:
             self.lm_head = RawBf16MatVecKernel(w.embed, max_batch=max_batch)
 
     # -- prefill: exact products --------------------------------------------
-    def prefill_weight(self, li: int, name: str) -> torch.Tensor:
+    def prefill_weight(self, li: int, *names: str) -> torch.Tensor:
+        """The BF16 weight of a projection, or of several stacked by rows (valid
+        until the next call: the SE12 backend decodes into its scratch)."""
         if self.kind == "se12":
-            k = self.layers[li][name]
-            return k.decode_into(self.scratch[: k.rows * k.cols].view(k.rows, k.cols))
-        return self.w.layers[li][name]
+            at, ks = 0, [self.layers[li][n] for n in names]
+            for k in ks:
+                k.decode_into(self.scratch[at: at + k.rows * k.cols].view(k.rows, k.cols))
+                at += k.rows * k.cols
+            return self.scratch[:at].view(-1, ks[0].cols)
+        if len(names) == 1:
+            return self.w.layers[li][names[0]]
+        if self.kind == "bf16":
+            return self.layers[li]["qkv" if names[0] == "q" else "gate_up"]
+        return torch.cat([self.w.layers[li][n] for n in names])
 
     # -- decode steps -------------------------------------------------------
     def grouped(self, li: int, names: tuple[str, ...], x: torch.Tensor) -> list[torch.Tensor]:
@@ -302,6 +313,69 @@ class Gemma2Decoder:
     def prefill(self, prompt: torch.Tensor) -> torch.Tensor:
         """Runs the prompt [batch, T] (exact products), fills the KV cache and
         returns the first generated token per sequence."""
+        T = prompt.shape[1]
+        h = self._prefill_kernels(prompt) if self._prefill_kernels_serve(T) else self._prefill_ops(prompt)
+        logits = self.be.logits(h)
+        logits = torch.tanh(logits / self.s.final_softcap) * self.s.final_softcap
+        self.last_logits.copy_(logits)
+        first = logits.argmax(-1)
+        self.ids.copy_(first)
+        self.pos.fill_(T)
+        self.tokens.zero_()
+        self.tokens[:, 0] = first
+        self.step_index.fill_(1)
+        return first
+
+    def _prefill_kernels_serve(self, T: int) -> bool:
+        """What se12_step_prefill_attention and se12_step_rmsnorm take; any
+        other shape runs the framework ops."""
+        s = self.s
+        return (s.head_dim in (64, 128, 256) and 0.0 < s.attn_softcap <= 64.0 and s.hidden <= 8192 and 0 < T <= self.max_len
+                and s.heads % s.kv_heads == 0)
+
+    def _prefill_kernels(self, prompt: torch.Tensor) -> torch.Tensor:
+        """The prompt pass with one library launch each for the norms, the
+        rotary embedding and cache slots, the attention and the MLP gate around
+        the products (11 to 16 launches per layer; the framework ops below take
+        ~85, each a pass over the activations or the T x T scores). Returns the
+        normalised hidden state of the last position [B, hidden]."""
+        s, B, T = self.s, self.batch, prompt.shape[1]
+        n, lib, st, ck = B * T, nat.lib(), nat.stream_ptr(), nat.step_check
+        bf16 = nat.STEP_BF16
+
+        def buf(*shape):
+            return torch.empty(shape, dtype=torch.bfloat16, device=self.dev)
+
+        x, h = buf(n, s.hidden), buf(n, s.hidden)
+        att, m = buf(n, s.heads * s.head_dim), buf(n, s.intermediate)
+        ws_bytes = lib.se12_step_prefill_workspace(B, T, s.heads, s.kv_heads, s.head_dim)
+        if ws_bytes < 0:
+            ck(ws_bytes)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=self.dev)
+        cos, sin = self._rope(torch.arange(T, device=self.dev))
+        emb = self.be.embed_rows(prompt)
+        ck(lib.se12_step_rmsnorm(nat.ptr(emb), bf16, s.hidden, nat.ptr(self.w.layers[0]["input_norm"]), nat.ptr(x), None,
+                                 nat.ptr(h), n, s.hidden, s.eps, float(self.embed_scale.item()), 0, st))
+
+        def norm(y, w1, w2):
+            ck(lib.se12_step_rmsnorm(nat.ptr(y), bf16, s.hidden, nat.ptr(w1), nat.ptr(x), nat.ptr(w2), nat.ptr(h), n,
+                                     s.hidden, s.eps, 0.0, 1, st))
+
+        for li, lw in enumerate(self.w.layers):
+            qkv = F.linear(h, self.be.prefill_weight(li, "q", "k", "v"))
+            ck(lib.se12_step_prefill_attention(
+                nat.ptr(qkv), qkv.shape[1], nat.ptr(cos), nat.ptr(sin), nat.ptr(self.kt[li]), nat.ptr(self.v[li]),
+                nat.ptr(att), B, T, s.heads, s.kv_heads, s.head_dim, self.max_len, self.scaling, s.attn_softcap,
+                0 if li % 2 else s.sliding_window, nat.ptr(ws), ws_bytes, st))
+            norm(F.linear(att, self.be.prefill_weight(li, "o")), lw["post_attn_norm"], lw["pre_ffw_norm"])
+            gu = F.linear(h, self.be.prefill_weight(li, "gate", "up"))
+            ck(lib.se12_step_gelu_mul(gu.data_ptr(), gu.data_ptr() + 2 * s.intermediate, bf16, 2 * s.intermediate, nat.ptr(m),
+                                      n, s.intermediate, st))
+            nxt = self.w.layers[li + 1]["input_norm"] if li + 1 < s.layers else self.w.final_norm
+            norm(F.linear(m, self.be.prefill_weight(li, "down")), lw["post_ffw_norm"], nxt)
+        return h.view(B, T, s.hidden)[:, -1].contiguous()
+
+    def _prefill_ops(self, prompt: torch.Tensor) -> torch.Tensor:
         s, B = self.s, self.batch
         T = prompt.shape[1]
         x = (self.be.embed_rows(prompt) * self.embed_scale).view(B, T, s.hidden)
@@ -332,15 +406,7 @@ class Gemma2Decoder:
             mm = F.gelu(F.linear(h, self.be.prefill_weight(li, "gate")), approximate="tanh") * \
                 F.linear(h, self.be.prefill_weight(li, "up"))
             x = x + rms_norm(F.linear(mm, self.be.prefill_weight(li, "down")), lw["post_ffw_norm"], s.eps)
-        logits = self._finish(x[:, -1, :].contiguous())
-        self.last_logits.copy_(logits)
-        first = logits.argmax(-1)
-        self.ids.copy_(first)
-        self.pos.fill_(T)
-        self.tokens.zero_()
-        self.tokens[:, 0] = first
-        self.step_index.fill_(1)
-        return first
+        return rms_norm(x[:, -1, :].contiguous(), self.w.final_norm, s.eps)
 
     # -- one decode step (captured) -----------------------------------------
     def _step(self) -> None:

@@ -170,3 +170,31 @@ def test_fused_tails_agree_with_separate_step_kernels(gpu):
     assert torch.equal(a.kt[0], b.kt[0]) and torch.equal(a.v[0], b.v[0])
     assert _close(a.kt[1][..., 10], b.kt[1][..., 10]) and _close(a.v[1][:, :, 10], b.v[1][:, :, 10])
     assert _close(a.residual, b.residual) and _close(a.last_logits, b.last_logits)
+
+
+@pytest.mark.parametrize("backend", ["se12", "bf16"])
+@pytest.mark.parametrize("head_dim,batch,length", [(64, 2, 45), (128, 1, 70), (256, 3, 9)])
+def test_prompt_pass_through_the_kernels_agrees_with_framework_ops(gpu, backend, head_dim, batch, length):
+    """The same last hidden state and caches as the framework-op pass within BF16 rounding (its scores go through BF16 four
+    times, the kernels' none), for heads the kernels take; others run the framework ops."""
+    sh = Gemma2Shape(layers=2, hidden=256, intermediate=512, heads=4, kv_heads=2, head_dim=head_dim, vocab=512, sliding_window=20)
+    w = Gemma2Weights.random(sh, gpu, seed=12)
+    enc = _encoded(w) if backend == "se12" else None
+    d = Gemma2Decoder(w, backend, batch, max_len=length + 3, encoded=enc)
+    assert d._prefill_kernels_serve(length) and not d._prefill_kernels_serve(d.max_len + 1)
+    prompt = _prompt(gpu, batch, length)
+    with torch.no_grad():
+        a = d._prefill_kernels(prompt)
+        kt, v = [t.clone() for t in d.kt], [t.clone() for t in d.v]
+        b = d._prefill_ops(prompt)
+    assert _close(a, b, 0.05)
+    assert torch.equal(kt[0], d.kt[0]) and torch.equal(v[0], d.v[0])     # layer 0: before any attention
+    assert _close(kt[1], d.kt[1], 0.05) and _close(v[1], d.v[1], 0.05)
+
+
+def test_prompt_pass_of_other_head_sizes(gpu):
+    sh = Gemma2Shape(layers=1, hidden=256, intermediate=512, heads=4, kv_heads=2, head_dim=32, vocab=512)
+    w = Gemma2Weights.random(sh, gpu, seed=13)
+    d = Gemma2Decoder(w, "se12", 1, max_len=24, encoded=_encoded(w))
+    assert not d._prefill_kernels_serve(9)
+    assert int(d.prefill(_prompt(gpu, 1, 9)).item()) == int(d.last_logits.float().argmax())

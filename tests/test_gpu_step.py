@@ -92,6 +92,82 @@ def test_gelu_mul(gpu, dtype):
     _ulp_close(out, ref)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,cols", [(57, 9216), (65, 8072), (600, 1000)])
+def test_gelu_mul_in_pieces_equals_element_by_element(gpu, rows, cols, dtype):
+    """Launches of 524,288 values and more take 8 per thread where they are aligned: the same bits as an output that is not."""
+    assert rows * cols >= 524288
+    g = _gen(gpu, rows)
+    gu = (torch.randn((rows, 2 * cols), generator=g, device=gpu) * 2).to(dtype)
+    gate, up = gu[:, :cols], gu[:, cols:]
+    d = nat.STEP_F32 if dtype == torch.float32 else nat.STEP_BF16
+    out = torch.empty((rows, cols), dtype=torch.bfloat16, device=gpu)
+    odd = torch.empty(rows * cols + 1, dtype=torch.bfloat16, device=gpu)[1:].view(rows, cols)
+    for o in (out, odd):
+        nat.step_check(nat.lib().se12_step_gelu_mul(nat.ptr(gate), nat.ptr(up), d, 2 * cols, nat.ptr(o), rows, cols,
+                                                    nat.stream_ptr()))
+    assert torch.equal(out, odd)
+    _ulp_close(out, F.gelu(gate.to(torch.bfloat16), approximate="tanh") * up.to(torch.bfloat16))
+
+
+# (batch, tokens, heads, kv heads, head dim, cache length, window): tokens at the edges of the 32-query blocks, 32-key tiles
+# and 64-token rope blocks, one query block per wave round and more, windows inside a tile and across several
+PREFILL_CASES = [
+    (1, 1, 4, 2, 64, 8, 0), (2, 31, 4, 4, 64, 40, 0), (1, 32, 8, 4, 256, 32, 0), (2, 33, 8, 1, 128, 64, 0),
+    (1, 63, 4, 2, 256, 64, 16), (1, 64, 2, 2, 128, 72, 33), (3, 65, 4, 2, 64, 72, 64), (1, 129, 8, 4, 256, 136, 0),
+    (2, 200, 8, 2, 128, 208, 31), (1, 513, 4, 2, 256, 520, 100), (1, 300, 16, 2, 64, 304, 4096),
+]
+
+
+@pytest.mark.parametrize("batch,T,heads,kvh,d,L,window", PREFILL_CASES)
+def test_prefill_attention(gpu, batch, T, heads, kvh, d, L, window):
+    """Against attention in 64 bits over the framework's rotated BF16 q and k. With u = 2^-8 (BF16's unit roundoff) the rounded
+    probabilities move the weighted sum by u sum p |v| and their total, and so the output, by u |out|, and the output is rounded
+    by u |out|: 3 u sum p |v| in all; FP32 scores up to 50 and their exponentials add 2e-5 of each probability twice."""
+    g = _gen(gpu, T + d)
+    stride = (heads + 2 * kvh) * d + 8
+    qkv = torch.randn((batch, T, stride), generator=g, device=gpu).to(torch.bfloat16)
+    q, k, v = (qkv[..., a * d: b * d].reshape(batch, T, -1, d).transpose(1, 2).clone()
+               for a, b in ((0, heads), (heads, heads + kvh), (heads + kvh, heads + 2 * kvh)))
+    inv = 1.0 / (10000.0 ** (torch.arange(0, d, 2, dtype=torch.int64, device=gpu).float() / d))
+    f = torch.arange(T, device=gpu).float()[:, None] * inv
+    emb = torch.cat((f, f), dim=-1)
+    cos, sin = emb.cos().to(torch.bfloat16), emb.sin().to(torch.bfloat16)
+    q, k = q * cos + rotate_half(q) * sin, k * cos + rotate_half(k) * sin
+    kt = torch.full((batch, kvh, d, L), 3.0, device=gpu).to(torch.bfloat16)
+    vc = torch.full((batch, kvh, L, d), 5.0, device=gpu).to(torch.bfloat16)
+    out = torch.full((batch, T, heads * d), float("nan"), device=gpu).to(torch.bfloat16)
+    n = nat.lib().se12_step_prefill_workspace(batch, T, heads, kvh, d)
+    ws = torch.full((n,), 255, dtype=torch.uint8, device=gpu)     # NaNs: the contents are indifferent
+    scaling = d ** -0.5
+    nat.step_check(nat.lib().se12_step_prefill_attention(
+        nat.ptr(qkv), stride, nat.ptr(cos), nat.ptr(sin), nat.ptr(kt), nat.ptr(vc), nat.ptr(out), batch, T, heads, kvh, d, L,
+        scaling, 50.0, window, nat.ptr(ws), n, nat.stream_ptr()))
+    assert torch.equal(kt[..., :T], k.transpose(2, 3)) and bool((kt[..., T:] == 3).all())
+    assert torch.equal(vc[:, :, :T], v) and bool((vc[:, :, T:] == 5).all())
+    qd, kd, vd = (t.double() for t in (q, k.repeat_interleave(heads // kvh, 1), v.repeat_interleave(heads // kvh, 1)))
+    sc = torch.tanh(qd @ kd.transpose(2, 3).contiguous() * scaling / 50.0) * 50.0
+    back = torch.arange(T, device=gpu)[:, None] - torch.arange(T, device=gpu)[None, :]
+    ok = (back >= 0) & (back < window) if window else back >= 0
+    p = torch.softmax(sc.masked_fill(~ok, float("-inf")), -1)
+    want = (p @ vd).transpose(1, 2).reshape(batch, T, -1)
+    bound = (3 * 2.0 ** -8 + 4e-5) * (p @ vd.abs()).transpose(1, 2).reshape(batch, T, -1)
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+
+def test_prefill_attention_refuses_bad_shapes(gpu):
+    t = torch.zeros(4096, dtype=torch.bfloat16, device=gpu)
+    lib = nat.lib()
+    assert lib.se12_step_prefill_workspace(1, 8, 4, 2, 96) < 0 and lib.se12_step_prefill_workspace(1, 8, 3, 2, 64) < 0
+
+    def call(T=2, L=8, softcap=50.0, ws=4096):
+        return lib.se12_step_prefill_attention(nat.ptr(t), 512, nat.ptr(t), nat.ptr(t), nat.ptr(t), nat.ptr(t), nat.ptr(t), 1,
+                                               T, 4, 2, 64, L, 1.0, softcap, 0, nat.ptr(t), ws, nat.stream_ptr())
+
+    for bad in (dict(T=9), dict(softcap=0.0), dict(softcap=100.0), dict(softcap=float("nan")), dict(ws=100), dict(L=12)):
+        assert call(**bad) == -1, bad
+
+
 def _attention_ref(q, k, v, kt, vc, inv_freq, pos, heads, kvh, d, scaling, softcap, window):
     """The eager step's attention at one position (gemma2.Gemma2Decoder._step)."""
     B = q.shape[0]
