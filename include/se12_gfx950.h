@@ -141,17 +141,20 @@ int se12_bind(const se12_streams* streams, int64_t rows, int64_t cols, int32_t m
 int se12_bind_raw_bf16(const uint16_t* w_dev, int64_t rows, int64_t cols, int32_t max_batch,
                        void* stream, se12_handle** out);
 
-/* The same in device memory of the caller (256-byte aligned, at least
- * se12_bind_workspace bytes for the shape and SE12_FORMAT_*, contents
- * indifferent, alive until the handle is released), which an allocator that
- * keeps its memory hands out without a driver call; only the raw copies of tiles
- * with more escapes than a side record lists are allocated here, where there
- * are any. */
-int64_t se12_bind_workspace(int64_t rows, int64_t cols, int32_t max_batch, int32_t format);
-int se12_bind_in(const se12_streams* streams, int64_t rows, int64_t cols, int32_t max_batch, void* workspace,
-                 int64_t workspace_bytes, void* stream, se12_handle** out);
-int se12_bind_raw_bf16_in(const uint16_t* w_dev, int64_t rows, int64_t cols, int32_t max_batch, void* workspace,
-                          int64_t workspace_bytes, void* stream, se12_handle** out);
+/* The same in device memory of the caller, which an allocator that keeps its
+ * memory hands out without a driver call: two blocks, 256-byte aligned, of at
+ * least the bytes se12_bind_workspace gives for the shape and SE12_FORMAT_*,
+ * contents indifferent, alive until the handle is released. `hot` is read by
+ * every launch (best beside other handles' hot blocks), `cold` by launches with
+ * K splits (its size may be 0, the pointer then NULL). Only the raw copies of
+ * tiles with more escapes than a side record lists are allocated here, where
+ * there are any. */
+int se12_bind_workspace(int64_t rows, int64_t cols, int32_t max_batch, int32_t format, int64_t* hot_bytes,
+                        int64_t* cold_bytes);
+int se12_bind_in(const se12_streams* streams, int64_t rows, int64_t cols, int32_t max_batch, void* hot, int64_t hot_bytes,
+                 void* cold, int64_t cold_bytes, void* stream, se12_handle** out);
+int se12_bind_raw_bf16_in(const uint16_t* w_dev, int64_t rows, int64_t cols, int32_t max_batch, void* hot,
+                          int64_t hot_bytes, void* cold, int64_t cold_bytes, void* stream, se12_handle** out);
 
 /* The 15 codebook bytes bind read from an SE12 handle's codebook_dev (host only). */
 int se12_handle_codebook(const se12_handle* h, uint8_t codebook_out[15]);

@@ -105,12 +105,13 @@ SIGNATURES = {
     "se12_device_info_get": (c_i32, [c_i32, ctypes.POINTER(DeviceInfo)]),
     "se12_bind": (c_i32, [ctypes.POINTER(Streams), c_i64, c_i64, c_i32, c_void_p, ctypes.POINTER(c_void_p)]),
     "se12_bind_raw_bf16": (c_i32, [c_void_p, c_i64, c_i64, c_i32, c_void_p, ctypes.POINTER(c_void_p)]),
-    "se12_bind_workspace": (c_i64, [c_i64, c_i64, c_i32, c_i32]),
+    "se12_bind_workspace": (c_i32, [c_i64, c_i64, c_i32, c_i32, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)]),
     "se12_bind_in": (
-        c_i32, [ctypes.POINTER(Streams), c_i64, c_i64, c_i32, c_void_p, c_i64, c_void_p, ctypes.POINTER(c_void_p)],
+        c_i32, [ctypes.POINTER(Streams), c_i64, c_i64, c_i32, c_void_p, c_i64, c_void_p, c_i64, c_void_p,
+                ctypes.POINTER(c_void_p)],
     ),
     "se12_bind_raw_bf16_in": (
-        c_i32, [c_void_p, c_i64, c_i64, c_i32, c_void_p, c_i64, c_void_p, ctypes.POINTER(c_void_p)],
+        c_i32, [c_void_p, c_i64, c_i64, c_i32, c_void_p, c_i64, c_void_p, c_i64, c_void_p, ctypes.POINTER(c_void_p)],
     ),
     "se12_handle_codebook": (c_i32, [c_void_p, c_u8p]),
     "se12_release": (c_i32, [c_void_p]),

@@ -74,12 +74,12 @@ def _require(t: Any, name: str, dtype: torch.dtype, shape: tuple, device: torch.
 
 
 class _Handle:
-    """Owns one se12_handle*; released when garbage-collected. `workspace` is
-    the tensor the library keeps the handle's device data in: it goes back to
+    """Owns one se12_handle*; released when garbage-collected. `workspace` are
+    the tensors the library keeps the handle's device data in: they go back to
     torch's allocator once the release has waited for the device, so no stream
-    the handle was used on can still read it."""
+    the handle was used on can still read them."""
 
-    def __init__(self, raw: ctypes.c_void_p, keepalive: tuple, workspace: torch.Tensor | None = None) -> None:
+    def __init__(self, raw: ctypes.c_void_p, keepalive: tuple, workspace: tuple = ()) -> None:
         self.raw = raw
         self._keepalive = keepalive  # the tensors the handle points into
         self._workspace = workspace
@@ -88,7 +88,7 @@ class _Handle:
         if self.raw:
             nat.lib().se12_release(self.raw)
             self.raw = ctypes.c_void_p(None)
-            self._workspace = None
+            self._workspace = ()
 
     def __del__(self) -> None:
         try:
@@ -115,9 +115,9 @@ def bind_se12(dt: Se12DeviceTensor, max_batch: int = nat.MAX_BATCH) -> _Handle:
     h = ctypes.c_void_p()
     lib = nat.lib()
     with torch.cuda.device(dt.sm.device):
-        ws = _bind_workspace(dt.rows, dt.cols, max_batch, nat.FORMAT_SE12, dt.sm.device)
-        nat.check(lib.se12_bind_in(ctypes.byref(s), dt.rows, dt.cols, max_batch, nat.ptr(ws), ws.numel(), nat.stream_ptr(),
-                                   ctypes.byref(h)))
+        ws = hot, cold = _bind_workspace(dt.rows, dt.cols, max_batch, nat.FORMAT_SE12, dt.sm.device)
+        nat.check(lib.se12_bind_in(ctypes.byref(s), dt.rows, dt.cols, max_batch, nat.ptr(hot), hot.numel(), nat.ptr(cold),
+                                   cold.numel(), nat.stream_ptr(), ctypes.byref(h)))
     handle = _Handle(h, (dt,), ws)
     cb = (ctypes.c_uint8 * CODEBOOK_SIZE)()
     nat.check(lib.se12_handle_codebook(h, cb))
@@ -125,11 +125,11 @@ def bind_se12(dt: Se12DeviceTensor, max_batch: int = nat.MAX_BATCH) -> _Handle:
     return handle
 
 
-def _bind_workspace(rows: int, cols: int, max_batch: int, fmt: int, device) -> torch.Tensor:
-    n = nat.lib().se12_bind_workspace(rows, cols, max_batch, fmt)
-    if n < 0:
-        nat.check(n)
-    return torch.empty(n, dtype=torch.uint8, device=device)
+def _bind_workspace(rows: int, cols: int, max_batch: int, fmt: int, device) -> tuple[torch.Tensor, torch.Tensor]:
+    hot, cold = ctypes.c_int64(), ctypes.c_int64()
+    nat.check(nat.lib().se12_bind_workspace(rows, cols, max_batch, fmt, ctypes.byref(hot), ctypes.byref(cold)))
+    return (torch.empty(hot.value, dtype=torch.uint8, device=device),
+            torch.empty(cold.value, dtype=torch.uint8, device=device))
 
 
 def bind_raw_bf16(w: torch.Tensor, max_batch: int = nat.MAX_BATCH) -> _Handle:
@@ -138,9 +138,9 @@ def bind_raw_bf16(w: torch.Tensor, max_batch: int = nat.MAX_BATCH) -> _Handle:
     w = w.contiguous()
     h = ctypes.c_void_p()
     with torch.cuda.device(w.device):
-        ws = _bind_workspace(w.shape[0], w.shape[1], max_batch, nat.FORMAT_RAW_BF16, w.device)
-        nat.check(nat.lib().se12_bind_raw_bf16_in(nat.ptr(w), w.shape[0], w.shape[1], max_batch, nat.ptr(ws), ws.numel(),
-                                                  nat.stream_ptr(), ctypes.byref(h)))
+        ws = hot, cold = _bind_workspace(w.shape[0], w.shape[1], max_batch, nat.FORMAT_RAW_BF16, w.device)
+        nat.check(nat.lib().se12_bind_raw_bf16_in(nat.ptr(w), w.shape[0], w.shape[1], max_batch, nat.ptr(hot), hot.numel(),
+                                                  nat.ptr(cold), cold.numel(), nat.stream_ptr(), ctypes.byref(h)))
     return _Handle(h, (w,), ws)
 
 
