@@ -16,6 +16,7 @@
 #include "se12_step.h"
 #include "se12_device.hpp"
 #include "se12_internal.hpp"
+#include "se12_step_math.hpp"
 
 using namespace se12;
 
@@ -1042,10 +1043,8 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
     if (pro && !fuse_pro) {
         // the norm as its own kernel into h_out, then the product of h_out
         hipStream_t st0 = static_cast<hipStream_t>(stream);
-        if (pro->res_out != pro->res_in)
-            SE12_HIP(hipMemcpyAsync(pro->res_out, pro->res_in, (size_t)batch * h0->K * 2, hipMemcpyDeviceToDevice, st0));
-        const int rc = se12_step_rmsnorm(pro->y_prev, SE12_STEP_F32, h0->K, pro->w1, pro->res_out, pro->w2, pro->h_out,
-                                         batch, (int32_t)h0->K, pro->eps, 0.0f, 1, st0);
+        const int rc = se12step::step_rmsnorm(pro->y_prev, SE12_STEP_F32, h0->K, pro->w1, pro->res_in, pro->res_out, pro->w2,
+                                              pro->h_out, batch, (int32_t)h0->K, pro->eps, 0.0f, 1, st0);
         if (rc != SE12_STEP_OK) return fail(SE12_E_HIP, "%s norm: %s", fn, se12_step_last_error());
         return gemv_group(fn, hs, count, pro->h_out, SE12_X_BF16, batch, ys, launch, stream, epi, nullptr);
     }
@@ -1102,6 +1101,8 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
             p.xn = true;
             p.lds = gemv_xn_lds_bytes(h0->K, bl, waves);
         }
+        // the tile rows' sums of squares, written by the waves that finish them
+        if (epi && mfma) g.epi.row_ss = epi->row_ss;
         if (fuse_epi) {
             g.epi = *epi;
             if (g.epi.out) g.epi.out += (size_t)b0 * h0->N;
@@ -1117,10 +1118,6 @@ static int gemv_group(const char* fn, se12_handle* const* hs, int32_t count, con
     }
     if (epi && !fuse_epi) {
         // the step runs as its own kernel after the product
-        if (epi->row_ss) {
-            const hipError_t e = launch_row_sumsq(ys[0], h0->N, h0->TR, batch, epi->row_ss, st);
-            if (e != hipSuccess) return fail(SE12_E_HIP, "%s row sums: %s", fn, hipGetErrorString(e));
-        }
         if (epi->kind != kEpiNone) {
             const int rc = epi->kind == kEpiGeluMul
                                ? se12_step_gelu_mul(ys[0], ys[1], SE12_STEP_F32, h0->N, epi->out, batch, (int32_t)h0->N, st)
@@ -1310,9 +1307,8 @@ int se12_gemv_prenorm(se12_handle* const* handles, int32_t count, const float* y
     if (!ok) {
         // same results through the separate kernels (in-place residual update)
         hipStream_t st = static_cast<hipStream_t>(stream);
-        if (ri != ro) SE12_HIP(hipMemcpyAsync(residual_out, residual_in, row_bytes, hipMemcpyDeviceToDevice, st));
-        const int rc = se12_step_rmsnorm(y_prev, SE12_STEP_F32, K, w1, residual_out, w2, h_out, batch, (int32_t)K, eps,
-                                         0.0f, 1, st);
+        const int rc = se12step::step_rmsnorm(y_prev, SE12_STEP_F32, K, w1, residual_in, residual_out, w2, h_out, batch,
+                                              (int32_t)K, eps, 0.0f, 1, st);
         if (rc != SE12_STEP_OK) return fail(SE12_E_HIP, "%s norm: %s", fn, se12_step_last_error());
         return gemv_group(fn, handles, count, h_out, SE12_X_BF16, batch, y, launch, stream, gelu_out ? &e : nullptr);
     }

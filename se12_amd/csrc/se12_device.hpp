@@ -597,6 +597,16 @@ __device__ __forceinline__ float row16_sum(float v) {
     return v;
 }
 
+// bf16(a)^2 + bf16(b)^2 + bf16(c)^2 + bf16(d)^2 of four consecutive tile rows, in
+// row16_sum's order; the sums of a tile row's four quads then add in pairs
+__device__ __forceinline__ float square_bf16(float v) {
+    const float t = __uint_as_float((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v) << 16);
+    return t * t;
+}
+__device__ __forceinline__ float quad_sumsq(const float v[4]) {
+    return (square_bf16(v[0]) + square_bf16(v[1])) + (square_bf16(v[2]) + square_bf16(v[3]));
+}
+
 // The half layout's loads of one tile for one lane: part p reads 8 bytes of
 // `sm` and 4 of `ec` (512 / 256 contiguous bytes per wave instruction).
 struct HalfTileLoads {

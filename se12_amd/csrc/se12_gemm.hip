@@ -602,6 +602,20 @@ __global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
     // accumulator layout: lane l holds D[4 * (l / 16) + e][l % 16] of each
     // batch group: tile row 4 * (l / 16) + e, batch row 16 * g + l % 16
     const int64_t n0 = (int64_t)tr * kTileRows + 4 * (int)(lane >> 4);
+    // the row's sum of squares (GemvEpilogue::row_ss): lanes l, l + 16, l + 32
+    // and l + 48 hold the quads of batch row 16 g + l; rows past N count 0
+    float* const row_ss = ga.epi.row_ss;
+    auto store_row_ss = [&](const float* sums, int g) {
+        if (!row_ss) return;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = n0 + e < a.N ? sums[e] : 0.0f;
+        float q = quad_sumsq(v);
+        q += __shfl_xor(q, 16, 64);
+        q += __shfl_xor(q, 32, 64);
+        const int b = 16 * g + (int)lane;
+        if (lane < 16u && b < batch) row_ss[(int64_t)b * a.TR + tr] = q;
+    };
     if (S == 1) {
 #pragma unroll
         for (int g = 0; g < BG; ++g) {
@@ -610,6 +624,8 @@ __global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (n0 + e < a.N) a.y[(int64_t)b * a.N + n0 + e] = acc[g][e];
+            const float sums[4] = {acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
+            store_row_ss(sums, g);
         }
         return;
     }
@@ -631,10 +647,10 @@ __global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
 #pragma unroll
     for (int g = 0; g < BG; ++g) {
         const int b = 16 * g + (int)(lane & 15u);
+        float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if (b < batch) {
             // every split's loads first (in groups of 8), then the adds in
             // ascending split order
-            float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
             for (int s0 = 0; s0 < S; s0 += 8) {
                 uint64_t lo[8], hi[8];
 #pragma unroll
@@ -659,6 +675,7 @@ __global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
             for (int e = 0; e < 4; ++e)
                 if (n0 + e < a.N) a.y[(int64_t)b * a.N + n0 + e] = sum[e];
         }
+        store_row_ss(sum, g);
     }
     if (lane == 0) __hip_atomic_store(&a.counters[tr], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

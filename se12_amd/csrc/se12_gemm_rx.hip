@@ -202,6 +202,16 @@ __attribute__((amdgpu_waves_per_eu(XG ? 2 : 3))) void gemm_rx_kernel(GemvGroupAr
         const int b = 16 * g + (int)(lane & 15u);
         xrow[g] = b < batch ? b : 0;
     }
+    // the row's sum of squares (GemvEpilogue::row_ss): lanes 4 i .. 4 i + 3 hold
+    // the row's quads of one batch row
+    float* const row_ss = ga.epi.row_ss;
+    auto store_row_ss = [&](const float v[4], int b, int tr) {
+        if (!row_ss) return;
+        float q = quad_sumsq(v);
+        q += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q), 0xB1, 0xF, 0xF, true));   // quad_perm 1,0,3,2
+        q += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q), 0x4E, 0xF, 0xF, true));   // quad_perm 2,3,0,1
+        if ((lane & 3u) == 0u && b < batch) row_ss[(int64_t)b * a.TR + tr] = q;
+    };
     // y as 16-byte pieces: N % 16 == 0 on this path, so a 16-byte aligned y
     // keeps every batch row aligned
     const bool y_vec = (reinterpret_cast<uintptr_t>(a.y) & 15u) == 0u;
@@ -220,6 +230,7 @@ __attribute__((amdgpu_waves_per_eu(XG ? 2 : 3))) void gemm_rx_kernel(GemvGroupAr
             for (int e = 0; e < 4; ++e)
                 v[e] = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(acc[g][e])));
             const int b = 16 * g + (int)(lane >> 2);
+            store_row_ss(v, b, tr);
             if (b < batch) {
                 float* yp = a.y + (int64_t)b * a.N + (int64_t)tr * kTileRows + 4 * (int)(lane & 3u);
                 if (y_vec) {
@@ -273,9 +284,9 @@ __attribute__((amdgpu_waves_per_eu(XG ? 2 : 3))) void gemm_rx_kernel(GemvGroupAr
 #pragma unroll
                 for (int g = 0; g < BG; ++g) {
                     const int b = 16 * g + (int)(lane >> 2);
+                    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                     if (b < batch) {
                         const int64_t n = (int64_t)tr * kTileRows + 4 * (int)(lane & 3u);
-                        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                         uint64_t lo[kRxMaxSplits], hi[kRxMaxSplits];
 #pragma unroll
                         for (int ss = 0; ss < kRxMaxSplits; ++ss) {
@@ -302,6 +313,7 @@ __attribute__((amdgpu_waves_per_eu(XG ? 2 : 3))) void gemm_rx_kernel(GemvGroupAr
                             for (int e = 0; e < 4; ++e) yp[e] = v[e];
                         }
                     }
+                    store_row_ss(v, b, tr);
                 }
                 if (lane == 0) __hip_atomic_store(&a.counters[tr], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }

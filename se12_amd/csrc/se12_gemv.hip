@@ -809,22 +809,6 @@ hipError_t launch_b(const GemvGroupArgs& a, const GemvPlan& p, hipStream_t strea
 
 }  // namespace
 
-// row_ss of a product whose launch did not write it (the MFMA kernel): the
-// same 16-lane tree over bf16(y)^2 as the dot2 tail, so the values agree
-// wherever y does. Grid (tile rows, batch rows), one wave per block.
-__global__ __launch_bounds__(64) void row_sumsq_kernel(const float* y, int64_t N, int32_t TR, float* row_ss) {
-    const int tr = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
-    const int64_t n = (int64_t)tr * kTileRows + (lane & 15);
-    const float t = (lane < 16 && n < N) ? se12step::round_bf16(y[(int64_t)b * N + n]) : 0.0f;
-    const float q = row16_sum(t * t);
-    if (lane == 0) row_ss[(int64_t)b * TR + tr] = q;
-}
-
-hipError_t launch_row_sumsq(const float* y, int64_t N, int32_t TR, int32_t batch, float* row_ss, hipStream_t stream) {
-    hipLaunchKernelGGL(row_sumsq_kernel, dim3(TR, batch), dim3(64), 0, stream, y, N, TR, row_ss);
-    return hipGetLastError();
-}
-
 hipError_t launch_gemv(const GemvGroupArgs& a, const GemvPlan& p, hipStream_t stream) {
     switch (p.batch * 2 + (p.raw ? 1 : 0)) {
         case 2: return launch_b<1, false>(a, p, stream);

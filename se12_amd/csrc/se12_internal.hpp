@@ -52,10 +52,12 @@ struct GemvEpilogue {
     const uint16_t* w2;       // [N] BF16
     uint16_t* residual;       // [B, N] BF16
     uint16_t* out;            // [B, N] BF16
-    // any kind, single-matrix dot2 launches: when not NULL, the block that
-    // completes tile row t also writes row_ss[b, t] = the sum over its 16
-    // rows n < N of bf16(y[b, n])^2 (a 16-lane DPP tree), the first sum of
-    // squares of the decoder's next norm
+    // any kind, single-matrix launches of every kernel: when not NULL, the
+    // block (MFMA kernels: the wave) that completes tile row t also writes
+    // row_ss[b, t] = the sum over its 16 rows n < N of bf16(y[b, n])^2 (rows in
+    // pairs, fours, eights: one order in every kernel), the first sum of
+    // squares of the decoder's next norm. As a launch of its own after the
+    // product it took 4 us.
     float* row_ss;            // [B, TR]
 };
 
@@ -212,7 +214,6 @@ constexpr int gemv_waves_per_simd(int batch, bool raw, int g, int pf, bool gener
 inline size_t gemv_lds_bytes(int waves, int batch) { return (size_t)waves * batch * 16 * sizeof(float); }
 
 hipError_t launch_gemv(const GemvGroupArgs& a, const GemvPlan& p, hipStream_t stream);
-hipError_t launch_row_sumsq(const float* y, int64_t N, int32_t TR, int32_t batch, float* row_ss, hipStream_t stream);
 
 // Batched path (se12_gemm.hip): BF16 x with kGemmMinBatch..32 rows runs one
 // MFMA launch over all rows (one pass over the weights) instead of one

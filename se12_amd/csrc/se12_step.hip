@@ -86,6 +86,7 @@ struct NormArgs {
     const void* in;
     int64_t in_stride;
     const uint16_t* w1;
+    const uint16_t* res_in;  // mode 1; residual itself, or another tensor
     uint16_t* residual;
     const uint16_t* w2;
     uint16_t* out;
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(kNormMaxThreads) void rmsnorm_kernel(NormArgs a) {
         x[k] = load_as_bf16<DT>(a.in, base + ic);
         w1[k] = bf16_to_f(a.w1[ic]);
         if constexpr (MODE == 1) {
-            res[k] = bf16_to_f(a.residual[rbase + ic]);
+            res[k] = bf16_to_f(a.res_in[rbase + ic]);
             w2[k] = bf16_to_f(a.w2[ic]);
         }
     }
@@ -1178,19 +1179,17 @@ ArgmaxLayout argmax_layout(int32_t rows, int32_t vocab) {
 
 }  // namespace
 
-extern "C" {
+namespace se12step {
 
-const char* se12_step_last_error(void) { return step_error(); }
-
-int se12_step_rmsnorm(const void* in, int32_t in_dtype, int64_t in_stride, const uint16_t* w1, uint16_t* residual,
-                      const uint16_t* w2, uint16_t* out, int32_t rows, int32_t hidden, float eps, float in_scale,
-                      int32_t mode, void* stream) {
+int step_rmsnorm(const void* in, int32_t in_dtype, int64_t in_stride, const uint16_t* w1, const uint16_t* res_in,
+                 uint16_t* res_out, const uint16_t* w2, uint16_t* out, int32_t rows, int32_t hidden, float eps,
+                 float in_scale, int32_t mode, void* stream) {
     if (!in || !w1 || !out || rows <= 0 || hidden <= 0 || !dtype_ok(in_dtype) || in_stride < hidden)
         return step_fail("se12_step_rmsnorm: bad argument");
-    if (mode == 1 && (!residual || !w2)) return step_fail("se12_step_rmsnorm: mode 1 needs residual and w2");
+    if (mode == 1 && (!res_in || !res_out || !w2)) return step_fail("se12_step_rmsnorm: mode 1 needs residual and w2");
     if (mode != 0 && mode != 1) return step_fail("se12_step_rmsnorm: mode must be 0 or 1");
     if (hidden > kNormPer * kNormMaxThreads) return step_fail("se12_step_rmsnorm: hidden above 8192");
-    NormArgs a{in, in_stride, w1, residual, w2, out, hidden, eps, in_scale};
+    NormArgs a{in, in_stride, w1, res_in, res_out, w2, out, hidden, eps, in_scale};
     const int threads = ((hidden + kNormPer - 1) / kNormPer + 63) / 64 * 64;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     const bool f32 = in_dtype == SE12_STEP_F32;
@@ -1206,6 +1205,18 @@ int se12_step_rmsnorm(const void* in, int32_t in_dtype, int64_t in_stride, const
             hipLaunchKernelGGL((rmsnorm_kernel<SE12_STEP_BF16, 1>), dim3(rows), dim3(threads), 0, st, a);
     }
     return step_launched();
+}
+
+}  // namespace se12step
+
+extern "C" {
+
+const char* se12_step_last_error(void) { return step_error(); }
+
+int se12_step_rmsnorm(const void* in, int32_t in_dtype, int64_t in_stride, const uint16_t* w1, uint16_t* residual,
+                      const uint16_t* w2, uint16_t* out, int32_t rows, int32_t hidden, float eps, float in_scale,
+                      int32_t mode, void* stream) {
+    return step_rmsnorm(in, in_dtype, in_stride, w1, residual, residual, w2, out, rows, hidden, eps, in_scale, mode, stream);
 }
 
 int64_t se12_step_attention_workspace(int32_t batch, int32_t heads, int32_t kv_heads, int32_t head_dim,

@@ -94,5 +94,10 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
 int step_fail(const char* msg);
 int step_fail(const char* who, const char* msg);
 int step_launched();
+// host: se12_step_rmsnorm with the residual read from res_in and written to
+// res_out (the same tensor, or disjoint ones)
+int step_rmsnorm(const void* in, int32_t in_dtype, int64_t in_stride, const uint16_t* w1, const uint16_t* res_in,
+                 uint16_t* res_out, const uint16_t* w2, uint16_t* out, int32_t rows, int32_t hidden, float eps,
+                 float in_scale, int32_t mode, void* stream);
 
 }  // namespace se12step

@@ -41,14 +41,14 @@ def _norm_close(got: torch.Tensor, want: torch.Tensor, min_exact: float = 0.99) 
     assert bool((err <= scale * 2.0 ** -7).all()), (err, scale)
 
 
-def _kernel(rows, cols, seed, fmt, gpu):
+def _kernel(rows, cols, seed, fmt, gpu, max_batch=8):
     from se12_amd.hip import RawBf16MatVecKernel, Se12MatVecKernel
 
     bits = o.normal_bf16(rows, cols, seed=seed, std=0.02)
     if fmt == "raw":
-        return RawBf16MatVecKernel(torch.from_numpy(bits).to(gpu).view(torch.bfloat16), max_batch=8)
+        return RawBf16MatVecKernel(torch.from_numpy(bits).to(gpu).view(torch.bfloat16), max_batch=max_batch)
     enc = o.encode(bits.reshape(-1), rows, cols)
-    return Se12MatVecKernel(to_device(enc, gpu), max_batch=8)
+    return Se12MatVecKernel(to_device(enc, gpu), max_batch=max_batch)
 
 
 def _x(batch, cols, gpu, seed, dtype=torch.bfloat16):
@@ -320,6 +320,38 @@ def test_rowss_sums_the_tile_rows_of_the_output(gpu, fmt, rows, cols, batch, dty
         torch.cuda.synchronize()
         assert torch.equal(y, k.multiply(x))
         torch.testing.assert_close(ss, _want_row_ss(y), rtol=1e-5, atol=1e-30)
+
+
+@pytest.mark.parametrize("fmt", ["se12", "raw"])
+@pytest.mark.parametrize("rows,cols,batch,dtype", [
+    (2304, 2048, 5, torch.bfloat16),    # resident x, one batch group
+    (2304, 2048, 17, torch.bfloat16),   # two batch groups, the second of one row
+    (2304, 9216, 8, torch.bfloat16),    # K splits, added by the last arrival
+    (2304, 9216, 32, torch.bfloat16),   # x slabs
+    (300, 512, 7, torch.bfloat16),      # a last tile row of 12 rows
+    (17, 300, 32, torch.bfloat16),      # of one row; a partial last tile
+    (2304, 9216, 6, torch.float32),     # FP32 x: planes
+    (1000, 700, 21, torch.float32),
+])
+def test_rowss_from_the_matrix_core_products(gpu, fmt, rows, cols, batch, dtype):
+    """Written by the wave that finishes a tile row: every word of row_ss, to the
+    bits of a fixed order (the squares of BF16 values are exact in FP32, so pairs,
+    fours, eights and sixteens are the only roundings), and none past it."""
+    k = _kernel(rows, cols, 70, fmt, gpu, max_batch=32)
+    tr = (rows + 15) // 16
+    x = _x(batch, cols, gpu, 75, dtype)
+    buf = torch.full((batch + 1, tr), float("nan"), device=gpu)
+    y = k.multiply_rowss(x, buf[:batch])
+    torch.cuda.synchronize()
+    assert torch.equal(y, k.multiply(x))
+    sq = torch.zeros((batch, tr * 16), dtype=torch.float32, device=gpu)
+    sq[:, :rows] = y.to(torch.bfloat16).float() ** 2
+    q = sq.view(batch, tr, 8, 2)
+    q = q[..., 0] + q[..., 1]
+    q = q[..., 0::2] + q[..., 1::2]
+    q = q[..., 0::2] + q[..., 1::2]
+    assert torch.equal(buf[:batch], q[..., 0] + q[..., 1])
+    assert buf[batch].isnan().all()
 
 
 @pytest.mark.parametrize("batch", [1, 2, 4])
