@@ -314,6 +314,10 @@ int se12_gemv_prenorm(se12_handle* const* handles, int32_t count, const float* y
  * kernel lws/adapters/cuda/kernels/se12_decode.cu:12-22). */
 int se12_decode(se12_handle* h, uint16_t* out_dev, void* stream);
 
+/* se12_decode of up to SE12_MAX_GROUP matrices of one device, each to its own
+ * output, in one launch (a layer's q, k, v ahead of its prompt product). */
+int se12_decode_group(se12_handle* const* handles, int32_t count, uint16_t* const* outs_dev, void* stream);
+
 /* Decodes `nrows` rows given by device int64 indices, in that order, to
  * [nrows, cols] BF16 bits; only the tiles covering those rows are read. An
  * index outside [0, rows) yields a row of zeros. Replaces

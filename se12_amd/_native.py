@@ -148,6 +148,7 @@ SIGNATURES = {
         c_i32, [c_void_p, c_void_p, c_i32, c_i32, c_void_p, c_void_p, ctypes.POINTER(Launch), c_void_p],
     ),
     "se12_decode": (c_i32, [c_void_p, c_void_p, c_void_p]),
+    "se12_decode_group": (c_i32, [ctypes.POINTER(c_void_p), c_i32, ctypes.POINTER(c_void_p), c_void_p]),
     "se12_decode_rows": (c_i32, [c_void_p, c_void_p, c_i64, c_void_p, c_void_p]),
     "se12_codebook_from_histogram": (c_i32, [ctypes.POINTER(ctypes.c_uint64), c_u8p]),
     "se12_decode_rows_scaled": (c_i32, [c_void_p, c_void_p, c_i64, ctypes.c_float, c_void_p, c_void_p]),

@@ -1336,16 +1336,31 @@ static DecodeArgs decode_args(const se12_handle* h, uint16_t* out) {
     return a;
 }
 
-int se12_decode(se12_handle* h, uint16_t* out, void* stream) {
-    if (!h || !out) return fail(SE12_E_INVALID, "se12_decode: NULL argument");
-    if (h->format != SE12_FORMAT_SE12) return fail(SE12_E_INVALID, "se12_decode: handle is not SE12");
+static int decode_group(const char* fn, se12_handle* const* hs, int32_t count, uint16_t* const* outs, void* stream) {
+    DecodeGroup g{};
+    for (int32_t i = 0; i < count; ++i) {
+        if (!hs[i] || !outs[i]) return fail(SE12_E_INVALID, "%s: NULL argument", fn);
+        if (hs[i]->format != SE12_FORMAT_SE12) return fail(SE12_E_INVALID, "%s: handle is not SE12", fn);
+        if (hs[i]->device != hs[0]->device) return fail(SE12_E_INVALID, "%s: matrices on different devices", fn);
+        g.m[i] = decode_args(hs[i], outs[i]);
+    }
+    g.count = count;
     DeviceScope ds;
-    SE12_HIP(ds.enter(h->device));
-    DecodeArgs a = decode_args(h, out);
-    a.items = h->T;
-    hipError_t e = launch_decode(a, static_cast<hipStream_t>(stream), h->cu_count);
-    if (e != hipSuccess) return fail(SE12_E_HIP, "se12_decode launch: %s", hipGetErrorString(e));
+    SE12_HIP(ds.enter(hs[0]->device));
+    hipError_t e = launch_decode(g, static_cast<hipStream_t>(stream), hs[0]->cu_count);
+    if (e != hipSuccess) return fail(SE12_E_HIP, "%s launch: %s", fn, hipGetErrorString(e));
     return SE12_OK;
+}
+
+int se12_decode(se12_handle* h, uint16_t* out, void* stream) {
+    return decode_group("se12_decode", &h, 1, &out, stream);
+}
+
+int se12_decode_group(se12_handle* const* handles, int32_t count, uint16_t* const* outs, void* stream) {
+    if (!handles || !outs) return fail(SE12_E_INVALID, "se12_decode_group: NULL argument");
+    if (count < 1 || count > kMaxGroup)
+        return fail(SE12_E_INVALID, "se12_decode_group: %d matrices outside [1, %d]", count, kMaxGroup);
+    return decode_group("se12_decode_group", handles, count, outs, stream);
 }
 
 static int decode_rows(const char* fn, se12_handle* h, const int64_t* rows, int64_t nrows, float scale, uint16_t* out,

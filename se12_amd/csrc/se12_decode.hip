@@ -62,15 +62,24 @@ __device__ __forceinline__ void store8(uint16_t* out_row, int64_t col, int64_t K
 // each write alternate halves of 32-byte pieces: 2304x9216 took 19.0 us
 // with it against 15.7 here, the stores nontemporal in both; 14336x3584
 // 39.0 against 33.5.)
-__global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(DecodeArgs a, int64_t nw) {
+//
+// Up to kMaxGroup matrices share a launch, each with blocks of its own (the pair
+// table in LDS is a matrix's): the
+// seven matrices of a Gemma-2-2B layer take 59.5 us in four launches against 70 in
+// seven, mostly on q, k, v (9.0 us), whose own launches end before they fill HBM.
+__global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(DecodeGroup grp) {
     SE12_DECLARE_LUT(lut);
+    int mi = 0;
+    while (mi + 1 < grp.count && (int)blockIdx.x >= grp.block0[mi + 1]) ++mi;
+    const DecodeArgs a = grp.m[mi];
+    const int64_t nw = grp.nw[mi];
     const int tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     // tile indices in 32 bits (the library refuses matrices of 2^31 tiles or
     // more), so the per-tile division is a 32-bit one
     const uint32_t T = (uint32_t)a.T, NW = (uint32_t)nw, TC = (uint32_t)a.TC;
-    const uint32_t g = blockIdx.x * kDecodeWaves + (uint32_t)w;
+    const uint32_t g = (blockIdx.x - (uint32_t)grp.block0[mi]) * kDecodeWaves + (uint32_t)w;
     const uint32_t n = g < NW && g < T ? (T - 1u - g) / NW + 1u : 0u;  // tiles of this wave
     struct Slot {
         TileSide side;
@@ -219,10 +228,18 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_rows_kernel(Decod
 // 14336x3584 33.5 / 36.5 / 33.6 / 33.9)
 constexpr int kDecodeStreamWavesPerCu = 4;
 
-hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream, int cu_count) {
-    const int64_t nw = std::min<int64_t>(a.T, (int64_t)std::max(1, cu_count) * kDecodeStreamWavesPerCu);
-    const int64_t blocks = (nw + kDecodeWaves - 1) / kDecodeWaves;
-    hipLaunchKernelGGL(decode_stream_kernel, dim3((uint32_t)blocks), dim3(kDecodeWaves * kWave), 0, stream, a, nw);
+// The waves are shared out by the matrices' tiles, in whole blocks.
+hipError_t launch_decode(DecodeGroup& g, hipStream_t stream, int cu_count) {
+    const int64_t waves = (int64_t)std::max(1, cu_count) * kDecodeStreamWavesPerCu;
+    int64_t tiles = 0;
+    for (int i = 0; i < g.count; ++i) tiles += g.m[i].T;
+    g.block0[0] = 0;
+    for (int i = 0; i < g.count; ++i) {
+        const int64_t share = std::max<int64_t>(kDecodeWaves, waves * g.m[i].T / tiles / kDecodeWaves * kDecodeWaves);
+        g.nw[i] = std::min<int64_t>(g.m[i].T, share);
+        g.block0[i + 1] = g.block0[i] + (int32_t)((g.nw[i] + kDecodeWaves - 1) / kDecodeWaves);
+    }
+    hipLaunchKernelGGL(decode_stream_kernel, dim3((uint32_t)g.block0[g.count]), dim3(kDecodeWaves * kWave), 0, stream, g);
     return hipGetLastError();
 }
 

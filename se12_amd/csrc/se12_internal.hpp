@@ -154,6 +154,15 @@ struct DecodeArgs {
     int32_t out_vec_ok;
 };
 
+// Whole matrices decoded by one launch: matrix i has the blocks block0[i] ..
+// block0[i + 1] - 1 and nw[i] waves on its tiles.
+struct DecodeGroup {
+    DecodeArgs m[kMaxGroup];
+    int64_t nw[kMaxGroup];
+    int32_t block0[kMaxGroup + 1];
+    int32_t count;
+};
+
 // Device scratch of the encoder (se12_encode_workspace bytes).
 constexpr int kEncodeHistBlocks = 512;
 struct EncodeWork {
@@ -297,7 +306,8 @@ constexpr size_t rx_lds_total(int64_t k, int staged, int batch, int waves, int k
     return rx_lds_bytes(k, staged) > sums ? rx_lds_bytes(k, staged) : sums;
 }
 hipError_t launch_gemm_rx(const GemvGroupArgs& a, int batch, const GemvPlan& p, hipStream_t stream);
-hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream, int cu_count);
+// m and count set; count 1..kMaxGroup
+hipError_t launch_decode(DecodeGroup& g, hipStream_t stream, int cu_count);
 // scale 0: the weights as they are
 hipError_t launch_decode_rows(const DecodeArgs& a, float scale, hipStream_t stream);
 // What bind reads back: zero before launch_bind_tiles (but the codebook).

@@ -163,10 +163,13 @@ class _Backend:
         """The BF16 weight of a projection, or of several stacked by rows (valid
         until the next call: the SE12 backend decodes into its scratch)."""
         if self.kind == "se12":
-            at, ks = 0, [self.layers[li][n] for n in names]
+            from .hip import decode_group
+
+            at, ks, outs = 0, [self.layers[li][n] for n in names], []
             for k in ks:
-                k.decode_into(self.scratch[at: at + k.rows * k.cols].view(k.rows, k.cols))
+                outs.append(self.scratch[at: at + k.rows * k.cols].view(k.rows, k.cols))
                 at += k.rows * k.cols
+            decode_group(ks, outs)
             return self.scratch[:at].view(-1, ks[0].cols)
         if len(names) == 1:
             return self.w.layers[li][names[0]]

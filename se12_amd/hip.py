@@ -423,6 +423,18 @@ def multiply_grouped(kernels, activations: torch.Tensor, launch: LaunchConfigura
     return outs
 
 
+def decode_group(kernels: list[Se12MatVecKernel], outs: list[torch.Tensor]) -> None:
+    """`decode_into` of up to 4 bound matrices of one device in one launch."""
+    n, k0 = len(kernels), kernels[0]
+    if not 1 <= n <= nat.MAX_GROUP or len(outs) != n:
+        raise ValueError(f"1..{nat.MAX_GROUP} matrices and as many outputs, got {n} and {len(outs)}")
+    for i, (k, o) in enumerate(zip(kernels, outs)):
+        _require(o, f"outs[{i}]", torch.bfloat16, (k.rows, k.cols), k0.device)
+    hs = (ctypes.c_void_p * n)(*[k.handle.raw.value for k in kernels])
+    ps = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
+    nat.check(nat.lib().se12_decode_group(hs, n, ps, nat.stream_ptr()))
+
+
 @dataclasses.dataclass(frozen=True)
 class RowIndices:
     """Row indices in request order (weight_decoder.py:18-23)."""

@@ -134,6 +134,28 @@ def test_bind_stats_count_the_raw_decoded_tiles(gpu):
     assert (a.value, b.value) == (0, 0)
 
 
+@pytest.mark.parametrize("shapes", [
+    [(33, 300)],
+    [(2048, 2304), (1024, 2304), (1024, 2304)],   # q, k, v
+    [(1, 1), (2304, 4096), (17, 257), (160, 2560)],  # one tile beside several per wave
+])
+def test_decode_group_equals_the_oracle(gpu, shapes):
+    """Each matrix of a launch decodes with its own codebook, to its own output."""
+    from se12_amd.hip import Se12MatVecKernel, decode_group
+
+    want = [uniform_bits(r, c, seed=i) if i == 0 and r * c < 65536 else o.normal_bf16(r, c, seed=i, std=0.02 * 4.0 ** i)
+            for i, (r, c) in enumerate(shapes)]
+    ks = [Se12MatVecKernel(to_device(o.encode(b.reshape(-1), r, c), gpu)) for b, (r, c) in zip(want, shapes)]
+    outs = [torch.full((r, c), float("nan"), dtype=torch.bfloat16, device=gpu) for r, c in shapes]
+    decode_group(ks, outs)
+    for b, out in zip(want, outs):
+        assert np.array_equal(out.view(torch.int16).cpu().numpy().reshape(-1), b.reshape(-1))
+    with pytest.raises(ValueError):
+        decode_group(ks, outs[:-1])
+    with pytest.raises(ValueError):
+        decode_group(ks * 5, outs * 5)
+
+
 @pytest.mark.parametrize("rows,cols,kind", [
     (1, 1, "normal"), (16, 15, "uniform"), (17, 256, "heavy"), (33, 257, "heavy"), (48, 1024, "heavy"),     # 1, 1, 1, 2, 4 K tiles
     (40, 1025, "uniform"), (64, 2304, "normal"), (64, 2304, "heavy"), (32, 1288, "uniform"),                # 5, 9, 9, 6
