@@ -356,7 +356,7 @@ class Gemma2Decoder:
             ck(ws_bytes)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=self.dev)
         cos, sin = self._rope(torch.arange(T, device=self.dev))
-        emb = self.be.embed_rows(prompt)
+        emb = self.be.embed_rows(prompt).view(n, s.hidden)   # refuses a prompt of another batch
         ck(lib.se12_step_rmsnorm(nat.ptr(emb), bf16, s.hidden, nat.ptr(self.w.layers[0]["input_norm"]), nat.ptr(x), None,
                                  nat.ptr(h), n, s.hidden, s.eps, float(self.embed_scale.item()), 0, st))
 

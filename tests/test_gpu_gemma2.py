@@ -198,3 +198,14 @@ def test_prompt_pass_of_other_head_sizes(gpu):
     d = Gemma2Decoder(w, "se12", 1, max_len=24, encoded=_encoded(w))
     assert not d._prefill_kernels_serve(9)
     assert int(d.prefill(_prompt(gpu, 1, 9)).item()) == int(d.last_logits.float().argmax())
+
+
+@pytest.mark.parametrize("backend", ["se12", "bf16"])
+def test_prompt_of_another_batch_is_refused(gpu, backend):
+    sh = Gemma2Shape(layers=1, hidden=256, intermediate=512, heads=4, kv_heads=2, head_dim=64, vocab=512)
+    w = Gemma2Weights.random(sh, gpu, seed=14)
+    d = Gemma2Decoder(w, backend, 2, max_len=24, encoded=_encoded(w) if backend == "se12" else None)
+    for batch in (1, 3):
+        with pytest.raises(RuntimeError, match="invalid for input"):
+            d.prefill(_prompt(gpu, batch, 9))
+    d.prefill(_prompt(gpu, 2, 9))
