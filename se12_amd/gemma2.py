@@ -254,6 +254,7 @@ class Gemma2Decoder:
         self.inv_freq = 1.0 / (s.rope_theta ** (torch.arange(0, s.head_dim, 2, dtype=torch.int64, device=dev).float() / s.head_dim))
         self.scaling = s.query_pre_attn_scalar ** -0.5
         self.embed_scale = torch.tensor(math.sqrt(s.hidden), dtype=torch.bfloat16, device=dev)
+        self.embed_scale_value = torch.tensor(math.sqrt(s.hidden), dtype=torch.bfloat16).item()   # without asking the device
         self.ids = torch.zeros(batch, dtype=torch.int64, device=dev)
         self.pos = torch.zeros((), dtype=torch.int64, device=dev)
         self.step_index = torch.zeros((), dtype=torch.int64, device=dev)
@@ -290,7 +291,6 @@ class Gemma2Decoder:
             self.o_out = buf(s.hidden) if f32 else None
             self.down_out = buf(s.hidden) if f32 else None
             self.logits_out = buf(s.vocab) if f32 else None
-            self.embed_scale_value = float(self.embed_scale.float().item())
             n = nat.lib().se12_step_attention_workspace(batch, s.heads, s.kv_heads, s.head_dim, max_len)
             if n < 0:
                 nat.step_check(n)
@@ -317,7 +317,11 @@ class Gemma2Decoder:
         """Runs the prompt [batch, T] (exact products), fills the KV cache and
         returns the first generated token per sequence."""
         T = prompt.shape[1]
-        h = self._prefill_kernels(prompt) if self._prefill_kernels_serve(T) else self._prefill_ops(prompt)
+        if self._prefill_kernels_serve(T):
+            with torch.cuda.device(self.dev):   # the kernels go to the current device
+                h = self._prefill_kernels(prompt)
+        else:
+            h = self._prefill_ops(prompt)
         logits = self.be.logits(h)
         logits = torch.tanh(logits / self.s.final_softcap) * self.s.final_softcap
         self.last_logits.copy_(logits)
@@ -331,10 +335,16 @@ class Gemma2Decoder:
 
     def _prefill_kernels_serve(self, T: int) -> bool:
         """What se12_step_prefill_attention and se12_step_rmsnorm take; any
-        other shape runs the framework ops."""
+        other shape, weights on the CPU or of other types run the framework
+        ops."""
         s = self.s
-        return (s.head_dim in (64, 128, 256) and 0.0 < s.attn_softcap <= 64.0 and s.hidden <= 8192 and 0 < T <= self.max_len
-                and s.heads % s.kv_heads == 0)
+        if not (self.dev.type == "cuda" and s.head_dim in (64, 128, 256) and 0.0 < s.attn_softcap <= 64.0
+                and s.hidden <= 8192 and 0 < T <= self.max_len and s.heads % s.kv_heads == 0):
+            return False
+        norms = [lw[n] for lw in self.w.layers for n in ("input_norm", "post_attn_norm", "pre_ffw_norm", "post_ffw_norm")]
+        return self.w.embed.dtype == torch.bfloat16 and all(
+            w.dtype == torch.bfloat16 and w.shape == (s.hidden,) and w.is_contiguous() and w.device == self.w.embed.device
+            for w in (*norms, self.w.final_norm))
 
     def _prefill_kernels(self, prompt: torch.Tensor) -> torch.Tensor:
         """The prompt pass with one library launch each for the norms, the
@@ -358,7 +368,7 @@ class Gemma2Decoder:
         cos, sin = self._rope(torch.arange(T, device=self.dev))
         emb = self.be.embed_rows(prompt).view(n, s.hidden)   # refuses a prompt of another batch
         ck(lib.se12_step_rmsnorm(nat.ptr(emb), bf16, s.hidden, nat.ptr(self.w.layers[0]["input_norm"]), nat.ptr(x), None,
-                                 nat.ptr(h), n, s.hidden, s.eps, float(self.embed_scale.item()), 0, st))
+                                 nat.ptr(h), n, s.hidden, s.eps, self.embed_scale_value, 0, st))
 
         def norm(y, w1, w2):
             ck(lib.se12_step_rmsnorm(nat.ptr(y), bf16, s.hidden, nat.ptr(w1), nat.ptr(x), nat.ptr(w2), nat.ptr(h), n,

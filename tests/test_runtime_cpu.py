@@ -153,3 +153,24 @@ def test_fused_mode_routes_decode_steps_to_the_kernel_and_prefill_to_exact():
     assert calls and all(c[0] == 2 for c in calls)   # decode steps at batch 2
     with pytest.raises(ValueError):
         runtime.load_packed(pm, mode="fast", device="cpu", config=cfg, kernel_factory=Counting, log=None)
+
+
+@pytest.mark.parametrize("other", ["cpu", "norm_dtype", "norm_view"])
+def test_prompt_pass_off_the_kernels_runs_the_framework_ops(other):
+    """Weights the step kernels cannot read (on the CPU; norms of another type or layout) never reach them."""
+    from se12_amd.gemma2 import Gemma2Decoder, Gemma2Shape, Gemma2Weights
+
+    sh = Gemma2Shape(layers=1, hidden=256, intermediate=512, heads=4, kv_heads=2, head_dim=64, vocab=300)
+    w = Gemma2Weights.random(sh, torch.device("cpu"), seed=3)
+    d = Gemma2Decoder(w, "bf16", 2, max_len=16, fused_step=False)
+    if other == "cpu":
+        first = d.prefill(torch.randint(0, sh.vocab, (2, 9), generator=torch.Generator().manual_seed(1)))
+        assert torch.equal(first, d.last_logits.argmax(-1)) and int(d.pos) == 9 and bool(d.kt[0][..., :9].any())
+        with pytest.raises(RuntimeError, match="invalid for input"):
+            d.prefill(torch.zeros((1, 9), dtype=torch.int64))
+    d.dev = torch.device("cuda", 0) if other != "cpu" else d.dev   # the rule alone: nothing is launched
+    if other != "cpu":
+        assert d._prefill_kernels_serve(9)
+        n = w.layers[0]["pre_ffw_norm"]
+        w.layers[0]["pre_ffw_norm"] = n.float() if other == "norm_dtype" else n.repeat_interleave(2)[::2]
+    assert not d._prefill_kernels_serve(9)
