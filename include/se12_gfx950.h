@@ -318,6 +318,18 @@ int se12_decode(se12_handle* h, uint16_t* out_dev, void* stream);
  * output, in one launch (a layer's q, k, v ahead of its prompt product). */
 int se12_decode_group(se12_handle* const* handles, int32_t count, uint16_t* const* outs_dev, void* stream);
 
+/* Decodes a whole matrix on the current device from its streams, without a
+ * handle: what se12_bind and se12_decode give, for a matrix that is decoded and
+ * not multiplied. check_host is pinned host memory of
+ * se12_decode_streams_check_bytes() bytes, 16-byte aligned, of this call alone:
+ * the fallback tiles are counted and the codebook read back, as by se12_bind,
+ * and the call returns once they are there (the decode may still run).
+ * With check_host and codebook_out NULL nothing is checked and the call does
+ * not wait: for streams that have passed before. */
+int64_t se12_decode_streams_check_bytes(void);
+int se12_decode_streams(const se12_streams* streams, int64_t rows, int64_t cols, uint16_t* out_dev, void* check_host,
+                        uint8_t codebook_out[15], void* stream);
+
 /* Decodes `nrows` rows given by device int64 indices, in that order, to
  * [nrows, cols] BF16 bits; only the tiles covering those rows are read. An
  * index outside [0, rows) yields a row of zeros. Replaces

@@ -149,6 +149,8 @@ SIGNATURES = {
     ),
     "se12_decode": (c_i32, [c_void_p, c_void_p, c_void_p]),
     "se12_decode_group": (c_i32, [ctypes.POINTER(c_void_p), c_i32, ctypes.POINTER(c_void_p), c_void_p]),
+    "se12_decode_streams_check_bytes": (c_i64, []),
+    "se12_decode_streams": (c_i32, [ctypes.POINTER(Streams), c_i64, c_i64, c_void_p, c_void_p, c_u8p, c_void_p]),
     "se12_decode_rows": (c_i32, [c_void_p, c_void_p, c_i64, c_void_p, c_void_p]),
     "se12_codebook_from_histogram": (c_i32, [ctypes.POINTER(ctypes.c_uint64), c_u8p]),
     "se12_decode_rows_scaled": (c_i32, [c_void_p, c_void_p, c_i64, ctypes.c_float, c_void_p, c_void_p]),

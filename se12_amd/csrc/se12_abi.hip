@@ -276,21 +276,26 @@ int se12_bind_workspace(int64_t rows, int64_t cols, int32_t max_batch, int32_t f
     return SE12_OK;
 }
 
+static int check_streams(const char* fn, const se12_streams* s) {
+    if (!s->sm_dev || !s->ec_dev || !s->esc_dev || !s->codebook_dev || !s->fallback_bitmap_dev)
+        return fail(SE12_E_INVALID, "%s: a required stream pointer is NULL", fn);
+    if (!aligned16(s->sm_dev) || !aligned16(s->ec_dev) || !aligned16(s->esc_dev) ||
+        (s->fallback_raw_dev && !aligned16(s->fallback_raw_dev)))
+        return fail(SE12_E_INVALID, "%s: sm/ec/esc/fallback_raw must be 16-byte aligned", fn);
+    if (s->fallback_raw_elems < 0 || s->fallback_raw_elems % SE12_TILE_SIZE != 0)
+        return fail(SE12_E_INVALID, "%s: fallback_raw has %lld elements, not a whole number of tiles", fn,
+                    (long long)s->fallback_raw_elems);
+    if (s->fallback_raw_elems > 0 && !s->fallback_raw_dev)
+        return fail(SE12_E_INVALID, "%s: fallback_raw is NULL but has elements", fn);
+    return SE12_OK;
+}
+
 static int bind_se12(const se12_streams* s, int64_t rows, int64_t cols, int32_t max_batch, const HandleMemory* mem,
                      void* stream, se12_handle** out) {
     if (!s || !out) return fail(SE12_E_INVALID, "se12_bind: NULL argument");
     *out = nullptr;
     if (int rc = check_shape(rows, cols, max_batch)) return rc;
-    if (!s->sm_dev || !s->ec_dev || !s->esc_dev || !s->codebook_dev || !s->fallback_bitmap_dev)
-        return fail(SE12_E_INVALID, "se12_bind: a required stream pointer is NULL");
-    if (!aligned16(s->sm_dev) || !aligned16(s->ec_dev) || !aligned16(s->esc_dev) ||
-        (s->fallback_raw_dev && !aligned16(s->fallback_raw_dev)))
-        return fail(SE12_E_INVALID, "se12_bind: sm/ec/esc/fallback_raw must be 16-byte aligned");
-    if (s->fallback_raw_elems < 0 || s->fallback_raw_elems % SE12_TILE_SIZE != 0)
-        return fail(SE12_E_INVALID, "se12_bind: fallback_raw has %lld elements, not a whole number of tiles",
-                    (long long)s->fallback_raw_elems);
-    if (s->fallback_raw_elems > 0 && !s->fallback_raw_dev)
-        return fail(SE12_E_INVALID, "se12_bind: fallback_raw is NULL but has elements");
+    if (int rc = check_streams("se12_bind", s)) return rc;
     se12_handle* h = new se12_handle();
     std::memset(h, 0, sizeof *h);
     h->format = SE12_FORMAT_SE12;
@@ -1363,6 +1368,67 @@ int se12_decode_group(se12_handle* const* handles, int32_t count, uint16_t* cons
     return decode_group("se12_decode_group", handles, count, outs, stream);
 }
 
+static int compute_units(int* cus) {
+    int dev = 0;
+    SE12_HIP(hipGetDevice(&dev));
+    SE12_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return SE12_OK;
+}
+
+int64_t se12_decode_streams_check_bytes(void) { return (int64_t)sizeof(BindResult); }
+
+int se12_decode_streams(const se12_streams* s, int64_t rows, int64_t cols, uint16_t* out, void* check_host,
+                        uint8_t codebook_out[15], void* stream) {
+    const char* fn = "se12_decode_streams";
+    if (!s || !out || !check_host != !codebook_out) return fail(SE12_E_INVALID, "%s: NULL argument", fn);
+    if (int rc = check_shape(rows, cols, 1)) return rc;
+    if (int rc = check_streams(fn, s)) return rc;
+    if (!aligned16(check_host)) return fail(SE12_E_INVALID, "%s: check_host must be 16-byte aligned", fn);
+    DecodeGroup g{};
+    DecodeArgs& a = g.m[0];
+    a.sm = s->sm_dev;
+    a.ec = s->ec_dev;
+    a.esc = s->esc_dev;
+    a.codebook = s->codebook_dev;
+    a.bitmap = s->fallback_bitmap_dev;
+    a.fb_raw = s->fallback_raw_dev;
+    a.raw_tiles = s->fallback_raw_elems / SE12_TILE_SIZE;
+    a.out = out;
+    a.N = rows;
+    a.K = cols;
+    a.TR = (int32_t)ceil_div(rows, SE12_TILE_ROWS);
+    a.TC = (int32_t)ceil_div(cols, SE12_TILE_COLS);
+    a.T = (int64_t)a.TR * a.TC;
+    a.out_vec_ok = (aligned16(out) && cols % 8 == 0) ? 1 : 0;
+    g.count = 1;
+    int cus = 0;
+    if (int rc = compute_units(&cus)) return rc;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!check_host) {
+        SE12_HIP(launch_decode_direct(g, st, cus));
+        return SE12_OK;
+    }
+    BindResult* r = static_cast<BindResult*>(check_host);
+    hipEvent_t checked;
+    SE12_HIP(hipEventCreateWithFlags(&checked, hipEventDisableTiming));
+    hipError_t e = launch_check_streams(a.bitmap, a.T, a.codebook, r, st);
+    if (e == hipSuccess) e = hipEventRecord(checked, st);
+    if (e == hipSuccess) e = launch_decode_direct(g, st, cus);
+    if (e == hipSuccess) e = hipEventSynchronize(checked);
+    (void)hipEventDestroy(checked);
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(st);   // nothing still reads the caller's memory
+        return fail(SE12_E_HIP, "%s: %s", fn, hipGetErrorString(e));
+    }
+    if ((int64_t)r->fallback_tiles != a.raw_tiles) {
+        (void)hipStreamSynchronize(st);
+        return fail(SE12_E_INVALID, "%s: bitmap marks %lld fallback tiles but fallback_raw holds %lld elements", fn,
+                    (long long)r->fallback_tiles, (long long)s->fallback_raw_elems);
+    }
+    std::memcpy(codebook_out, r->codebook, SE12_CODEBOOK_SIZE);
+    return SE12_OK;
+}
+
 static int decode_rows(const char* fn, se12_handle* h, const int64_t* rows, int64_t nrows, float scale, uint16_t* out,
                        void* stream) {
     if (!h) return fail(SE12_E_INVALID, "%s: NULL handle", fn);
@@ -1439,13 +1505,6 @@ static int encode_streams_args(EncodeArgs& a, const se12_streams_out* out) {
     a.bitmap = out->fallback_bitmap_dev;
     a.raw = out->fallback_raw_dev;
     a.raw_tiles = out->fallback_raw_tiles;
-    return SE12_OK;
-}
-
-static int compute_units(int* cus) {
-    int dev = 0;
-    SE12_HIP(hipGetDevice(&dev));
-    SE12_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
     return SE12_OK;
 }
 

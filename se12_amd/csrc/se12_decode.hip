@@ -47,6 +47,34 @@ __device__ __forceinline__ void store8(uint16_t* out_row, int64_t col, int64_t K
     }
 }
 
+// Patches the escapes of a tile in the half layout as its ec words show them:
+// parts, then lanes, then weights are the row-major order in which escapes take
+// the esc slots (past the 15th: the last, like the reference's clip). Scalar work
+// per escape; a tile of N(0, 0.02) weights holds less than one. esc: lane k holds
+// word k of the slots.
+__device__ __forceinline__ void patch_found_escapes(uint32_t pat[4][8], const HalfTileLoads& t, uint32_t esc, uint32_t lane) {
+    uint32_t found[8], any = 0;
+#pragma unroll
+    for (int p = 0; p < 8; ++p) any |= found[p] = escape_nibbles(t.ec[p]);
+    if (!wave_any(any != 0u)) return;
+    uint32_t r = 0;
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+        uint32_t* q = &pat[p >> 1][4 * (p & 1)];
+        for (uint64_t lanes = __builtin_amdgcn_ballot_w64(found[p] != 0u); lanes != 0; lanes &= lanes - 1) {
+            const int owner = __builtin_ctzll(lanes);
+            uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)found[p], owner);
+            for (; m != 0u; m &= m - 1u, ++r) {
+                const uint32_t c = (uint32_t)__builtin_ctz(m) >> 2, slot = r < 15u ? r : 15u;
+                const uint32_t e = ((uint32_t)__builtin_amdgcn_readlane((int)esc, (int)(slot >> 2)) >> (8u * (slot & 3u))) & 0xFFu;
+                const uint32_t v = (int)lane == owner ? e << ((c & 1u) ? 23u : 7u) : 0u;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) q[i] |= (c >> 1) == i ? v : 0u;
+            }
+        }
+    }
+}
+
 // Whole-matrix decode: nw waves stream the tiles, wave g taking tiles g,
 // g + nw, ... (the waves read a moving window of the tile-major streams),
 // each with the next tile's loads in flight while it decodes and stores the
@@ -67,6 +95,12 @@ __device__ __forceinline__ void store8(uint16_t* out_row, int64_t col, int64_t K
 // table in LDS is a matrix's): the
 // seven matrices of a Gemma-2-2B layer take 59.5 us in four launches against 70 in
 // seven, mostly on q, k, v (9.0 us), whose own launches end before they fill HBM.
+//
+// DIRECT: from the format's streams alone, for a matrix that is decoded once and
+// never bound: the fallback bit and the 16 esc bytes are read per tile, the
+// escapes found in the ec words that the tile holds anyway. A fallback rank past
+// raw_tiles gives zeros (the caller refuses such streams).
+template <bool DIRECT>
 __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(DecodeGroup grp) {
     SE12_DECLARE_LUT(lut);
     int mi = 0;
@@ -82,12 +116,18 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Dec
     const uint32_t g = (blockIdx.x - (uint32_t)grp.block0[mi]) * kDecodeWaves + (uint32_t)w;
     const uint32_t n = g < NW && g < T ? (T - 1u - g) / NW + 1u : 0u;  // tiles of this wave
     struct Slot {
-        TileSide side;
+        TileSide side;        // DIRECT: lane k % 4 the k-th word of the esc slots
         HalfTileLoads t;
+        uint32_t bits;        // DIRECT: the tile's byte of the bitmap
     };
     auto load = [&](Slot& sl, uint32_t i) {
         const uint32_t tile = min(g + i * NW, T - 1u);
-        load_side(sl.side, a.side, tile, lane);
+        if constexpr (DIRECT) {
+            sl.side.rec = reinterpret_cast<const uint32_t*>(a.esc + (int64_t)tile * kEscBudget)[lane & 3u];
+            sl.bits = a.bitmap[tile >> 3];
+        } else {
+            load_side(sl.side, a.side, tile, lane);
+        }
         load_tile_half(sl.t, a.sm, a.ec, tile, lane);
     };
     const bool vec_ok = a.out_vec_ok != 0;
@@ -97,7 +137,9 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Dec
         const int kt = (int)(tile - (uint32_t)tr * TC);
         const int64_t col = (int64_t)kt * kTileCols + 8 * (lane & 31u);
         const int64_t row0 = (int64_t)tr * kTileRows + (lane >> 5);
-        const uint32_t info = side_info(sl.side, 0);
+        const bool direct_fallback =
+            DIRECT && ((__builtin_amdgcn_readfirstlane((int)sl.bits) >> (7u - (tile & 7u))) & 1) != 0;
+        const uint32_t info = DIRECT ? (direct_fallback ? kInfoFallback : 0u) : side_info(sl.side, 0);
         // wave-uniform: a tile inside the matrix whose rows take whole
         // 16-byte stores needs no per-lane guard
         const bool full = vec_ok && (int64_t)(tr + 1) * kTileRows <= a.N && (int64_t)(kt + 1) * kTileCols <= a.K;
@@ -113,10 +155,16 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Dec
         };
         if (info_is_fallback(info)) {
             // a tile read as raw BF16 (tile-local row-major, like sm)
-            const int16_t* raw = raw_tile_ptr(info, a.fb_raw, a.ovf_raw) + 8 * lane;
             uint4 r[8];
+            const int64_t rank = DIRECT ? fallback_rank(a.bitmap, tile, lane) : 0;
+            if (!DIRECT || rank < a.raw_tiles) {
+                const int16_t* raw = (DIRECT ? a.fb_raw + rank * kTile : raw_tile_ptr(info, a.fb_raw, a.ovf_raw)) + 8 * lane;
 #pragma unroll
-            for (int p = 0; p < 8; ++p) r[p] = stream_load(reinterpret_cast<const uint4*>(raw + 512 * p));
+                for (int p = 0; p < 8; ++p) r[p] = stream_load(reinterpret_cast<const uint4*>(raw + 512 * p));
+            } else {
+#pragma unroll
+                for (int p = 0; p < 8; ++p) r[p] = make_uint4(0u, 0u, 0u, 0u);
+            }
             wait_vector_loads();  // rare path: keeps the common path's waits exact
 #pragma unroll
             for (int p = 0; p < 8; ++p) {
@@ -126,7 +174,10 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Dec
         } else {
             uint32_t pat[4][8];
             lookup_tile_half(lut, sl.t, pat);
-            patch_tile_escapes<kHalfLayout>(pat, info, sl.side, 0, lane);
+            if constexpr (DIRECT)
+                patch_found_escapes(pat, sl.t, sl.side.rec, lane);
+            else
+                patch_tile_escapes<kHalfLayout>(pat, info, sl.side, 0, lane);
 #pragma unroll
             for (int p = 0; p < 8; ++p) {
                 uint32_t wv[4];
@@ -137,10 +188,21 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Dec
     };
     // the pair table, then the first tile (a wave past the grid's waves
     // re-loads tile g's clamp, so that the table's wait count is exact)
-    const uint4 lutv = reinterpret_cast<const uint4*>(a.lut)[lane];
+    static_assert(kDecodeWaves * kWave == 256, "a thread per entry of the pair table");
+    uint4 lutv = make_uint4(0u, 0u, 0u, 0u);
+    uint8_t code[2];
+    if constexpr (DIRECT) {
+        code[0] = a.codebook[min(tid & 15, kCodebook - 1)];
+        code[1] = a.codebook[min(tid >> 4, kCodebook - 1)];
+    } else {
+        lutv = reinterpret_cast<const uint4*>(a.lut)[lane];
+    }
     Slot s0, s1;
     load(s0, 0);
-    store_block_lut(lut, lutv, lane);
+    if constexpr (DIRECT)
+        lut[tid] = ((tid & 15) < kCodebook ? (uint32_t)code[0] << 7 : 0u) | ((tid >> 4) < kCodebook ? (uint32_t)code[1] << 23 : 0u);
+    else
+        store_block_lut(lut, lutv, lane);
     lds_barrier();
     if (n == 0) return;
     uint32_t i = 0;
@@ -229,7 +291,7 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_rows_kernel(Decod
 constexpr int kDecodeStreamWavesPerCu = 4;
 
 // The waves are shared out by the matrices' tiles, in whole blocks.
-hipError_t launch_decode(DecodeGroup& g, hipStream_t stream, int cu_count) {
+static void share_waves(DecodeGroup& g, int cu_count) {
     const int64_t waves = (int64_t)std::max(1, cu_count) * kDecodeStreamWavesPerCu;
     int64_t tiles = 0;
     for (int i = 0; i < g.count; ++i) tiles += g.m[i].T;
@@ -239,7 +301,57 @@ hipError_t launch_decode(DecodeGroup& g, hipStream_t stream, int cu_count) {
         g.nw[i] = std::min<int64_t>(g.m[i].T, share);
         g.block0[i + 1] = g.block0[i] + (int32_t)((g.nw[i] + kDecodeWaves - 1) / kDecodeWaves);
     }
-    hipLaunchKernelGGL(decode_stream_kernel, dim3((uint32_t)g.block0[g.count]), dim3(kDecodeWaves * kWave), 0, stream, g);
+}
+
+hipError_t launch_decode(DecodeGroup& g, hipStream_t stream, int cu_count) {
+    share_waves(g, cu_count);
+    hipLaunchKernelGGL(decode_stream_kernel<false>, dim3((uint32_t)g.block0[g.count]), dim3(kDecodeWaves * kWave), 0, stream, g);
+    return hipGetLastError();
+}
+
+hipError_t launch_decode_direct(DecodeGroup& g, hipStream_t stream, int cu_count) {
+    share_waves(g, cu_count);
+    hipLaunchKernelGGL(decode_stream_kernel<true>, dim3((uint32_t)g.block0[g.count]), dim3(kDecodeWaves * kWave), 0, stream, g);
+    return hipGetLastError();
+}
+
+// One block: the fallback tiles of the bitmap and the codebook, into memory that
+// the host reads (system-scope stores). Ahead of a direct decode, so that the
+// host has its answer while that still runs.
+constexpr int kCheckThreads = 1024;
+
+__global__ __launch_bounds__(kCheckThreads) void check_streams_kernel(const uint8_t* bitmap, int64_t T, const uint8_t* codebook,
+                                                                       BindResult* out) {
+    __shared__ unsigned long long sum[kCheckThreads / kWave];
+    const int tid = threadIdx.x;
+    const int64_t bytes = T >> 3;
+    unsigned long long n = 0;
+    for (int64_t b = 8 * (int64_t)tid; b < bytes; b += 8 * kCheckThreads) {
+        if (b + 8 <= bytes) {
+            uint64_t v;
+            __builtin_memcpy(&v, bitmap + b, sizeof v);
+            n += __popcll(v);
+        } else {
+            for (int64_t i = b; i < bytes; ++i) n += __popc((uint32_t)bitmap[i]);
+        }
+    }
+    if (tid == 0 && (T & 7)) n += __popc((uint32_t)bitmap[bytes] >> (8 - (T & 7)));
+    for (int o = 32; o > 0; o /= 2) n += __shfl_xor(n, o, 64);
+    if ((tid & 63) == 0) sum[tid >> 6] = n;
+    __syncthreads();
+    if (tid < 16) {
+        const uint8_t c = tid < kCodebook ? codebook[tid] : 0;
+        __hip_atomic_store(&out->codebook[tid], c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (tid == 0) {
+        n = 0;
+        for (int k = 0; k < kCheckThreads / kWave; ++k) n += sum[k];
+        __hip_atomic_store(&out->fallback_tiles, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+hipError_t launch_check_streams(const uint8_t* bitmap, int64_t T, const uint8_t* codebook, BindResult* out, hipStream_t stream) {
+    hipLaunchKernelGGL(check_streams_kernel, dim3(1), dim3(kCheckThreads), 0, stream, bitmap, T, codebook, out);
     return hipGetLastError();
 }
 

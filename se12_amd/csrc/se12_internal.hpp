@@ -150,6 +150,7 @@ struct DecodeArgs {
     const int64_t* rows;      // decode_rows only
     uint16_t* out;
     int64_t N, K, T, nrows, items;
+    int64_t raw_tiles;        // direct decode only: tiles fb_raw holds
     int32_t TR, TC;
     int32_t out_vec_ok;
 };
@@ -318,6 +319,10 @@ struct BindResult {
 };
 hipError_t launch_bind_tiles(const uint8_t* bitmap, const uint8_t* ec, const uint8_t* esc, const uint8_t* codebook, int64_t T,
                              uint32_t* side, uint32_t* lut, BindResult* result, hipStream_t stream);
+// a whole matrix from its streams (no lut, side or ovf_raw), and what a caller
+// checks of them (overflow_tiles is not written)
+hipError_t launch_decode_direct(DecodeGroup& g, hipStream_t stream, int cu_count);
+hipError_t launch_check_streams(const uint8_t* bitmap, int64_t T, const uint8_t* codebook, BindResult* out, hipStream_t stream);
 hipError_t launch_overflow_decode(const DecodeArgs& a, int16_t* raw, hipStream_t stream);
 // histogram and codebook (also to codebook_out on the device unless NULL)
 hipError_t launch_encode_histogram(const EncodeArgs& a, int cu_count, uint8_t* codebook_out, hipStream_t stream);

@@ -181,3 +181,62 @@ def test_decode_rows_equals_the_oracle_at_tile_edges(gpu, rows, cols, kind):
         assert torch.equal(scaled.nan_to_num(), ref.nan_to_num())      # (0 == -0 in a row outside the matrix)
     with pytest.raises(Exception):
         k.decode_rows_scaled_into(idx, out, float("inf"))
+
+
+@pytest.mark.parametrize("rows,cols,kind", [(1, 1, "tail"), (36, 300, "tail"), (48, 768, "uniform"), (17, 257, "uniform"),
+                                            (2049, 1024, "tail"), (1, 214, "uniform"), (4096, 4104, "tail")])
+def test_decode_from_the_streams_equals_decode_of_the_bound_matrix(gpu, rows, cols, kind):
+    """Fallback tiles, tiles past the listed escapes, part tiles, more tiles than waves, bitmaps that end inside a byte; the
+    unchecked repeat gives the same bits."""
+    from se12_amd.hip import HipSe12WeightDecoder, Se12MatVecKernel, encode_on_device
+
+    bits = uniform_bits(rows, cols, seed=rows) if kind == "uniform" else heavy_tailed_bf16(rows, cols, seed=cols)
+    dt = encode_on_device(bf16_tensor(bits, gpu))
+    dec = HipSe12WeightDecoder()
+    first, again = dec.decode_to_device(dt), dec.decode_to_device(dt)
+    bound = Se12MatVecKernel(dt, max_batch=1).decode_into(torch.empty((rows, cols), dtype=torch.bfloat16, device=gpu))
+    for got in (first, again, bound):
+        assert np.array_equal(got.view(torch.int16).cpu().numpy(), bits)
+
+
+def test_decode_from_the_streams_refuses_what_bind_refuses(gpu):
+    import dataclasses
+
+    from se12_amd.hip import HipSe12WeightDecoder, encode_on_device
+
+    dt = encode_on_device(bf16_tensor(uniform_bits(64, 512, seed=7), gpu))
+    assert dt.fallback_raw.numel() > 4096
+    dec = HipSe12WeightDecoder()
+    with pytest.raises(Exception, match="fallback tiles"):
+        dec.decode_to_device(dataclasses.replace(dt, fallback_raw=dt.fallback_raw[4096:].contiguous()))
+    with pytest.raises(ValueError, match="codebook"):
+        dec.decode_to_device(dataclasses.replace(dt, codebook_host=tuple(reversed(dt.codebook_host))))
+    assert dec.decode_to_device(dt).shape == (64, 512)
+
+
+def test_decoder_on_two_streams_and_two_threads(gpu):
+    import threading
+
+    from se12_amd.hip import HipSe12WeightDecoder, RowIndices, encode_on_device
+
+    cases = [heavy_tailed_bf16(512, 1024 + 256 * i, seed=i) for i in range(4)]
+    dec, bad = HipSe12WeightDecoder(), []
+
+    def work(k):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for bits in cases[k::2] * 3:
+                out = dec.decode_to_device(encode_on_device(bf16_tensor(bits, gpu)))
+                s.synchronize()
+                if not np.array_equal(out.view(torch.int16).cpu().numpy(), bits):
+                    bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad
+    dt = encode_on_device(bf16_tensor(cases[0], gpu))
+    assert np.array_equal(dec.decode_to_device(dt).view(torch.int16).cpu().numpy(), cases[0])
+    assert np.array_equal(dec.decode_rows(dt, RowIndices((3, 500))).bit_pattern.reshape(2, -1), cases[0][[3, 500]])
