@@ -364,18 +364,24 @@ int se12_encode(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld,
                 const uint8_t codebook[15], const se12_streams_out* out, int64_t* fallback_tiles_out,
                 void* stream);
 
-/* The whole encoder in one call: histogram, codebook, sm / ec / esc and the
- * fallback bitmap of w, without a round trip to the host in between. Writes the
- * streams of `out` except fallback_raw (out->fallback_raw_* may be NULL / 0),
- * the codebook to codebook_dev[15] (device) and codebook_out (host) and the
- * number of fallback tiles; the caller then gives se12_encode_fallback a buffer
- * of that many tiles. `workspace`: device memory of se12_encode_workspace()
- * bytes, 16-byte aligned, contents indifferent. Synchronizes `stream` (the count
- * and the codebook are results). Same bytes as se12_encode_prepare +
- * se12_encode, which allocate their own scratch and read w twice more. */
+/* The encoder without a round trip to the host in the middle, in two calls on
+ * one stream. se12_encode_codebook counts the exponents of w and chooses the
+ * codebook (to codebook_dev[15] and `workspace`; asynchronous, so the caller
+ * can allocate the streams while it runs). se12_encode_streams then writes the
+ * streams of `out` except fallback_raw (out->fallback_raw_* may be NULL / 0)
+ * and returns the codebook and the number of fallback tiles; the caller gives
+ * se12_encode_fallback a buffer of that many tiles. `workspace`: device memory
+ * of se12_encode_workspace() bytes, 16-byte aligned, contents indifferent, the
+ * same in both calls; `result_host`: pinned host memory of
+ * se12_encode_result_bytes() bytes, 16-byte aligned, of this call alone.
+ * Synchronizes `stream`. Same bytes as se12_encode_prepare + se12_encode, which
+ * allocate their own scratch and read w twice more. */
 int64_t se12_encode_workspace(void);
+int64_t se12_encode_result_bytes(void);
+int se12_encode_codebook(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld, uint8_t* codebook_dev,
+                         void* workspace, int64_t workspace_bytes, void* stream);
 int se12_encode_streams(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld, const se12_streams_out* out,
-                        uint8_t* codebook_dev, uint8_t codebook_out[15], int64_t* fallback_tiles_out, void* workspace,
+                        uint8_t codebook_out[15], int64_t* fallback_tiles_out, void* result_host, void* workspace,
                         int64_t workspace_bytes, void* stream);
 
 /* The raw bits of the tiles that fallback_bitmap_dev marks, in tile order, to

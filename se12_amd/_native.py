@@ -155,8 +155,10 @@ SIGNATURES = {
     "se12_codebook_from_histogram": (c_i32, [ctypes.POINTER(ctypes.c_uint64), c_u8p]),
     "se12_decode_rows_scaled": (c_i32, [c_void_p, c_void_p, c_i64, ctypes.c_float, c_void_p, c_void_p]),
     "se12_encode_workspace": (c_i64, []),
+    "se12_encode_result_bytes": (c_i64, []),
+    "se12_encode_codebook": (c_i32, [c_void_p, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_i64, c_void_p]),
     "se12_encode_streams": (
-        c_i32, [c_void_p, c_i64, c_i64, c_i64, ctypes.POINTER(StreamsOut), c_void_p, c_u8p, ctypes.POINTER(c_i64), c_void_p,
+        c_i32, [c_void_p, c_i64, c_i64, c_i64, ctypes.POINTER(StreamsOut), c_u8p, ctypes.POINTER(c_i64), c_void_p, c_void_p,
                 c_i64, c_void_p],
     ),
     "se12_encode_fallback": (c_i32, [c_void_p, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_i64, c_void_p]),

@@ -1509,11 +1509,6 @@ static int encode_streams_args(EncodeArgs& a, const se12_streams_out* out) {
 }
 
 namespace {
-// what the host reads of an EncodeWork, in one copy
-struct EncodeResult {
-    uint8_t codebook[16];
-    unsigned long long fallback_tiles;
-};
 static_assert(offsetof(EncodeWork, fallback_tiles) == offsetof(EncodeWork, codebook) + offsetof(EncodeResult, fallback_tiles),
               "EncodeResult mirrors EncodeWork");
 hipError_t read_result(EncodeResult* r, const EncodeWork* ws, hipStream_t st) {
@@ -1524,26 +1519,45 @@ hipError_t read_result(EncodeResult* r, const EncodeWork* ws, hipStream_t st) {
 
 int64_t se12_encode_workspace(void) { return (int64_t)sizeof(EncodeWork); }
 
+int64_t se12_encode_result_bytes(void) { return (int64_t)sizeof(EncodeResult); }
+
+static int encode_workspace(const char* fn, EncodeArgs& a, void* workspace, int64_t workspace_bytes) {
+    if (!workspace || workspace_bytes < (int64_t)sizeof(EncodeWork) || !aligned16(workspace))
+        return fail(SE12_E_CAPACITY, "%s: needs a 16-byte aligned workspace of %zu bytes", fn, sizeof(EncodeWork));
+    a.ws = static_cast<EncodeWork*>(workspace);
+    return SE12_OK;
+}
+
+int se12_encode_codebook(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, uint8_t* codebook_dev, void* workspace,
+                         int64_t workspace_bytes, void* stream) {
+    if (!codebook_dev) return fail(SE12_E_INVALID, "se12_encode_codebook: NULL argument");
+    EncodeArgs a;
+    if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
+    if (int rc = encode_workspace("se12_encode_codebook", a, workspace, workspace_bytes)) return rc;
+    int cus = 0;
+    if (int rc = compute_units(&cus)) return rc;
+    SE12_HIP(launch_encode_histogram(a, cus, codebook_dev, static_cast<hipStream_t>(stream)));
+    return SE12_OK;
+}
+
 int se12_encode_streams(const uint16_t* w, int64_t rows, int64_t cols, int64_t ld, const se12_streams_out* out,
-                        uint8_t* codebook_dev, uint8_t codebook_out[15], int64_t* fallback_tiles_out, void* workspace,
+                        uint8_t codebook_out[15], int64_t* fallback_tiles_out, void* result_host, void* workspace,
                         int64_t workspace_bytes, void* stream) {
-    if (!out || !codebook_dev || !codebook_out || !fallback_tiles_out || !workspace)
-        return fail(SE12_E_INVALID, "se12_encode_streams: NULL argument");
-    if (workspace_bytes < (int64_t)sizeof(EncodeWork) || !aligned16(workspace))
-        return fail(SE12_E_CAPACITY, "se12_encode_streams: needs a 16-byte aligned workspace of %zu bytes", sizeof(EncodeWork));
+    if (!out || !codebook_out || !fallback_tiles_out || !result_host || !aligned16(result_host))
+        return fail(SE12_E_INVALID, "se12_encode_streams: NULL or misaligned argument");
     EncodeArgs a;
     if (int rc = encode_args(a, w, rows, cols, ld)) return rc;
     if (int rc = encode_streams_args(a, out)) return rc;
-    int cus = 0;
-    if (int rc = compute_units(&cus)) return rc;
+    if (int rc = encode_workspace("se12_encode_streams", a, workspace, workspace_bytes)) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    a.ws = static_cast<EncodeWork*>(workspace);
-    EncodeResult r;
-    SE12_HIP(launch_encode_histogram(a, cus, codebook_dev, st));
-    SE12_HIP(launch_encode_tiles(a, true, st));
-    SE12_HIP(read_result(&r, a.ws, st));
-    std::memcpy(codebook_out, r.codebook, SE12_CODEBOOK_SIZE);
-    *fallback_tiles_out = (int64_t)r.fallback_tiles;
+    EncodeResult* r = static_cast<EncodeResult*>(result_host);
+    hipError_t e = launch_encode_tiles(a, true, st);
+    if (e == hipSuccess) e = launch_encode_result(a, r, st);
+    const hipError_t waited = hipStreamSynchronize(st);   // nothing still writes the caller's memory
+    if (e == hipSuccess) e = waited;
+    if (e != hipSuccess) return fail(SE12_E_HIP, "se12_encode_streams: %s", hipGetErrorString(e));
+    std::memcpy(codebook_out, r->codebook, SE12_CODEBOOK_SIZE);
+    *fallback_tiles_out = (int64_t)r->fallback_tiles;
     return SE12_OK;
 }
 

@@ -18,11 +18,13 @@
 //
 // Bound by the weights' bytes: read once for the histogram, once (from the
 // last-level cache where they fit) for the streams.
-// 9216x2304 as the packer's call issues it 253 -> 73 us (histogram 78 -> 10.2:
+// 9216x2304 as the packer's call issues it 253 -> 58 us (histogram 78 -> 10.2:
 // it read 2 bytes per load, divided 64-bit indexes and queued on shared LDS
-// counters; select 7.2; tiles 17.2 + 2 x 11 of counting + 9.4 of scanning ->
-// 19; the rest is the call's one synchronisation, was 4, and its allocations);
-// 256000x2304 2,024 -> 626 us, 5.2 TB/s of weights read twice and streams.
+// counters; select 6.5; tiles 17.2 + 2 x 11 of counting + 9.4 of scanning ->
+// 18.5; the result's way to the host 4.0; the rest is the call's one
+// synchronisation, was 4, and its allocations, most of them made while the
+// first two kernels run); 256000x2304 2,024 -> 621 us, 5.2 TB/s of weights read
+// twice and streams.
 #include <algorithm>
 
 #include "se12_device.hpp"
@@ -105,26 +107,36 @@ __global__ __launch_bounds__(kHistThreads) void encode_histogram_kernel(EncodeAr
 __global__ __launch_bounds__(kHistThreads) void encode_select_kernel(EncodeWork* ws, int blocks, uint8_t* codebook_out) {
     __shared__ uint64_t part[kHistThreads];
     __shared__ __attribute__((aligned(16))) uint64_t key[kBins];   // count << 8 | exponent
+    constexpr int kGroups = kBins / 4, kRuns = kHistThreads / kGroups, kFlight = 16;
+    __shared__ uint64_t sums[kRuns * kBins];
     const int tid = threadIdx.x, e = tid & (kBins - 1), s = tid / kBins;
-    constexpr int kSlices = kHistThreads / kBins, kFlight = 32;
-    uint64_t n = 0;
-    // one block waits for its loads alone: many in flight (7.2 us with 32 and
-    // the one-key ranks below, 20.6 with 16 and two-field ranks)
-    for (int b0 = s; b0 < blocks; b0 += kSlices * kFlight) {
-        uint32_t v[kFlight];
+    constexpr int kSlices = kHistThreads / kBins;
+    // one block waits for its loads alone, so 256 blocks' counts are all in
+    // flight at once: four bins per load, 16 loads per thread (7.1 -> 6.5 us)
+    uint64_t n4[4] = {0, 0, 0, 0};
+    for (int b0 = tid / kGroups; b0 < blocks; b0 += kRuns * kFlight) {
+        uint4 v[kFlight];
 #pragma unroll
         for (int k = 0; k < kFlight; ++k) {
-            const int b = b0 + k * kSlices;
-            v[k] = ws->partial[(int64_t)(b < blocks ? b : s) * kBins + e];
+            const int b = b0 + k * kRuns;
+            v[k] = reinterpret_cast<const uint4*>(ws->partial + (int64_t)(b < blocks ? b : b0) * kBins)[tid & (kGroups - 1)];
         }
 #pragma unroll
-        for (int k = 0; k < kFlight; ++k) n += b0 + k * kSlices < blocks ? v[k] : 0u;
+        for (int k = 0; k < kFlight; ++k) {
+            if (b0 + k * kRuns >= blocks) continue;
+            n4[0] += v[k].x;
+            n4[1] += v[k].y;
+            n4[2] += v[k].z;
+            n4[3] += v[k].w;
+        }
     }
-    part[tid] = n;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sums[4 * tid + i] = n4[i];
     __syncthreads();
     if (tid < kBins) {
+        uint64_t n = 0;
 #pragma unroll
-        for (int k = 1; k < kSlices; ++k) n += part[tid + k * kBins];
+        for (int k = 0; k < kRuns; ++k) n += sums[k * kBins + tid];
         key[tid] = (n << 8) | (uint64_t)tid;
         ws->histogram[tid] = n;
     }
@@ -352,6 +364,20 @@ hipError_t launch_encode_tiles(const EncodeArgs& a, bool write, hipStream_t stre
         hipLaunchKernelGGL(encode_tiles_kernel<true>, grid, block, 0, stream, a);
     else
         hipLaunchKernelGGL(encode_tiles_kernel<false>, grid, block, 0, stream, a);
+    return hipGetLastError();
+}
+
+// What the host reads of a call, into memory that it can: a copy of the
+// runtime's takes 4.2 us on the device and as long again to issue.
+__global__ void encode_result_kernel(const EncodeWork* ws, EncodeResult* host) {
+    const int tid = threadIdx.x;
+    if (tid < 16) __hip_atomic_store(&host->codebook[tid], ws->codebook[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (tid == 16)
+        __hip_atomic_store(&host->fallback_tiles, ws->fallback_tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t launch_encode_result(const EncodeArgs& a, EncodeResult* host, hipStream_t stream) {
+    hipLaunchKernelGGL(encode_result_kernel, dim3(1), dim3(kWave), 0, stream, a.ws, host);
     return hipGetLastError();
 }
 

@@ -171,7 +171,13 @@ struct EncodeWork {
     uint8_t code_of[256];
     uint8_t codebook[16];                 // read back by the host with fallback_tiles
     unsigned long long fallback_tiles;
-    uint32_t partial[kEncodeHistBlocks * 256];
+    alignas(16) uint32_t partial[kEncodeHistBlocks * 256];
+};
+
+// what the host reads of an EncodeWork (laid out alike)
+struct EncodeResult {
+    uint8_t codebook[16];
+    unsigned long long fallback_tiles;
 };
 
 struct EncodeArgs {
@@ -328,6 +334,7 @@ hipError_t launch_overflow_decode(const DecodeArgs& a, int16_t* raw, hipStream_t
 hipError_t launch_encode_histogram(const EncodeArgs& a, int cu_count, uint8_t* codebook_out, hipStream_t stream);
 hipError_t launch_encode_codes(const EncodeArgs& a, const uint8_t codebook[16], hipStream_t stream);
 hipError_t launch_encode_tiles(const EncodeArgs& a, bool write, hipStream_t stream);
+hipError_t launch_encode_result(const EncodeArgs& a, EncodeResult* host, hipStream_t stream);
 hipError_t launch_encode_raw(const EncodeArgs& a, hipStream_t stream);
 // Streaming-read probe (se12_probe.hip): its grid for a device and the launch.
 int64_t read_probe_blocks(int32_t compute_units);

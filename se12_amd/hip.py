@@ -563,18 +563,21 @@ def encode_on_device(weights: torch.Tensor) -> Se12DeviceTensor:
     lib = nat.lib()
     with torch.cuda.device(dev):
         st = nat.stream_ptr()
+        codebook_dev = torch.empty(CODEBOOK_SIZE, dtype=torch.uint8, device=dev)
+        ws = torch.empty(lib.se12_encode_workspace(), dtype=torch.uint8, device=dev)
+        nat.check(lib.se12_encode_codebook(nat.ptr(w), rows, cols, cols, nat.ptr(codebook_dev), nat.ptr(ws), ws.numel(), st))
+        # (while that runs)
         sm = torch.empty(t * TILE_SIZE, dtype=torch.uint8, device=dev)
         ec = torch.empty(t * TILE_SIZE // 2, dtype=torch.uint8, device=dev)
         esc = torch.empty(t * ESCAPE_BUDGET, dtype=torch.uint8, device=dev)
         bitmap = torch.empty(bitmap_bytes(t), dtype=torch.uint8, device=dev)
-        codebook_dev = torch.empty(CODEBOOK_SIZE, dtype=torch.uint8, device=dev)
-        ws = torch.empty(lib.se12_encode_workspace(), dtype=torch.uint8, device=dev)
+        result = torch.empty(lib.se12_encode_result_bytes(), dtype=torch.uint8, pin_memory=True)
         out = nat.StreamsOut(
             sm_dev=sm.data_ptr(), ec_dev=ec.data_ptr(), esc_dev=esc.data_ptr(), fallback_bitmap_dev=bitmap.data_ptr(),
             fallback_raw_dev=None, fallback_raw_tiles=0,
         )
-        nat.check(lib.se12_encode_streams(nat.ptr(w), rows, cols, cols, ctypes.byref(out), nat.ptr(codebook_dev), cb,
-                                          ctypes.byref(nfb), nat.ptr(ws), ws.numel(), st))
+        nat.check(lib.se12_encode_streams(nat.ptr(w), rows, cols, cols, ctypes.byref(out), cb, ctypes.byref(nfb),
+                                          nat.ptr(result), nat.ptr(ws), ws.numel(), st))
         raw = torch.empty(nfb.value * TILE_SIZE, dtype=torch.int16, device=dev)
         if nfb.value:
             nat.check(lib.se12_encode_fallback(nat.ptr(w), rows, cols, cols, nat.ptr(bitmap), nat.ptr(raw), nfb.value, st))
