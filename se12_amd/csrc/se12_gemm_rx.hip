@@ -230,7 +230,6 @@ __attribute__((amdgpu_waves_per_eu(XG ? 2 : 3))) void gemm_rx_kernel(GemvGroupAr
             for (int e = 0; e < 4; ++e)
                 v[e] = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(acc[g][e])));
             const int b = 16 * g + (int)(lane >> 2);
-            store_row_ss(v, b, tr);
             if (b < batch) {
                 float* yp = a.y + (int64_t)b * a.N + (int64_t)tr * kTileRows + 4 * (int)(lane & 3u);
                 if (y_vec) {
@@ -240,6 +239,7 @@ __attribute__((amdgpu_waves_per_eu(XG ? 2 : 3))) void gemm_rx_kernel(GemvGroupAr
                     for (int e = 0; e < 4; ++e) yp[e] = v[e];
                 }
             }
+            store_row_ss(v, b, tr);   // after y's stores, which wait for nothing of it
         }
     };
 
