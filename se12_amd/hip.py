@@ -482,6 +482,12 @@ class HipSe12WeightDecoder:
         self._last: _Decoded | None = None
         self._lock = threading.RLock()   # a decode is launched before another thread's replaces its tensor
 
+    def __getstate__(self) -> dict:   # copies and pickles have a lock of their own
+        return {k: v for k, v in self.__dict__.items() if k != "_lock"}
+
+    def __setstate__(self, state: dict) -> None:
+        self.__dict__.update(state, _lock=threading.RLock())
+
     def _known(self, tensor: Any) -> _Decoded | None:
         return self._last if self._last is not None and self._last.tensor is tensor else None
 

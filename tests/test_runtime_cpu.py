@@ -174,3 +174,14 @@ def test_prompt_pass_off_the_kernels_runs_the_framework_ops(other):
         n = w.layers[0]["pre_ffw_norm"]
         w.layers[0]["pre_ffw_norm"] = n.float() if other == "norm_dtype" else n.repeat_interleave(2)[::2]
     assert not d._prefill_kernels_serve(9)
+
+
+def test_a_decoder_can_be_copied_and_pickled():
+    import copy
+    import pickle
+
+    from se12_amd.hip import HipSe12WeightDecoder
+
+    d = HipSe12WeightDecoder()
+    for other in (copy.deepcopy(d), pickle.loads(pickle.dumps(d))):
+        assert other._known(object()) is None and other._lock is not d._lock
