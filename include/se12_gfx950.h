@@ -386,7 +386,8 @@ int se12_encode_streams(const uint16_t* w_dev, int64_t rows, int64_t cols, int64
 
 /* The raw bits of the tiles that fallback_bitmap_dev marks, in tile order, to
  * fallback_raw_dev [fallback_raw_tiles * 4096] (tiles past its capacity are
- * left out). Asynchronous on `stream`. */
+ * left out). Synchronizes `stream`: the streams of an encoded matrix are used
+ * on other streams, and w given back, as soon as its encoder calls return. */
 int se12_encode_fallback(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld,
                          const uint8_t* fallback_bitmap_dev, int16_t* fallback_raw_dev, int64_t fallback_raw_tiles,
                          void* stream);

@@ -1571,7 +1571,11 @@ int se12_encode_fallback(const uint16_t* w, int64_t rows, int64_t cols, int64_t 
     a.bitmap = const_cast<uint8_t*>(fallback_bitmap_dev);
     a.raw = fallback_raw_dev;
     a.raw_tiles = fallback_raw_tiles;
-    SE12_HIP(launch_encode_raw(a, static_cast<hipStream_t>(stream)));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipError_t e = launch_encode_raw(a, st);
+    const hipError_t waited = hipStreamSynchronize(st);   // nothing still reads w
+    if (e == hipSuccess) e = waited;
+    if (e != hipSuccess) return fail(SE12_E_HIP, "se12_encode_fallback: %s", hipGetErrorString(e));
     return SE12_OK;
 }
 

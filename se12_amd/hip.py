@@ -556,7 +556,9 @@ class HipSe12WeightDecoder:
 
 def encode_on_device(weights: torch.Tensor) -> Se12DeviceTensor:
     """SE12-encodes a [rows, cols] BF16 device tensor on the GPU; the streams are
-    byte-identical to the reference encoder's (codec.py:111-141)."""
+    byte-identical to the reference encoder's (codec.py:111-141). Nothing of the
+    call is pending when it returns or raises: the result can be used on any
+    stream, and the weights given back, at once."""
     if weights.dtype != torch.bfloat16 or weights.dim() != 2:
         raise ValueError("encode_on_device needs a 2-D bfloat16 tensor")
     w = weights.contiguous()
@@ -572,21 +574,24 @@ def encode_on_device(weights: torch.Tensor) -> Se12DeviceTensor:
         codebook_dev = torch.empty(CODEBOOK_SIZE, dtype=torch.uint8, device=dev)
         ws = torch.empty(lib.se12_encode_workspace(), dtype=torch.uint8, device=dev)
         nat.check(lib.se12_encode_codebook(nat.ptr(w), rows, cols, cols, nat.ptr(codebook_dev), nat.ptr(ws), ws.numel(), st))
-        # (while that runs)
-        sm = torch.empty(t * TILE_SIZE, dtype=torch.uint8, device=dev)
-        ec = torch.empty(t * TILE_SIZE // 2, dtype=torch.uint8, device=dev)
-        esc = torch.empty(t * ESCAPE_BUDGET, dtype=torch.uint8, device=dev)
-        bitmap = torch.empty(bitmap_bytes(t), dtype=torch.uint8, device=dev)
-        result = torch.empty(lib.se12_encode_result_bytes(), dtype=torch.uint8, pin_memory=True)
-        out = nat.StreamsOut(
-            sm_dev=sm.data_ptr(), ec_dev=ec.data_ptr(), esc_dev=esc.data_ptr(), fallback_bitmap_dev=bitmap.data_ptr(),
-            fallback_raw_dev=None, fallback_raw_tiles=0,
-        )
-        nat.check(lib.se12_encode_streams(nat.ptr(w), rows, cols, cols, ctypes.byref(out), cb, ctypes.byref(nfb),
-                                          nat.ptr(result), nat.ptr(ws), ws.numel(), st))
-        raw = torch.empty(nfb.value * TILE_SIZE, dtype=torch.int16, device=dev)
-        if nfb.value:
-            nat.check(lib.se12_encode_fallback(nat.ptr(w), rows, cols, cols, nat.ptr(bitmap), nat.ptr(raw), nfb.value, st))
+        try:   # (while that runs)
+            sm = torch.empty(t * TILE_SIZE, dtype=torch.uint8, device=dev)
+            ec = torch.empty(t * TILE_SIZE // 2, dtype=torch.uint8, device=dev)
+            esc = torch.empty(t * ESCAPE_BUDGET, dtype=torch.uint8, device=dev)
+            bitmap = torch.empty(bitmap_bytes(t), dtype=torch.uint8, device=dev)
+            result = torch.empty(lib.se12_encode_result_bytes(), dtype=torch.uint8, pin_memory=True)
+            out = nat.StreamsOut(
+                sm_dev=sm.data_ptr(), ec_dev=ec.data_ptr(), esc_dev=esc.data_ptr(), fallback_bitmap_dev=bitmap.data_ptr(),
+                fallback_raw_dev=None, fallback_raw_tiles=0,
+            )
+            nat.check(lib.se12_encode_streams(nat.ptr(w), rows, cols, cols, ctypes.byref(out), cb, ctypes.byref(nfb),
+                                              nat.ptr(result), nat.ptr(ws), ws.numel(), st))
+            raw = torch.empty(nfb.value * TILE_SIZE, dtype=torch.int16, device=dev)
+            if nfb.value:
+                nat.check(lib.se12_encode_fallback(nat.ptr(w), rows, cols, cols, nat.ptr(bitmap), nat.ptr(raw), nfb.value, st))
+        except BaseException:
+            torch.cuda.current_stream().synchronize()
+            raise
     return Se12DeviceTensor(
         sm=sm, ec=ec, esc=esc, codebook=codebook_dev, fallback_bitmap=bitmap, fallback_raw=raw, rows=int(rows),
         cols=int(cols), codebook_host=tuple(cb),

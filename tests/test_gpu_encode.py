@@ -105,3 +105,28 @@ def test_encoder_at_tile_and_bitmap_edges(gpu, rows, cols, kind):
     for k in got:
         if k != "codebook":
             assert torch.equal(got[k], aligned[k]), k
+
+
+def test_nothing_is_pending_after_an_encode(gpu):
+    """A matrix of fallback tiles packed on a side stream is complete when the
+    call returns: another stream decodes it, and the weights' memory is given
+    back, without a wait of the caller's."""
+    import torch
+
+    from se12_amd.hip import HipSe12WeightDecoder, encode_on_device
+
+    g = torch.Generator(device=gpu)
+    g.manual_seed(5)
+    bits = torch.randint(-32768, 32768, (32768, 2304), generator=g, device=gpu, dtype=torch.int16)
+    w = bits.clone().view(torch.bfloat16)
+    torch.cuda.synchronize()
+    side, other = torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)
+    with torch.cuda.stream(side):
+        t = encode_on_device(w)
+    assert side.query()
+    assert t.fallback_raw.numel() == bits.numel()      # every tile is raw
+    w.zero_()
+    with torch.cuda.stream(other):
+        got = HipSe12WeightDecoder().decode_to_device(t)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), bits)
