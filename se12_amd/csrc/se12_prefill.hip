@@ -167,11 +167,18 @@ __global__ __launch_bounds__(kRopeThreads) void prefill_rope_kernel(RopeArgs a) 
 // the scores of a lane, as they come out of the first product, the B operand
 // of the second (key of A row m: kKeyOfRow), so probabilities never leave
 // their lane.
-// The soft-capped scores lie within +-softcap (at most kMaxSoftcap), so
-// exp(s) neither overflows nor vanishes in FP32 and no running maximum is
-// needed: the sums of different key tiles just add. Scores, capping and
-// sums are FP32; a probability is rounded to BF16 for the second product, and
-// their sum is that of the rounded ones, so that the weights add up to one.
+// Scores, capping and sums are FP32; a probability is rounded to BF16 for the
+// second product, and their sum is that of the rounded ones, so that the weights
+// add up to one. A query's weights are 2^(s - m - shift): s its scores (base 2),
+// m the largest of them seen, or up to kMaxSlack below it. m starts at the
+// wave's first tile; a tile that passes it by more than kMaxSlack moves m and
+// what is summed, and starts again. shift makes the weights add up to less than
+// one, so the sums of any finite V stay finite, as with weights normalised
+// first, and the largest weight stays above 2^-45: V down to 1e-24 keeps its
+// bits. (e^s itself fits FP32 with |s| <= softcap, and summing it needs no m,
+// but V above 6e16 then overflows at a softcap of 50: 1,024 / 4,096 positions, 8
+// heads of 256, both launches, 32.8 / 147 us that way, 33.8 / 157 this, 40 where
+// scores of a standard deviation of 16 make tiles start again.)
 // K and V^T operands come straight from L2, 1 KB of consecutive bytes per
 // instruction in the order prefill_rope_kernel left them; with K and V^T
 // row-major, 32 bytes of each of 32 rows per instruction, the first-level cache
@@ -181,6 +188,7 @@ __global__ __launch_bounds__(kRopeThreads) void prefill_rope_kernel(RopeArgs a) 
 constexpr int kPrefillThreads = 256;
 constexpr int kPrefillRows = 32;
 constexpr float kMaxSoftcap = 64.0f;
+constexpr float kMaxSlack = 16.0f;      // base 2
 
 struct PrefillAttnArgs {
     const uint16_t* qkv;     // [B, T, stride], rotated
@@ -191,6 +199,7 @@ struct PrefillAttnArgs {
     int T, Tp, heads, kvh, window;
     float c1;                // 2 scaling / softcap, base 2
     float c2;                // softcap, base 2
+    float shift;             // log2 of the keys of a query (rounded up) + 1 + kMaxSlack
 };
 
 template <int D>
@@ -198,6 +207,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_attention_kernel(Pref
     constexpr int kSteps = D / 16;     // inner steps of the first product
     constexpr int kTiles = D / 32;     // row tiles of the second
     extern __shared__ __attribute__((aligned(16))) float sums[];   // [2][kTiles * 16 + 1][64]
+    __shared__ float maxima[kPrefillThreads / 64][32];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int head = blockIdx.y, b = blockIdx.z, kh = head / (a.heads / a.kvh);
     // the blocks with the most keys first
@@ -218,7 +228,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_attention_kernel(Pref
     for (int i = 0; i < kTiles; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] = 0.0f;
-    float l = 0.0f;
+    float l = 0.0f, m = -a.c2;     // no score is lower
 
     const int last = min(q0 + kPrefillRows, a.T) - 1;   // the block's last query sees keys up to itself
     const int lo = a.window > 0 ? max(0, q0 - a.window + 1) : 0;
@@ -231,93 +241,139 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_attention_kernel(Pref
     auto load_k = [&](int t) {
         const uint16_t* p = kp + (int64_t)min(t, t_last) * (32 * D);
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) kf[s] = *reinterpret_cast<const bf16x8_t*>(p + 512 * s);
+        for (int s = 0; s < kSteps; ++s) {
+            kf[s] = *reinterpret_cast<const bf16x8_t*>(p + 512 * s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     auto load_v = [&](int t) {
         const uint16_t* p = vp + (int64_t)min(t, t_last) * (32 * D);
 #pragma unroll
         for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
+            for (int s = 0; s < 2; ++s) {
                 vf[i][s] = *reinterpret_cast<const bf16x8_t*>(p + 512 * (2 * i + s));
+                __builtin_amdgcn_sched_barrier(0);
+            }
     };
     constexpr int kWaves = kPrefillThreads / 64;
-    int kt = lo / 32 + w;
+    const int kt0 = lo / 32 + w;
+    int kt = kt0;
+    float top = 0.0f;
     load_k(kt);
+    __builtin_amdgcn_sched_barrier(0);   // the order of the loop's loads, and so its waits
     load_v(kt);
-    for (; kt <= t_last; kt += kWaves) {
-        const int k0 = 32 * kt;
-        floatx16_t sc;
+    while (true) {
+        bool higher = false;
+        for (; kt <= t_last; kt += kWaves) {
+            const int k0 = 32 * kt;
+            floatx16_t sc;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) sc[e] = 0.0f;
+            for (int e = 0; e < 16; ++e) sc[e] = 0.0f;
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qf[s], sc, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        load_k(kt + kWaves);
-        __builtin_amdgcn_sched_barrier(0);
-        float p[16];
+            for (int s = 0; s < kSteps; ++s) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qf[s], sc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            load_k(kt + kWaves);
+            __builtin_amdgcn_sched_barrier(0);
+            // softcap tanh(x) = softcap (1 - 2 r), r = 1 / (1 + e^2x), base 2
+            float r[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            // softcap tanh(x) = softcap (1 - 2 / (1 + e^2x)), then e^ of it
-            const float ex = __builtin_amdgcn_exp2f(sc[e] * a.c1);
-            p[e] = __builtin_amdgcn_exp2f(a.c2 - 2.0f * a.c2 * __builtin_amdgcn_rcpf(1.0f + ex));
-        }
-        const bool inside = k0 + 31 <= q0 && (a.window <= 0 || last - k0 < a.window);
-        if (!inside) {
+            for (int e = 0; e < 16; ++e)
+                r[e] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sc[e] * a.c1));
+            const bool inside = k0 + 31 <= q0 && (a.window <= 0 || last - k0 < a.window);
+            if (!inside) {
+                const int reach = a.window > 0 ? a.window : INT32_MAX;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int key = k0 + 16 * (e >> 3) + 8 * half + (e & 7);
-                if (key > q || (a.window > 0 && q - key >= a.window)) p[e] = 0.0f;
+                for (int e = 0; e < 16; ++e) {
+                    const int key = k0 + 16 * (e >> 3) + 8 * half + (e & 7);
+                    r[e] = ((key > q) | (q - key >= reach)) ? INFINITY : r[e];
+                }
             }
-        }
-        bf16x8_t pf[2];
+            float least[5];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            uint32_t u[4];
+            for (int e = 0; e < 5; ++e) least[e] = fminf(fminf(r[3 * e], r[3 * e + 1]), r[3 * e + 2]);
+            top = a.c2 - 2.0f * a.c2 * fminf(fminf(fminf(least[0], least[1]), least[2]), fminf(fminf(least[3], least[4]), r[15]));
+            // (the two lanes of a query keep one maximum)
+            if (kt == kt0) m = fmaxf(m, fmaxf(top, __shfl_xor(top, 32, 64)));
+            const float base = a.c2 - (m + a.shift);
+            bf16x8_t pf[2];
+            float tile_l = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                u[k] = f_to_bf16x2(p[8 * s + 2 * k], p[8 * s + 2 * k + 1]);
-                l += __uint_as_float(u[k] << 16) + __uint_as_float(u[k] & 0xFFFF0000u);
+            for (int s = 0; s < 2; ++s) {
+                uint32_t u[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    u[k] = f_to_bf16x2(__builtin_amdgcn_exp2f(base - 2.0f * a.c2 * r[8 * s + 2 * k]),
+                                       __builtin_amdgcn_exp2f(base - 2.0f * a.c2 * r[8 * s + 2 * k + 1]));
+                    tile_l += __uint_as_float(u[k] << 16) + __uint_as_float(u[k] & 0xFFFF0000u);
+                }
+                pf[s] = __builtin_bit_cast(bf16x8_t, make_uint4(u[0], u[1], u[2], u[3]));
             }
-            pf[s] = __builtin_bit_cast(bf16x8_t, make_uint4(u[0], u[1], u[2], u[3]));
+            higher = __builtin_amdgcn_ballot_w64(top > m + kMaxSlack) != 0;
+            if (!higher) {
+                l += tile_l;
+#pragma unroll
+                for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s)
+                        o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i][s], pf[s], o[i], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            load_v(higher ? kt : kt + kWaves);   // on both paths, so that the waits stay exact
+            if (higher) break;
         }
+        if (!higher) break;
+        // the tile passes the maximum: what is summed moves to the new one, and
+        // the tile starts again (outside the loop over the tiles, so that the
+        // sums stay in accumulation registers there)
+        const float to = fmaxf(m, fmaxf(top, __shfl_xor(top, 32, 64)));
+        const float scale = __builtin_amdgcn_exp2f(m - to);
+        m = to;
+        l *= scale;
 #pragma unroll
         for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i][s], pf[s], o[i], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        load_v(kt + kWaves);
+            for (int e = 0; e < 16; ++e) o[i][e] *= scale;
+        load_k(kt);
+        __builtin_amdgcn_s_waitcnt(0);   // rare: keeps the loop's waits exact
     }
     l += __shfl_xor(l, 32, 64);
+    // the waves' sums on one maximum
+    if (half == 0) maxima[w][col] = m;
+    __syncthreads();
+    float all = maxima[0][col];
+#pragma unroll
+    for (int k = 1; k < kWaves; ++k) all = fmaxf(all, maxima[k][col]);
+    const float scale = __builtin_amdgcn_exp2f(m - all);
 
     // waves 2, 3 hand their sums to 0, 1, then 1 to 0: (w0 + w2) + (w1 + w3)
     constexpr int kValues = kTiles * 16 + 1;
-    auto put = [&](int slot) {
+    auto put = [&](int slot, float by) {
         float* to = sums + (size_t)slot * kValues * 64 + lane;
 #pragma unroll
         for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) to[(16 * i + e) * 64] = o[i][e];
-        to[(kValues - 1) * 64] = l;
+            for (int e = 0; e < 16; ++e) to[(16 * i + e) * 64] = o[i][e] * by;
+        to[(kValues - 1) * 64] = l * by;
     };
-    auto add = [&](int slot) {
+    auto add = [&](int slot, float by) {
         const float* from = sums + (size_t)slot * kValues * 64 + lane;
 #pragma unroll
         for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) o[i][e] += from[(16 * i + e) * 64];
-        l += from[(kValues - 1) * 64];
+            for (int e = 0; e < 16; ++e) o[i][e] = o[i][e] * by + from[(16 * i + e) * 64];
+        l = l * by + from[(kValues - 1) * 64];
     };
-    if (w >= 2) put(w - 2);
+    if (w >= 2) put(w - 2, scale);
     __syncthreads();
-    if (w < 2) add(w);
+    if (w < 2) add(w, scale);
     __syncthreads();
-    if (w == 1) put(0);
+    if (w == 1) put(0, 1.0f);
     __syncthreads();
     if (w > 0 || q >= a.T) {
         return;
     }
-    add(0);
+    add(0, 1.0f);
     const float inv = 1.0f / l;
     uint16_t* op = a.out + (seq + q) * (int64_t)a.heads * D + (int64_t)head * D + 4 * half;
 #pragma unroll
@@ -386,8 +442,11 @@ int se12_step_prefill_attention(uint16_t* qkv, int64_t stride, const uint16_t* c
     const size_t rope_lds = (size_t)kRopeTokens * (2 * head_dim + 16);
     hipLaunchKernelGGL(prefill_rope_kernel, rope_grid, dim3(kRopeThreads), rope_lds, st, r);
     constexpr float kLog2E = 1.4426950408889634f;
+    const int64_t keys = window > 0 ? std::min(window, tokens) : tokens;
+    int keys_log2 = 0;
+    while (((int64_t)1 << keys_log2) < keys) ++keys_log2;
     const PrefillAttnArgs a{qkv, stride, ko, vo, out, tokens, Tp, heads, kv_heads, window,
-                            2.0f * scaling / softcap * kLog2E, softcap * kLog2E};
+                            2.0f * scaling / softcap * kLog2E, softcap * kLog2E, (float)keys_log2 + 1.0f + kMaxSlack};
     if (head_dim == 64)
         launch_prefill_attention<64>(a, batch, st);
     else if (head_dim == 128)

@@ -155,6 +155,48 @@ def test_prefill_attention(gpu, batch, T, heads, kvh, d, L, window):
     assert bool(((out.double() - want).abs() <= bound).all())
 
 
+# what a query's scores do: spread over the whole capped range, all at its lower end, rising along the keys
+@pytest.mark.parametrize("scores", ["wide", "low", "rising"])
+@pytest.mark.parametrize("T,heads,kvh,d,window,log2_v", [(200, 4, 2, 64, 0, 125), (97, 4, 1, 128, 40, 125), (161, 2, 2, 256, 0, 125),
+                                                         (130, 4, 2, 256, 0, -100)])
+def test_prefill_attention_over_the_range_of_v(gpu, T, heads, kvh, d, window, log2_v, scores):
+    """Values up to 2e38, where unnormalised weights of e^score overflow FP32, and down to 1e-30, against 64 bits. The bound is
+    test_prefill_attention's with 1e-4 for the scores: q . k reaches 100 here, its FP32 sum 1e-5 of that."""
+    g = _gen(gpu, T + d + log2_v)
+    stride = (heads + 2 * kvh) * d
+    qkv = torch.randn((1, T, stride), generator=g, device=gpu)
+    q, k, v = qkv[..., :heads * d], qkv[..., heads * d:(heads + kvh) * d], qkv[..., (heads + kvh) * d:]
+    v *= 2.0 ** log2_v
+    if scores == "wide":
+        q *= 8.0
+    else:
+        q.fill_(4.0)
+        k.fill_(-4.0)
+        if scores == "rising":
+            k *= 1.0 - 2.0 * torch.arange(T, device=gpu)[None, :, None] / T
+    qkv = qkv.to(torch.bfloat16)
+    one, zero = torch.ones((T, d), dtype=torch.bfloat16, device=gpu), torch.zeros((T, d), dtype=torch.bfloat16, device=gpu)
+    L = -(-T // 8) * 8
+    kt = torch.zeros((1, kvh, d, L), dtype=torch.bfloat16, device=gpu)
+    vc = torch.zeros((1, kvh, L, d), dtype=torch.bfloat16, device=gpu)
+    out = torch.empty((1, T, heads * d), dtype=torch.bfloat16, device=gpu)
+    n = nat.lib().se12_step_prefill_workspace(1, T, heads, kvh, d)
+    ws = torch.empty(n, dtype=torch.uint8, device=gpu)
+    nat.step_check(nat.lib().se12_step_prefill_attention(
+        nat.ptr(qkv), stride, nat.ptr(one), nat.ptr(zero), nat.ptr(kt), nat.ptr(vc), nat.ptr(out), 1, T, heads, kvh, d, L,
+        d ** -0.5, 50.0, window, nat.ptr(ws), n, nat.stream_ptr()))
+    qd, kd, vd = (qkv[..., a * d: b * d].reshape(T, -1, d).transpose(0, 1).double()
+                  for a, b in ((0, heads), (heads, heads + kvh), (heads + kvh, heads + 2 * kvh)))
+    kd, vd = kd.repeat_interleave(heads // kvh, 0), vd.repeat_interleave(heads // kvh, 0)
+    sc = torch.tanh(qd @ kd.transpose(1, 2).contiguous() * d ** -0.5 / 50.0) * 50.0
+    back = torch.arange(T, device=gpu)[:, None] - torch.arange(T, device=gpu)[None, :]
+    ok = (back >= 0) & (back < window) if window else back >= 0
+    p = torch.softmax(sc.masked_fill(~ok, float("-inf")), -1)
+    want = (p @ vd).transpose(0, 1).reshape(1, T, -1)
+    bound = (3 * 2.0 ** -8 + 2e-4) * (p @ vd.abs()).transpose(0, 1).reshape(1, T, -1)
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+
 def test_prefill_attention_refuses_bad_shapes(gpu):
     t = torch.zeros(4096, dtype=torch.bfloat16, device=gpu)
     lib = nat.lib()
