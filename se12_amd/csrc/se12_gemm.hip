@@ -73,17 +73,19 @@ constexpr int x_slab_bytes() {
 // kXEdge, BF16 of any K and alignment; kXF32, FP32 of any K.
 enum XMode { kXFast, kXEdge, kXF32 };
 
-// FP32 x goes to LDS as three BF16 planes, x = h + m + l exactly: each plane
+// FP32 x goes to LDS as three BF16 planes, x = h + 2^-7 (m + 2^-8 l): each plane
 // is the top 16 bits of what the ones before it leave (8 of the 24
-// significand bits). The product is then three MFMAs per part whose BF16
-// products are exact, summed in FP32: h in one accumulator that is emptied
-// into the row's sum after each K tile, m and l (2^-8 and 2^-16 of it) in
-// another. The edge-handling dot2 kernel it replaces at 5 and more rows reads
-// the weights once per 4 rows. Bound by the conversion and LDS traffic of the
+// significand bits), m and l scaled up to at most x's own size, so that no bit
+// of them falls below BF16's range where x is small (unscaled, x of 2^-116 kept
+// 18 bits and x below 2^-133 none). The product is then three MFMAs per part
+// whose BF16 products are exact, summed in FP32 per K tile and, h apart from m
+// and l, over the tiles. The edge-handling dot2 kernel it replaces at 5 and more
+// rows reads the weights once per 4 rows. Bound by the conversion and LDS traffic of the
 // planes beside the weights' stream. Cold weights, before and after: 3584x14336
-// at 8 / 16 / 32 rows 214 / 427 / 855 -> 28.4 / 34 / 53 us, 2304x9216 100 / 200 /
-// 400 -> 18.4 / 22 / 37, 14336x3584 210 / 420 / 840 -> 27.7 / 32 / 45; error
-// against 64 bits 1.0e-7 to 1.2e-7 (1.0e-7 to 2.8e-7 before).
+// at 8 / 16 / 32 rows 214 / 427 / 855 -> 28.7 / 34.4 / 53 us, 2304x9216 100 / 200
+// / 400 -> 17.6 / 22 / 37, 14336x3584 210 / 420 / 840 -> 28 / 33 / 46 (unscaled
+// planes 27.5 / 33.4 / 52, 17.2 / 21.5 / 37, 27.6 / 32.3 / 45); error against 64
+// bits 1.2e-7 from x of 2^-120 up (1.5e-7 to 2.8e-7 before).
 constexpr int x_planes(XMode xm) { return xm == kXF32 ? 3 : 1; }
 // a piece is 16 bytes of x: 8 BF16 or 4 FP32 columns of one batch row
 constexpr int x_piece_cols(XMode xm) { return xm == kXF32 ? 4 : 8; }
@@ -174,16 +176,21 @@ __device__ __forceinline__ uint4 cut_piece(uint4 v, int shift, int valid) {
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// One FP32 value as three BF16 planes (bits in the high half): h + m + l == x
-// for every finite x whose l is not below BF16's range; an infinity or a NaN
-// goes to h alone (a NaN quiet, so that it stays one in 16 bits).
+// One FP32 value as three BF16 planes (bits in the high half): h + kPlaneM (m +
+// kPlaneL l) == x for every finite x (to 2^-148: the last bit of a subnormal one
+// may fall); an infinity or a NaN goes to h alone (a NaN quiet, so that it
+// stays one in 16 bits).
+constexpr float kPlaneM = 0x1p-7f, kPlaneL = 0x1p-8f;
 __device__ __forceinline__ void split3(uint32_t u, uint32_t& h, uint32_t& m, uint32_t& l) {
     const float x = __uint_as_float(u);
-    const bool finite = (u & 0x7F800000u) != 0x7F800000u;
-    h = x != x ? 0x7FC00000u : (u & 0xFFFF0000u);
-    const float r = finite ? x - __uint_as_float(u & 0xFFFF0000u) : 0.0f;
+    // (a subnormal x, which may be too small for BF16, keeps h from zero, so
+    // that an infinite weight meets none; m takes the difference back)
+    const uint32_t top = (u & 0xFFFF0000u) | (2u * u - 1u < 0x00FFFFFFu ? 0x10000u : 0u);
+    h = x != x ? 0x7FC00000u : top;
+    float r = x - __uint_as_float(top);
+    r = r != r ? 0.0f : r * (1.0f / kPlaneM);
     m = __float_as_uint(r) & 0xFFFF0000u;
-    l = __float_as_uint(r - __uint_as_float(m));
+    l = __float_as_uint((r - __uint_as_float(m)) * (1.0f / kPlaneL));
 }
 
 // pieces past the step's slabs repeat the last piece: the same bytes to the
@@ -340,7 +347,7 @@ __global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
     floatx4_t acc[BG];
 #pragma unroll
     for (int g = 0; g < BG; ++g) acc[g] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    floatx4_t low[XM == kXF32 ? BG : 1];  // the m and l planes' sums
+    floatx4_t low[XM == kXF32 ? BG : 1];  // the m and l planes' sums, times 1 / kPlaneM
     if constexpr (XM == kXF32) {
 #pragma unroll
         for (int g = 0; g < BG; ++g) low[g] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -387,12 +394,17 @@ __global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
                         for (int q = 0; q < 8; ++q) wv[p][q] = finite_pair(wv[p][q]);
                 }
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    mfma_block_part<BG>(wv[p], xb + plane_bytes, p, lane, low);
-                    mfma_block_part<BG>(wv[p], xb + 2 * plane_bytes, p, lane, low);
+                for (int g = 0; g < BG; ++g) {
+                    acc[g] += tile[g];
+                    tile[g] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
                 }
+                if constexpr (BG > 1) __builtin_amdgcn_sched_barrier(0);   // no registers for both at once
 #pragma unroll
-                for (int g = 0; g < BG; ++g) acc[g] += tile[g];
+                for (int p = 0; p < 4; ++p) mfma_block_part<BG>(wv[p], xb + 2 * plane_bytes, p, lane, tile);
+#pragma unroll
+                for (int p = 0; p < 4; ++p) mfma_block_part<BG>(wv[p], xb + plane_bytes, p, lane, low);
+#pragma unroll
+                for (int g = 0; g < BG; ++g) low[g] += tile[g] * kPlaneL;
             }
         };
         // raw words: looked at one by one (FP32 x only)
@@ -574,7 +586,7 @@ __global__ __launch_bounds__(kGemmMaxThreads) void gemm_kernel(GemvGroupArgs ga,
     }
     if constexpr (XM == kXF32) {
 #pragma unroll
-        for (int g = 0; g < BG; ++g) acc[g] += low[g];
+        for (int g = 0; g < BG; ++g) acc[g] += low[g] * kPlaneM;
     }
     // the K groups of a tile row: groups 1..KG-1 hand their sums to group 0
     // through LDS (the x slabs are no longer read: every wave passed the

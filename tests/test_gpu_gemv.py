@@ -189,6 +189,37 @@ def test_float32_activations_keep_infinities_and_nans(gpu, batch):
     assert bool(((y.double() - ref).abs()[small] <= bound[small]).all()) and int(small.sum()) > 60 * (batch - 3)
 
 
+@pytest.mark.parametrize("batch", [5, 16, 32])
+def test_small_float32_activations_keep_their_bits(gpu, batch):
+    """x times 2^-116 gives the results times 2^-116 (but for products under FP32's range, K of 2^-148, and what they turn in a
+    rounding, 2^-22 of the largest result); subnormal x is within the bound of _edge_check and of FP32's range, and of x's last
+    bit (2^-148 of each weight); under an infinite weight it gives an infinity."""
+    from se12_amd.hip import RawBf16MatVecKernel, Se12MatVecKernel, encode_on_device
+
+    rows, cols = 80, 700
+    g = torch.Generator(device=gpu)
+    g.manual_seed(batch)
+    w = (torch.randn((rows, cols), generator=g, device=gpu) * 0.02).to(torch.bfloat16)
+    k, r = Se12MatVecKernel(encode_on_device(w)), RawBf16MatVecKernel(w)
+    x = torch.randn((batch, cols), generator=g, device=gpu)
+    y = k.multiply(x).double()
+    small = k.multiply(x * 2.0 ** -116)
+    assert torch.equal(small, r.multiply(x * 2.0 ** -116))
+    assert bool(((small.double() - y * 2.0 ** -116).abs() <= 2.0 ** -22 * 2.0 ** -116 * y.abs().max() + cols * 2.0 ** -148).all())
+    for e in (-126, -132):
+        xs = torch.ldexp(x, torch.tensor(e, device=gpu))
+        got, x64, w64 = k.multiply(xs), xs.double(), w.double().t().contiguous()
+        assert torch.equal(got, r.multiply(xs))
+        bound = (cols + 16) * (2.0 ** -23 * (x64.abs() @ w64.abs()) + 2.0 ** -149) + 2.0 ** -148 * w64.abs().sum(0)
+        assert bool(((got.double() - x64 @ w64).abs() <= bound).all()), e
+    w[3, 5], w[70, 699] = float("inf"), float("-inf")
+    x[0, 5], x[1, 5], x[0, 699] = 1e-42, -1e-45, 2.0 ** -130
+    k, r = Se12MatVecKernel(encode_on_device(w)), RawBf16MatVecKernel(w)
+    y = k.multiply(x)
+    assert torch.equal(y, r.multiply(x))
+    assert y[0, 3] == float("inf") and y[1, 3] == float("-inf") and y[0, 70] == float("-inf")
+
+
 def test_float32_activations_grouped_and_without_allocation(gpu):
     """The FP32 MFMA path under a grouped launch and in the static scratch: the results of single calls."""
     from se12_amd.hip import Se12MatVecKernel, encode_on_device, multiply_grouped
