@@ -276,11 +276,15 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_rows_kernel(Decod
         v[4] = r1.x; v[5] = r1.y; v[6] = r1.z; v[7] = r1.w;
     }
     if (!here || kt >= a.TC) return;
+    // (a NaN is the framework's, 0x7FC0 whatever the weight's sign and payload)
+    auto scaled = [&](uint32_t w) {
+        const float f = __uint_as_float(w) * scale;
+        return f != f ? __uint_as_float(0x7FC00000u) : f;
+    };
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        if constexpr (SCALED)
-            v[i] = se12step::f_to_bf16x2(__uint_as_float(v[i] << 16) * scale, __uint_as_float(v[i] & 0xFFFF0000u) * scale);
         if (!inside) v[i] = 0u;
+        if constexpr (SCALED) v[i] = se12step::f_to_bf16x2(scaled(v[i] << 16), scaled(v[i] & 0xFFFF0000u));
     }
     store16(a.out + ri * a.K, (int64_t)kt * kTileCols + 16 * c, a.K, a.out_vec_ok != 0, v);
 }

@@ -240,3 +240,18 @@ def test_decoder_on_two_streams_and_two_threads(gpu):
     dt = encode_on_device(bf16_tensor(cases[0], gpu))
     assert np.array_equal(dec.decode_to_device(dt).view(torch.int16).cpu().numpy(), cases[0])
     assert np.array_equal(dec.decode_rows(dt, RowIndices((3, 500))).bit_pattern.reshape(2, -1), cases[0][[3, 500]])
+
+
+@pytest.mark.parametrize("scale", [48.0, -3.5, 1e-30, 2.0 ** -133, 1e38])
+def test_scaled_lookup_gives_the_framework_product_of_every_weight(gpu, scale):
+    """All 65,536 BF16 patterns, NaNs of every payload among them, and rows outside the matrix: the bits of the separate
+    multiply."""
+    from se12_amd.hip import Se12MatVecKernel, encode_on_device
+    from se12_amd.runtime import CompressedEmbedding
+
+    w = torch.arange(65536, device=gpu, dtype=torch.int32).to(torch.int16).view(256, 256).view(torch.bfloat16)
+    k = Se12MatVecKernel(encode_on_device(w))
+    ids = torch.arange(-1, 257, device=gpu)
+    plain = k.decode_rows_into(ids, torch.empty((258, 256), dtype=torch.bfloat16, device=gpu))
+    got = CompressedEmbedding(k, scale=scale)(ids)
+    assert torch.equal(got.view(torch.int16), (plain * torch.tensor(scale, dtype=torch.bfloat16, device=gpu)).view(torch.int16))
