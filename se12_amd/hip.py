@@ -482,8 +482,10 @@ class HipSe12WeightDecoder:
         self._last: _Decoded | None = None
         self._lock = threading.RLock()   # a decode is launched before another thread's replaces its tensor
 
-    def __getstate__(self) -> dict:   # copies and pickles have a lock of their own
-        return {k: v for k, v in self.__dict__.items() if k != "_lock"}
+    # copies and pickles have a lock of their own and have seen no tensor: what is
+    # kept of one belongs to the decoder that waits for its streams
+    def __getstate__(self) -> dict:
+        return {**{k: v for k, v in self.__dict__.items() if k != "_lock"}, "_last": None}
 
     def __setstate__(self, state: dict) -> None:
         self.__dict__.update(state, _lock=threading.RLock())

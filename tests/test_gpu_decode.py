@@ -255,3 +255,22 @@ def test_scaled_lookup_gives_the_framework_product_of_every_weight(gpu, scale):
     plain = k.decode_rows_into(ids, torch.empty((258, 256), dtype=torch.bfloat16, device=gpu))
     got = CompressedEmbedding(k, scale=scale)(ids)
     assert torch.equal(got.view(torch.int16), (plain * torch.tensor(scale, dtype=torch.bfloat16, device=gpu)).view(torch.int16))
+
+
+@pytest.mark.parametrize("use", ["decode_to_device", "decode_rows"])
+def test_copies_and_pickles_of_a_decoder_start_afresh(gpu, use):
+    import copy
+    import pickle
+
+    from se12_amd.hip import HipSe12WeightDecoder, RowIndices, encode_on_device
+
+    bits = heavy_tailed_bf16(64, 512, seed=1)
+    dt = encode_on_device(bf16_tensor(bits, gpu))
+    dec = HipSe12WeightDecoder()
+    dec.decode_to_device(dt) if use == "decode_to_device" else dec.decode_rows(dt, RowIndices((1, 2)))
+    small = len(pickle.dumps(HipSe12WeightDecoder()))
+    assert len(pickle.dumps(dec)) == small                  # no streams travel with it
+    for other in (copy.copy(dec), copy.deepcopy(dec), pickle.loads(pickle.dumps(dec))):
+        assert other._known(dt) is None and other._lock is not dec._lock
+        assert np.array_equal(other.decode_to_device(dt).view(torch.int16).cpu().numpy(), bits)
+    assert dec._known(dt) is not None

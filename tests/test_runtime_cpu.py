@@ -185,3 +185,16 @@ def test_a_decoder_can_be_copied_and_pickled():
     d = HipSe12WeightDecoder()
     for other in (copy.deepcopy(d), pickle.loads(pickle.dumps(d))):
         assert other._known(object()) is None and other._lock is not d._lock
+
+
+def test_what_a_decoder_keeps_of_a_tensor_stays_with_it():
+    import copy
+    import pickle
+    import threading
+
+    from se12_amd.hip import HipSe12WeightDecoder
+
+    d = HipSe12WeightDecoder()
+    d._last = threading.Lock()       # as a handle, nothing that could be copied or pickled
+    for other in (copy.copy(d), copy.deepcopy(d), pickle.loads(pickle.dumps(d))):
+        assert other._last is None and other._lock is not d._lock
