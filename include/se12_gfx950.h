@@ -373,7 +373,8 @@ int se12_encode(const uint16_t* w_dev, int64_t rows, int64_t cols, int64_t ld,
  * se12_encode_fallback a buffer of that many tiles. `workspace`: device memory
  * of se12_encode_workspace() bytes, 16-byte aligned, contents indifferent, the
  * same in both calls; `result_host`: pinned host memory of
- * se12_encode_result_bytes() bytes, 16-byte aligned, of this call alone.
+ * se12_encode_result_bytes() bytes, 16-byte aligned, of this call alone. After
+ * one se12_encode_codebook, se12_encode_streams may be called again.
  * Synchronizes `stream`. Same bytes as se12_encode_prepare + se12_encode, which
  * allocate their own scratch and read w twice more. */
 int64_t se12_encode_workspace(void);

@@ -369,11 +369,14 @@ hipError_t launch_encode_tiles(const EncodeArgs& a, bool write, hipStream_t stre
 
 // What the host reads of a call, into memory that it can: a copy of the
 // runtime's takes 4.2 us on the device and as long again to issue.
-__global__ void encode_result_kernel(const EncodeWork* ws, EncodeResult* host) {
+// The count starts again at zero, for another pass over the tiles.
+__global__ void encode_result_kernel(EncodeWork* ws, EncodeResult* host) {
     const int tid = threadIdx.x;
     if (tid < 16) __hip_atomic_store(&host->codebook[tid], ws->codebook[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (tid == 16)
+    if (tid == 16) {
         __hip_atomic_store(&host->fallback_tiles, ws->fallback_tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        ws->fallback_tiles = 0;
+    }
 }
 
 hipError_t launch_encode_result(const EncodeArgs& a, EncodeResult* host, hipStream_t stream) {

@@ -130,3 +130,30 @@ def test_nothing_is_pending_after_an_encode(gpu):
         got = HipSe12WeightDecoder().decode_to_device(t)
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), bits)
+
+
+def test_streams_can_be_written_again_from_one_codebook(gpu):
+    import ctypes
+
+    import torch
+
+    from se12_amd import _native as nat
+    from se12_amd.hip import encode_on_device
+
+    rows, cols = 100, 1000
+    w = bf16_tensor(uniform_bits(rows, cols, seed=3), gpu)
+    want = encode_on_device(w)
+    lib, st = nat.lib(), nat.stream_ptr()
+    cb_dev = torch.empty(15, dtype=torch.uint8, device=gpu)
+    ws = torch.empty(lib.se12_encode_workspace(), dtype=torch.uint8, device=gpu)
+    nat.check(lib.se12_encode_codebook(nat.ptr(w), rows, cols, cols, nat.ptr(cb_dev), nat.ptr(ws), ws.numel(), st))
+    for _ in range(3):
+        sm, ec, esc, bitmap = (torch.empty_like(t) for t in (want.sm, want.ec, want.esc, want.fallback_bitmap))
+        out = nat.StreamsOut(sm_dev=sm.data_ptr(), ec_dev=ec.data_ptr(), esc_dev=esc.data_ptr(),
+                             fallback_bitmap_dev=bitmap.data_ptr(), fallback_raw_dev=None, fallback_raw_tiles=0)
+        result = torch.empty(lib.se12_encode_result_bytes(), dtype=torch.uint8, pin_memory=True)
+        cb, n = (ctypes.c_uint8 * 15)(), ctypes.c_int64()
+        nat.check(lib.se12_encode_streams(nat.ptr(w), rows, cols, cols, ctypes.byref(out), cb, ctypes.byref(n), nat.ptr(result),
+                                          nat.ptr(ws), ws.numel(), st))
+        assert n.value * 4096 == want.fallback_raw.numel() > 0 and tuple(cb) == want.codebook_host
+        assert torch.equal(sm, want.sm) and torch.equal(bitmap, want.fallback_bitmap)
