@@ -138,7 +138,6 @@ __global__ __launch_bounds__(kHistThreads) void encode_select_kernel(EncodeWork*
 #pragma unroll
         for (int k = 0; k < kRuns; ++k) n += sums[k * kBins + tid];
         key[tid] = (n << 8) | (uint64_t)tid;
-        ws->histogram[tid] = n;
     }
     __syncthreads();
     // four threads per exponent, each against a quarter of the others

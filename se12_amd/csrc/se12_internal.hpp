@@ -167,8 +167,7 @@ struct DecodeGroup {
 // Device scratch of the encoder (se12_encode_workspace bytes).
 constexpr int kEncodeHistBlocks = 512;
 struct EncodeWork {
-    uint64_t histogram[256];
-    uint8_t code_of[256];
+    alignas(16) uint8_t code_of[256];
     uint8_t codebook[16];                 // read back by the host with fallback_tiles
     unsigned long long fallback_tiles;
     alignas(16) uint32_t partial[kEncodeHistBlocks * 256];
