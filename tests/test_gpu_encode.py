@@ -157,3 +157,32 @@ def test_streams_can_be_written_again_from_one_codebook(gpu):
                                           nat.ptr(ws), ws.numel(), st))
         assert n.value * 4096 == want.fallback_raw.numel() > 0 and tuple(cb) == want.codebook_host
         assert torch.equal(sm, want.sm) and torch.equal(bitmap, want.fallback_bitmap)
+
+
+# rows of fewer columns than a load, than a group of 8 lanes' loads, than a wave's, and of several of a wave's; fewer rows
+# than groups of lanes (segments) and more than there are of 8 or 64 lanes
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (40000, 5), (40000, 8), (9, 63), (300, 64), (300, 65), (5000, 511),
+                                       (5000, 513), (3, 40000), (1, 70001), (17, 8192)])
+def test_histogram_of_rows_with_gaps(gpu, rows, cols):
+    """The codebook and the fallback count of rows further apart than their length, NaNs between them, are those of the rows
+    alone."""
+    import ctypes
+
+    import torch
+
+    from se12_amd import _native as nat
+    from se12_amd.hip import encode_on_device
+
+    g = torch.Generator(device=gpu)
+    g.manual_seed(rows + cols)
+    w = (torch.randn((rows, cols), generator=g, device=gpu) * 10.0 ** torch.randint(-4, 4, (rows, 1), generator=g,
+                                                                                     device=gpu)).to(torch.bfloat16)
+    want = encode_on_device(w)
+    counts = torch.bincount((w.view(torch.int16).to(torch.int32).reshape(-1) >> 7) & 0xFF, minlength=256)
+    order = sorted(range(256), key=lambda e: (-int(counts[e]), -e))
+    assert want.codebook_host == tuple(order[:15])
+    wide = torch.full((rows, cols + 3), float("nan"), dtype=torch.bfloat16, device=gpu)
+    wide[:, :cols] = w
+    cb, n = (ctypes.c_uint8 * 15)(), ctypes.c_int64()
+    nat.check(nat.lib().se12_encode_prepare(nat.ptr(wide), rows, cols, cols + 3, cb, ctypes.byref(n), nat.stream_ptr()))
+    assert tuple(cb) == want.codebook_host and n.value * 4096 == want.fallback_raw.numel()
