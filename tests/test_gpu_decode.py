@@ -274,3 +274,40 @@ def test_copies_and_pickles_of_a_decoder_start_afresh(gpu, use):
         assert other._known(dt) is None and other._lock is not dec._lock
         assert np.array_equal(other.decode_to_device(dt).view(torch.int16).cpu().numpy(), bits)
     assert dec._known(dt) is not None
+
+
+@pytest.mark.parametrize("kind", ["normal", "heavy", "uniform"])
+def test_a_matrix_decoded_again_is_bound(gpu, kind):
+    """Decoded from its streams the first time and while a graph captures, from the binding's records after that."""
+    from se12_amd.hip import HipSe12WeightDecoder, encode_on_device
+
+    bits = {"normal": lambda: o.normal_bf16(300, 1100, seed=1, std=0.02), "heavy": lambda: heavy_tailed_bf16(300, 1100, seed=2),
+            "uniform": lambda: uniform_bits(300, 1100, seed=3)}[kind]()
+    dt = encode_on_device(bf16_tensor(bits, gpu))
+    dec = HipSe12WeightDecoder()
+
+    def check(out):
+        torch.cuda.synchronize()
+        assert np.array_equal(out.view(torch.int16).cpu().numpy(), bits)
+
+    check(dec.decode_to_device(dt))
+    assert dec._last.handle is None
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = dec.decode_to_device(dt)
+    assert dec._last.handle is None
+    for _ in range(2):
+        out.zero_()
+        g.replay()
+        check(out)
+    check(dec.decode_to_device(dt))
+    handle = dec._last.handle
+    assert handle is not None
+    check(dec.decode_to_device(dt))
+    side = torch.cuda.Stream(gpu)
+    with torch.cuda.stream(side):
+        again = dec.decode_to_device(dt)
+    check(again)
+    assert dec._last.handle is handle
+    other = encode_on_device(bf16_tensor(np.ascontiguousarray(bits[:64]), gpu))
+    assert dec.decode_to_device(other).shape == (64, 1100) and dec._last.handle is None
