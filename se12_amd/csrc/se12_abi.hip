@@ -1384,8 +1384,7 @@ int se12_decode_streams(const se12_streams* s, int64_t rows, int64_t cols, uint1
     if (int rc = check_shape(rows, cols, 1)) return rc;
     if (int rc = check_streams(fn, s)) return rc;
     if (!aligned16(check_host)) return fail(SE12_E_INVALID, "%s: check_host must be 16-byte aligned", fn);
-    DecodeGroup g{};
-    DecodeArgs& a = g.m[0];
+    DecodeArgs a{};
     a.sm = s->sm_dev;
     a.ec = s->ec_dev;
     a.esc = s->esc_dev;
@@ -1400,12 +1399,11 @@ int se12_decode_streams(const se12_streams* s, int64_t rows, int64_t cols, uint1
     a.TC = (int32_t)ceil_div(cols, SE12_TILE_COLS);
     a.T = (int64_t)a.TR * a.TC;
     a.out_vec_ok = (aligned16(out) && cols % 8 == 0) ? 1 : 0;
-    g.count = 1;
     int cus = 0;
     if (int rc = compute_units(&cus)) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (!check_host) {
-        SE12_HIP(launch_decode_direct(g, st, cus));
+        SE12_HIP(launch_decode_direct(a, st, cus));
         return SE12_OK;
     }
     BindResult* r = static_cast<BindResult*>(check_host);
@@ -1413,7 +1411,7 @@ int se12_decode_streams(const se12_streams* s, int64_t rows, int64_t cols, uint1
     SE12_HIP(hipEventCreateWithFlags(&checked, hipEventDisableTiming));
     hipError_t e = launch_check_streams(a.bitmap, a.T, a.codebook, r, st);
     if (e == hipSuccess) e = hipEventRecord(checked, st);
-    if (e == hipSuccess) e = launch_decode_direct(g, st, cus);
+    if (e == hipSuccess) e = launch_decode_direct(a, st, cus);
     if (e == hipSuccess) e = hipEventSynchronize(checked);
     (void)hipEventDestroy(checked);
     if (e != hipSuccess) {

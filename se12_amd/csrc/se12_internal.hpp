@@ -326,7 +326,7 @@ hipError_t launch_bind_tiles(const uint8_t* bitmap, const uint8_t* ec, const uin
                              uint32_t* side, uint32_t* lut, BindResult* result, hipStream_t stream);
 // a whole matrix from its streams (no lut, side or ovf_raw), and what a caller
 // checks of them (overflow_tiles is not written)
-hipError_t launch_decode_direct(DecodeGroup& g, hipStream_t stream, int cu_count);
+hipError_t launch_decode_direct(const DecodeArgs& a, hipStream_t stream, int cu_count);
 hipError_t launch_check_streams(const uint8_t* bitmap, int64_t T, const uint8_t* codebook, BindResult* out, hipStream_t stream);
 hipError_t launch_overflow_decode(const DecodeArgs& a, int16_t* raw, hipStream_t stream);
 // histogram and codebook (also to codebook_out on the device unless NULL)
