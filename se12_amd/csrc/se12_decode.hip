@@ -146,6 +146,7 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Arg
         load_tile_half(sl.t, a.sm, a.ec, tile, lane);
     };
     const bool vec_ok = a.out_vec_ok != 0;
+    RankCursor ranked;   // DIRECT
     auto emit = [&](const Slot& sl, uint32_t i) {
         const uint32_t tile = g + i * NW;
         const int tr = (int)(tile / TC);
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(kDecodeWaves * kWave) void decode_stream_kernel(Arg
         if (info_is_fallback(info)) {
             // a tile read as raw BF16 (tile-local row-major, like sm)
             uint4 r[8];
-            const int64_t rank = DIRECT ? fallback_rank(a.bitmap, tile, lane) : 0;
+            const int64_t rank = DIRECT ? fallback_rank(a.bitmap, tile, lane, ranked) : 0;
             if (!DIRECT || rank < a.raw_tiles) {
                 const int16_t* raw = (DIRECT ? a.fb_raw + rank * kTile : raw_tile_ptr(info, a.fb_raw, a.ovf_raw)) + 8 * lane;
 #pragma unroll
@@ -397,8 +398,8 @@ hipError_t launch_decode_rows(const DecodeArgs& args, float scale, hipStream_t s
 // One wave per tile. Escapes are ranked in row-major order (chunk, then lane,
 // then weight within the lane), the order in which they take the tile's esc
 // slots; the first kListedEscapes positions go into the tile's record. A
-// fallback tile's word holds its rank in the bitmap (counted by its wave:
-// there are few), a tile with more escapes than listed the next free place
+// fallback tile's word holds its rank in the bitmap (counted by its wave),
+// a tile with more escapes than listed the next free place
 // of the raw buffer bind decodes those into (in no fixed order: the place is
 // only looked up). One kernel for what were a one-block scan of the bitmap, the
 // escape positions, a one-block scan of the counts and the record writes:
@@ -407,7 +408,8 @@ constexpr int kBindThreads = 512;
 
 __global__ __launch_bounds__(kBindThreads) void bind_tiles_kernel(const uint8_t* bitmap, const uint8_t* ec,
                                                                    const uint8_t* esc, const uint8_t* codebook, int64_t T,
-                                                                   uint32_t* side, uint32_t* lut, BindResult* result) {
+                                                                   int64_t run_bytes, uint32_t* side, uint32_t* lut,
+                                                                   BindResult* result) {
     constexpr int kWaves = kBindThreads / kWave;
     __shared__ uint32_t pos[kWaves][kListedEscapes / 2];
     __shared__ uint32_t over[kWaves], fall[kWaves], base;
@@ -418,76 +420,81 @@ __global__ __launch_bounds__(kBindThreads) void bind_tiles_kernel(const uint8_t*
         if (tid < 256) lut[tid] = pair_lut_entry(codebook, (uint32_t)tid);
         if (tid < kCodebook) result->codebook[tid] = codebook[tid];
     }
-    const int64_t tile = (int64_t)blockIdx.x * kWaves + w;
-    const bool here = tile < T;
-    const int64_t t = here ? tile : T - 1;   // a wave past the last tile works on it, and stores nothing
-    const uint8_t* ect = ec + t * (kTile / 2) + 8u * lane;
-    uint2 e[4];
+    RankCursor ranked;
+    const int64_t byte0 = (int64_t)blockIdx.x * run_bytes;
+    for (int64_t byte = byte0; byte < byte0 + run_bytes && byte * kWaves < T; ++byte) {
+        if (byte > byte0) __syncthreads();   // the last turn's counts are read
+        const int64_t tile = byte * kWaves + w;
+        const bool here = tile < T;
+        const int64_t t = here ? tile : T - 1;   // a wave past the last tile works on it, and stores nothing
+        const uint8_t* ect = ec + t * (kTile / 2) + 8u * lane;
+        uint2 e[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) e[j] = *reinterpret_cast<const uint2*>(ect + 512 * j);
-    const uint32_t slots = reinterpret_cast<const uint32_t*>(esc + t * kEscBudget)[(lane - 1u) & 3u];
-    const bool fallback = here && ((bitmap[t >> 3] >> (7 - (t & 7))) & 1u) != 0u;
-    if (lane < kListedEscapes / 2) pos[w][lane] = 0u;
-    __builtin_amdgcn_wave_barrier();
-    uint16_t* listed = reinterpret_cast<uint16_t*>(pos[w]);
-    uint32_t mask = 0, run = 0;
+        for (int j = 0; j < 4; ++j) e[j] = *reinterpret_cast<const uint2*>(ect + 512 * j);
+        const uint32_t slots = reinterpret_cast<const uint32_t*>(esc + t * kEscBudget)[(lane - 1u) & 3u];
+        const bool fallback = here && ((bitmap[t >> 3] >> (7 - (t & 7))) & 1u) != 0u;
+        if (lane < kListedEscapes / 2) pos[w][lane] = 0u;
+        __builtin_amdgcn_wave_barrier();
+        uint16_t* listed = reinterpret_cast<uint16_t*>(pos[w]);
+        uint32_t mask = 0, run = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        uint32_t t0 = escape_nibbles(e[j].x), t1 = escape_nibbles(e[j].y);
-        const uint32_t cnt = __popc(t0) + __popc(t1);
-        const uint32_t incl = wave_incl_scan(cnt);
-        const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
-        if (total) mask |= 1u << j;
-        uint32_t r = run + incl - cnt;
-        const uint32_t first = (4u * j + (lane >> 4)) * kTileCols + 16u * (lane & 15u);
-        while (t0 | t1) {
-            uint32_t p;
-            if (t0) {
-                p = (uint32_t)__builtin_ctz(t0) >> 2;
-                t0 &= t0 - 1u;
-            } else {
-                p = 8u + ((uint32_t)__builtin_ctz(t1) >> 2);
-                t1 &= t1 - 1u;
+        for (int j = 0; j < 4; ++j) {
+            uint32_t t0 = escape_nibbles(e[j].x), t1 = escape_nibbles(e[j].y);
+            const uint32_t cnt = __popc(t0) + __popc(t1);
+            const uint32_t incl = wave_incl_scan(cnt);
+            const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
+            if (total) mask |= 1u << j;
+            uint32_t r = run + incl - cnt;
+            const uint32_t first = (4u * j + (lane >> 4)) * kTileCols + 16u * (lane & 15u);
+            while (t0 | t1) {
+                uint32_t p;
+                if (t0) {
+                    p = (uint32_t)__builtin_ctz(t0) >> 2;
+                    t0 &= t0 - 1u;
+                } else {
+                    p = 8u + ((uint32_t)__builtin_ctz(t1) >> 2);
+                    t1 &= t1 - 1u;
+                }
+                if (r < kListedEscapes) listed[r] = (uint16_t)(first + p);
+                ++r;
             }
-            if (r < kListedEscapes) listed[r] = (uint16_t)(first + p);
-            ++r;
+            run += total;
         }
-        run += total;
-    }
-    const bool too_many = here && !fallback && run > kListedEscapes;
-    if (lane == 0) {
-        over[w] = too_many ? 1u : 0u;
-        fall[w] = fallback ? 1u : 0u;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        uint32_t n_over = 0, n_fall = 0;
+        const bool too_many = here && !fallback && run > kListedEscapes;
+        if (lane == 0) {
+            over[w] = too_many ? 1u : 0u;
+            fall[w] = fallback ? 1u : 0u;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            uint32_t n_over = 0, n_fall = 0;
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) {
-            n_over += over[k];
-            n_fall += fall[k];
+            for (int k = 0; k < kWaves; ++k) {
+                n_over += over[k];
+                n_fall += fall[k];
+            }
+            base = n_over ? (uint32_t)__hip_atomic_fetch_add(&result->overflow_tiles, (unsigned long long)n_over,
+                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                          : 0u;
+            if (n_fall)
+                __hip_atomic_fetch_add(&result->fallback_tiles, (unsigned long long)n_fall, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
         }
-        base = n_over ? (uint32_t)__hip_atomic_fetch_add(&result->overflow_tiles, (unsigned long long)n_over,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                      : 0u;
-        if (n_fall)
-            __hip_atomic_fetch_add(&result->fallback_tiles, (unsigned long long)n_fall, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        uint32_t info = mask | ((run < kInfoCountMax ? run : kInfoCountMax) << kInfoCountShift);
+        if (fallback) {
+            info = kInfoFallback | (uint32_t)fallback_rank(bitmap, t, lane, ranked);
+        } else if (too_many) {
+            uint32_t rank = base;
+            for (int k = 0; k < w; ++k) rank += over[k];
+            info = kInfoFallback | kInfoOverflow | rank;
+        }
+        if (here && lane < kSideWords)
+            side[tile * kSideWords + lane] = lane == 0   ? info
+                                             : lane <= 4 ? slots
+                                             : lane <= 8 ? pos[w][lane - 5]
+                                                         : 0u;
     }
-    __syncthreads();
-    uint32_t info = mask | ((run < kInfoCountMax ? run : kInfoCountMax) << kInfoCountShift);
-    if (fallback) {
-        info = kInfoFallback | (uint32_t)fallback_rank(bitmap, t, lane);
-    } else if (too_many) {
-        uint32_t rank = base;
-        for (int k = 0; k < w; ++k) rank += over[k];
-        info = kInfoFallback | kInfoOverflow | rank;
-    }
-    if (here && lane < kSideWords)
-        side[tile * kSideWords + lane] = lane == 0   ? info
-                                         : lane <= 4 ? slots
-                                         : lane <= 8 ? pos[w][lane - 5]
-                                                     : 0u;
 }
 
 // Decodes every tile with more than the listed escapes into raw[rank]
@@ -529,9 +536,10 @@ hipError_t launch_overflow_decode(const DecodeArgs& a, int16_t* raw, hipStream_t
 
 hipError_t launch_bind_tiles(const uint8_t* bitmap, const uint8_t* ec, const uint8_t* esc, const uint8_t* codebook, int64_t T,
                              uint32_t* side, uint32_t* lut, BindResult* result, hipStream_t stream) {
-    const int64_t blocks = (T + kBindThreads / kWave - 1) / (kBindThreads / kWave);
-    hipLaunchKernelGGL(bind_tiles_kernel, dim3((uint32_t)blocks), dim3(kBindThreads), 0, stream, bitmap, ec, esc, codebook, T,
-                       side, lut, result);
+    static_assert(kBindThreads / kWave == 8, "a byte of the bitmap per block and turn");
+    const int64_t bytes = (T + 7) / 8, run = rank_run(bytes);
+    hipLaunchKernelGGL(bind_tiles_kernel, dim3((uint32_t)((bytes + run - 1) / run)), dim3(kBindThreads), 0, stream, bitmap, ec,
+                       esc, codebook, T, run, side, lut, result);
     return hipGetLastError();
 }
 

@@ -115,11 +115,19 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
 }
 
 // The rank of fallback tile `tile` (the set bits before it in the MSB-first
-// bitmap), counted by a whole wave: 8 bytes per lane and step.
-__device__ __forceinline__ int64_t fallback_rank(const uint8_t* bitmap, int64_t tile, uint32_t lane) {
+// bitmap), counted by a whole wave from the last tile it ranked on (`at`: the
+// bytes counted, and their bits), 8 bytes per lane and step: a wave that takes
+// its tiles in ascending order reads the bitmap once, however many are fallback
+// tiles. (From the start for each, a 2,000,000 x 4096 matrix of them took 75 ms
+// to decode and 14.6 to bind, 7.5 and 4.7 this way.)
+struct RankCursor {
+    int64_t bytes = 0;
+    uint32_t count = 0;
+};
+__device__ __forceinline__ int64_t fallback_rank(const uint8_t* bitmap, int64_t tile, uint32_t lane, RankCursor& at) {
     const int64_t bytes = tile >> 3;
     uint32_t n = 0;
-    for (int64_t b = 8 * (int64_t)lane; b < bytes; b += 8 * kWave) {
+    for (int64_t b = at.bytes + 8 * (int64_t)lane; b < bytes; b += 8 * kWave) {
         if (b + 8 <= bytes) {
             uint64_t v;
             __builtin_memcpy(&v, bitmap + b, sizeof v);
@@ -128,9 +136,16 @@ __device__ __forceinline__ int64_t fallback_rank(const uint8_t* bitmap, int64_t 
             for (int64_t i = b; i < bytes; ++i) n += __popc((uint32_t)bitmap[i]);
         }
     }
-    const uint32_t total = __builtin_amdgcn_readlane(wave_incl_scan(n), kWave - 1);
-    return (int64_t)total + __popc((uint32_t)bitmap[bytes] >> (8 - (tile & 7)));
+    at.count += __builtin_amdgcn_readlane(wave_incl_scan(n), kWave - 1);
+    at.bytes = bytes;
+    return (int64_t)at.count + __popc((uint32_t)bitmap[bytes] >> (8 - (tile & 7)));
 }
+
+// Blocks of a kernel whose waves take tiles 8 by 8 (a byte of the bitmap per
+// block and turn): at most kRankBlocks, each with a run of consecutive bytes, so
+// that the waves' passes over the bitmap stay few.
+constexpr int64_t kRankBlocks = 32768;
+inline int64_t rank_run(int64_t bytes) { return (bytes + kRankBlocks - 1) / kRankBlocks; }
 
 // LDS barrier that does not wait for outstanding global loads (a plain
 // __syncthreads would also drain vmcnt and kill the prefetch).

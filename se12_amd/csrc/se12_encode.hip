@@ -325,25 +325,31 @@ __global__ __launch_bounds__(kTilesThreads) __attribute__((amdgpu_waves_per_eu(4
     }
 }
 
-// One wave per tile: a fallback tile's rank is the number of set bitmap bits
-// before it, counted by the wave.
-__global__ __launch_bounds__(kTilesThreads) void encode_raw_kernel(EncodeArgs a) {
+// One wave per tile and turn: a fallback tile's rank is the number of set
+// bitmap bits before it, counted by the wave.
+__global__ __launch_bounds__(kTilesThreads) void encode_raw_kernel(EncodeArgs a, int64_t run_bytes) {
     const uint32_t lane = threadIdx.x & 63;
-    const int64_t tile = (int64_t)blockIdx.x * (kTilesThreads / kWave) + (threadIdx.x >> 6);
-    if (tile >= a.T || !((a.bitmap[tile >> 3] >> (7 - (tile & 7))) & 1u)) return;
-    const int64_t rank = fallback_rank(a.bitmap, tile, lane);
-    if (rank >= a.raw_tiles) return;
-    const int tr = (int)(tile / a.TC);
-    const int kt = (int)(tile - (int64_t)tr * a.TC);
-    const int64_t col = (int64_t)kt * kTileCols + 16 * (lane & 15u);
-    int16_t* raw = a.raw + rank * kTile;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    RankCursor ranked;
+    const int64_t byte0 = (int64_t)blockIdx.x * run_bytes;
+    for (int64_t byte = byte0; byte < byte0 + run_bytes; ++byte) {
+        const int64_t tile = byte * 8 + w;
+        if (tile >= a.T) return;
+        if (!((a.bitmap[byte] >> (7 - w)) & 1u)) continue;
+        const int64_t rank = fallback_rank(a.bitmap, tile, lane, ranked);
+        if (rank >= a.raw_tiles) return;
+        const int tr = (int)(tile / a.TC);
+        const int kt = (int)(tile - (int64_t)tr * a.TC);
+        const int64_t col = (int64_t)kt * kTileCols + 16 * (lane & 15u);
+        int16_t* raw = a.raw + rank * kTile;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        uint32_t v[8];
-        load_weights16(a, (int64_t)tr * kTileRows + 4 * j + (lane >> 4), col, v);
-        uint4* p = reinterpret_cast<uint4*>(raw + 1024 * j + 16 * lane);
-        p[0] = make_uint4(v[0], v[1], v[2], v[3]);
-        p[1] = make_uint4(v[4], v[5], v[6], v[7]);
+        for (int j = 0; j < 4; ++j) {
+            uint32_t v[8];
+            load_weights16(a, (int64_t)tr * kTileRows + 4 * j + (lane >> 4), col, v);
+            uint4* p = reinterpret_cast<uint4*>(raw + 1024 * j + 16 * lane);
+            p[0] = make_uint4(v[0], v[1], v[2], v[3]);
+            p[1] = make_uint4(v[4], v[5], v[6], v[7]);
+        }
     }
 }
 
@@ -394,8 +400,9 @@ hipError_t launch_encode_result(const EncodeArgs& a, EncodeResult* host, hipStre
 }
 
 hipError_t launch_encode_raw(const EncodeArgs& a, hipStream_t stream) {
-    const dim3 grid((uint32_t)((a.T + kTilesThreads / kWave - 1) / (kTilesThreads / kWave)));
-    hipLaunchKernelGGL(encode_raw_kernel, grid, dim3(kTilesThreads), 0, stream, a);
+    static_assert(kTilesThreads / kWave == 8, "a byte of the bitmap per block and turn");
+    const int64_t bytes = (a.T + 7) / 8, run = rank_run(bytes);
+    hipLaunchKernelGGL(encode_raw_kernel, dim3((uint32_t)((bytes + run - 1) / run)), dim3(kTilesThreads), 0, stream, a, run);
     return hipGetLastError();
 }
 

@@ -311,3 +311,26 @@ def test_a_matrix_decoded_again_is_bound(gpu, kind):
     assert dec._last.handle is handle
     other = encode_on_device(bf16_tensor(np.ascontiguousarray(bits[:64]), gpu))
     assert dec.decode_to_device(other).shape == (64, 1100) and dec._last.handle is None
+
+
+@pytest.mark.parametrize("rows,share", [(64032, 0.02), (64032, 0.5), (64032, 1.0), (480000, 0.3)])
+def test_raw_tiles_of_a_matrix_of_many(gpu, rows, share):
+    """36,018 tiles (36 per wave of the decode) and 270,000 (two turns per block of bind and of the raw copy), `share` of them
+    raw at random: packed, decoded from the streams and from a binding, and looked up by row."""
+    from se12_amd.hip import HipSe12WeightDecoder, Se12MatVecKernel, encode_on_device
+
+    cols = 2304
+    g = torch.Generator(device=gpu)
+    g.manual_seed(int(100 * share))
+    w = (torch.randn((rows, cols), generator=g, device=gpu) * 0.02).to(torch.bfloat16).view(torch.int16)
+    raw = torch.rand((rows // 16, cols // 256), generator=g, device=gpu) < share
+    mask = raw.repeat_interleave(16, 0).repeat_interleave(256, 1)
+    w = torch.where(mask, torch.randint(-32768, 32768, (rows, cols), generator=g, device=gpu, dtype=torch.int16), w)
+    dt = encode_on_device(w.view(torch.bfloat16))
+    assert dt.fallback_raw.numel() >= 4096 * int(raw.sum())
+    assert torch.equal(HipSe12WeightDecoder().decode_to_device(dt).view(torch.int16), w)
+    k = Se12MatVecKernel(dt, max_batch=1)
+    out = torch.empty((rows, cols), dtype=torch.bfloat16, device=gpu)
+    assert torch.equal(k.decode_into(out).view(torch.int16), w)
+    idx = torch.randint(0, rows, (500,), generator=g, device=gpu)
+    assert torch.equal(k.decode_rows_into(idx, torch.empty((500, cols), dtype=torch.bfloat16, device=gpu)).view(torch.int16), w[idx])
