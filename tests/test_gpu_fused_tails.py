@@ -60,7 +60,7 @@ def _x(batch, cols, gpu, seed, dtype=torch.bfloat16):
     (512, 768, 1, torch.bfloat16),      # FAST, one launch
     (9216, 2304, 1, torch.bfloat16),    # Gemma-2-2B gate / up
     (200, 300, 3, torch.bfloat16),      # edge-handling variant, ragged rows
-    (256, 512, 6, torch.float32),       # FP32 x: two dot2 launches (4 + 2 rows)
+    (256, 512, 6, torch.float32),       # FP32 x: one MFMA launch, then the separate kernel
     (384, 512, 8, torch.bfloat16),      # MFMA product, then the separate kernel
 ])
 def test_gelu_mul_tail_equals_the_separate_kernel(gpu, fmt, rows, cols, batch, dtype):
@@ -104,7 +104,7 @@ def _separate_norm(y, w1, w2, res, eps):
     (100, 256, 2, torch.bfloat16),      # one K tile: no split-K
     (300, 700, 3, torch.bfloat16),      # edge-handling variant, ragged rows
     (298, 512, 1, torch.bfloat16),      # rows % 4 != 0: separate kernel
-    (256, 1024, 5, torch.float32),      # FP32 x: two dot2 launches (4 + 1 rows)
+    (256, 1024, 5, torch.float32),      # FP32 x: one MFMA launch, then the separate kernel
     (512, 512, 8, torch.bfloat16),      # MFMA product, then the separate kernel
     (8192, 256, 1, torch.bfloat16),     # 80 KiB of LDS for the tail (gfx950 blocks may take 160 KiB)
 ])
@@ -125,6 +125,42 @@ def test_rmsnorm_tail_matches_the_separate_kernel(gpu, fmt, rows, cols, batch, d
         _norm_close(out, want_out)
         if call < 2:
             want_res, want_out = _separate_norm(want_y, w1, w2, res, eps)
+
+
+@pytest.mark.parametrize("fmt", ["se12", "raw"])
+@pytest.mark.parametrize("batch,waves,splits", [(5, 1, 1), (6, 2, 2), (8, 3, 3)])
+def test_tails_over_two_dot2_launches(gpu, fmt, batch, waves, splits):
+    """FP32 x under a launch configuration runs the dot2 kernel, 4 rows per launch: each tail's rows and counters in the second
+    launch, against the product of the same configuration and the separate kernels."""
+    from se12_amd.hip import multiply_gelu_mul, multiply_grouped
+    from se12_amd.launch import configuration
+
+    rows, cols, eps = 512, 768, 1e-6
+    gate, up = _kernel(rows, cols, 81, fmt, gpu), _kernel(rows, cols, 82, fmt, gpu)
+    two = configuration(waves, splits, 2 * rows, batch, float32_activations=True)
+    one = configuration(waves, splits, rows, batch, float32_activations=True)
+    w1, w2, res0 = _norm_inputs(batch, rows, gpu, 83)
+    res, want_res = res0.clone(), res0
+    for call in range(3):  # the counters reset themselves; the residual accumulates
+        x = _x(batch, cols, gpu, 84 + call, torch.float32)
+        want_y = multiply_grouped([gate, up], x, launch=two)
+        want = torch.empty((batch, rows), dtype=torch.bfloat16, device=gpu)
+        nat.step_check(nat.lib().se12_step_gelu_mul(nat.ptr(want_y[0]), nat.ptr(want_y[1]), nat.STEP_F32, rows, nat.ptr(want),
+                                                    batch, rows, nat.stream_ptr()))
+        out = torch.full((batch, rows), float("nan"), dtype=torch.bfloat16, device=gpu)
+        ys = multiply_gelu_mul(gate, up, x, out, launch=two)
+        assert torch.equal(ys[0], want_y[0]) and torch.equal(ys[1], want_y[1]), call
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), call
+        y = gate.multiply(x, launch=one)
+        want_res, want_out = _separate_norm(y, w1, w2, want_res, eps)
+        out.fill_(float("nan"))
+        assert torch.equal(gate.multiply_rmsnorm(x, w1, w2, res, out, eps, launch=one), y), call
+        _norm_close(res, want_res)
+        _norm_close(out, want_out)
+        want_res = res.clone()
+        ss = torch.full((batch, rows // 16), float("nan"), device=gpu)
+        assert torch.equal(gate.multiply_rowss(x, ss, launch=one), y), call
+        torch.testing.assert_close(ss, _want_row_ss(y), rtol=1e-5, atol=1e-30)
 
 
 def test_tails_replay_in_a_graph(gpu):
@@ -307,7 +343,7 @@ def _want_row_ss(y: torch.Tensor) -> torch.Tensor:
     (2304, 9216, 1, torch.bfloat16),    # down_proj, split-K
     (2304, 9216, 4, torch.bfloat16),
     (300, 512, 3, torch.bfloat16),      # a partial last tile row
-    (256, 1024, 6, torch.bfloat16),     # MFMA product, row sums after it
+    (256, 1024, 6, torch.bfloat16),     # MFMA product, row sums in its waves
     (512, 768, 2, torch.float32),       # FP32 x
 ])
 def test_rowss_sums_the_tile_rows_of_the_output(gpu, fmt, rows, cols, batch, dtype):
