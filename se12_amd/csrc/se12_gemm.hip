@@ -82,9 +82,9 @@ enum XMode { kXFast, kXEdge, kXF32 };
 // and l, over the tiles. The edge-handling dot2 kernel it replaces at 5 and more
 // rows reads the weights once per 4 rows. Bound by the conversion and LDS traffic of the
 // planes beside the weights' stream. Cold weights, before and after: 3584x14336
-// at 8 / 16 / 32 rows 214 / 427 / 855 -> 28.7 / 34.4 / 53 us, 2304x9216 100 / 200
-// / 400 -> 17.6 / 22 / 37, 14336x3584 210 / 420 / 840 -> 28 / 33 / 46 (unscaled
-// planes 27.5 / 33.4 / 52, 17.2 / 21.5 / 37, 27.6 / 32.3 / 45); error against 64
+// at 8 / 16 / 32 rows 214 / 427 / 855 -> 28 / 33.7 / 52 us, 2304x9216 100 / 200 /
+// 400 -> 17.5 / 21.8 / 37, 14336x3584 210 / 420 / 840 -> 28 / 33.7 / 45.5 (unscaled
+// planes 27.7 / 33.4 / 52, 17.2 / 21.5 / 37, 27.7 / 32.6 / 45); error against 64
 // bits 1.2e-7 from x of 2^-120 up (1.5e-7 to 2.8e-7 before).
 constexpr int x_planes(XMode xm) { return xm == kXF32 ? 3 : 1; }
 // a piece is 16 bytes of x: 8 BF16 or 4 FP32 columns of one batch row
@@ -178,17 +178,15 @@ __device__ __forceinline__ uint4 cut_piece(uint4 v, int shift, int valid) {
 
 // One FP32 value as three BF16 planes (bits in the high half): h + kPlaneM (m +
 // kPlaneL l) == x for every finite x (to 2^-148: the last bit of a subnormal one
-// may fall); an infinity or a NaN goes to h alone (a NaN quiet, so that it
-// stays one in 16 bits).
+// may fall). An infinity goes to h alone; a NaN's m is a NaN, which no finite
+// weight takes away.
 constexpr float kPlaneM = 0x1p-7f, kPlaneL = 0x1p-8f;
 __device__ __forceinline__ void split3(uint32_t u, uint32_t& h, uint32_t& m, uint32_t& l) {
     const float x = __uint_as_float(u);
     // (a subnormal x, which may be too small for BF16, keeps h from zero, so
     // that an infinite weight meets none; m takes the difference back)
-    const uint32_t top = (u & 0xFFFF0000u) | (2u * u - 1u < 0x00FFFFFFu ? 0x10000u : 0u);
-    h = x != x ? 0x7FC00000u : top;
-    float r = x - __uint_as_float(top);
-    r = r != r ? 0.0f : r * (1.0f / kPlaneM);
+    h = (u & 0xFFFF0000u) | (2u * u - 1u < 0x00FFFFFFu ? 0x10000u : 0u);
+    const float r = __builtin_fabsf(x) == INFINITY ? 0.0f : (x - __uint_as_float(h)) * (1.0f / kPlaneM);
     m = __float_as_uint(r) & 0xFFFF0000u;
     l = __float_as_uint((r - __uint_as_float(m)) * (1.0f / kPlaneL));
 }
