@@ -75,7 +75,7 @@ typedef struct se12_streams_out {
  * names the dot2 kernel's shape at any batch; without one, 5 rows and more
  * run the x-slab MFMA kernel on three BF16 planes of x, which together hold
  * every bit of it):
- *  - dot2 kernel (batch 1..4 per launch, FP32 x): 1..16 waves, `blocks` =
+ *  - dot2 kernel (batch 1..4 per launch; FP32 x at any batch): 1..16 waves, `blocks` =
  *    tile_rows * k_splits, k_splits cutting the K tiles into contiguous
  *    ranges;
  *  - x-slab MFMA kernel (BF16 x, 5..32 rows): a multiple of ceil(batch / 8)
@@ -274,8 +274,8 @@ int se12_gemv_rmsnorm(se12_handle* h, const void* x_dev, int32_t x_dtype, int32_
 /* se12_gemv with the sums of squares of the output's tile rows (no reference
  * counterpart; for the decoder's norms): y as se12_gemv, and
  * row_ss[b, t] = sum over the 16 rows n of tile row t of bf16(y[b, n])^2
- * (FP32 [batch, tile rows]), written by the blocks completing each tile row
- * (dot2 launches) or by a small kernel after the product (MFMA launches).
+ * (FP32 [batch, tile rows]), written by the block (dot2 launches) or the wave
+ * (MFMA launches) that completes each tile row.
  * Same stream, allocation and ordering rules as se12_gemv. */
 int se12_gemv_rowss(se12_handle* h, const void* x_dev, int32_t x_dtype, int32_t batch, float* y_dev,
                     float* row_ss_dev, const se12_launch* launch, void* stream);

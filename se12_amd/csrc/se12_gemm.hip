@@ -1,12 +1,13 @@
 // Batched fused SE12 decode + matrix product for gfx950: Y[b, n] =
-// sum_k W[n, k] X[b, k] for up to 32 BF16 batch rows in ONE pass over the
+// sum_k W[n, k] X[b, k] for up to 32 batch rows (BF16, or FP32) in ONE pass over the
 // weights (the dot2 kernel in se12_gemv.hip takes 4 rows per launch and so
 // re-reads W once per 4 rows). Same semantics as the reference kernel
 // lws/adapters/cuda/kernels/gemv_se12.cu:50-142 at batch B, which runs one
 // warp per (row, batch) element and reads W B times.
 //
 // Grid: block = R x KG wave64s: R consecutive tile rows (R = ceil(batch / 8), 4 in place of 3,
-// the fewest waves whose threads load an x slab in one go) times KG K groups;
+// the fewest waves whose threads load an x slab in one go; FP32 x 4, or 8 above
+// 16 rows) times KG K groups;
 // wave w owns tile row R * row_block + w % R and, of the split's K tiles, the
 // ones of K group w / R (every KG-th tile). blockIdx.y = K split s covering
 // the K tiles [s*TC/S, (s+1)*TC/S). A grouped launch serves up to 4 matrices

@@ -252,7 +252,7 @@ constexpr int kGemmXPieces = 4;
 // B = 32 26.2 with 4)
 // FP32 x: 4 rows share each conversion to planes (8 rows where 32 batch rows
 // need their threads): 3584x14336, 8 batch rows, 28.3 us with 4, 30.9 with 8,
-// 43 with 2; 2304x9216 18.4 / 21.8 / 25.0
+// 43 with 2; 2304x9216 18.4 / 21.8 / 25.0 (cold weights, planes not scaled)
 constexpr int gemm_min_waves(int batch, bool xf32 = false) {
     if (xf32) return batch > 16 ? 8 : 4;
     const int fewest = (batch * 32 + 64 * kGemmXPieces - 1) / (64 * kGemmXPieces);

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kRopeThreads) void prefill_rope_kernel(RopeArgs a) 
 // and takes every 4th tile of 32 keys; the four waves' sums meet once at the
 // end, through LDS. The keys of a tile are loaded in the order that leaves
 // the scores of a lane, as they come out of the first product, the B operand
-// of the second (key of A row m: kKeyOfRow), so probabilities never leave
+// of the second (key of A row m: key_of_row), so probabilities never leave
 // their lane.
 // Scores, capping and sums are FP32; a probability is rounded to BF16 for the
 // second product, and their sum is that of the rounded ones, so that the weights
@@ -182,9 +182,9 @@ __global__ __launch_bounds__(kRopeThreads) void prefill_rope_kernel(RopeArgs a) 
 // K and V^T operands come straight from L2, 1 KB of consecutive bytes per
 // instruction in the order prefill_rope_kernel left them; with K and V^T
 // row-major, 32 bytes of each of 32 rows per instruction, the first-level cache
-// kept missing: 1,024 positions, 8 heads of 256, 37.5 us against 19.2 (0.22
-// PFLOP/s of the causal half; a block per CU whose longest walks 32 tiles); the
-// framework ops took ~120 us for the same.
+// kept missing: 1,024 positions, 8 heads of 256, 37.5 us against 19.2, both
+// without the maximum, 20.3 with it (0.21 PFLOP/s of the causal half; a block per
+// CU whose longest walks 32 tiles); the framework ops took ~120 us for the same.
 constexpr int kPrefillThreads = 256;
 constexpr int kPrefillRows = 32;
 constexpr float kMaxSoftcap = 64.0f;
