@@ -587,15 +587,15 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(const int64_t* po
 }
 
 // ---------------------------------------------------------------------------
-// attention over many positions: launches of more score blocks than
-// kLongBlocks (sequences x KV heads x chunks), e.g. a batch over a long
-// cache. The blocks of the kernels above load their share of the cache before
-// they know the position, one round trip less on a cache nearly all in use,
-// but a launch of many blocks then reads the whole cache whatever part is in
-// use, rotates q once per 64 positions, and computes each probability once
-// per 8 columns. Here a block reads the position first (other blocks of the
-// CU hide that), and the positions in use, not the cache's length, are cut
-// among the grid's blocks:
+// attention over many positions: launches of kLongBlocks score blocks
+// (sequences x KV heads x chunks) or more, e.g. a batch over a long cache. The
+// blocks of the kernels above load their share of the cache before they know
+// the position, one round trip less on a cache nearly all in use, but a launch
+// of many blocks then reads the whole cache whatever part is in use, rotates q
+// once per 64 positions, and computes each probability once per 8 columns.
+// Here a block reads the position first (other blocks of the CU hide that),
+// and the positions in use, not the cache's length, are cut among the grid's
+// blocks:
 //   scores  a run of units of 64 to 256 positions per block (by head_dim,
 //           so that a unit is a few KB of keys per wave): q rotated once, the
 //           next batch of keys in flight while one is used, a wave for each
@@ -604,20 +604,34 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(const int64_t* po
 //           V rows per load, each probability computed once and shared
 //           through LDS; the runs' FP32 sums meet as the spans above do.
 // Bound by the cache's bytes in use. Two launches in a graph, cold cache, the
-// short kernels above against these: 8 sequences x 8 KV heads of 256 x 2
-// queries, cache of 8,192: position 8,190 145.6 -> 136 us (3.9 TB/s; the key
-// rows are 16 KB apart, and a cache of 8,064 takes 17 us less), 3,000 121 ->
-// 56 us, 300 114 -> 18.6, a window of 1,024 at 8,000 128 -> 32; 32 x 8 x 128,
-// 2,048 long at 700 68 -> 31; 32 x 8 x 64, 4,096 long at 4,000 80 -> 66. Units
-// of 128 / 256 at head_dim 256 took 60 / 62 us at position 3,000, 64 / 128 at
-// head_dim 64 79 / 69; 2,048 blocks instead of 1,024 3-7% more, nontemporal
-// loads 126 at 8,190 but 40 and 97 on the smaller caches. Below kLongBlocks the
-// short kernels stay: at 512-1,024 blocks these took 29 / 34 / 41 us against
-// 19 / 25 / 24 (4 x 4 x 2,048, 8 x 8 x 1,024, 1 x 4 x 8,192).
+// short kernels above against these, in us at a full cache / position 3,000 or
+// half / 300 / full with a window of an eighth:
+//   8 seq x 8 KV heads x 256 x 1 query, 8,192 long  136/116/111/123 -> 126/57/18/30
+//                            x 2                    152/123/114/129 -> 136/60/20/35
+//                            x 8                    413/218/139/179 -> 273/122/38/72
+//   32 x 8 x 128 x 2, 2,048 long                     86/ 75/ 68/ 72 ->  74/52/22/23
+//   32 x 8 x  64 x 2, 4,096 long                    102/ 87/ 70/ 79 ->  73/58/19/22
+//   1 x 1 x 256 x 8, 400,000 long                  1885/107/107/270 -> 490/41/36/168
+// (136 us is 3.9 TB/s; the key rows are 16 KB apart, and a cache of 8,064
+// takes 17 us less). Units of 128 / 256 at head_dim 256 took 60 / 62 us at
+// position 3,000, 64 / 128 at head_dim 64 79 / 69; nontemporal loads 126 at a
+// full cache but 40 and 97 on smaller ones.
+// The grid is what the CUs hold at once: 1,024 blocks whatever the number of
+// query heads took 298 us in the third line (2 blocks of 8 queries fit a CU)
+// and 760 in the last, where each block of a wide grid also left a span of 64
+// positions for one block to add up.
+// The line between the two kernels: a short cache that is full is the case
+// where reading the position first costs most. From kLongBlocks these kernels
+// take at most 1.03 times the short ones there (2 queries 8 x 8 x 256 x 4,096:
+// 81 -> 79 us, and 61 -> 20 at 300); on 1,152 blocks (9 x 8 x 256 x 1,024) 31
+// -> 35 us at 2 queries and 68 -> 91 at 8. One query head per KV head leaves
+// pv the least work per row, .91 to .98 of the short kernels' speed at 4,096
+// blocks and 1.0 at kLongBlocks1; rows shorter than kLongDim leave most of a
+// unit's lanes without elements (head_dim 8: .73 to .97).
 // ---------------------------------------------------------------------------
 
-constexpr int kLongBlocks = 1024;
-constexpr int kLongGrid = 1024;    // blocks aimed at, over all (sequence, KV head) pairs
+constexpr int kLongBlocks = 4000, kLongBlocks1 = 5000;   // the second with one query head per KV head
+constexpr int kLongDim = 32;
 constexpr int kUnitLoads = 8;      // 16-byte loads of one batch per thread, two batches in flight
 constexpr int kPvStep = 64;        // positions of one step of a pv block: 8 V rows per thread, two steps in flight
 
@@ -767,7 +781,10 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_long_kernel(AttnArgs a) 
     const int p = (int)p64, lo = window_lo(p, a.window);
     // span sp of the positions in use: whole steps, the same for every block
     const int len = p - lo + 1;
-    const int span = ((len + Y - 1) / Y + kPvStep - 1) / kPvStep * kPvStep;
+    // (kPvStep at least, more on a wide grid: one block adds up the spans' sums)
+    const int least = kPvStep * (Y > 128 ? Y / 128 : 1);
+    const int even = ((len + Y - 1) / Y + kPvStep - 1) / kPvStep * kPvStep;
+    const int span = even > least ? even : least;
     const int nspans = (len + span - 1) / span;
     if (sp >= nspans) return;
     const int j0 = lo + sp * span, j1 = j0 + span < p + 1 ? j0 + span : p + 1;
@@ -1135,10 +1152,13 @@ void launch_scores_long(const AttnArgs& a, dim3 grid, hipStream_t stream) {
 
 template <int G>
 void launch_attention(const AttnArgs& a, int blocks_x, hipStream_t stream) {
-    if ((int64_t)blocks_x * a.chunks > kLongBlocks) {
-        // a chunk, and a step of the pv kernel, is the least a block takes
-        const int y = std::max(1, std::min(a.chunks, kLongGrid / blocks_x));
-        const dim3 grid(blocks_x, y);
+    if (a.d >= kLongDim && (int64_t)blocks_x * a.chunks >= (G == 1 ? kLongBlocks1 : kLongBlocks)) {
+        // whole units, the same number per block, on as many blocks as the CUs
+        // hold at once
+        constexpr int kResident = 256 * (G <= 2 ? 4 : G == 4 ? 3 : 2);
+        const int64_t unit = a.d > 128 ? 64 : a.d > 64 ? 128 : 256, units = (a.max_len + unit - 1) / unit;
+        const int64_t most = std::max(1, kResident / blocks_x), per_block = (units + most - 1) / most;
+        const dim3 grid(blocks_x, (uint32_t)((units + per_block - 1) / per_block));
         // about 16 K key elements per unit
         if (a.d > 128)
             launch_scores_long<G, 64>(a, grid, stream);

@@ -310,9 +310,9 @@ def test_attention_step(gpu, batch, heads, kvh, d, L, pos, window, dtype):
     assert torch.equal(out, out2)
 
 
-# more than 1,024 (sequence, KV head, 64-position chunk) blocks, the kernels for long caches: positions at the edges of
-# units (64 / 128 / 256 at head_dim 256 / 128 / up to 64), of pv steps and spans, windows across them, head dims whose
-# value rows leave threads idle, every query-group size, a cache length off the unit
+# more than 1,024 (sequence, KV head, 64-position chunk) blocks, several per CU slot, of the kernels that load their
+# share of the cache before they know the position (the larger ones take the kernels for long caches): positions at the
+# edges of chunks and spans, windows across them, head dims whose value rows leave threads idle, every query-group size
 ATTN_LONG_CASES = [
     (32, 16, 8, 256, 320, 0, 0, torch.float32),
     (32, 16, 8, 256, 320, 63, 0, torch.bfloat16),
@@ -338,6 +338,56 @@ def test_attention_step_over_many_blocks(gpu, batch, heads, kvh, d, L, pos, wind
 
 def test_attention_over_many_blocks_position_outside_the_cache_touches_nothing(gpu):
     batch, heads, kvh, d, L = 64, 8, 4, 64, 384
+    q = torch.ones((batch, heads * d), device=gpu)
+    k = torch.ones((batch, kvh * d), device=gpu)
+    kt = torch.full((batch, kvh, d, L), 3.0, device=gpu).to(torch.bfloat16)
+    vc = torch.full((batch, kvh, L, d), 5.0, device=gpu).to(torch.bfloat16)
+    out = torch.full((batch, heads * d), 7.0, device=gpu).to(torch.bfloat16)
+    ws = _workspace(gpu, batch, heads, kvh, d, L)
+    for p in (L, -1):
+        _attention(q, k, k, torch.float32, heads * d, kvh * d, kt, vc, torch.ones(d // 2, device=gpu),
+                   torch.tensor(p, dtype=torch.int64, device=gpu), out, batch, heads, kvh, d, L, 1.0, 0.0, 0, ws)
+        torch.cuda.synchronize()
+        assert bool((out == 0).all()) and bool((kt == 3).all()) and bool((vc == 5).all())
+    assert bool((ws == 0).all())
+
+
+# the kernels for long caches, from 4,000 blocks (5,000 with one query head per KV head, head dims from 32): positions
+# at the edges of units (64 / 128 / 256 positions at head_dim 256 / 128 / up to 64), of pv steps and spans, windows
+# across them, a cache length off the unit, value rows that leave threads idle, every query-group size, grids of one
+# block up to several hundred per KV head, where a span has a least length
+ATTN_LONGEST_CASES = [
+    (50, 16, 8, 256, 640, 0, 0, torch.float32),           # exactly 4,000
+    (50, 16, 8, 256, 640, 63, 0, torch.bfloat16),
+    (50, 16, 8, 256, 640, 64, 0, torch.float32),
+    (63, 16, 8, 256, 520, 519, 100, torch.float32),
+    (63, 16, 8, 256, 520, 384, 65, torch.bfloat16),
+    (8, 16, 8, 256, 4096, 4095, 0, torch.float32),
+    (16, 16, 4, 128, 4104, 4103, 0, torch.float32),
+    (16, 16, 4, 128, 4104, 384, 129, torch.bfloat16),
+    (16, 8, 4, 96, 4104, 2000, 0, torch.float32),
+    (4, 16, 2, 256, 32768, 32767, 0, torch.float32),
+    (4, 16, 2, 256, 32768, 511, 0, torch.bfloat16),
+    (64, 64, 8, 64, 512, 255, 0, torch.float32),
+    (64, 64, 8, 64, 512, 256, 0, torch.float32),
+    (40, 8, 8, 40, 1000, 777, 500, torch.float32),
+    (40, 8, 8, 32, 1000, 999, 0, torch.bfloat16),
+    (1, 1, 1, 64, 320064, 320063, 0, torch.float32),
+    (1, 1, 1, 64, 320064, 100000, 70001, torch.float32),
+    (1, 8, 1, 256, 262144, 262143, 0, torch.float32),
+    (1, 8, 1, 256, 262144, 30000, 4096, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("batch,heads,kvh,d,L,pos,window,dtype", ATTN_LONGEST_CASES)
+def test_attention_step_over_long_caches(gpu, batch, heads, kvh, d, L, pos, window, dtype):
+    assert d >= 32 and batch * kvh * -(-L // 64) >= (4000 if heads > kvh else 5000)
+    test_attention_step(gpu, batch, heads, kvh, d, L, pos, window, dtype)
+
+
+@pytest.mark.parametrize("heads", [4, 8])
+def test_attention_over_long_caches_position_outside_the_cache_touches_nothing(gpu, heads):
+    batch, kvh, d, L = 64, 4, 64, 1280
     q = torch.ones((batch, heads * d), device=gpu)
     k = torch.ones((batch, kvh * d), device=gpu)
     kt = torch.full((batch, kvh, d, L), 3.0, device=gpu).to(torch.bfloat16)
