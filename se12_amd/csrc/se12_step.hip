@@ -940,7 +940,7 @@ __device__ __forceinline__ void load8_as_bf16(const void* p, int64_t i, float* v
 }
 
 // Rows of whole 8-column pieces (cols and stride multiples of 8, 16-byte
-// aligned tensors) on more values than a wave per CU holds: a piece per
+// aligned tensors) on a launch of kGelu8Min values and more: a piece per
 // thread, the row from the grid. Bound by the bytes and the tanh: 1,024 x 9,216
 // BF16 18.7 -> 11.4 us (5 TB/s) against an element per thread.
 template <int DT>
@@ -1114,8 +1114,14 @@ bool dtype_ok(int32_t d) { return d == SE12_STEP_F32 || d == SE12_STEP_BF16; }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
-// values from which gelu_mul8_kernel fills the CUs (256 x 4 waves x 64 lanes x 8)
-constexpr int64_t kGelu8Min = 524288;
+// gelu_mul8_kernel's line: two waves per SIMD of 8 values per lane, so that one
+// loads while the other computes (a value per thread gives 8 times the waves),
+// in rows that fill a wave of pieces. FP32 / BF16, a value per thread -> 8:
+// 114 x 9,216 3.55 / 3.63 -> 3.43 / 3.34 us, but 57 x 9,216 2.70 / 2.67 -> 2.97
+// / 2.80; 3,000 x 512 4.62 / 4.50 -> 4.20 / 4.09, but 4,000 x 384 4.59 / 4.51
+// -> 4.74 / 4.57.
+constexpr int64_t kGelu8Min = 1048576;
+constexpr int32_t kGelu8Cols = 512;
 
 int64_t up256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
@@ -1303,8 +1309,8 @@ int se12_step_gelu_mul(const void* gate, const void* up, int32_t dtype, int64_t 
     const int64_t n = (int64_t)rows * cols;
     const dim3 grid((unsigned)((n + 255) / 256));
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    if (n >= kGelu8Min && rows <= 65535 && cols % 8 == 0 && stride % 8 == 0 && aligned16(gate) && aligned16(up) &&
-        aligned16(out)) {
+    if (n >= kGelu8Min && cols >= kGelu8Cols && rows <= 65535 && cols % 8 == 0 && stride % 8 == 0 &&
+        aligned16(gate) && aligned16(up) && aligned16(out)) {
         const dim3 grid8((unsigned)((cols / 8 + 255) / 256), rows);
         if (dtype == SE12_STEP_F32)
             hipLaunchKernelGGL(gelu_mul8_kernel<SE12_STEP_F32>, grid8, dim3(256), 0, st, gate, up, stride, out, cols);

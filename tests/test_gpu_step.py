@@ -95,7 +95,7 @@ def test_gelu_mul(gpu, dtype):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows,cols", [(57, 9216), (65, 8072), (600, 1000)])
 def test_gelu_mul_in_pieces_equals_element_by_element(gpu, rows, cols, dtype):
-    """Launches of 524,288 values and more take 8 per thread where they are aligned: the same bits as an output that is not."""
+    """Large launches take 8 values per thread where they are aligned: the same bits as an output that is not."""
     assert rows * cols >= 524288
     g = _gen(gpu, rows)
     gu = (torch.randn((rows, 2 * cols), generator=g, device=gpu) * 2).to(dtype)
@@ -108,6 +108,13 @@ def test_gelu_mul_in_pieces_equals_element_by_element(gpu, rows, cols, dtype):
                                                     nat.stream_ptr()))
     assert torch.equal(out, odd)
     _ulp_close(out, F.gelu(gate.to(torch.bfloat16), approximate="tanh") * up.to(torch.bfloat16))
+
+
+# either side of 1,048,576 values and of 512 columns, the line from which 8 values per thread are taken
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,cols", [(2048, 512), (2047, 512), (2081, 504), (128, 8192), (129, 8184), (1, 1048576)])
+def test_gelu_mul_either_side_of_the_line_for_pieces(gpu, rows, cols, dtype):
+    test_gelu_mul_in_pieces_equals_element_by_element(gpu, rows, cols, dtype)
 
 
 # (batch, tokens, heads, kv heads, head dim, cache length, window): tokens at the edges of the 32-query blocks, 32-key tiles
