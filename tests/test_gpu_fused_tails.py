@@ -364,6 +364,8 @@ def test_rowss_sums_the_tile_rows_of_the_output(gpu, fmt, rows, cols, batch, dty
     (2304, 2048, 17, torch.bfloat16),   # two batch groups, the second of one row
     (2304, 9216, 8, torch.bfloat16),    # K splits, added by the last arrival
     (2304, 9216, 32, torch.bfloat16),   # x slabs
+    (1000, 4096, 27, torch.bfloat16),   # resident x, the second batch group's from global memory
+    (4608, 4096, 20, torch.bfloat16),   # two batch groups in K splits
     (300, 512, 7, torch.bfloat16),      # a last tile row of 12 rows
     (17, 300, 32, torch.bfloat16),      # of one row; a partial last tile
     (2304, 9216, 6, torch.float32),     # FP32 x: planes
